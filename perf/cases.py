@@ -157,6 +157,63 @@ def run(state):
     return packed, quadmul_amd.unpack_int4(packed)
 
 
+def _nibbles(packed):
+    """Bytes of int4 pairs -> their values in float64, even k from the low nibble."""
+    u = packed.view(torch.uint8).to(torch.int16)
+    both = torch.stack((u & 15, u >> 4), dim=-1).reshape(u.shape[0], -1)
+    return torch.where(both > 7, both - 16, both).double()
+
+
+def _bytes(values):
+    v = values.to(torch.int16) & 15
+    return (v[:, 0::2] | (v[:, 1::2] << 4)).to(torch.uint8).view(torch.int8)
+
+
+def _rows_to_int4(x):
+    """The rule of the quantisation: amax / 7 per row, the multiplication with its inverse in 32 bits where x has no more
+    (so the integers are the rule's own, ties too), round to even.  Integers and scales in float64."""
+    wide = x if x.dtype == torch.float64 else x.float()
+    amax = wide.abs().amax(dim=1, keepdim=True)
+    inv = torch.where(amax > 0, 7.0 / amax, torch.zeros_like(amax))
+    return torch.round(wide * inv).clamp(-7, 7).double(), amax.double() / 7.0
+
+
+def _linear64(x, weight, bias=None):
+    (xq, xs), (wq, ws) = _rows_to_int4(x), _rows_to_int4(weight)
+    y = (xq @ wq.T) * xs * ws.T
+    return y if bias is None else y + bias.double()
+
+
+def exact(case, seed):
+    """What ``run`` returns, in 64 bits from the same inputs, with plain torch."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(seed)
+    kind, m, k = case["kind"], case["m"], case["k"]
+    if kind == "gemm":
+        weights = [_packed(gen, case["n"], k) for _ in range(case["calls"])]
+        a = _nibbles(_packed(gen, m, k))
+        return [a @ _nibbles(b).T for b in weights]  # below 2^53: the integers themselves
+    if kind == "pack":
+        values = torch.randint(-8, 8, (m, k), dtype=torch.int8, device="cuda", generator=gen)
+        return _bytes(values), values
+    dtype = DTYPES[case["dtype"]]
+    x = _activations(gen, m, k, dtype)
+    if kind == "quantize":
+        q, scales = _rows_to_int4(x)
+        return _bytes(q), scales[:, 0]
+
+    def drawn(n, k, bias):  # as _layer draws them
+        weight = torch.randn(n, k, device="cuda", generator=gen) * (1.0 / math.sqrt(k))
+        b = torch.randn(n, device="cuda", generator=gen) * 0.1 if bias else None
+        return weight.to(dtype), b if b is None else b.to(dtype)
+
+    if kind == "linear":
+        return _linear64(x, *drawn(case["n"], k, case["bias"]))
+    wide, down = drawn(2 * case["n"], k, False)[0], drawn(k, case["n"], False)[0]
+    gate, up = _linear64(x, wide).chunk(2, dim=-1)
+    return _linear64(torch.nn.functional.silu(gate) * up, down)
+
+
 def work(case):
     kind, m, k = case["kind"], case["m"], case["k"]
     if kind == "gemm":
