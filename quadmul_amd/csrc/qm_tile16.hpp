@@ -537,7 +537,8 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
     // instruction just before this statement -- v_readlane, when it keeps scalar registers in
     // the lanes of a vector one -- and a memory instruction must not read such a register
     // within five wait states; the compiler sees to that for its own instructions and cannot
-    // for the store in here.)
+    // for the store in here.  scc: s_and_b64 writes it, and it carries the low half of a 64-bit
+    // address into the high half when the compiler places the statement between the two.)
     auto store_lanes = [&](char *const base, const uint32_t lane_off, const auto v, auto row_, auto col_) __attribute__((always_inline)) {
         constexpr int row = decltype(row_)::value, col = decltype(col_)::value;
         const int rl = rows_left, cl = cols_left;   // (an asm operand cannot name a captured variable)
@@ -545,11 +546,11 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
         if constexpr (sizeof(v) == 16)
             asm volatile("s_nop 4\n\tv_cmp_lt_i32_e32 vcc, %7, %5\n\ts_mov_b64 %1, vcc\n\tv_cmp_lt_i32_e32 vcc, %8, %6\n\ts_and_b64 %1, %1, vcc\n\t"
                          "s_mov_b64 %0, exec\n\ts_mov_b64 exec, %1\n\tglobal_store_dwordx4 %2, %3, %4\n\ts_mov_b64 exec, %0"
-                         : "=&s"(saved), "=&s"(on) : "v"(lane_off), "v"(v), "s"(base), "v"(rl), "v"(cl), "n"(row), "n"(col) : "memory", "vcc");
+                         : "=&s"(saved), "=&s"(on) : "v"(lane_off), "v"(v), "s"(base), "v"(rl), "v"(cl), "n"(row), "n"(col) : "memory", "vcc", "scc");
         else
             asm volatile("s_nop 4\n\tv_cmp_lt_i32_e32 vcc, %7, %5\n\ts_mov_b64 %1, vcc\n\tv_cmp_lt_i32_e32 vcc, %8, %6\n\ts_and_b64 %1, %1, vcc\n\t"
                          "s_mov_b64 %0, exec\n\ts_mov_b64 exec, %1\n\tglobal_store_dwordx2 %2, %3, %4\n\ts_mov_b64 exec, %0"
-                         : "=&s"(saved), "=&s"(on) : "v"(lane_off), "v"(v), "s"(base), "v"(rl), "v"(cl), "n"(row), "n"(col) : "memory", "vcc");
+                         : "=&s"(saved), "=&s"(on) : "v"(lane_off), "v"(v), "s"(base), "v"(rl), "v"(cl), "n"(row), "n"(col) : "memory", "vcc", "scc");
     };
     // Whole tile, through the LDS: part t = 0..7 of blocks (ib, 4*grp .. 4*grp+3), one part per
     // MFMA slot.  Parts 0..3 write one block each; the read-back of row quartet k and its
