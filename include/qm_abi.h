@@ -134,6 +134,12 @@ int qm_gemm_i4_ws(const void *A, const void *B, void *C, int m, int n, int k, vo
 int qm_gemm_i4_scaled_ws(const void *A, const void *B, void *D, int m, int n, int k, const float *row_scale,
                          const float *col_scale, int out_dtype, void *stream, int cfg, void *workspace,
                          size_t workspace_bytes);
+/* The scaled form with a bias: D[m][n] = round16(D[m][n] as above + bias[n]), bias [N] in D's
+ * 16-bit type (2-byte aligned device pointer, or NULL for none) -- two roundings, the values a
+ * separate in-place addition to D gives, without its pass over D. */
+int qm_gemm_i4_scaled_bias_ws(const void *A, const void *B, void *D, int m, int n, int k, const float *row_scale,
+                              const float *col_scale, const void *bias, int out_dtype, void *stream, int cfg,
+                              void *workspace, size_t workspace_bytes);
 size_t qm_gemm_workspace_bytes(int m, int n, int k, int ptr_align, int cfg, int scaled);
 
 /*

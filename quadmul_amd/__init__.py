@@ -35,7 +35,7 @@ CFG_AUTO = -1
 #: every symbol include/qm_abi.h declares
 ABI_SYMBOLS = (
     "qm_gemm_i4", "qm_gemm_i4_cfg", "qm_gemm_i4_scaled", "qm_gemm_i4_scaled_cfg", "qm_config_has_scaled",
-    "qm_gemm_i4_ws", "qm_gemm_i4_static", "qm_gemm_i4_scaled_ws", "qm_gemm_workspace_bytes", "qm_quantize_pack_i4", "qm_select_config", "qm_select_config_ex", "qm_num_configs", "qm_config_name",
+    "qm_gemm_i4_ws", "qm_gemm_i4_static", "qm_gemm_i4_scaled_ws", "qm_gemm_i4_scaled_bias_ws", "qm_gemm_workspace_bytes", "qm_quantize_pack_i4", "qm_select_config", "qm_select_config_ex", "qm_num_configs", "qm_config_name",
     "qm_config_supports", "qm_pack_i4", "qm_unpack_i4", "qm_status_string", "qm_last_hip_error", "qm_version", "qm_init",
     "qm_debug_set_operand_limit",
 )
@@ -74,6 +74,8 @@ def library() -> ctypes.CDLL:
     lib.qm_gemm_i4_static.restype = ci
     lib.qm_gemm_i4_scaled_ws.argtypes = [vp, vp, vp, ci, ci, ci, vp, vp, ci, vp, ci, vp, ctypes.c_size_t]
     lib.qm_gemm_i4_scaled_ws.restype = ci
+    lib.qm_gemm_i4_scaled_bias_ws.argtypes = [vp, vp, vp, ci, ci, ci, vp, vp, vp, ci, vp, ci, vp, ctypes.c_size_t]
+    lib.qm_gemm_i4_scaled_bias_ws.restype = ci
     lib.qm_gemm_workspace_bytes.argtypes = [ci, ci, ci, ci, ci, ci]
     lib.qm_gemm_workspace_bytes.restype = ctypes.c_size_t
     lib.qm_config_has_scaled.argtypes = [ci]
@@ -189,25 +191,29 @@ def gemm_cfg(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, m: int, n: int, 
 
 def gemm_scaled(a: torch.Tensor, b: torch.Tensor, d: torch.Tensor, m: int, n: int, k: int,
                 row_scale: Optional[torch.Tensor] = None, col_scale: Optional[torch.Tensor] = None, cfg: int = CFG_AUTO,
-                workspace=True) -> None:
+                workspace=True, bias: Optional[torch.Tensor] = None) -> None:
     """The GEMM with the dequantising epilogue fused in (no counterpart in the reference's
     code; README.md:7 names the idea): ``d[m,n] = round(((float)c[m,n] * row_scale[m]) *
     col_scale[n])`` with ``c`` the exact int32 product; ``d`` is float16 or bfloat16 and is
-    overwritten; the scales are float32 vectors on the same device, None = all ones.
-    ``workspace``: see :func:`gemm`."""
+    overwritten; the scales are float32 vectors on the same device, None = all ones.  ``bias``
+    (``[n]``, ``d``'s type): added to the rounded value and rounded again, what ``d += bias``
+    after the call gives.  ``workspace``: see :func:`gemm`."""
     _check_operands(a, b, d, m, n, k, c_dtypes=(torch.float16, torch.bfloat16))
     for s_, cnt, what in ((row_scale, m, "row_scale"), (col_scale, n, "col_scale")):
         if s_ is None:
             continue
         if not (s_.is_cuda and s_.device == a.device and s_.dtype == torch.float32 and s_.is_contiguous() and s_.numel() == cnt):
             raise QuadmulError(f"gemm_scaled: {what} must be a contiguous float32 vector of {cnt} elements on a's device")
+    if bias is not None and not (bias.is_cuda and bias.device == a.device and bias.dtype == d.dtype and bias.is_contiguous() and bias.numel() == n):
+        raise QuadmulError(f"gemm_scaled: bias must be a contiguous {d.dtype} vector of {n} elements on a's device")
     out = 1 if d.dtype == torch.float16 else 2
     ws, ws_bytes, _keep = _workspace(workspace, a, b, m, n, k, cfg, True)
     with torch.cuda.device(a.device):
-        st = library().qm_gemm_i4_scaled_ws(a.data_ptr(), b.data_ptr(), d.data_ptr(), m, n, k,
-                                            None if row_scale is None else row_scale.data_ptr(),
-                                            None if col_scale is None else col_scale.data_ptr(), out, _stream_ptr(a), cfg,
-                                            ws, ws_bytes)
+        st = library().qm_gemm_i4_scaled_bias_ws(a.data_ptr(), b.data_ptr(), d.data_ptr(), m, n, k,
+                                                 None if row_scale is None else row_scale.data_ptr(),
+                                                 None if col_scale is None else col_scale.data_ptr(),
+                                                 None if bias is None else bias.data_ptr(), out, _stream_ptr(a), cfg,
+                                                 ws, ws_bytes)
     _check(st, "qm_gemm_i4_scaled_ws")
 
 

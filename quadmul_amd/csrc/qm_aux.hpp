@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(256) gemm_generic_kernel(const GemmArgs p, con
     if (m < p.M && n < p.N) {
         const size_t at = (size_t)m * c_stride(p) + n;
         if (p.out == OUT_I32) p.C[at] = sum;
-        else reinterpret_cast<uint16_t *>(p.C)[at] = round16(scaled(sum, scale_at(p.row_scale, m, p.M), scale_at(p.col_scale, n, p.N)), p.out);
+        else reinterpret_cast<uint16_t *>(p.C)[at] = finish16(p, sum, scale_at(p.row_scale, m, p.M), n);
     }
 }
 
@@ -65,6 +65,13 @@ static hipError_t launch_generic(const GemmArgs &p, hipStream_t stream, int)
 __global__ void fill_zero16_kernel(uint16_t *dst, size_t n)
 {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) dst[i] = 0;
+}
+
+// k == 0 with a bias: zero plus the bias (which turns a bias of -0 into +0)
+__global__ void fill_bias16_kernel(uint16_t *dst, const uint16_t *bias, int ncols, int ldc, size_t n, int out)
+{
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+        dst[i / ncols * ldc + i % ncols] = add16(0, bias[i % ncols], out);
 }
 
 __global__ void fill_zero_kernel(int32_t *dst, size_t n)
@@ -132,6 +139,7 @@ struct SplitReduceArgs {
     int tiles_m, tiles_n, group_m, ksplit;
     int BM, BN, WGN, FM, FN, waves;
     const float *row_scale, *col_scale;
+    const uint16_t *bias;
     int out;
 };
 
@@ -184,11 +192,16 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitReduceArg
     } else {
         uint16_t *drow = static_cast<uint16_t *>(q.C) + (size_t)m * q.N;
         const float rs = scale_at(q.row_scale, m, q.M);
+        GemmArgs f{};
+        f.N = q.N;
+        f.col_scale = q.col_scale;
+        f.bias = q.bias;
+        f.out = q.out;
         uint16_t h[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int c = sum[e];
-            h[e] = round16(scaled(c, rs, scale_at(q.col_scale, n + e, q.N)), q.out);
+            h[e] = finish16(f, c, rs, n + e);
         }
         if ((q.N & 3) == 0 && ((uintptr_t)q.C & 7) == 0) {
             *reinterpret_cast<v2i *>(drow + n) = v2i{(int)(h[0] | ((uint32_t)h[1] << 16)), (int)(h[2] | ((uint32_t)h[3] << 16))};

@@ -28,6 +28,9 @@ struct GemmArgs {
     // a null pointer standing for all ones
     const float *row_scale = nullptr;  // [M]
     const float *col_scale = nullptr;  // [N]
+    // scaled output only: added per column to the rounded value, in the output's type, and rounded
+    // again (what a separate in-place addition of a bias to D gives); null: nothing is added
+    const uint16_t *bias = nullptr;  // [N]
     int out = OUT_I32;
     // K split over several work items per tile (pipelined kernel): where the partial sums go.
     // Null: they meet in C by atomic adds (C zero-filled beforehand).  Otherwise item i of the
@@ -66,12 +69,61 @@ __device__ __forceinline__ uint16_t round16(float x)
 }
 __device__ __forceinline__ uint16_t round16(float x, int out) { return out == OUT_F16 ? round16<OUT_F16>(x) : round16<OUT_BF16>(x); }
 
+// The sum of two 16-bit floats, rounded to nearest even: two bf16 (or fp16) values add up in
+// fp32 with enough digits to spare that rounding the fp32 sum is rounding the exact one.
+__device__ __forceinline__ uint16_t add16(uint16_t h, uint16_t b, int out)
+{
+    if (out == OUT_F16) return __builtin_bit_cast(uint16_t, (_Float16)(__builtin_bit_cast(_Float16, h) + __builtin_bit_cast(_Float16, b)));
+    return round16<OUT_BF16>(__builtin_bit_cast(float, (uint32_t)h << 16) + __builtin_bit_cast(float, (uint32_t)b << 16));
+}
+
 // the scaled value of one element, in the one order of operations everything here uses
 __device__ __forceinline__ float scaled(int c, float rs, float cs)
 {
 #pragma clang fp contract(off)
     const float t = (float)c * rs;
     return t * cs;
+}
+
+// Two values at once, the first in the low half.  bf16: one v_cvt_pk_bf16_f32, which gives what
+// round16 gives for every one of the 2^32 inputs (checked on the device), NaNs included.
+template <int OUT>
+__device__ __forceinline__ uint32_t round16_pair(float x, float y)
+{
+    if constexpr (OUT == OUT_BF16) {
+        typedef float f2 __attribute__((ext_vector_type(2)));
+        typedef __bf16 h2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{x, y}), h2));
+    } else {
+        return (uint32_t)round16<OUT_F16>(x) | ((uint32_t)round16<OUT_F16>(y) << 16);
+    }
+}
+template <int OUT>
+__device__ __forceinline__ uint32_t add16_pair(uint32_t h, uint32_t b)
+{
+    if constexpr (OUT == OUT_BF16) {
+        return round16_pair<OUT_BF16>(__builtin_bit_cast(float, h << 16) + __builtin_bit_cast(float, b << 16),
+                                      __builtin_bit_cast(float, h & 0xFFFF0000u) + __builtin_bit_cast(float, b & 0xFFFF0000u));
+    } else {
+        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, (h2)(__builtin_bit_cast(h2, h) + __builtin_bit_cast(h2, b)));
+    }
+}
+// The bias of columns n .. n+3 as two packed pairs; -0 (which adds nothing to any value, to a
+// zero of either sign included) past the last column and without a bias.
+__device__ __forceinline__ v2i bias4_at(const GemmArgs &p, int n)
+{
+    uint32_t b[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b[e] = (p.bias != nullptr && n + e < p.N) ? p.bias[n + e] : 0x8000u;
+    return v2i{(int)(b[0] | (b[1] << 16)), (int)(b[2] | (b[3] << 16))};
+}
+
+// the element (.., n) of a 16-bit output: scaled, rounded, the bias (if any) added
+__device__ __forceinline__ uint16_t finish16(const GemmArgs &p, int c, float rs, int n)
+{
+    const uint16_t h = round16(scaled(c, rs, scale_at(p.col_scale, n, p.N)), p.out);
+    return p.bias != nullptr && n < p.N ? add16(h, p.bias[n], p.out) : h;
 }
 
 // gfx950 has no int4 MFMA, so nibbles are widened to int8 -- but scaled by 16,

@@ -46,7 +46,7 @@ static hipError_t launch_dot(const GemmArgs &p, hipStream_t stream, int opt)
 {
     if (opt & QM_OPT_PREPARE) return hipSuccess;
     const int blocks = (p.N + Cfg::BN - 1) / Cfg::BN;
-    gemm_dot_kernel<Cfg><<<dim3(blocks), dim3(Cfg::THREADS), 0, stream>>>(p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out, p.row_scale, p.col_scale);
+    gemm_dot_kernel<Cfg><<<dim3(blocks), dim3(Cfg::THREADS), 0, stream>>>(p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out, p.row_scale, p.col_scale, p.bias);
     return hipGetLastError();
 }
 #define QM_DOT(MR, FN, NW, U) \
@@ -60,7 +60,7 @@ static hipError_t launch_skinny_dma(const GemmArgs &p, hipStream_t stream, int o
     if (opt & QM_OPT_PREPARE) return hipSuccess;
     const int blocks = (p.N + Cfg::BN - 1) / Cfg::BN, row_blocks = (p.M + Cfg::MAX_M - 1) / Cfg::MAX_M;
     if (row_blocks > 65535) return hipErrorInvalidValue;
-    gemm_skinny_dma_kernel<Cfg><<<dim3(blocks, row_blocks), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out, p.row_scale, p.col_scale);
+    gemm_skinny_dma_kernel<Cfg><<<dim3(blocks, row_blocks), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out, p.row_scale, p.col_scale, p.bias);
     return hipGetLastError();
 }
 // Compute units of the current device (asked once per device).
@@ -95,7 +95,7 @@ static hipError_t launch_skinny_stream_dma(const GemmArgs &p, hipStream_t stream
     const int resident = cus * (160 * 1024 / Cfg::LDS_BYTES);  // workgroups the device holds at once (the LDS decides)
     const int grid = blocks < resident ? blocks : resident;
     gemm_skinny_stream_dma_kernel<Cfg><<<dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(
-        p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out | (grid << 8), blocks, p.row_scale, p.col_scale);
+        p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out | (grid << 8), blocks, p.row_scale, p.col_scale, p.bias);
     return hipGetLastError();
 }
 #define QM_SKINNYP(FM, FN, NW, D, R) \
@@ -236,9 +236,11 @@ static hipError_t launch_split_with_workspace(GemmArgs p, const Choice &ch, void
     q.waves = d.waves;
     q.row_scale = p.row_scale;
     q.col_scale = p.col_scale;
+    q.bias = p.bias;
     q.out = p.out;
     p.out = OUT_I32;
     p.row_scale = p.col_scale = nullptr;
+    p.bias = nullptr;
     p.ws = static_cast<int32_t *>(ws);
     hipError_t e = d.launch(p, s, ch.group_m | (ch.ksplit << 8) | (ch.spread << 16));
     if (e != hipSuccess) return e;
@@ -285,14 +287,16 @@ static int col_block_for_large_b(int m, int n, int k, int ptr_align)
 // place: a K split whose partial sums have no workspace to meet in falls back to atomic adds
 // into a zero-filled C for int32, and is not taken at all for a rounded output.
 static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k, const float *row_scale,
-                    const float *col_scale, int out, hipStream_t s, int cfg, void *workspace, size_t workspace_bytes, int ldc = 0)
+                    const float *col_scale, int out, hipStream_t s, int cfg, void *workspace, size_t workspace_bytes, int ldc = 0,
+                    const uint16_t *bias = nullptr)
 {
     const bool scaled = out != OUT_I32;
     const size_t cnt = (size_t)m * (size_t)n;
     const int row_stride = ldc != 0 ? ldc : n;   // of the output, in elements
     const bool strided = row_stride != n;        // a block of columns of a wider output
     if (k == 0) {
-        if (scaled) fill_zero16_kernel<<<dim3(flat_grid(cnt, 256)), dim3(256), 0, s>>>(static_cast<uint16_t *>(dst), cnt);
+        if (scaled && bias) fill_bias16_kernel<<<dim3(flat_grid(cnt, 256)), dim3(256), 0, s>>>(static_cast<uint16_t *>(dst), bias, n, row_stride, cnt, out);
+        else if (scaled) fill_zero16_kernel<<<dim3(flat_grid(cnt, 256)), dim3(256), 0, s>>>(static_cast<uint16_t *>(dst), cnt);
         else fill_zero_kernel<<<dim3(flat_grid(cnt, 256)), dim3(256), 0, s>>>(static_cast<int32_t *>(dst), cnt);
         const hipError_t e = hipGetLastError();
         return e == hipSuccess ? QM_OK : fail_launch(e);
@@ -302,7 +306,7 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
         for (int r0 = 0; r0 < m; r0 += rb) {
             const int st = run_gemm(static_cast<const uint8_t *>(A) + (size_t)r0 * (size_t)(k / 2), B,
                                     static_cast<uint8_t *>(dst) + (size_t)r0 * (size_t)row_stride * (scaled ? 2 : 4), m - r0 < rb ? m - r0 : rb,
-                                    n, k, row_scale ? row_scale + r0 : nullptr, col_scale, out, s, cfg, workspace, workspace_bytes, ldc);
+                                    n, k, row_scale ? row_scale + r0 : nullptr, col_scale, out, s, cfg, workspace, workspace_bytes, ldc, bias);
             if (st != QM_OK) return st;
         }
         return QM_OK;
@@ -311,7 +315,8 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
         for (int c0 = 0; c0 < n; c0 += cb) {
             const int st = run_gemm(A, static_cast<const uint8_t *>(B) + (size_t)c0 * (size_t)(k / 2),
                                     static_cast<uint8_t *>(dst) + (size_t)c0 * (scaled ? 2 : 4), m, n - c0 < cb ? n - c0 : cb, k, row_scale,
-                                    col_scale ? col_scale + c0 : nullptr, out, s, cfg, workspace, workspace_bytes, row_stride);
+                                    col_scale ? col_scale + c0 : nullptr, out, s, cfg, workspace, workspace_bytes, row_stride,
+                                    bias ? bias + c0 : nullptr);
             if (st != QM_OK) return st;
         }
         return QM_OK;
@@ -320,6 +325,7 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
     GemmArgs p{static_cast<const uint8_t *>(A), static_cast<const uint8_t *>(B), static_cast<int32_t *>(dst), m, n, k};
     p.row_scale = row_scale;
     p.col_scale = col_scale;
+    p.bias = bias;
     p.out = out;
     p.ldc = strided ? row_stride : 0;
     if (strided && cfg != QM_CFG_AUTO) return QM_ERR_CONFIG;
@@ -434,18 +440,25 @@ QM_EXPORT int qm_gemm_i4_cfg(const void *A, const void *B, void *C, int m, int n
     return qm_gemm_i4_ws(A, B, C, m, n, k, stream, cfg, nullptr, 0);
 }
 
-QM_EXPORT int qm_gemm_i4_scaled_ws(const void *A, const void *B, void *D, int m, int n, int k, const float *row_scale,
-                                   const float *col_scale, int out_dtype, void *stream, int cfg, void *workspace,
-                                   size_t workspace_bytes)
+QM_EXPORT int qm_gemm_i4_scaled_bias_ws(const void *A, const void *B, void *D, int m, int n, int k, const float *row_scale,
+                                        const float *col_scale, const void *bias, int out_dtype, void *stream, int cfg,
+                                        void *workspace, size_t workspace_bytes)
 {
     if (out_dtype != QM_OUT_F16 && out_dtype != QM_OUT_BF16) return QM_ERR_DTYPE;
     if (m < 0 || n < 0 || k < 0 || (k & 1)) return QM_ERR_SHAPE;
     if (m == 0 || n == 0) return QM_OK;
     if (!D) return QM_ERR_NULL;
-    if ((uintptr_t)D & 1) return QM_ERR_ALIGN;
+    if (((uintptr_t)D & 1) || ((uintptr_t)bias & 1)) return QM_ERR_ALIGN;
     if (k > 0 && (!A || !B)) return QM_ERR_NULL;
     return run_gemm(A, B, D, m, n, k, row_scale, col_scale, out_dtype == QM_OUT_F16 ? OUT_F16 : OUT_BF16,
-                    reinterpret_cast<hipStream_t>(stream), cfg, workspace, workspace_bytes);
+                    reinterpret_cast<hipStream_t>(stream), cfg, workspace, workspace_bytes, 0, static_cast<const uint16_t *>(bias));
+}
+
+QM_EXPORT int qm_gemm_i4_scaled_ws(const void *A, const void *B, void *D, int m, int n, int k, const float *row_scale,
+                                   const float *col_scale, int out_dtype, void *stream, int cfg, void *workspace,
+                                   size_t workspace_bytes)
+{
+    return qm_gemm_i4_scaled_bias_ws(A, B, D, m, n, k, row_scale, col_scale, nullptr, out_dtype, stream, cfg, workspace, workspace_bytes);
 }
 
 QM_EXPORT int qm_gemm_i4_scaled_cfg(const void *A, const void *B, void *D, int m, int n, int k, const float *row_scale,

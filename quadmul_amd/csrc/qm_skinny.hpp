@@ -188,7 +188,7 @@ gemm_skinny_kernel(const GemmArgs p)
         if (m < p.M && n < p.N) {
             const size_t at = (size_t)m * c_stride(p) + n;
             if (p.out == OUT_I32) p.C[at] = s >> 8;
-            else reinterpret_cast<uint16_t *>(p.C)[at] = round16(scaled(s >> 8, scale_at(p.row_scale, m, p.M), scale_at(p.col_scale, n, p.N)), p.out);
+            else reinterpret_cast<uint16_t *>(p.C)[at] = finish16(p, s >> 8, scale_at(p.row_scale, m, p.M), n);
         }
     }
 }
@@ -308,7 +308,7 @@ gemm_skinny_stream_kernel(const GemmArgs p, const int nblocks)
             if (m < p.M && n < p.N) {
                 const size_t at = (size_t)m * c_stride(p) + n;
                 if (p.out == OUT_I32) p.C[at] = s >> 8;
-                else reinterpret_cast<uint16_t *>(p.C)[at] = round16(scaled(s >> 8, scale_at(p.row_scale, m, p.M), scale_at(p.col_scale, n, p.N)), p.out);
+                else reinterpret_cast<uint16_t *>(p.C)[at] = finish16(p, s >> 8, scale_at(p.row_scale, m, p.M), n);
             }
         }
 #pragma unroll
@@ -342,12 +342,13 @@ struct DotCfg {
 template <class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS)
 gemm_dot_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int M, const int N, const int K, const int ldc, const int out,
-                       const float *row_scale, const float *col_scale)
+                       const float *row_scale, const float *col_scale, const uint16_t *bias)
 {
     // (scalar arguments: preloaded into SGPRs before the first wave starts, see gemm_skinny_stream_dma_kernel)
     GemmArgs p{A, B, C, M, N, K};
     p.row_scale = row_scale;
     p.col_scale = col_scale;
+    p.bias = bias;
     p.out = out;
     p.ldc = ldc;
     constexpr int MR = Cfg::MR, FN = Cfg::FN, NW = Cfg::NW, U = Cfg::U;
@@ -425,7 +426,7 @@ gemm_dot_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int M, con
             for (int w = 0; w < NW; ++w) s += (&red[w][0][0])[idx];
             const size_t at = (size_t)m * c_stride(p) + n;
             if (p.out == OUT_I32) p.C[at] = s;
-            else reinterpret_cast<uint16_t *>(p.C)[at] = round16(scaled(s, scale_at(p.row_scale, m, p.M), scale_at(p.col_scale, n, p.N)), p.out);
+            else reinterpret_cast<uint16_t *>(p.C)[at] = finish16(p, s, scale_at(p.row_scale, m, p.M), n);
         }
     }
 }

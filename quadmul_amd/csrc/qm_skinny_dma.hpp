@@ -65,12 +65,13 @@ struct SkinnyDmaCfg {
 template <class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS)
 gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int M, const int N, const int K, const int ldc, const int out,
-                       const float *row_scale, const float *col_scale)
+                       const float *row_scale, const float *col_scale, const uint16_t *bias)
 {
     // (scalar arguments: preloaded into SGPRs before the first wave starts, see gemm_skinny_stream_dma_kernel)
     GemmArgs p{A, B, C, M, N, K};
     p.row_scale = row_scale;
     p.col_scale = col_scale;
+    p.bias = bias;
     p.out = out;
     p.ldc = ldc;
     constexpr int FM = Cfg::FM, FN = Cfg::FN, NW = Cfg::NW, D = Cfg::D, LPR = Cfg::LOADS_PER_RUN;
@@ -245,7 +246,7 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int c = s[e];
-                h[e] = round16(scaled(c, rs, scale_at(p.col_scale, n + e, p.N)), p.out);
+                h[e] = finish16(p, c, rs, n + e);
             }
             if (vec_ok) {
                 *reinterpret_cast<v2i *>(d) = v2i{(int)(h[0] | ((uint32_t)h[1] << 16)), (int)(h[2] | ((uint32_t)h[3] << 16))};
@@ -300,7 +301,8 @@ struct SkinnyStreamCfg {
 template <class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS)
 gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int M, const int N, const int K, const int ldc,
-                              const int out_and_grid, const int nblocks, const float *row_scale, const float *col_scale)  // 16 dwords: all preloaded
+                              const int out_and_grid, const int nblocks, const float *row_scale, const float *col_scale,  // 16 dwords up to here: all preloaded
+                              const uint16_t *bias)
 {
     // (out_and_grid: the output form in bits 0..7, the number of workgroups above.  gridDim.x
     // is a hidden kernel argument beyond the preloaded ones: read from there it is a scalar
@@ -308,6 +310,7 @@ gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, co
     GemmArgs p{A, B, C, M, N, K};
     p.row_scale = row_scale;
     p.col_scale = col_scale;
+    p.bias = bias;
     p.out = out_and_grid & 0xFF;
     p.ldc = ldc;
     constexpr int FM = Cfg::FM, FN = Cfg::FN, NW = Cfg::NW, D = Cfg::D, R = Cfg::R, LPU = Cfg::LOADS_PER_UNIT;
@@ -496,7 +499,7 @@ gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, co
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int c = s[e];
-                    h[e] = round16(scaled(c, rs, scale_at(p.col_scale, n + e, p.N)), p.out);
+                    h[e] = finish16(p, c, rs, n + e);
                 }
                 if (vec_ok) {
                     *reinterpret_cast<v2i *>(d) = v2i{(int)(h[0] | ((uint32_t)h[1] << 16)), (int)(h[2] | ((uint32_t)h[3] << 16))};

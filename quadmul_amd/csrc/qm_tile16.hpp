@@ -218,7 +218,12 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
     // K-step.
     const int ldc = c_stride(p);  // row stride of C in elements (N, unless this call computes a block of columns of a wider C)
     const bool vec_ok = (ldc & 3) == 0 && ((uintptr_t)p.C & (4 * ESZ - 1)) == 0;  // 4 elements per store
-    const bool plain_c = vec_ok && ksplit == 1 && ldc < (1 << 21);
+    // (The bias of a 16-bit output waits in registers for that; a configuration with no room for it
+    // -- 256 x 256 with the deepest ring: sixteen registers, one spilt -- writes the tiles of a call
+    // that has one through the guarded code.)
+    constexpr int NBIAS = Cfg::XPOSE ? FN / 4 : Cfg::XHALF ? FN / 2 : FN;  // column quartets of a lane
+    constexpr bool BIAS_REGS = OUT != OUT_I32 && NBIAS <= 4;
+    const bool plain_c = vec_ok && ksplit == 1 && ldc < (1 << 21) && (OUT == OUT_I32 || BIAS_REGS || p.bias == nullptr);
     const int full_m = p.M / BM, full_n = p.N / BN;
     const int nwhole = __builtin_amdgcn_readfirstlane(plain_c ? full_m * full_n : 0);
     auto locate = [&](const int item, int &m0, int &n0, int &kt0, int &KT) __attribute__((always_inline)) {
@@ -482,6 +487,11 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
     typedef float v4f __attribute__((ext_vector_type(4)));
     float rs_reg[OUT != OUT_I32 ? FM : 1];
     v4f cs_reg[OUT != OUT_I32 ? FN : 1];
+    // ... and the bias of the four columns it stores of every 64-column group (whole tiles through
+    // the LDS) or of every block, packed in the output's type.  No bias: -0, the value that
+    // changes nothing when it is added, so that the write-out has no branch.  (In registers
+    // because a load in the last K-step would drain the ring, see below.)
+    v2i bias_reg[OUT != OUT_I32 ? NBIAS : 1];
     v4i zero4;
     asm volatile("v_mov_b32 %0, 0" : "=v"(zero4.x));  // (opaque, so the MFMA operand is a plain register tuple)
     zero4.y = zero4.z = zero4.w = zero4.x;
@@ -502,13 +512,18 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
     };
     // four fp32 bit patterns -> four 16-bit floats in two registers
     auto pack16 = [&](const v4i v) __attribute__((always_inline)) -> v2i {
-        uint32_t h[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int bits = v[e];  // (by value: a bit cast applied to the vector element itself reads element 0)
-            h[e] = round16<OUT == OUT_I32 ? OUT_F16 : OUT>(__builtin_bit_cast(float, bits));
-        }
-        return v2i{(int)(h[0] | (h[1] << 16)), (int)(h[2] | (h[3] << 16))};
+        const int e0 = v[0], e1 = v[1], e2 = v[2], e3 = v[3];  // (by value: a bit cast applied to the vector element itself reads element 0)
+        const uint32_t lo = round16_pair<OUT == OUT_I32 ? OUT_F16 : OUT>(__builtin_bit_cast(float, e0), __builtin_bit_cast(float, e1));
+        const uint32_t hi = round16_pair<OUT == OUT_I32 ? OUT_F16 : OUT>(__builtin_bit_cast(float, e2), __builtin_bit_cast(float, e3));
+        return v2i{(int)lo, (int)hi};
+    };
+    // the same plus the bias of their four columns
+    auto with_bias = [&](const v2i o, const v2i b) __attribute__((always_inline)) -> v2i {
+        return v2i{(int)add16_pair<OUT>((uint32_t)o.x, (uint32_t)b.x), (int)add16_pair<OUT>((uint32_t)o.y, (uint32_t)b.y)};
+    };
+    auto pack_block = [&](const v4i v, auto j_) __attribute__((always_inline)) -> v2i {
+        if constexpr (BIAS_REGS) return with_bias(pack16(v), bias_reg[decltype(j_)::value]);
+        else return pack16(v);
     };
     // byte offsets of this lane from the tile's corner (32 bits are enough for the rows of one
     // tile when N is below 2^21): as the MFMA leaves a block, and as the LDS area is read back
@@ -571,8 +586,8 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
                 if constexpr (edge) store_lanes(at, lane_row, v, std::integral_constant<int, ib * 16 + 4 * k>{}, std::integral_constant<int, grp * 64>{});
                 else *reinterpret_cast<v4i *>(at + lane_row) = v;
             } else {
-                if constexpr (edge) store_lanes(at, lane_row, pack16(xr[k]), std::integral_constant<int, ib * 16 + 4 * k>{}, std::integral_constant<int, grp * 64>{});
-                else *reinterpret_cast<v2i *>(at + lane_row) = pack16(xr[k]);
+                if constexpr (edge) store_lanes(at, lane_row, with_bias(pack16(xr[k]), bias_reg[grp]), std::integral_constant<int, ib * 16 + 4 * k>{}, std::integral_constant<int, grp * 64>{});
+                else *reinterpret_cast<v2i *>(at + lane_row) = with_bias(pack16(xr[k]), bias_reg[grp]);
             }
         };
         if constexpr (t < 4) {
@@ -610,8 +625,8 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
             if constexpr (edge) store_lanes(at, lane_half, v, std::integral_constant<int, ib * 16 + 8 * k>{}, std::integral_constant<int, h * 32>{});
             else *reinterpret_cast<v4i *>(at + lane_half) = v;
         } else {
-            if constexpr (edge) store_lanes(at, lane_half, pack16(xr[k]), std::integral_constant<int, ib * 16 + 8 * k>{}, std::integral_constant<int, h * 32>{});
-            else *reinterpret_cast<v2i *>(at + lane_half) = pack16(xr[k]);
+            if constexpr (edge) store_lanes(at, lane_half, with_bias(pack16(xr[k]), bias_reg[h]), std::integral_constant<int, ib * 16 + 8 * k>{}, std::integral_constant<int, h * 32>{});
+            else *reinterpret_cast<v2i *>(at + lane_half) = with_bias(pack16(xr[k]), bias_reg[h]);
         }
     };
     auto write_half = [&](auto ib_, auto h_, auto t_, auto edge_) __attribute__((always_inline)) {
@@ -644,10 +659,10 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
             char *const at = tile_c + ((size_t)(ib * 16) * ldc + j * 16) * ESZ;  // wave-uniform
             if constexpr (decltype(edge_)::value) {
                 if constexpr (OUT == OUT_I32) store_lanes(at, lane_blk, xr[0], std::integral_constant<int, ib * 16>{}, std::integral_constant<int, j * 16>{});
-                else store_lanes(at, lane_blk, pack16(xr[0]), std::integral_constant<int, ib * 16>{}, std::integral_constant<int, j * 16>{});
+                else store_lanes(at, lane_blk, pack_block(xr[0], j_), std::integral_constant<int, ib * 16>{}, std::integral_constant<int, j * 16>{});
             } else {
                 if constexpr (OUT == OUT_I32) *reinterpret_cast<v4i *>(at + lane_blk) = xr[0];
-                else *reinterpret_cast<v2i *>(at + lane_blk) = pack16(xr[0]);
+                else *reinterpret_cast<v2i *>(at + lane_blk) = pack_block(xr[0], j_);
             }
         }
     };
@@ -674,7 +689,9 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
         if constexpr (OUT != OUT_I32) {
             if (m < p.M) {
                 uint16_t *drow = reinterpret_cast<uint16_t *>(p.C) + (size_t)m * ldc;
-                const v2i o = pack16(v);
+                // (the columns of a block, not the order whole tiles are stored in: the bias is
+                // fetched here)
+                const v2i o = with_bias(pack16(v), bias4_at(p, n));
                 if (vec_ok && n + 3 < p.N) {
                     *reinterpret_cast<v2i *>(drow + n) = o;
                 } else if (n + 3 < p.N) {
@@ -873,6 +890,14 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
             for (int j = 0; j < FN; ++j)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) keep_here_f(cs_reg[j][e]);
+            if constexpr (BIAS_REGS) {
+                const int bias_n = c_n0 + wn * Cfg::WN + (Cfg::XPOSE ? (lane & 15) * 4 : Cfg::XHALF ? (lane & 7) * 4 : g * 4);
+                constexpr int bias_step = Cfg::XPOSE ? 64 : Cfg::XHALF ? 32 : 16;
+#pragma unroll
+                for (int j = 0; j < NBIAS; ++j) bias_reg[j] = bias4_at(p, bias_n + j * bias_step);
+#pragma unroll
+                for (int j = 0; j < NBIAS; ++j) asm volatile("" ::"v"(bias_reg[j]));
+            }
         }
         // (the masks are made opaque: knowing one to be all-ones-per-nibble or zero, the
         // compiler would hoist the whole widening of B out of the MFMA slots into a branch)

@@ -289,3 +289,69 @@ def test_tiles_that_stick_out_of_c_on_every_pipelined_configuration(oracle_mod, 
                 assert torch.isnan(buf16[:pad]).all() and torch.isnan(buf16[pad + m * n:]).all(), name
         ran += 1
     assert ran >= 8
+
+
+# every epilogue: the dot, wave-level and persistent kernels (1 to 64 rows), the generic kernel (K % 32,
+# and too small to pad), zero-padded copies, each tile through its own way of writing whole tiles,
+# tiles that stick out of C, odd N, a short last K-step, a K split added up out of a workspace, k = 0
+BIAS_SHAPES = [(1, 33, 256), (2, 64, 4096), (9, 130, 8192), (40, 96, 1152), (70, 33, 162), (2048, 520, 130), (256, 512, 256), (520, 780, 384),
+               (300, 1021, 416), (257, 258, 640), (6, 10, 0)]
+
+
+@pytest.mark.parametrize("shape", BIAS_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_bias_in_every_epilogue(oracle_mod, shape):
+    """The bias added in the epilogue gives, bit for bit, the rounded value plus the bias rounded
+    once more; without one, a zero with a negative scale stays -0."""
+    m, n, k = shape
+    a, b = make_operands(m, n, max(k, 2), SEED_BASE + 7600 + m + n + k)
+    ap, bp = pack_cpu(a), pack_cpu(b)
+    if k == 0:
+        ap, bp = ap[:, :0].contiguous(), bp[:, :0].contiguous()
+    ap[0] = 0                                        # zero products: -0 under the negative scales
+    rs, cs = make_scales(m, n, SEED_BASE + 7601 + m)
+    cs[::3] *= -1
+    c = oracle_mod.gemm_i4(ap.numpy(), bp.numpy()) if k else np.zeros((m, n), np.int32)
+    a_d, b_d, rs_d, cs_d = ap.to(DEV), bp.to(DEV), rs.to(DEV), cs.to(DEV)
+    for dtype, out in DTYPES:
+        bias = torch.randn(n, generator=torch.Generator().manual_seed(n)).to(dtype)
+        bias[1::5] = 0.0
+        bias[2::5] = -0.0
+        plain = torch.from_numpy(oracle_mod.scale_round16(c, rs.numpy(), cs.numpy(), out).view(np.int16)).view(dtype) if k else torch.zeros((m, n), dtype=dtype)
+        want = plain + bias
+        codes = [qm.CFG_AUTO]
+        if k:
+            for cfg in range(qm.num_configs()):
+                if qm.config_supports(cfg, m, n, k) and qm.config_has_scaled(cfg):
+                    codes.append(cfg | (2 << 16))
+                    if k >= 640 and qm.config_name(cfg).startswith("q"):
+                        codes.append(cfg | (2 << 16) | (2 << 24))
+        for code in codes:
+            name = "auto" if code < 0 else qm.config_name(code & 0xFFFF)
+            for b_, w_ in ((bias.to(DEV), want), (None, plain)):
+                d = poisoned_d(m, n, dtype)
+                qm.gemm_scaled(a_d, b_d, d, m, n, k, rs_d, cs_d, code, bias=b_)
+                torch.cuda.synchronize()
+                assert (bits(d) == bits(w_)).all(), (name, code >> 16, dtype, b_ is None)
+    with pytest.raises(qm.QuadmulError):
+        qm.gemm_scaled(a_d, b_d, d, m, n, k, rs_d, cs_d, bias=torch.zeros(n + 1, dtype=d.dtype, device=DEV))
+
+
+def test_linear_bias_that_the_kernel_cannot_take(oracle_mod):
+    """A bias that autograd follows, or of another type than the output, is added apart as ever."""
+    from quadmul_amd.linear import W4A4Linear
+
+    n, k = 64, 256
+    g = torch.Generator().manual_seed(SEED_BASE + 7700)
+    w, x = torch.randn((n, k), generator=g).to(DEV), torch.randn((3, k), generator=g).to(DEV)
+    bias = torch.randn(n, generator=g).to(DEV)
+    layer = W4A4Linear.from_float(w, bias)
+    y = layer(x)
+    layer.bias = layer.bias.clone().requires_grad_(True)
+    z = layer(x)
+    assert z.requires_grad and torch.equal(z.detach(), y)
+    z.float().sum().backward()
+    assert torch.equal(layer.bias.grad, torch.full((n,), 3.0, dtype=torch.float16, device=DEV))
+    layer.bias = bias                                # float32 beside a float16 output
+    bare = W4A4Linear(layer.weight_packed, layer.weight_scale)(x)
+    bare += bias
+    assert torch.equal(layer(x), bare)
