@@ -60,9 +60,9 @@ extern "C" {
  *     per tile through the workspace: here the best unsplit configuration runs instead.
  *     Two shapes of the reference's table are left that split K: 256 x 8192 x 28672, 59.3 us
  *     against 55.8 (1.06x), and 512 x 8192 x 28672, 96-105 us against 92-95 (1.04-1.11x);
- *   - K % 32 != 0, or A or B not 16-byte aligned: no 16-byte loads, the one-thread-per-element
- *     kernel runs (2048 x 4096 x 4100: 3.3 ms, against 44 us on zero-padded copies in a
- *     workspace).  Weight matrices of the reference's table all have K % 32 == 0.
+ *   - K % 32 != 0, or A or B not 16-byte aligned: the kernel for operands at any address runs,
+ *     several times slower on many rows than the zero-padded copies in a workspace.  Weight
+ *     matrices of the reference's table all have K % 32 == 0.
  * A caller that can lend device memory should bind qm_gemm_i4_ws; one that cannot allocate,
  * qm_gemm_i4_static.
  */
@@ -115,7 +115,7 @@ int qm_config_has_scaled(int cfg); /* 1 / 0 */
  * C.  The second use (cfg = QM_CFG_AUTO only): large shapes whose K is not a multiple of
  * 32, or whose operands are not 16-byte aligned, get copies of A and B in the workspace
  * with every row padded with zeros to whole 128-nibble steps, and run on the pipelined
- * kernel instead of the generic one.  Results are identical to the forms without a
+ * kernel, except where the kernel for operands at any address is faster.  Results are identical to the forms without a
  * workspace.
  *   workspace        device memory, 16-byte aligned, or NULL; used by the kernels of this
  *                    call only (in stream order): calls that may overlap on the GPU need

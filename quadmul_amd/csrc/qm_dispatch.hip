@@ -12,6 +12,7 @@
 #include "qm_launch.hpp"
 #include "qm_skinny.hpp"
 #include "qm_skinny_dma.hpp"
+#include "qm_ragged.hpp"
 #include "qm_aux.hpp"
 
 #define QM_EXPORT extern "C" __attribute__((visibility("default")))
@@ -202,6 +203,54 @@ static hipError_t launch_padded(GemmArgs &p, const PadPlan &pl, void *ws, hipStr
     return hipSuccess;
 }
 
+// The automatic choice where none of the aligned kernels takes the operands (the "generic"
+// configuration: K % 32 != 0, or A or B not 16-byte aligned): the matrix-core kernel of
+// qm_ragged.hpp if K and the operands' sizes are within what it addresses -- else, as for an
+// explicit "generic", one thread per element.
+static bool ragged_fits(int m, int n, int k)
+{
+    const long long kb = k / 2;
+    return k >= 32 && k <= QM_MAX_K_X16 && (long long)m * kb < 0x7fffffffLL && (long long)n * kb < 0x7fffffffLL && (m + 15) / 16 <= 65535;
+}
+
+template <class Cfg>
+static hipError_t launch_ragged(const GemmArgs &p, hipStream_t s)
+{
+    const dim3 grid((p.N + Cfg::BN - 1) / Cfg::BN, (p.M + Cfg::MAX_M - 1) / Cfg::MAX_M);
+    gemm_ragged_kernel<Cfg><<<grid, dim3(Cfg::THREADS), 0, s>>>(p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out, p.row_scale, p.col_scale, p.bias);
+    return hipGetLastError();
+}
+
+// With a workspace a large product can also run on zero-padded copies of A and B on the
+// aligned kernels.  The copies cost a launch and 2 x (M + N) K / 2 bytes whatever M is; the kernel
+// here costs more with every block of rows.  us, here / on copies: 3 x 9000 x 9000 12 / 38, 17 x 5001
+// x 2050 8.7 / 10.5, 17 x 3307 x 4100 10.0 / 12.1, 64 x 9000 x 9000 34 / 46, 64 x 8191 x 1030 8.3 / 10.3;
+// 33 x 3307 x 4100 16.1 / 12.4, 33 x 700 x 8998 18.1 / 15.3, 100 x 9000 x 9000 50 / 53, 100 x 5001 x 2050
+// 18.5 / 13.8, 200 x 8191 x 1030 19.8 / 15.1.  A small product on a short K is over before the copies
+// are: 200 x 1001 x 1002 4.3 / 9.8, 500 x 1001 x 1002 5.7 / 9.8.
+static bool ragged_before_copies(int m, int n, int k)
+{
+    return m <= 32 || (m <= 64 && n >= 6000) || (k <= 2048 && (long long)m * n * k < (1LL << 29));
+}
+
+// The largest block that leaves more than half of the 256 CUs a workgroup of their own: it reads
+// (rows + columns) x K / 2 bytes per rows x columns of C, but a workgroup's time is its K loop
+// and an idle CU helps nobody.  us, on blocks of 2x1, 2x2, 4x2 and 4x4 times 16: 17 x 3307 x 4100 10.0,
+// 13.2, 15.4, 21.8; 64 x 3307 x 4100 23.0, 16.1, 23.5, 30.1; 200 x 3307 x 4100 59, 43, 44, 31; 100 x 1001 x
+// 1002 3.5, 4.2, 5.3, 6.7; 64 x 9000 x 9000 64, 45, 53, 34.  Up to 16 rows, 1x1 and 1x2: 16 x 3307 x 4100 8.9,
+// 12.1; 16 x 5001 x 2050 9.5, 7.8.  One thread per element, which these calls used to run on: 1 x 9000
+// x 9000 264 us (here 14.5), 16 x 700 x 8998 195 (12.6), 64 x 1001 x 1002 19 (3.4).
+static hipError_t launch_ragged(const GemmArgs &p, hipStream_t s)
+{
+    const auto crowded = [&](int fm, int fn) { return (long long)((p.N + 16 * fn - 1) / (16 * fn)) * ((p.M + 16 * fm - 1) / (16 * fm)) > 128; };
+    if (p.M <= 16 && crowded(1, 2)) return launch_ragged<RaggedCfg<1, 2, 8, 2>>(p, s);
+    if (p.M <= 16) return launch_ragged<RaggedCfg<1, 1, 16, 2>>(p, s);
+    if (p.M > 32 && crowded(4, 4)) return launch_ragged<RaggedCfg<4, 4, 8, 1>>(p, s);
+    if (p.M > 32 && crowded(4, 2)) return launch_ragged<RaggedCfg<4, 2, 8, 2>>(p, s);
+    if (crowded(2, 2)) return launch_ragged<RaggedCfg<2, 2, 8, 2>>(p, s);
+    return launch_ragged<RaggedCfg<2, 1, 16, 2>>(p, s);
+}
+
 static Choice choice_from_code(int cfg)
 {
     Choice ch;
@@ -359,7 +408,8 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
         ch = select_scaled(m, n, k, align, false);
         ch.ksplit = 1;
     }
-    if (cfg == QM_CFG_AUTO && has_ws) {
+    const bool ragged = cfg == QM_CFG_AUTO && g_configs[ch.cfg].kind == KIND_GENERIC && ragged_fits(m, n, k);
+    if (cfg == QM_CFG_AUTO && has_ws && !(ragged && ragged_before_copies(m, n, k))) {
         PadPlan pl = plan_padded_k(m, n, k, align, ch);
         if (pl.on && !launcher(pl.ch.cfg)) {
             // a pipelined configuration that has the scaled output, if the shape is one for those
@@ -371,6 +421,10 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
             if (e == hipSuccess) e = launcher(pl.ch.cfg)(p, s, pl.ch.group_m | (1 << 8) | (pl.ch.spread << 16));
             return e == hipSuccess ? QM_OK : fail_launch(e);
         }
+    }
+    if (ragged) {
+        const hipError_t e = launch_ragged(p, s);
+        return e == hipSuccess ? QM_OK : fail_launch(e);
     }
     if (ch.ksplit > 1) {
         // int32, no workspace: the partial sums meet in C by integer atomic adds, C starts from zero

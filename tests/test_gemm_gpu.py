@@ -758,3 +758,49 @@ def test_every_config_on_random_shapes_against_the_generic_kernel():
         assert torch.equal(want, got), (names[cfg], ksplit, m, n, k, f"operand seed {seed}")
         ran[names[cfg]] = ran.get(names[cfg], 0) + 1
     assert len(ran) == len(names) - 1 and min(ran.values()) >= 10, ran
+
+
+# rows either side of every change of block (16, 32, 64) and of the rule against padded copies; K from the
+# 16 bytes a lane loads up, around whole chunks of 64 bytes, one chunk more than the waves of a workgroup
+RAGGED_SHAPES = [(1, 1, 32 + 2), (16, 33, 34), (17, 15, 62), (32, 31, 126), (33, 64, 130), (65, 130, 254), (3, 2500, 258), (1, 4100, 2050),
+                 (16, 4200, 2178), (17, 5000, 1030), (31, 300, 4102), (40, 9000, 514), (64, 8300, 4098), (100, 4200, 386), (300, 500, 1000)]
+
+
+@pytest.mark.parametrize("shape", RAGGED_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_any_even_k_at_any_address(oracle_mod, shape):
+    """The kernel for operands that are not 16-byte aligned: int32, fp16 and bf16 with scales and
+    bias, operands at odd addresses between bytes that must not count, without a workspace and
+    with one, and the memory around C as it was."""
+    m, n, k = shape
+    a, b = make_operands(m, n, k, SEED_BASE + 9700 + m + n + k)
+    ap, bp = pack_cpu(a), pack_cpu(b)
+    want = oracle_mod.gemm_i4(ap.numpy(), bp.numpy())
+
+    def at(t, off):
+        buf = torch.full((t.numel() + off + 64,), 0x77, dtype=torch.int8, device=DEV)
+        v = buf[off:off + t.numel()].view(t.shape)
+        v.copy_(t)
+        return v
+
+    pad = 512
+    rs, cs = torch.rand(m, device=DEV) * 0.02, torch.rand(n, device=DEV) * 0.05 - 0.02
+    for oa, ob in ((0, 0), (3, 5), (16, 1)):
+        a_d, b_d = at(ap, oa), at(bp, ob)
+        for ws in (None, True):
+            buf = torch.full((m * n + 2 * pad,), 0x7F7F7F7F, dtype=torch.int32, device=DEV)
+            qm.gemm(a_d, b_d, buf[pad:pad + m * n].view(m, n), m, n, k, workspace=ws)
+            torch.cuda.synchronize()
+            bad = oracle_mod.compare(buf[pad:pad + m * n].view(m, n).cpu().numpy(), want)
+            assert bad == -1, (oa, ob, ws, bad)
+            assert (buf[:pad] == 0x7F7F7F7F).all() and (buf[pad + m * n:] == 0x7F7F7F7F).all()
+        for dtype, out in ((torch.float16, oracle_mod.OUT_F16), (torch.bfloat16, oracle_mod.OUT_BF16)):
+            bias = torch.randn(n, device=DEV).to(dtype)
+            d = torch.full((m, n), float("nan"), dtype=dtype, device=DEV)
+            qm.gemm_scaled(a_d, b_d, d, m, n, k, rs, cs, bias=bias)
+            torch.cuda.synchronize()
+            w = torch.from_numpy(oracle_mod.scale_round16(want, rs.cpu().numpy(), cs.cpu().numpy(), out).view(np.int16)).view(dtype) + bias.cpu()
+            assert torch.equal(d.cpu().view(torch.int16), w.view(torch.int16)), (oa, ob, dtype)
+    lo = torch.full((m, k), -8, dtype=torch.int8)
+    c_d = poisoned_c(m, n, DEV)
+    qm.gemm(at(pack_cpu(lo), 1), at(pack_cpu(torch.full((n, k), 7, dtype=torch.int8)), 2), c_d, m, n, k)
+    assert (c_d == -56 * k).all()
