@@ -270,119 +270,143 @@ __global__ void unpack_i4_byte_kernel(const uint8_t *__restrict__ src, int8_t *_
 }
 
 // --------------------------------------------------------------------------
-// Per-row symmetric quantisation to int4 fused with the packing: one workgroup per row,
-// the row held in registers between the two passes over it (maximum, then quantise), so
-// HBM is read once.  x is fp16, bf16 or fp32; 8 elements (4 packed bytes) per thread-chunk.
+// Per-row symmetric quantisation to int4 fused with the packing, the row held in registers
+// between the two passes over it (maximum, then quantise), so HBM is read once.  x is fp16,
+// bf16 or fp32; 8 elements (4 packed bytes) per lane and chunk.
+//
+// Any even k from 8 up and any address: rows are loaded and stored at whatever alignment they
+// have (the memory pipeline splits at cache lines), and the last chunk of a row is its last 8
+// elements -- those that the chunk before has too are quantised twice to the same bytes.
+// Lanes without a chunk load that last one as well and store nothing, so all loads of a
+// lane are in flight together (behind a branch per chunk each waited for the one before).
 // --------------------------------------------------------------------------
 template <int IN> struct QuantIn;
 template <> struct QuantIn<QM_IN_F16> {
-    static constexpr int BYTES = 2;
+    static constexpr int BYTES = 2, WORDS = 4;  // of an element, and 32-bit words per chunk
     static __device__ __forceinline__ float widen(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 };
 template <> struct QuantIn<QM_IN_BF16> {
-    static constexpr int BYTES = 2;
+    static constexpr int BYTES = 2, WORDS = 4;
     static __device__ __forceinline__ float widen(uint16_t h) { return __builtin_bit_cast(float, (uint32_t)h << 16); }
 };
 template <> struct QuantIn<QM_IN_F32> {
-    static constexpr int BYTES = 4;
+    static constexpr int BYTES = 4, WORDS = 8;
 };
 
 template <int IN>
-__device__ __forceinline__ void load8(const uint8_t *src, float (&v)[8])
-{
-    if constexpr (IN == QM_IN_F32) {
-        const v4i lo = *reinterpret_cast<const v4i *>(src), hi = *reinterpret_cast<const v4i *>(src + 16);
+struct Chunk8 {
+    v4i w[QuantIn<IN>::WORDS / 4];
+    __device__ __forceinline__ void load(const uint8_t *src)
+    {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int a = lo[e], b = hi[e];
-            v[e] = __builtin_bit_cast(float, a);
-            v[4 + e] = __builtin_bit_cast(float, b);
-        }
-    } else {
-        const v4i w = *reinterpret_cast<const v4i *>(src);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t d = (uint32_t)w[e];
-            v[2 * e] = QuantIn<IN>::widen((uint16_t)(d & 0xFFFFu));
-            v[2 * e + 1] = QuantIn<IN>::widen((uint16_t)(d >> 16));
+        for (int i = 0; i < QuantIn<IN>::WORDS / 4; ++i) {
+            if constexpr (IN == QM_IN_F32) w[i] = *reinterpret_cast<const v4i_elem_aligned *>(src + 16 * i);
+            else w[i] = *reinterpret_cast<const v4i_half_aligned *>(src + 16 * i);
         }
     }
+    __device__ __forceinline__ float at(int e) const
+    {
+        if constexpr (IN == QM_IN_F32) {
+            const int d = w[e >> 2][e & 3];
+            return __builtin_bit_cast(float, d);
+        } else {
+            const uint32_t d = (uint32_t)w[0][e >> 1];
+            return QuantIn<IN>::widen((uint16_t)((e & 1) ? d >> 16 : d & 0xFFFFu));
+        }
+    }
+    __device__ __forceinline__ float amax(float m) const
+    {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(at(e)));
+        return m;
+    }
+};
+
+// 8 elements -> 8 nibbles, element e in nibble e (low nibble = even k, test.py:8,14).  The clamp is
+// one v_med3_f32, which takes a NaN to -7 as fmin(fmax()) does.  The rounded values are
+// small integers, put together in fp32 four at a time without any rounding:
+// 2^23 + sum((n_e + 8) 16^e) < 2^24, whose low 16 bits are the nibbles with their sign bits inverted.
+__device__ __forceinline__ uint32_t quant4(float r0, float r1, float r2, float r3)
+{
+    float t = __builtin_fmaf(r3, 16.0f, r2);
+    t = __builtin_fmaf(t, 16.0f, r1);
+    t = __builtin_fmaf(t, 16.0f, r0 + (8388608.0f + 34952.0f));
+    return __builtin_bit_cast(uint32_t, t);
 }
 
-__device__ __forceinline__ uint32_t quant8(const float (&v)[8], float inv)
+template <int IN>
+__device__ __forceinline__ uint32_t quant8(const Chunk8<IN> &c, float inv)
 {
 #pragma clang fp contract(off)
-    uint32_t out = 0;
+    float r[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        float r = __builtin_rintf(v[e] * inv);  // round half to even
-        r = fminf(fmaxf(r, -7.0f), 7.0f);
-        out |= ((uint32_t)(int)r & 0xFu) << (4 * e);  // element e -> nibble e: low nibble = even k (test.py:8,14)
-    }
-    return out;
+    for (int e = 0; e < 8; ++e) r[e] = __builtin_amdgcn_fmed3f(__builtin_rintf(c.at(e) * inv), -7.0f, 7.0f);  // (round half to even)
+    const uint32_t lo = quant4(r[0], r[1], r[2], r[3]), hi = quant4(r[4], r[5], r[6], r[7]);
+    return __builtin_amdgcn_perm(hi, lo, 0x05040100u) ^ 0x88888888u;
 }
 
-// workgroup-wide maximum of non-negative floats
-__device__ __forceinline__ float block_max(float x, float *lds)
+// maximum over the NW waves that share a row (one row per workgroup unless NW == 1)
+template <int NW>
+__device__ __forceinline__ float row_max(float x, float *lds)
 {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) x = fmaxf(x, __shfl_xor(x, off));
-    const int wave = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) lds[wave] = x;
-    __syncthreads();
-    float m = lds[0];
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) m = fmaxf(m, lds[w]);
-    __syncthreads();
-    return m;
+    if constexpr (NW > 1) {
+        if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = x;
+        __syncthreads();
+        x = lds[0];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) x = fmaxf(x, lds[w]);
+    }
+    return x;
 }
 
-// NC: chunks of 8 elements a thread keeps in registers (k <= 2048 * NC); NC == 0: any k that is
-// a multiple of 8, the row read twice (the second time out of the L2)
-template <int IN, int NC>
-__global__ void __launch_bounds__(256) quantize_pack_kernel(const uint8_t *__restrict__ x, uint8_t *__restrict__ dst, float *__restrict__ scales, int k)
+// NW waves per row (4 rows per workgroup if one), NC chunks of 8 elements per lane: k <= 512 * NW * NC.
+// NC == 0: any k, the row read twice (the second time out of the L2).
+template <int IN, int NW, int NC>
+__global__ void __launch_bounds__(NW == 1 ? 256 : 64 * NW) quantize_pack_kernel(const uint8_t *__restrict__ x, uint8_t *__restrict__ dst, float *__restrict__ scales, int rows, int k)
 {
-    __shared__ float red[4];
-    const int row = blockIdx.x, tid = threadIdx.x, nchunks = k >> 3;
+    __shared__ float red[NW];
+    const int row = NW == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+    const int lane = NW == 1 ? threadIdx.x & 63 : threadIdx.x;  // within the row
+    if (NW == 1 && row >= rows) return;
+    const int nchunks = (k + 7) >> 3;
     const uint8_t *xr = x + (size_t)row * k * QuantIn<IN>::BYTES;
-    uint32_t *out = reinterpret_cast<uint32_t *>(dst + (size_t)row * (k >> 1));
+    uint8_t *out = dst + (size_t)row * (k >> 1);
+    const auto first = [&](int c) { return min(8 * c, k - 8); };
     float amax = 0.0f;
     if constexpr (NC > 0) {
-        float v[NC][8];
+        Chunk8<IN> v[NC];
 #pragma unroll
-        for (int i = 0; i < NC; ++i) {
-            const int c = tid + i * 256;
-            if (c < nchunks) {
-                load8<IN>(xr + (size_t)c * 8 * QuantIn<IN>::BYTES, v[i]);
+        for (int i = 0; i < NC; ++i) v[i].load(xr + first(lane + i * 64 * NW) * QuantIn<IN>::BYTES);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[i][e]));
-            }
-        }
-        amax = block_max(amax, red);
+        for (int i = 0; i < NC; ++i) amax = v[i].amax(amax);
+        amax = row_max<NW>(amax, red);
         const float inv = amax > 0.0f ? 7.0f / amax : 0.0f;
-        if (tid == 0) scales[row] = amax / 7.0f;
+        if (lane == 0) scales[row] = amax / 7.0f;
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
-            const int c = tid + i * 256;
-            if (c < nchunks) out[c] = quant8(v[i], inv);
+            const int c = lane + i * 64 * NW;
+            const uint32_t q = quant8(v[i], inv);
+            if (c < nchunks) *reinterpret_cast<u32_any_aligned *>(out + (first(c) >> 1)) = q;
         }
     } else {
-        float v[8];
-        for (int c = tid; c < nchunks; c += 256) {
-            load8<IN>(xr + (size_t)c * 8 * QuantIn<IN>::BYTES, v);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[e]));
+        Chunk8<IN> v;
+        for (int c = lane; c < nchunks; c += 64 * NW) {
+            v.load(xr + (size_t)first(c) * QuantIn<IN>::BYTES);
+            amax = v.amax(amax);
         }
-        amax = block_max(amax, red);
+        amax = row_max<NW>(amax, red);
         const float inv = amax > 0.0f ? 7.0f / amax : 0.0f;
-        if (tid == 0) scales[row] = amax / 7.0f;
-        for (int c = tid; c < nchunks; c += 256) {
-            load8<IN>(xr + (size_t)c * 8 * QuantIn<IN>::BYTES, v);
-            out[c] = quant8(v, inv);
+        if (lane == 0) scales[row] = amax / 7.0f;
+        for (int c = lane; c < nchunks; c += 64 * NW) {
+            v.load(xr + (size_t)first(c) * QuantIn<IN>::BYTES);
+            *reinterpret_cast<u32_any_aligned *>(out + (first(c) >> 1)) = quant8(v, inv);
         }
     }
 }
 
-// any even k, any alignment: one pair of elements per thread and pass
+// k < 8: one pair of elements per thread and pass
 template <int IN>
 __global__ void __launch_bounds__(256) quantize_pack_scalar_kernel(const uint8_t *__restrict__ x, uint8_t *__restrict__ dst, float *__restrict__ scales, int k)
 {
@@ -398,7 +422,7 @@ __global__ void __launch_bounds__(256) quantize_pack_scalar_kernel(const uint8_t
     };
     float amax = 0.0f;
     for (int j = tid; j < k; j += 256) amax = fmaxf(amax, fabsf(at(j)));
-    amax = block_max(amax, red);
+    amax = row_max<4>(amax, red);
     const float inv = amax > 0.0f ? 7.0f / amax : 0.0f;
     if (tid == 0) scales[row] = amax / 7.0f;
     for (int j = 2 * tid; j < k; j += 512) {
@@ -407,24 +431,51 @@ __global__ void __launch_bounds__(256) quantize_pack_scalar_kernel(const uint8_t
     }
 }
 
+template <int IN, int NW, int NC>
+static void launch_quantize_rows(const uint8_t *x, uint8_t *dst, float *scales, int rows, int k, hipStream_t s)
+{
+    constexpr int threads = NW == 1 ? 256 : 64 * NW, rows_per_block = NW == 1 ? 4 : 1;
+    constexpr int most = (1 << 21) * rows_per_block;  // a grid has less than 2^32 threads
+    for (int r0 = 0; r0 < rows; r0 += most) {
+        const int n = rows - r0 < most ? rows - r0 : most;
+        quantize_pack_kernel<IN, NW, NC><<<dim3((unsigned)(n + rows_per_block - 1) / rows_per_block), dim3(threads), 0, s>>>(
+            x + (size_t)r0 * k * QuantIn<IN>::BYTES, dst + (size_t)r0 * (k / 2), scales + r0, n, k);
+        if (r0 > 0x7fffffff - most) break;
+    }
+}
+
+// Four waves per row: as many chunks per lane as the row takes, none of them empty.  A workgroup per row is
+// as much dispatch as work on thousands of rows below 1536 elements, where each wave has
+// a row of its own (us, wave / workgroup per row: 8191 x 1030 bf16 6.3 / 8.7, 2048 x 1024 2.85 / 3.2, but
+// 2048 x 4096 6.0 / 5.5, 256 x 4096 3.1 / 2.6); beyond 12288 sixteen waves hold a row in two chunks per lane
+// (sixteen / four: 8192 x 14336 f32 94.5 / 103.5, 64 x 14336 3.0 / 3.2, but 2048 x 8192 11.1 / 9.0).
+// Against one chunk after the other, and one element per thread where k % 8 != 0: 2048 x 8192 bf16
+// 12.1 -> 9.0 us (4.6 TB/s), 8 x 11008 3.5 -> 2.65, 2048 x 8194 24.8 -> 9.4, 8191 x 1030 18.5 -> 6.3.
 template <int IN>
 static hipError_t launch_quantize_pack(const void *x, void *dst, float *scales, int rows, int k, hipStream_t s)
 {
     const uint8_t *xb = static_cast<const uint8_t *>(x);
     uint8_t *db = static_cast<uint8_t *>(dst);
-    const bool vec = k % 8 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)dst & 3) == 0;
-    if (!vec) quantize_pack_scalar_kernel<IN><<<dim3(rows), dim3(256), 0, s>>>(xb, db, scales, k);
-    else if (k <= 2048 * 2) quantize_pack_kernel<IN, 2><<<dim3(rows), dim3(256), 0, s>>>(xb, db, scales, k);
-    else if (k <= 2048 * 8) quantize_pack_kernel<IN, 8><<<dim3(rows), dim3(256), 0, s>>>(xb, db, scales, k);
-    else quantize_pack_kernel<IN, 0><<<dim3(rows), dim3(256), 0, s>>>(xb, db, scales, k);
+    if (k < 8) quantize_pack_scalar_kernel<IN><<<dim3(rows), dim3(256), 0, s>>>(xb, db, scales, k);
+    else if (k > 16384) launch_quantize_rows<IN, 16, 0>(xb, db, scales, rows, k, s);
+    else if (k > 12288) launch_quantize_rows<IN, 16, 2>(xb, db, scales, rows, k, s);
+    else if (rows > 1024 && k <= 512) launch_quantize_rows<IN, 1, 1>(xb, db, scales, rows, k, s);
+    else if (rows > 1024 && k <= 1024) launch_quantize_rows<IN, 1, 2>(xb, db, scales, rows, k, s);
+    else if (rows > 1024 && k <= 1536) launch_quantize_rows<IN, 1, 3>(xb, db, scales, rows, k, s);
+    else if (k <= 2048) launch_quantize_rows<IN, 4, 1>(xb, db, scales, rows, k, s);
+    else if (k <= 4096) launch_quantize_rows<IN, 4, 2>(xb, db, scales, rows, k, s);
+    else if (k <= 6144) launch_quantize_rows<IN, 4, 3>(xb, db, scales, rows, k, s);
+    else if (k <= 8192) launch_quantize_rows<IN, 4, 4>(xb, db, scales, rows, k, s);
+    else if (k <= 10240) launch_quantize_rows<IN, 4, 5>(xb, db, scales, rows, k, s);
+    else launch_quantize_rows<IN, 4, 6>(xb, db, scales, rows, k, s);
     return hipGetLastError();
 }
 
-static unsigned flat_grid(size_t items, unsigned block)
+static unsigned flat_grid(size_t items, unsigned block, size_t most = 256u * 32u)
 {
     size_t g = (items + block - 1) / block;
     if (g < 1) g = 1;
-    if (g > 256u * 32u) g = 256u * 32u;
+    if (g > most) g = most;
     return (unsigned)g;
 }
 

@@ -13,6 +13,11 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 // apart from the next lane's, ran at a third of the speed (1444 x 31702 x 128: 104 us).
 typedef v4i v4i_elem_aligned __attribute__((aligned(4)));
 typedef v2i v2i_half_aligned __attribute__((aligned(2)));
+typedef v4i v4i_half_aligned __attribute__((aligned(2)));
+// ... and at any byte address.
+typedef v4i v4i_any_aligned __attribute__((aligned(1)));
+typedef v2i v2i_any_aligned __attribute__((aligned(1)));
+typedef uint32_t u32_any_aligned __attribute__((aligned(1)));
 
 // Output forms: the exact int32 product, or the product scaled per row and per column in
 // fp32 and rounded to a 16-bit float (the "dequantise on the way out" use the reference's

@@ -24,8 +24,6 @@
 
 namespace qm {
 
-typedef v4i v4i_any_aligned __attribute__((aligned(1)));
-
 template <int FM_, int FN_, int NW_, int U_>
 struct RaggedCfg {
     static constexpr int FM = FM_, FN = FN_, NW = NW_, U = U_;

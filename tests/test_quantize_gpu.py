@@ -49,6 +49,51 @@ def test_quantize_pack_unaligned_input(oracle_mod):
     assert (packed.cpu().numpy().view(np.uint8) == want_p).all() and (scales.cpu().numpy() == want_s).all()
 
 
+# k that is no multiple of 8 (the last chunk of a row overlaps the one before), either side of every change of
+# waves per row and chunks per lane, rows around the four of a workgroup
+ANY_ROW = [(1, 8), (1025, 10), (1026, 512), (1027, 514), (1025, 1026), (1026, 1536), (1030, 1538), (1024, 514), (3, 2046), (2, 2050), (3, 4098),
+           (2, 6146), (3, 8190), (2, 8194), (3, 10242), (2, 12288), (3, 12290), (2, 16382), (3, 16386)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("shape", ANY_ROW, ids=lambda s: "x".join(map(str, s)))
+def test_quantize_pack_any_row(oracle_mod, shape, dtype):
+    """Input one element and output one byte off alignment, the bytes around the output untouched."""
+    rows, k = shape
+    x = make_x(rows, k, dtype, SEED_BASE + 8300 + rows + k)
+    buf = torch.zeros(rows * k + 1, dtype=dtype, device=DEV)
+    buf[1:].copy_(x.reshape(-1))
+    out = torch.full((rows * k // 2 + 33,), 0x5A, dtype=torch.uint8, device=DEV)
+    scales = torch.empty(rows, device=DEV)
+    kind = {torch.float16: 1, torch.bfloat16: 2, torch.float32: 3}[dtype]
+    st = qm.library().qm_quantize_pack_i4(buf.data_ptr() + x.element_size(), kind, out.data_ptr() + 17, scales.data_ptr(), rows, k,
+                                          torch.cuda.current_stream().cuda_stream)
+    assert st == 0
+    want_p, want_s = oracle_mod.quantize_pack(x.to(torch.float32).numpy())
+    got = out.cpu().numpy()
+    assert (got[17:17 + rows * k // 2].reshape(rows, -1) == want_p).all() and (scales.cpu().numpy() == want_s).all()
+    assert (got[:17] == 0x5A).all() and (got[17 + rows * k // 2:] == 0x5A).all()
+
+
+@pytest.mark.parametrize("k", [6, 600, 2600])
+def test_quantize_pack_special_values(k):
+    """A NaN counts for nothing in a row's maximum and becomes -7; an infinity makes the scale infinite and
+    everything finite 0; where 7 / amax overflows the values saturate (and a zero, times infinity, is a NaN)."""
+    x = torch.ones((1100, k))
+    x[0, 1] = float("nan")
+    x[1] = float("nan")
+    x[2, 2], x[2, 3] = float("inf"), -2.0
+    x[3] = 1e-39
+    x[3, 4], x[3, 5] = 0.0, -1e-39
+    packed, scales = qm.quantize_pack(x.to(DEV))
+    v = qm.unpack_int4(packed).cpu()
+    assert v[0, 1] == -7 and (v[0, 2:] == 7).all() and (v[1] == -7).all()
+    assert v[2, 2] == -7 and v[2, 3] == 0 and (v[2, 4:] == 0).all()
+    assert v[3, 4] == -7 and v[3, 5] == -7 and v[3, 0] == 7
+    s = scales.cpu()
+    assert s[0] == np.float32(1) / np.float32(7) and s[1] == 0 and s[2] == float("inf")
+
+
 def test_int4_linear_layer_end_to_end(oracle_mod):
     """activations -> quantize_pack -> gemm_scaled(row_scale = activation scales, col_scale =
     weight scales) against the oracle's chain of the same three steps (bit-exact), and against
