@@ -603,8 +603,8 @@ QM_EXPORT int qm_pack_i4(const void *src_i8, void *dst_packed, int rows, int k, 
     if (nbytes == 0) return QM_OK;
     if (!src_i8 || !dst_packed) return QM_ERR_NULL;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (nbytes % 8 == 0 && ((uintptr_t)src_i8 & 15) == 0 && ((uintptr_t)dst_packed & 7) == 0)
-        pack_i4_vec_kernel<<<dim3(flat_grid(nbytes / 8, 256)), dim3(256), 0, s>>>(static_cast<const v4i *>(src_i8), static_cast<v2i *>(dst_packed), nbytes / 8);
+    if (nbytes >= 8)
+        pack_i4_vec_kernel<<<dim3(flat_grid(nbytes, 8 * PACK_PIECES * PACK_THREADS, 1u << 22)), dim3(PACK_THREADS), 0, s>>>(static_cast<const uint8_t *>(src_i8), static_cast<uint8_t *>(dst_packed), nbytes);
     else
         pack_i4_byte_kernel<<<dim3(flat_grid(nbytes, 256)), dim3(256), 0, s>>>(static_cast<const uint8_t *>(src_i8), static_cast<uint8_t *>(dst_packed), nbytes);
     const hipError_t e = hipGetLastError();
@@ -633,8 +633,8 @@ QM_EXPORT int qm_unpack_i4(const void *src_packed, void *dst_i8, int rows, int k
     if (nbytes == 0) return QM_OK;
     if (!src_packed || !dst_i8) return QM_ERR_NULL;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (nbytes % 4 == 0 && ((uintptr_t)src_packed & 3) == 0 && ((uintptr_t)dst_i8 & 7) == 0)
-        unpack_i4_vec_kernel<<<dim3(flat_grid(nbytes / 4, 256)), dim3(256), 0, s>>>(static_cast<const uint32_t *>(src_packed), static_cast<v2i *>(dst_i8), nbytes / 4);
+    if (nbytes >= 8)
+        unpack_i4_vec_kernel<<<dim3(flat_grid(nbytes, 8 * PACK_THREADS, 1u << 22)), dim3(PACK_THREADS), 0, s>>>(static_cast<const uint8_t *>(src_packed), static_cast<uint8_t *>(dst_i8), nbytes);
     else
         unpack_i4_byte_kernel<<<dim3(flat_grid(nbytes, 256)), dim3(256), 0, s>>>(static_cast<const uint8_t *>(src_packed), static_cast<int8_t *>(dst_i8), nbytes);
     const hipError_t e = hipGetLastError();

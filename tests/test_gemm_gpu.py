@@ -239,6 +239,26 @@ def test_pack_unpack_kernels(oracle_mod):
     assert torch.equal(qm.pack_int4(qm.unpack_int4(allb)).view(torch.uint8), allb)
 
 
+@pytest.mark.parametrize("nbytes", [1, 7, 8, 9, 15, 2047, 2049, 4095, 4096, 4103, 100001])
+@pytest.mark.parametrize("off", [0, 1, 3])
+def test_pack_unpack_any_address(oracle_mod, nbytes, off):
+    """Sizes around the pieces of a thread and of a workgroup, at any address, the bytes around the output untouched."""
+    g = torch.Generator().manual_seed(SEED_BASE + 4100 + nbytes)
+    v = torch.randint(-8, 8, (1, 2 * nbytes), dtype=torch.int8, generator=g)
+    want = oracle_mod.pack_i4(v.numpy()).reshape(-1)
+    src = torch.zeros(2 * nbytes + off, dtype=torch.int8, device=DEV)
+    src[off:] = v[0].to(DEV)
+    out = torch.full((nbytes + 24,), 0x5A, dtype=torch.uint8, device=DEV)
+    back = torch.full((2 * nbytes + 24,), 0x5A, dtype=torch.int8, device=DEV)
+    lib, s = qm.library(), torch.cuda.current_stream().cuda_stream
+    assert lib.qm_pack_i4(src.data_ptr() + off, out.data_ptr() + 8 + off, 1, 2 * nbytes, s) == 0
+    assert lib.qm_unpack_i4(out.data_ptr() + 8 + off, back.data_ptr() + 8 + off, 1, 2 * nbytes, s) == 0
+    o, b = out.cpu().numpy(), back.cpu()
+    assert (o[8 + off:8 + off + nbytes] == want).all() and torch.equal(b[8 + off:8 + off + 2 * nbytes], v[0])
+    assert (o[:8 + off] == 0x5A).all() and (o[8 + off + nbytes:] == 0x5A).all()
+    assert (b[:8 + off] == 0x5A).all() and (b[8 + off + 2 * nbytes:] == 0x5A).all()
+
+
 # ------------------------------------------------------------------ the named workloads
 NAMED_SHAPES = [
     (0, 1024, 1024, 1024), (1, 4096, 4096, 4096),
