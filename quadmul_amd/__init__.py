@@ -7,7 +7,8 @@ Two ways in, both ending in the same C ABI (``include/qm_abi.h``,
   reference's module of the same name: ``quadmul.gemm(a, b, c, m, n, k)``
   (extension.cpp:8-29, call site test.py:40);
 * this package, which binds the C ABI with ctypes and takes torch tensors only to
-  borrow their device pointers and the current stream.
+  borrow their device pointers and the current stream; quantising, packing and the linear
+  layer go through the extension module, whose host side costs less per call.
 
 There is no CPU or eager fallback for the GEMM: if the HIP library has not been
 built, every call raises.
@@ -108,6 +109,27 @@ def library() -> ctypes.CDLL:
     lib.qm_debug_set_operand_limit.restype = ctypes.c_longlong
     _lib = lib
     return lib
+
+
+_ext = None
+
+
+def _native(name: str, *args):
+    """The extension module's function of this name.  From Python the same call costs two to three times as
+    much on the host (device guard, stream, allocations, ctypes), more than a small one takes on the GPU."""
+    global _ext
+    if _ext is None:
+        try:
+            import quadmul
+        except ImportError as e:
+            raise QuadmulError(f"the extension module quadmul cannot be imported ({e}): build it with `python -m quadmul_amd.build`") from e
+        _ext = quadmul
+    try:
+        return getattr(_ext, name)(*args)
+    except RuntimeError as e:
+        if type(e) is RuntimeError:
+            raise QuadmulError(str(e)) from None
+        raise
 
 
 def _check(status: int, what: str) -> None:
@@ -224,18 +246,11 @@ def quantize_pack(x: torch.Tensor):
     [rows])`` with ``scales = amax / 7`` -- the ``row_scale`` of ``gemm_scaled``."""
     if not (x.is_cuda and x.dim() == 2 and x.is_contiguous()):
         raise QuadmulError("quantize_pack: x must be a contiguous 2-d GPU tensor")
-    kinds = {torch.float16: 1, torch.bfloat16: 2, torch.float32: 3}
-    if x.dtype not in kinds:
+    if x.dtype not in (torch.float16, torch.bfloat16, torch.float32):
         raise QuadmulError("quantize_pack: x must be float16, bfloat16 or float32")
-    rows, k = x.shape
-    if k % 2:
+    if x.shape[1] % 2:
         raise QuadmulError("quantize_pack: k must be even")
-    packed = torch.empty((rows, k // 2), dtype=torch.int8, device=x.device)
-    scales = torch.empty((rows,), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
-        st = library().qm_quantize_pack_i4(x.data_ptr(), kinds[x.dtype], packed.data_ptr(), scales.data_ptr(), rows, k, _stream_ptr(x))
-    _check(st, "qm_quantize_pack_i4")
-    return packed, scales
+    return _native("quantize_pack", x)
 
 
 def config_has_scaled(cfg: int) -> bool:
@@ -280,11 +295,7 @@ def pack_int4(values: torch.Tensor) -> torch.Tensor:
         raise QuadmulError("pack_int4: K must be even")
     v = values.contiguous()
     if v.is_cuda:
-        out = torch.empty((rows, k // 2), dtype=torch.int8, device=v.device)
-        with torch.cuda.device(v.device):
-            st = library().qm_pack_i4(v.data_ptr(), out.data_ptr(), rows, k, _stream_ptr(v))
-        _check(st, "qm_pack_i4")
-        return out
+        return _native("pack", v)
     u = v.view(torch.uint8).reshape(-1)
     return ((u[0::2] & 0x0F) | ((u[1::2] & 0x0F) << 4)).reshape(rows, k // 2).view(torch.int8).contiguous()
 
@@ -297,11 +308,7 @@ def unpack_int4(packed: torch.Tensor) -> torch.Tensor:
     p = packed.contiguous()
     rows, half = p.shape
     if p.is_cuda:
-        out = torch.empty((rows, 2 * half), dtype=torch.int8, device=p.device)
-        with torch.cuda.device(p.device):
-            st = library().qm_unpack_i4(p.data_ptr(), out.data_ptr(), rows, 2 * half, _stream_ptr(p))
-        _check(st, "qm_unpack_i4")
-        return out
+        return _native("unpack", p)
     u = p.view(torch.uint8)
     lo = (u & 0x0F).to(torch.int16)
     hi = (u >> 4).to(torch.int16)

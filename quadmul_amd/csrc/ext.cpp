@@ -10,6 +10,8 @@
 #include <torch/extension.h>
 #include <torch/library.h>
 
+#include <algorithm>
+
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
@@ -144,6 +146,42 @@ std::tuple<torch::Tensor, torch::Tensor> quantize_pack(torch::Tensor x)
     return {packed, scales};
 }
 
+// The W4A4 linear layer (quadmul_amd/linear.py) in one call: quantise + pack the rows of x, then the
+// GEMM with the scaled output and the bias.  The packed rows, their scales and the workspace of a K split
+// share one allocation.
+torch::Tensor linear(torch::Tensor x, torch::Tensor weight, int64_t n, c10::optional<torch::Tensor> weight_scale, c10::optional<torch::Tensor> bias, bool bf16)
+{
+    const auto t = x.scalar_type();
+    TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous(), "quadmul.linear: x must be a contiguous 2-D GPU tensor");
+    TORCH_CHECK(t == torch::kFloat16 || t == torch::kBFloat16 || t == torch::kFloat32, "quadmul.linear: x must be float16, bfloat16 or float32");
+    TORCH_CHECK(weight.is_cuda() && weight.device() == x.device() && is_byte(weight) && weight.is_contiguous(),
+                "quadmul.linear: the weight must be a contiguous int8 or uint8 tensor (packed int4) on x's device");
+    const int64_t m = x.size(0), k = x.size(1);
+    TORCH_CHECK(n >= 0 && k % 2 == 0 && weight.numel() == n * (k / 2), "quadmul.linear: the weight must hold ", n, " rows of ", k, " / 2 bytes");
+    TORCH_CHECK(m <= INT32_MAX && n <= INT32_MAX && k <= INT32_MAX, "quadmul.linear: m, n, k must fit in int32");
+    check_scale(weight_scale, x, n, "weight_scale");
+    const auto out = bf16 ? torch::kBFloat16 : torch::kFloat16;
+    TORCH_CHECK(!bias.has_value() || (bias->device() == x.device() && bias->scalar_type() == out && bias->is_contiguous() && bias->numel() == n),
+                "quadmul.linear: the bias must be a contiguous vector of ", n, " elements of the output's type on x's device");
+    c10::OptionalDeviceGuard guard(x.device());
+    auto y = torch::empty({m, n}, x.options().dtype(out));
+    const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    const size_t packed_bytes = up((size_t)m * (k / 2)), scale_bytes = up((size_t)m * sizeof(float));
+    const int align = (int)std::min<uintptr_t>(256, weight.data_ptr() ? (uintptr_t)weight.data_ptr() & -(uintptr_t)weight.data_ptr() : 256);
+    const size_t ws_bytes = qm_gemm_workspace_bytes((int)m, (int)n, (int)k, align, QM_CFG_AUTO, 1);
+    auto scratch = torch::empty({(int64_t)(packed_bytes + scale_bytes + ws_bytes)}, x.options().dtype(torch::kUInt8));
+    uint8_t *const xq = scratch.data_ptr<uint8_t>();
+    float *const xs = reinterpret_cast<float *>(xq + packed_bytes);
+    const int in = t == torch::kFloat16 ? QM_IN_F16 : (t == torch::kBFloat16 ? QM_IN_BF16 : QM_IN_F32);
+    check_status(qm_quantize_pack_i4(x.data_ptr(), in, xq, xs, (int)m, (int)k, stream_of(x)), "quadmul.linear");
+    check_status(qm_gemm_i4_scaled_bias_ws(xq, weight.data_ptr(), y.data_ptr(), (int)m, (int)n, (int)k, xs,
+                                           weight_scale.has_value() ? weight_scale->data_ptr<float>() : nullptr,
+                                           bias.has_value() ? bias->data_ptr() : nullptr, bf16 ? QM_OUT_BF16 : QM_OUT_F16, stream_of(x), QM_CFG_AUTO,
+                                           ws_bytes ? xq + packed_bytes + scale_bytes : nullptr, ws_bytes),
+                 "quadmul.linear");
+    return y;
+}
+
 // Device-side unpack_int4_matrix (kernel.cu:389-408): [rows, K/2] bytes -> [rows, K] int8.
 torch::Tensor unpack(torch::Tensor packed)
 {
@@ -204,9 +242,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("gemm_scaled", &gemm_scaled, "Int4xInt4 GEMM with per-row and per-column fp32 scales, fp16 / bf16 output", py::arg("a"), py::arg("b"),
           py::arg("d"), py::arg("m"), py::arg("n"), py::arg("k"), py::arg("row_scale") = py::none(), py::arg("col_scale") = py::none());
     m.def("gemm_cfg", &gemm_cfg, "gemm with an explicit kernel configuration id (autotuning)");
-    m.def("pack", &pack, "Pack a [rows, K] int8 tensor of int4 values into [rows, K/2] bytes on the GPU");
-    m.def("quantize_pack", &quantize_pack, "Per-row symmetric int4 quantisation of a [rows, K] float tensor, packed; returns (packed, scales)");
-    m.def("unpack", &unpack, "Unpack [rows, K/2] bytes into a [rows, K] int8 tensor on the GPU");
+    // (the launches of these may wait for room in the stream's queue: without the interpreter's lock)
+    using nogil = py::call_guard<py::gil_scoped_release>;
+    m.def("linear", &linear, "W4A4 linear layer: quantise + pack the rows of x, GEMM with scaled 16-bit float output, bias", py::arg("x"), py::arg("weight"),
+          py::arg("out_features"), py::arg("weight_scale"), py::arg("bias"), py::arg("bf16"), nogil());
+    m.def("pack", &pack, nogil(), "Pack a [rows, K] int8 tensor of int4 values into [rows, K/2] bytes on the GPU");
+    m.def("quantize_pack", &quantize_pack, nogil(), "Per-row symmetric int4 quantisation of a [rows, K] float tensor, packed; returns (packed, scales)");
+    m.def("unpack", &unpack, nogil(), "Unpack [rows, K/2] bytes into a [rows, K] int8 tensor on the GPU");
     m.def("num_configs", &qm_num_configs);
     m.def("config_name", [](int cfg) { const char *s = qm_config_name(cfg); return std::string(s ? s : ""); });
     m.def("select_config", &qm_select_config);

@@ -4,7 +4,7 @@
     y[t, n] = round16((sum_k xq[t, k] * wq[n, k]) * x_scale[t] * w_scale[n]) (+ bias[n])
 
 with ``xq, x_scale = quantize_pack(x)`` (per-token symmetric int4, scale = amax / 7) and
-``wq, w_scale`` the same quantisation of the weight rows, done once.  Two launches per
+``wq, w_scale`` the same quantisation of the weight rows, done once.  Two launches out of one native
 call: quantise + pack the activations, and the GEMM with the dequantising epilogue, which adds
 the bias too; the int32 product never reaches memory.
 """
@@ -15,12 +15,12 @@ from typing import Optional
 import torch
 from torch.autograd import forward_ad
 
-from . import QuadmulError, gemm_scaled, quantize_pack
+from . import QuadmulError, _native, quantize_pack
 
 
-def _fusable(bias: Optional[torch.Tensor], y: torch.Tensor, n: int) -> bool:
-    return (bias is not None and type(bias) in (torch.Tensor, torch.nn.Parameter) and not bias.requires_grad
-            and bias.dtype == y.dtype and bias.device == y.device and bias.shape == (n,) and bias.is_contiguous()
+def _fusable(bias: torch.Tensor, x: torch.Tensor, out_dtype: torch.dtype, n: int) -> bool:
+    return (type(bias) in (torch.Tensor, torch.nn.Parameter) and not bias.requires_grad
+            and bias.dtype == out_dtype and bias.device == x.device and bias.shape == (n,) and bias.is_contiguous()
             and forward_ad._current_level < 0)
 
 
@@ -57,24 +57,24 @@ class W4A4Linear(torch.nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if x.shape[-1] != self.in_features:
             raise QuadmulError(f"W4A4Linear: last dimension of x must be {self.in_features}")
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, self.in_features)
+        flat = x.dim() == 2 and self.in_features > 0
+        x2 = x if flat else x.reshape(-1, self.in_features)
         if not x2.is_contiguous():
             x2 = x2.contiguous()
-        m = x2.shape[0]
-        y = torch.empty((m, self.out_features), dtype=self.out_dtype, device=x.device)
-        if m:
-            xq, xs = quantize_pack(x2)
+        if x2.shape[0]:
+            if self.out_dtype not in (torch.float16, torch.bfloat16):
+                raise QuadmulError("W4A4Linear: out_dtype must be float16 or bfloat16")
             bias = self.bias
             # in the GEMM's epilogue: a separate addition reads and writes all of y once more
             # (2048 x 11008: 21 us beside a GEMM of 73).  A bias that the kernel cannot take as
             # it is -- moved or cast after construction -- or that autograd follows is added apart.
-            fused = _fusable(bias, y, self.out_features)
-            gemm_scaled(xq, self.weight_packed, y, m, self.out_features, self.in_features, xs, self.weight_scale,
-                        bias=bias if fused else None)
+            fused = bias is not None and _fusable(bias, x2, self.out_dtype, self.out_features)
+            y = _native("linear", x2, self.weight_packed, self.out_features, self.weight_scale, bias if fused else None, self.out_dtype == torch.bfloat16)
             if bias is not None and not fused:
                 y += bias
-        return y.reshape(*lead, self.out_features)
+        else:
+            y = torch.empty((0, self.out_features), dtype=self.out_dtype, device=x.device)
+        return y if flat else y.reshape(*x.shape[:-1], self.out_features)
 
     def extra_repr(self) -> str:
         return f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, out_dtype={self.out_dtype}"

@@ -148,6 +148,41 @@ def test_w4a4_linear_module(oracle_mod, out_dtype):
         layer(torch.zeros((2, k + 2), dtype=torch.float16, device=DEV))
 
 
+def test_w4a4_linear_forms_taken_and_refused():
+    """The one native call behind the module: every form of input it takes gives the bits of the 2-D contiguous
+    one, what does not fit is refused before anything is launched."""
+    from quadmul_amd.linear import W4A4Linear
+
+    n, k = 96, 320
+    g = torch.Generator().manual_seed(SEED_BASE + 8700)
+    w, x = torch.randn((n, k), generator=g).half().to(DEV), torch.randn((6, k), generator=g).half().to(DEV)
+    layer = W4A4Linear.from_float(w)
+    y = layer(x)
+    xq, xs = qm.quantize_pack(x)
+    want = torch.empty((6, n), dtype=torch.float16, device=DEV)
+    qm.gemm_scaled(xq, layer.weight_packed, want, 6, n, k, xs, layer.weight_scale)
+    assert torch.equal(y, want)
+    assert torch.equal(layer(x[0]), y[0]) and torch.equal(layer(x.view(2, 3, k)), y.view(2, 3, n))
+    assert torch.equal(layer(x.t().contiguous().t()), y) and torch.equal(layer(x[::2]), y[::2])
+    assert torch.equal(layer(x.clone().requires_grad_()), y) and not layer(x.clone().requires_grad_()).requires_grad
+    assert torch.equal(layer(x.float()), y)
+    assert layer(x[:0].view(2, 0, k)).shape == (2, 0, n)
+    assert torch.equal(W4A4Linear(layer.weight_packed.view(torch.uint8), layer.weight_scale)(x), y)
+    assert torch.equal(torch.compile(layer, backend="aot_eager")(x), y)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        again = layer(x)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(again, y)
+    for bad in (x.double(), x.to(torch.int8), x.cpu()):
+        with pytest.raises(qm.QuadmulError):
+            layer(bad)
+    halved = W4A4Linear.from_float(w).half()   # the scales are no float32 any more
+    with pytest.raises(qm.QuadmulError):
+        halved(x)
+
+
 def test_linear_chain_through_dispatcher_ops_traced(oracle_mod):
     """quantize_pack and gemm_scaled as dispatcher ops: the whole linear chain stays in one
     traced graph (aot_eager: fake tensors go through the Meta implementations) and gives the
