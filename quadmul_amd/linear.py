@@ -19,7 +19,7 @@ from . import QuadmulError, _native, quantize_pack
 
 
 def _fusable(bias: torch.Tensor, x: torch.Tensor, out_dtype: torch.dtype, n: int) -> bool:
-    return (type(bias) in (torch.Tensor, torch.nn.Parameter) and not bias.requires_grad
+    return (type(bias) in (torch.Tensor, torch.nn.Parameter) and bias.layout is torch.strided and not bias.requires_grad and not bias.is_neg()
             and bias.dtype == out_dtype and bias.device == x.device and bias.shape == (n,) and bias.is_contiguous()
             and forward_ad._current_level < 0)
 

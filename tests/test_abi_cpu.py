@@ -348,3 +348,12 @@ def test_the_build_scans_for_scalar_operands_written_just_before_an_asm_load_or_
     found = scalar_operand_hazards(str(isa))
     assert [f[0] for f in found] == [4, 12], found
     assert "v_readlane_b32 s11" in found[0][1] and "v_readfirstlane_b32 s20" in found[1][1]
+
+
+def test_bias_that_the_kernel_cannot_read_as_it_is_is_added_apart():
+    from quadmul_amd.linear import _fusable
+
+    x, b = torch.zeros(2, 8, dtype=torch.float16), torch.arange(4, dtype=torch.float16)
+    assert _fusable(b, x, torch.float16, 4) and _fusable(torch.nn.Parameter(b, requires_grad=False), x, torch.float16, 4)
+    for other in (torch._neg_view(b), b.to_sparse(), b.float(), b[:3], torch.zeros(8, dtype=torch.float16)[::2], b.reshape(1, 4), torch.nn.Parameter(b)):
+        assert not _fusable(other, x, torch.float16, 4)
