@@ -85,42 +85,54 @@ __global__ void fill_zero_kernel(int32_t *dst, size_t n)
 // K is not a multiple of 32, or whose operands are not 16-byte aligned, out of a
 // caller-provided workspace.  Both operands in one launch (a second dependent launch costs
 // more than the copy of a small operand): rows 0 .. rows_a-1 are A's, the rest B's.
-// Source rows may start at any byte: one wave per row, one 32-bit word of the copy per
-// lane and turn, put together from the two aligned source words that hold its bytes
-// (consecutive lanes read consecutive words), the bytes past the end of the row zeroed.  An
-// aligned word that holds at least one byte of a matrix lies in the same page as that byte,
-// so reading it whole is safe; a word wholly past the end of the matrix is not read.
-// kb: bytes per source row; kbp4: 32-bit words per row of the copy.
+// Source rows may start at any byte: one 16-byte piece of the copy per thread, loaded at whatever address
+// it has.  Where the row ends inside a piece, the load runs on into the next row and those bytes are
+// zeroed; a piece that would run past the end of the operand is read byte by byte.  No byte outside
+// the operands is read.
+// kb: bytes per source row; ppr: 16-byte pieces per row of the copy.
+// Bound: HBM on large operands (4096 x 11008 x 4094 13.6 us, 4.6 TB/s of bytes read and written), the
+// launch on small ones.  With one wave per row and 4 bytes per lane and turn, put together from
+// two aligned words, these took (us, before -> now): 33 x 3307 x 4100 5.5 -> 3.6, 1531 x 3307 x 4100
+// 6.3 -> 5.3, 100 x 9000 x 9000 29.1 -> 14.5, 4096 x 11008 x 4094 16.6 -> 13.6.  Non-temporal loads are
+// slower (6.2, 1531 x 3307 x 4100), non-temporal stores 0.3 us faster there and 1 us slower on 100 x 9000 x 9000.
 // --------------------------------------------------------------------------
 struct PadRowsArgs {
     const uint8_t *src_a, *src_b;
-    uint32_t *dst_a, *dst_b;
-    int rows_a, rows_b, kb, kbp4;
+    v4i *dst_a, *dst_b;
+    int rows_a, rows_b, kb, ppr;
 };
 
 __global__ void __launch_bounds__(256) pad_rows_kernel(const PadRowsArgs q)
 {
-    const int lane = threadIdx.x & 63;
-    for (int r = blockIdx.x * 4 + (threadIdx.x >> 6); r < q.rows_a + q.rows_b; r += gridDim.x * 4) {
-        const bool is_a = r < q.rows_a;
-        const uint8_t *src = is_a ? q.src_a : q.src_b;
-        const int row = is_a ? r : r - q.rows_a;
-        const uintptr_t end = (uintptr_t)src + (size_t)(is_a ? q.rows_a : q.rows_b) * q.kb;
-        const uintptr_t at = (uintptr_t)src + (size_t)row * q.kb;
-        const uint32_t *w = reinterpret_cast<const uint32_t *>(at & ~(uintptr_t)3);
-        const uint32_t shift = (uint32_t)(at & 3);
-        uint32_t *out = (is_a ? q.dst_a : q.dst_b) + (size_t)row * q.kbp4;
-        for (int i = lane; i < q.kbp4; i += 64) {
-            const int keep = q.kb - 4 * i;  // bytes of the row from this word on
-            uint32_t v = 0;
-            if (keep > 0) {
-                const uint32_t x0 = w[i];
-                const uint32_t x1 = (uintptr_t)(w + i + 1) < end ? w[i + 1] : 0u;
-                v = __builtin_amdgcn_alignbyte(x1, x0, shift) & (keep >= 4 ? 0xffffffffu : (1u << (8 * keep)) - 1u);
+    const uint32_t piece = blockIdx.x * 256u + threadIdx.x;  // (below 2^28: either copy is below 2 GiB)
+    const uint32_t r = piece / (uint32_t)q.ppr;
+    if (r >= (uint32_t)(q.rows_a + q.rows_b)) return;
+    const int at = 16 * (int)(piece - r * (uint32_t)q.ppr);
+    const bool is_a = r < (uint32_t)q.rows_a;
+    const int row = is_a ? (int)r : (int)r - q.rows_a, rows = is_a ? q.rows_a : q.rows_b;
+    const uint8_t *src = (is_a ? q.src_a : q.src_b) + (size_t)row * q.kb + at;
+    v4i *out = (is_a ? q.dst_a : q.dst_b) + (size_t)row * q.ppr + (at >> 4);
+    const int keep = q.kb - at;  // bytes of the row from this piece on
+    v4i v{0, 0, 0, 0};
+    if (keep > 0) {
+        if ((long long)(rows - row) * q.kb - at >= 16) {
+            v = *reinterpret_cast<const v4i_any_aligned *>(src);
+        } else {
+            uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 15; ++e)  // (fewer than 16 are left)
+                if (e < keep) w[e >> 2] |= (uint32_t)src[e] << (8 * (e & 3));
+            v = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+        }
+        if (keep < 16) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int b = min(max(keep - 4 * e, 0), 4);
+                v[e] = b >= 4 ? v[e] : (int)((uint32_t)v[e] & ((1u << (8 * b)) - 1u));
             }
-            out[i] = v;
         }
     }
+    *out = v;
 }
 
 // --------------------------------------------------------------------------

@@ -192,9 +192,9 @@ static PadPlan plan_padded_k(int m, int n, int k, int ptr_align, const Choice &d
 static hipError_t launch_padded(GemmArgs &p, const PadPlan &pl, void *ws, hipStream_t s)
 {
     uint8_t *a_p = static_cast<uint8_t *>(ws), *b_p = a_p + pl.a_bytes;
-    const PadRowsArgs q{p.A, p.B, reinterpret_cast<uint32_t *>(a_p), reinterpret_cast<uint32_t *>(b_p), p.M, p.N, p.K / 2, pl.kp / 8};
-    const long long rows = (long long)p.M + p.N;
-    pad_rows_kernel<<<dim3((unsigned)std::min<long long>((rows + 3) / 4, 256 * 32)), dim3(256), 0, s>>>(q);
+    const PadRowsArgs q{p.A, p.B, reinterpret_cast<v4i *>(a_p), reinterpret_cast<v4i *>(b_p), p.M, p.N, p.K / 2, pl.kp / 32};
+    const long long pieces = ((long long)p.M + p.N) * q.ppr;
+    pad_rows_kernel<<<dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, s>>>(q);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     p.A = a_p;
