@@ -209,13 +209,19 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
     // (readfirstlane: the quotients are computed on the vector ALU; everything derived from
     // them is wave-uniform and belongs in scalar registers)
     //
-    // When C takes plain 16-byte stores and K is not split, a tile's write-out is folded into
-    // its last K-step.  The items are then numbered in two ranges: [0, nwhole) the tiles that
+    // When K is not split, a tile's write-out is folded into its last K-step.  The items are then numbered in two ranges: [0, nwhole) the tiles that
     // lie wholly inside the matrix, [nwhole, nitems) the ragged right column and bottom row of
     // tiles, whose stores are under the condition that their rows and columns exist.  A
     // workgroup's items ascend, so it runs its whole tiles first.  Otherwise (nwhole is 0: K
-    // split, odd N, unaligned C) every item is written out by the guarded code after its last
-    // K-step.
+    // split, fewer than BN columns of unaligned rows) every item is written out by the guarded
+    // code after its last K-step.
+    //
+    // Rows of C that are not 16-byte aligned (N % 4 != 0, or C itself) take the same stores -- the
+    // device has them at any alignment -- except that no lane's four columns may lie across the
+    // end of a row: the right column of tiles is moved left to end where C does, and the columns
+    // it shares with its neighbour are written by both, with the same values.  us,
+    // against writing every tile of such a C after its last K-step: 1531 x 3307 x 4224 33.8 -> 30.0 (3308
+    // columns: 29.8); calls with N % 4 == 0 and an aligned C run the code that they ran.
     const int ldc = c_stride(p);  // row stride of C in elements (N, unless this call computes a block of columns of a wider C)
     const bool vec_ok = (ldc & 3) == 0 && ((uintptr_t)p.C & (4 * ESZ - 1)) == 0;  // 4 elements per store
     // (The bias of a 16-bit output waits in registers for that; a configuration with no room for it
@@ -223,7 +229,8 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
     // that has one through the guarded code.)
     constexpr int NBIAS = Cfg::XPOSE ? FN / 4 : Cfg::XHALF ? FN / 2 : FN;  // column quartets of a lane
     constexpr bool BIAS_REGS = OUT != OUT_I32 && NBIAS <= 4;
-    const bool plain_c = vec_ok && ksplit == 1 && ldc < (1 << 21) && (OUT == OUT_I32 || BIAS_REGS || p.bias == nullptr);
+    const int last_n0 = vec_ok ? p.N : p.N - BN;  // no tile begins further right
+    const bool plain_c = last_n0 >= 0 && ksplit == 1 && ldc < (1 << 21) && (OUT == OUT_I32 || BIAS_REGS || p.bias == nullptr);
     const int full_m = p.M / BM, full_n = p.N / BN;
     const int nwhole = __builtin_amdgcn_readfirstlane(plain_c ? full_m * full_n : 0);
     auto locate = [&](const int item, int &m0, int &n0, int &kt0, int &KT) __attribute__((always_inline)) {
@@ -256,6 +263,7 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
         const int tm_b = r1 > r0 ? r0 : full_m, tn_b = r1 > r0 ? full_n : q - r0;
         m0 = (ragged ? tm_b : tm_a) * BM;
         n0 = (ragged ? tn_b : tn_a) * BN;
+        if (plain_c) n0 = min(n0, last_n0);
         kt0 = __builtin_amdgcn_readfirstlane(min(ks * kps, kt_all - 1));
         KT = __builtin_amdgcn_readfirstlane(max(min(kps, kt_all - ks * kps), 1));
     };
@@ -539,7 +547,7 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
     // (with branches between the MFMA slots the register allocator spills), and the address
     // stays base register + 32-bit lane offset.  rows_left / cols_left are what the matrix has
     // from this lane's first row and column of the tile on, in the order the stores below use
-    // (set per item; N % 4 == 0, so a lane's four columns are inside or outside together).
+    // (set per item; a lane's four columns are inside or outside together).
     // A store whose lanes are all off may or may not count as issued, so the last K-step of
     // such a tile allows for none of its stores in its wait.  Whole tiles keep their plain
     // stores (the conditions cost ten instructions a store: 1 to 10 % on whole-tile shapes
@@ -584,10 +592,10 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
                 v4i v = xr[k];
                 v.x >>= 8; v.y >>= 8; v.z >>= 8; v.w >>= 8;
                 if constexpr (edge) store_lanes(at, lane_row, v, std::integral_constant<int, ib * 16 + 4 * k>{}, std::integral_constant<int, grp * 64>{});
-                else *reinterpret_cast<v4i *>(at + lane_row) = v;
+                else *reinterpret_cast<v4i_elem_aligned *>(at + lane_row) = v;
             } else {
                 if constexpr (edge) store_lanes(at, lane_row, with_bias(pack16(xr[k]), bias_reg[grp]), std::integral_constant<int, ib * 16 + 4 * k>{}, std::integral_constant<int, grp * 64>{});
-                else *reinterpret_cast<v2i *>(at + lane_row) = with_bias(pack16(xr[k]), bias_reg[grp]);
+                else *reinterpret_cast<v2i_half_aligned *>(at + lane_row) = with_bias(pack16(xr[k]), bias_reg[grp]);
             }
         };
         if constexpr (t < 4) {
@@ -623,10 +631,10 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
             v4i v = xr[k];
             v.x >>= 8; v.y >>= 8; v.z >>= 8; v.w >>= 8;
             if constexpr (edge) store_lanes(at, lane_half, v, std::integral_constant<int, ib * 16 + 8 * k>{}, std::integral_constant<int, h * 32>{});
-            else *reinterpret_cast<v4i *>(at + lane_half) = v;
+            else *reinterpret_cast<v4i_elem_aligned *>(at + lane_half) = v;
         } else {
             if constexpr (edge) store_lanes(at, lane_half, with_bias(pack16(xr[k]), bias_reg[h]), std::integral_constant<int, ib * 16 + 8 * k>{}, std::integral_constant<int, h * 32>{});
-            else *reinterpret_cast<v2i *>(at + lane_half) = with_bias(pack16(xr[k]), bias_reg[h]);
+            else *reinterpret_cast<v2i_half_aligned *>(at + lane_half) = with_bias(pack16(xr[k]), bias_reg[h]);
         }
     };
     auto write_half = [&](auto ib_, auto h_, auto t_, auto edge_) __attribute__((always_inline)) {
@@ -661,8 +669,8 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
                 if constexpr (OUT == OUT_I32) store_lanes(at, lane_blk, xr[0], std::integral_constant<int, ib * 16>{}, std::integral_constant<int, j * 16>{});
                 else store_lanes(at, lane_blk, pack_block(xr[0], j_), std::integral_constant<int, ib * 16>{}, std::integral_constant<int, j * 16>{});
             } else {
-                if constexpr (OUT == OUT_I32) *reinterpret_cast<v4i *>(at + lane_blk) = xr[0];
-                else *reinterpret_cast<v2i *>(at + lane_blk) = pack_block(xr[0], j_);
+                if constexpr (OUT == OUT_I32) *reinterpret_cast<v4i_elem_aligned *>(at + lane_blk) = xr[0];
+                else *reinterpret_cast<v2i_half_aligned *>(at + lane_blk) = pack_block(xr[0], j_);
             }
         }
     };
@@ -673,7 +681,7 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
         else if constexpr (Cfg::XHALF) write_half(ib_, std::integral_constant<int, s / 4>{}, std::integral_constant<int, s % 4>{}, edge_);
         else write_block(ib_, std::integral_constant<int, s / 2>{}, std::integral_constant<int, s % 2>{}, edge_);
     };
-    // Any tile: guarded stores (ragged edges, odd N or unaligned C, K-split partial sums)
+    // Any tile: guarded stores (K-split partial sums, few columns of unaligned rows)
     auto write_guarded = [&](auto ib_, auto j_) __attribute__((always_inline)) {
         constexpr int ib = decltype(ib_)::value, j = decltype(j_)::value;
         const v4i v = take_block(ib_, j_);
@@ -863,8 +871,7 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
     auto run_item = [&](auto mode_) __attribute__((always_inline)) {
         // mode 1: a whole tile, written out with plain stores inside its last K-step; 2: a tile
         // that sticks out of C, the same with every store under its lanes' conditions;
-        // 0: guarded stores after the last K-step (K split, or a C that does not take plain
-        // 16-byte stores)
+        // 0: guarded stores after the last K-step (K split, or few columns of unaligned rows)
         constexpr int mode = decltype(mode_)::value;
         constexpr bool whole = mode != 0, edge = mode == 2;
         locate(c_item, c_m0, c_n0, c_kt0, c_KT);

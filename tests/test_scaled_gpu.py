@@ -291,6 +291,51 @@ def test_tiles_that_stick_out_of_c_on_every_pipelined_configuration(oracle_mod, 
     assert ran >= 8
 
 
+# N % 4 = 1, 2, 3, and N % 4 == 0 with C itself off; N a multiple of no tile, one column more than one, less than one
+UNALIGNED_C = [((700, 1301, 512), 0), ((512, 1026, 384), 0), ((1290, 519, 256 + 32), 3), ((300, 4097, 1024), 1), ((257, 130, 640), 0), ((520, 65, 256), 0),
+               ((200, 63, 384), 0), ((512, 512, 384), 1)]
+
+
+@pytest.mark.parametrize("shape,off", UNALIGNED_C, ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else f"off{s}")
+def test_unaligned_rows_of_c_on_every_pipelined_configuration(oracle_mod, shape, off):
+    """The right column of tiles moved left to end where C does, int32 and both 16-bit outputs, these with and
+    without a bias, against the oracle; and the memory around the output stays as it was."""
+    m, n, k = shape
+    a, b = make_operands(m, n, k, SEED_BASE + 8600 + m + n)
+    ap, bp = pack_cpu(a), pack_cpu(b)
+    rs, cs = make_scales(m, n, SEED_BASE + 8700 + m)
+    c = oracle_mod.gemm_i4(ap.numpy(), bp.numpy())
+    a_d, b_d, rs_d, cs_d = ap.to(DEV), bp.to(DEV), rs.to(DEV), cs.to(DEV)
+    pad = 4096
+    ran = 0
+    for cfg, name in enumerate(qm.config_names()):
+        if not name.startswith("q") or not qm.config_supports(cfg, m, n, k):
+            continue
+        for gm, spread in [(4, 0), (2, 1)]:
+            code = cfg | (gm << 16) | (spread << 30)
+            buf = torch.full((m * n + 2 * pad,), 0x7F7F7F7F, dtype=torch.int32, device=DEV)
+            at = pad + off
+            qm.gemm_cfg(a_d, b_d, buf[at:at + m * n].view(m, n), m, n, k, code)
+            torch.cuda.synchronize()
+            bad = oracle_mod.compare(buf[at:at + m * n].view(m, n).cpu().numpy(), c)
+            assert bad == -1, f"{name} group_m={gm} spread={spread}: first mismatch at row {bad // n}, column {bad % n}"
+            assert (buf[:at] == 0x7F7F7F7F).all() and (buf[at + m * n:] == 0x7F7F7F7F).all(), name
+            if not qm.config_has_scaled(cfg):
+                continue
+            for dtype, out in DTYPES:
+                want = torch.from_numpy(oracle_mod.scale_round16(c, rs.numpy(), cs.numpy(), out).view(np.int16)).view(dtype)
+                bias = torch.randn(n, generator=torch.Generator().manual_seed(SEED_BASE + n)).to(dtype)
+                for bias_d, w in ((None, want), (bias.to(DEV), want + bias)):
+                    buf16 = torch.full((m * n + 2 * pad,), float("nan"), dtype=dtype, device=DEV)
+                    d_d = buf16[at:at + m * n].view(m, n)
+                    qm.gemm_scaled(a_d, b_d, d_d, m, n, k, rs_d, cs_d, code, bias=bias_d)
+                    torch.cuda.synchronize()
+                    assert torch.equal(d_d.cpu().view(torch.int16), w.view(torch.int16)), f"{name} {dtype} group_m={gm} spread={spread} bias={bias_d is not None}"
+                    assert torch.isnan(buf16[:at]).all() and torch.isnan(buf16[at + m * n:]).all(), name
+        ran += 1
+    assert ran >= 8
+
+
 # every epilogue: the dot, wave-level and persistent kernels (1 to 64 rows), the generic kernel (K % 32,
 # and too small to pad), zero-padded copies, each tile through its own way of writing whole tiles,
 # tiles that stick out of C, odd N, a short last K-step, a K split added up out of a workspace, k = 0
