@@ -26,8 +26,8 @@ much a partly filled last round costs (1: as much as a full one -- one workgroup
 towards 0: in proportion -- several small workgroups per CU, where the ones left speed up);
 ``busy_us`` is what a K-step slows down by as the device fills up (shared L2s, fabric and
 power); ``odd_us`` is added per round when N % 4 != 0 (rows of C that are not 16-byte aligned:
-the pipelined kernel then writes every tile after its last K-step, none of it folded into
-that step); ``ragged_us`` per round of tiles that stick out of C (they are written through
+in the committed timings the pipelined kernel writes every tile of such a C after its last
+K-step, none of it folded into that step); ``ragged_us`` per round of tiles that stick out of C (they are written through
 guarded stores after the last K-step); ``reread_us`` per megabyte of B that the second and
 later blocks of rows of the wave-level kernel read again after the L2s have lost it;
 ``skew_us`` is what a K-step costs more when the rows of A and B are not whole 128-byte
