@@ -48,6 +48,15 @@ inline hipError_t ensure_dynamic_lds(KernelPtr kernel, int bytes, std::atomic<bo
     return hipSuccess;
 }
 
+// Bytes of a kernel's argument buffer, for kernels whose arguments must fit in the preloaded SGPRs.
+template <class... Args>
+constexpr size_t kernarg_bytes(void (*)(Args...))
+{
+    size_t at = 0;
+    ((at = (at + alignof(Args) - 1) / alignof(Args) * alignof(Args) + sizeof(Args)), ...);
+    return at;
+}
+
 // The address, on the current device, of the library's own scratch array (qm_scratch.hip).
 hipError_t static_scratch(void **out);
 

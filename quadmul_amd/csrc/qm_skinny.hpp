@@ -341,15 +341,15 @@ struct DotCfg {
 
 template <class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS)
-gemm_dot_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int M, const int N, const int K, const int ldc, const int out,
+gemm_dot_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int rows_out, const int N, const int K, const int ldc,
                        const float *row_scale, const float *col_scale, const uint16_t *bias)
 {
-    // (scalar arguments: preloaded into SGPRs before the first wave starts, see gemm_skinny_stream_dma_kernel)
-    GemmArgs p{A, B, C, M, N, K};
+    // (scalar arguments, 16 dwords: preloaded into SGPRs before the first wave starts, see gemm_skinny_stream_dma_kernel)
+    GemmArgs p{A, B, C, packed_rows(rows_out), N, K};
     p.row_scale = row_scale;
     p.col_scale = col_scale;
     p.bias = bias;
-    p.out = out;
+    p.out = packed_out(rows_out);
     p.ldc = ldc;
     constexpr int MR = Cfg::MR, FN = Cfg::FN, NW = Cfg::NW, U = Cfg::U;
     __shared__ int32_t red[NW][MR][FN * 16];  // every wave's sums, added up after one barrier (nothing to clear, no barrier in front of the loads)

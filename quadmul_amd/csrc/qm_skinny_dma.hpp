@@ -64,15 +64,15 @@ struct SkinnyDmaCfg {
 
 template <class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS)
-gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int M, const int N, const int K, const int ldc, const int out,
+gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int rows_out, const int N, const int K, const int ldc,
                        const float *row_scale, const float *col_scale, const uint16_t *bias)
 {
-    // (scalar arguments: preloaded into SGPRs before the first wave starts, see gemm_skinny_stream_dma_kernel)
-    GemmArgs p{A, B, C, M, N, K};
+    // (scalar arguments, 16 dwords: preloaded into SGPRs before the first wave starts, see gemm_skinny_stream_dma_kernel)
+    GemmArgs p{A, B, C, packed_rows(rows_out), N, K};
     p.row_scale = row_scale;
     p.col_scale = col_scale;
     p.bias = bias;
-    p.out = out;
+    p.out = packed_out(rows_out);
     p.ldc = ldc;
     constexpr int FM = Cfg::FM, FN = Cfg::FN, NW = Cfg::NW, D = Cfg::D, LPR = Cfg::LOADS_PER_RUN;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -82,7 +82,7 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
     const int n0 = blockIdx.x * Cfg::BN, m0 = blockIdx.y * Cfg::MAX_M;
-    const bool b_read_once = M <= Cfg::MAX_M;  // one block of rows (gridDim.y == 1, without fetching the grid's size)
+    const bool b_read_once = p.M <= Cfg::MAX_M;  // one block of rows (gridDim.y == 1, without fetching the grid's size)
     const int Kb = p.K >> 1;             // bytes per row; a multiple of 16
     const int nruns = (Kb + 127) >> 7;   // 128-byte runs per row, the last one possibly short
     // this wave's runs: wave, wave + NW, ...
@@ -300,18 +300,18 @@ struct SkinnyStreamCfg {
 // measured 1.5 % at M = 16, N = K = 4096 with B from HBM.)
 template <class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS)
-gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int M, const int N, const int K, const int ldc,
-                              const int out_and_grid, const int nblocks, const float *row_scale, const float *col_scale,  // 16 dwords up to here: all preloaded
-                              const uint16_t *bias)
+gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int grid_rows_out, const int N, const int K, const int ldc,
+                              const float *row_scale, const float *col_scale, const uint16_t *bias)  // 16 dwords: all preloaded
 {
-    // (out_and_grid: the output form in bits 0..7, the number of workgroups above.  gridDim.x
-    // is a hidden kernel argument beyond the preloaded ones: read from there it is a scalar
-    // load that every wave waits for before it can issue its first load.)
-    GemmArgs p{A, B, C, M, N, K};
+    // (grid_rows_out: the output form in bits 0..1, the rows in bits 2..7, the number of workgroups
+    // above.  gridDim.x is a hidden kernel argument beyond the preloaded ones: read from there
+    // it is a scalar load that every wave waits for before it can issue its first load.)
+    static_assert(Cfg::MAX_M < 64, "six bits for the rows");
+    GemmArgs p{A, B, C, (grid_rows_out >> 2) & 63, N, K};
     p.row_scale = row_scale;
     p.col_scale = col_scale;
     p.bias = bias;
-    p.out = out_and_grid & 0xFF;
+    p.out = grid_rows_out & 3;
     p.ldc = ldc;
     constexpr int FM = Cfg::FM, FN = Cfg::FN, NW = Cfg::NW, D = Cfg::D, R = Cfg::R, LPU = Cfg::LOADS_PER_UNIT;
     extern __shared__ __align__(16) uint8_t smem[];
@@ -371,7 +371,8 @@ gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, co
         }
     {
         // (the asm keeps the compiler from starting on the division before A's loads above)
-        int grid = out_and_grid >> 8;
+        int grid = grid_rows_out >> 8;
+        const int nblocks = (N + Cfg::BN - 1) / Cfg::BN;
         asm volatile("" : "+s"(grid));
         G = grid;
         // one block per workgroup whenever the device holds them all at once: no division then
