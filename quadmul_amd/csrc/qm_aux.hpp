@@ -210,11 +210,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const SplitReduceArg
         f.bias = q.bias;
         f.out = q.out;
         uint16_t h[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int c = sum[e];
-            h[e] = finish16(f, c, rs, n + e);
-        }
+        finish16x4(f, sum, rs, n, h);
         if ((q.N & 3) == 0 && ((uintptr_t)q.C & 7) == 0) {
             *reinterpret_cast<v2i *>(drow + n) = v2i{(int)(h[0] | ((uint32_t)h[1] << 16)), (int)(h[2] | ((uint32_t)h[3] << 16))};
         } else if (n + 3 < q.N) {

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace qm {
 
@@ -139,6 +140,36 @@ __device__ __forceinline__ uint16_t finish16(const GemmArgs &p, int c, float rs,
 {
     const uint16_t h = round16(scaled(c, rs, scale_at(p.col_scale, n, p.N)), p.out);
     return p.bias != nullptr && n < p.N ? add16(h, p.bias[n], p.out) : h;
+}
+
+// The elements (.., n .. n+3), n < N.  The scales and the biases of all four are fetched before the first
+// is used: with one element after the other, each behind its own conditions, every load is waited
+// for by itself -- four round trips to the L2 for a block, and four more for the bias.
+__device__ __forceinline__ void finish16x4(const GemmArgs &p, const v4i c, float rs, int n, uint16_t (&h)[4])
+{
+    float cs[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+    uint16_t b[4] = {0, 0, 0, 0};
+    if (p.col_scale != nullptr) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) cs[e] = p.col_scale[min(n + e, p.N - 1)];
+    }
+    if (p.bias != nullptr) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) b[e] = p.bias[min(n + e, p.N - 1)];
+    }
+    const auto finish = [&](auto out_) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int ce = c[e];
+            h[e] = round16<decltype(out_)::value>(scaled(ce, rs, cs[e]));
+        }
+        if (p.bias != nullptr) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = add16(h[e], b[e], decltype(out_)::value);
+        }
+    };
+    if (p.out == OUT_F16) finish(std::integral_constant<int, OUT_F16>{});
+    else finish(std::integral_constant<int, OUT_BF16>{});
 }
 
 // gfx950 has no int4 MFMA, so nibbles are widened to int8 -- but scaled by 16,

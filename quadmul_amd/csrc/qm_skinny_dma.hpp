@@ -243,11 +243,7 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
             uint16_t *const d = reinterpret_cast<uint16_t *>(p.C) + at;
             const float rs = scale_at(p.row_scale, m, p.M);
             uint16_t h[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int c = s[e];
-                h[e] = finish16(p, c, rs, n + e);
-            }
+            finish16x4(p, s, rs, n, h);
             if (vec_ok) {
                 *reinterpret_cast<v2i *>(d) = v2i{(int)(h[0] | ((uint32_t)h[1] << 16)), (int)(h[2] | ((uint32_t)h[3] << 16))};
             } else if (n + 3 < p.N) {
@@ -497,11 +493,7 @@ gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, co
                 uint16_t *const d = reinterpret_cast<uint16_t *>(p.C) + at;
                 const float rs = scale_at(p.row_scale, m, p.M);
                 uint16_t h[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int c = s[e];
-                    h[e] = finish16(p, c, rs, n + e);
-                }
+                finish16x4(p, s, rs, n, h);
                 if (vec_ok) {
                     *reinterpret_cast<v2i *>(d) = v2i{(int)(h[0] | ((uint32_t)h[1] << 16)), (int)(h[2] | ((uint32_t)h[3] << 16))};
                 } else if (n + 3 < p.N) {

@@ -338,9 +338,10 @@ def test_unaligned_rows_of_c_on_every_pipelined_configuration(oracle_mod, shape,
 
 # every epilogue: the dot, wave-level and persistent kernels (1 to 64 rows), the generic kernel (K % 32,
 # and too small to pad), zero-padded copies, each tile through its own way of writing whole tiles,
-# tiles that stick out of C, odd N, a short last K-step, a K split added up out of a workspace, k = 0
+# tiles that stick out of C, odd N, a short last K-step, a K split added up out of a workspace, k = 0,
+# several blocks of columns per workgroup of the persistent kernel with the last one cut short
 BIAS_SHAPES = [(1, 33, 256), (2, 64, 4096), (9, 130, 8192), (40, 96, 1152), (70, 33, 162), (2048, 520, 130), (256, 512, 256), (520, 780, 384),
-               (300, 1021, 416), (257, 258, 640), (6, 10, 0)]
+               (300, 1021, 416), (257, 258, 640), (6, 10, 0), (5, 8263, 384)]
 
 
 @pytest.mark.parametrize("shape", BIAS_SHAPES, ids=lambda s: "x".join(map(str, s)))
