@@ -227,14 +227,31 @@ static hipError_t launch_ragged(const GemmArgs &p, hipStream_t s)
 
 // With a workspace a large product can also run on zero-padded copies of A and B on the
 // aligned kernels.  The copies cost a launch and 2 x (M + N) K / 2 bytes whatever M is; the kernel
-// here costs more with every block of rows.  us, here / on copies: 3 x 9000 x 9000 12 / 38, 17 x 5001
-// x 2050 8.7 / 10.5, 17 x 3307 x 4100 10.0 / 12.1, 64 x 9000 x 9000 34 / 46, 64 x 8191 x 1030 8.3 / 10.3;
-// 33 x 3307 x 4100 16.1 / 12.4, 33 x 700 x 8998 18.1 / 15.3, 100 x 9000 x 9000 50 / 53, 100 x 5001 x 2050
-// 18.5 / 13.8, 200 x 8191 x 1030 19.8 / 15.1.  A small product on a short K is over before the copies
-// are: 200 x 1001 x 1002 4.3 / 9.8, 500 x 1001 x 1002 5.7 / 9.8.
-static bool ragged_before_copies(int m, int n, int k)
+// here costs more with every block of rows, and by how the rows lie:
+//   - on multiples of four bytes its loads are whole (us, here / on copies: 64 x 9000 x 9000 18.5 / 32,
+//     100 x 9000 x 9000 29 / 38, 300 x 5001 x 2056 15.2 / 19.5, 400 x 8191 x 1032 19.8 / 16.1, 64 x 28672 x 8200 49 / 77,
+//     129 x 28672 x 8200 99 / 90, 200 x 8192 x 28672 122 / 100), whatever K is up to 64 rows;
+//   - else every 16 bytes of a lane are split: 16 x 6001 x 4100 11.8 / 11.9, 32 x 6000 x 3002 8.4 / 11.4, 32 x 1000 x 6002
+//     11.6 / 7.5, 32 x 28672 x 8194 116 / 70, 48 x 8191 x 1030 7.4 / 8.8, 512 x 1001 x 1002 6.1 / 6.9, 512 x 8191 x 1030
+//     36 / 17;
+//   - and a few bytes off a multiple of 1024 from row to row the pieces of a block's rows meet
+//     in the same sets of the L1: 16 x 9000 x 2050 13.5 / 11.3, 32 x 5001 x 2050 10.2 / 9.3, 32 x 4100 x 4098
+//     17.1 / 11.0, 48 x 1500 x 2046 7.3 / 6.4.
+// One or two rows never take the copies, which are as large as the weights and at most a
+// fifth faster there (1 x 28672 x 8194 61 / 60, 1 x 11008 x 14338 53 / 44, 1 x 65536 x 4100 55 / 71).  A K of one or
+// two steps is mostly write-out: 160 x 5000 x 130 5.0 / 6.5, 300 x 5000 x 130 8.3 / 7.7.  Over 1088 products of
+// 1500 rows, this rule is 0.6 % behind the better of the two in the mean; one that took no account
+// of how the rows lie was 8 % behind.
+static bool ragged_before_copies(int m, int n, int k, int ptr_align)
 {
-    return m <= 32 || (m <= 64 && n >= 6000) || (k <= 2048 && (long long)m * n * k < (1LL << 29));
+    const long long outs = (long long)m * n;
+    if (m <= 2) return true;
+    if (k < 256) return outs <= (5 << 18);
+    const int kb = k / 2, off = kb & 1023;
+    if (kb % 4 == 0 && ptr_align >= 4) return m <= 64 || (m <= 512 && outs <= (k <= 10240 ? 3 << 20 : 1 << 20));
+    const bool near_1024 = off != 0 && (off < 8 || off >= 1016);
+    if (m <= (near_1024 ? 16 : 32) && (k <= 4224 || off == 0)) return true;
+    return k <= 2176 && outs * k < (near_1024 ? 1LL << 27 : 1LL << 29);
 }
 
 // The largest block that leaves more than half of the 256 CUs a workgroup of their own: it reads
@@ -413,7 +430,7 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
         ch.ksplit = 1;
     }
     const bool ragged = cfg == QM_CFG_AUTO && g_configs[ch.cfg].kind == KIND_GENERIC && ragged_fits(m, n, k);
-    if (cfg == QM_CFG_AUTO && has_ws && !(ragged && ragged_before_copies(m, n, k))) {
+    if (cfg == QM_CFG_AUTO && has_ws && !(ragged && ragged_before_copies(m, n, k, align))) {
         PadPlan pl = plan_padded_k(m, n, k, align, ch);
         if (pl.on && !launcher(pl.ch.cfg)) {
             // a pipelined configuration that has the scaled output, if the shape is one for those
