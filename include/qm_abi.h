@@ -127,7 +127,8 @@ int qm_config_has_scaled(int cfg); /* 1 / 0 */
  * cfg as for qm_gemm_i4_cfg (QM_CFG_AUTO included); with a workspace the scaled form also
  * takes K splits, on every "q" configuration.
  * qm_gemm_workspace_bytes: what the call with these arguments uses at most (0 when it
- * needs none); scaled = 1 for the scaled form.
+ * needs none, which includes calls that run on the kernel for operands at any address);
+ * ptr_align is the smallest alignment in bytes shared by A and B; scaled = 1 for the scaled form.
  */
 int qm_gemm_i4_ws(const void *A, const void *B, void *C, int m, int n, int k, void *stream, int cfg,
                   void *workspace, size_t workspace_bytes);

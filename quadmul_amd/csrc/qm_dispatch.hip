@@ -160,53 +160,6 @@ static bool workspace_fits(const ConfigDesc &d, int m, int n, int ksplit, const 
     return ws != nullptr && ((uintptr_t)ws & 15) == 0 && ws_bytes >= split_workspace_bytes(d, m, n, ksplit);
 }
 
-// Automatic choice only: K padded to a multiple of 128 (operands copied into the workspace) so
-// that the pipelined kernel can run instead of the generic one.  Worth it when the shape is
-// large -- the copy is (M + N) K / 2 bytes twice over.  `direct` is the choice without padding.
-struct PadPlan {
-    bool on = false;
-    int kp = 0;
-    Choice ch{};
-    size_t a_bytes = 0, b_bytes = 0;
-    size_t bytes() const { return a_bytes + b_bytes; }
-};
-
-static PadPlan plan_padded_k(int m, int n, int k, int ptr_align, const Choice &direct)
-{
-    PadPlan pl;
-    const int kind = g_configs[direct.cfg].kind;
-    if (kind == KIND_TILE16 || kind == KIND_SKINNY) return pl;
-    const int kp = (k + 127) / 128 * 128;
-    if (kp > QM_MAX_K_X16 || !fast_path_ok(m, n, kp, 256)) return pl;
-    const long long outs = (long long)m * n;
-    if (outs * kp < (1LL << 27)) return pl;  // (kp: a K below one K-step counts as the step it is padded to)
-    (void)ptr_align;
-    Choice ch = heuristic(m, n, kp, 256, false);
-    if (g_configs[ch.cfg].kind == KIND_GENERIC) return pl;
-    ch.ksplit = 1;
-    pl.on = true;
-    pl.kp = kp;
-    pl.ch = ch;
-    pl.a_bytes = ((size_t)m * (kp / 2) + 255) / 256 * 256;
-    pl.b_bytes = ((size_t)n * (kp / 2) + 255) / 256 * 256;
-    return pl;
-}
-
-// The padded copies of A and B in the workspace, and the arguments of the GEMM on them.
-static hipError_t launch_padded(GemmArgs &p, const PadPlan &pl, void *ws, hipStream_t s)
-{
-    uint8_t *a_p = static_cast<uint8_t *>(ws), *b_p = a_p + pl.a_bytes;
-    const PadRowsArgs q{p.A, p.B, reinterpret_cast<v4i *>(a_p), reinterpret_cast<v4i *>(b_p), p.M, p.N, p.K / 2, pl.kp / 32};
-    const long long pieces = ((long long)p.M + p.N) * q.ppr;
-    pad_rows_kernel<<<dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, s>>>(q);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    p.A = a_p;
-    p.B = b_p;
-    p.K = pl.kp;
-    return hipSuccess;
-}
-
 // The automatic choice where none of the aligned kernels takes the operands (the "generic"
 // configuration: K % 32 != 0, or A or B not 16-byte aligned): the matrix-core kernel of
 // qm_ragged.hpp if K and the operands' sizes are within what it addresses -- else, as for an
@@ -215,14 +168,6 @@ static bool ragged_fits(int m, int n, int k)
 {
     const long long kb = k / 2;
     return k >= 32 && k <= QM_MAX_K_X16 && (long long)m * kb < 0x7fffffffLL && (long long)n * kb < 0x7fffffffLL && (m + 15) / 16 <= 65535;
-}
-
-template <class Cfg>
-static hipError_t launch_ragged(const GemmArgs &p, hipStream_t s)
-{
-    const dim3 grid((p.N + Cfg::BN - 1) / Cfg::BN, (p.M + Cfg::MAX_M - 1) / Cfg::MAX_M);
-    gemm_ragged_kernel<Cfg><<<grid, dim3(Cfg::THREADS), 0, s>>>(p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out, p.row_scale, p.col_scale, p.bias);
-    return hipGetLastError();
 }
 
 // With a workspace a large product can also run on zero-padded copies of A and B on the
@@ -252,6 +197,64 @@ static bool ragged_before_copies(int m, int n, int k, int ptr_align)
     const bool near_1024 = off != 0 && (off < 8 || off >= 1016);
     if (m <= (near_1024 ? 16 : 32) && (k <= 4224 || off == 0)) return true;
     return k <= 2176 && outs * k < (near_1024 ? 1LL << 27 : 1LL << 29);
+}
+
+// Automatic choice only: K padded to a multiple of 128 (operands copied into the workspace) so
+// that the pipelined kernel can run instead of the generic one.  Worth it when the shape is
+// large -- the copy is (M + N) K / 2 bytes twice over -- and the kernel for operands at any
+// address is not the faster one.  `direct` is the choice without padding.  The size of the
+// workspace (qm_gemm_workspace_bytes) and the launch (run_gemm) both come from this plan: a
+// call is never asked for memory that it then leaves alone.
+struct PadPlan {
+    bool on = false;
+    int kp = 0;
+    Choice ch{};
+    size_t a_bytes = 0, b_bytes = 0;
+    size_t bytes() const { return a_bytes + b_bytes; }
+};
+
+static PadPlan plan_padded_k(int m, int n, int k, int ptr_align, const Choice &direct)
+{
+    PadPlan pl;
+    const int kind = g_configs[direct.cfg].kind;
+    if (kind == KIND_TILE16 || kind == KIND_SKINNY) return pl;
+    if (ragged_fits(m, n, k) && ragged_before_copies(m, n, k, ptr_align)) return pl;
+    const int kp = (k + 127) / 128 * 128;
+    if (kp > QM_MAX_K_X16 || !fast_path_ok(m, n, kp, 256)) return pl;
+    const long long outs = (long long)m * n;
+    if (outs * kp < (1LL << 27)) return pl;  // (kp: a K below one K-step counts as the step it is padded to)
+    Choice ch = heuristic(m, n, kp, 256, false);
+    if (g_configs[ch.cfg].kind == KIND_GENERIC) return pl;
+    ch.ksplit = 1;
+    pl.on = true;
+    pl.kp = kp;
+    pl.ch = ch;
+    pl.a_bytes = ((size_t)m * (kp / 2) + 255) / 256 * 256;
+    pl.b_bytes = ((size_t)n * (kp / 2) + 255) / 256 * 256;
+    return pl;
+}
+
+// The padded copies of A and B in the workspace, and the arguments of the GEMM on them.
+static hipError_t launch_padded(GemmArgs &p, const PadPlan &pl, void *ws, hipStream_t s)
+{
+    uint8_t *a_p = static_cast<uint8_t *>(ws), *b_p = a_p + pl.a_bytes;
+    const PadRowsArgs q{p.A, p.B, reinterpret_cast<v4i *>(a_p), reinterpret_cast<v4i *>(b_p), p.M, p.N, p.K / 2, pl.kp / 32};
+    const long long pieces = ((long long)p.M + p.N) * q.ppr;
+    pad_rows_kernel<<<dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, s>>>(q);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    p.A = a_p;
+    p.B = b_p;
+    p.K = pl.kp;
+    return hipSuccess;
+}
+
+template <class Cfg>
+static hipError_t launch_ragged(const GemmArgs &p, hipStream_t s)
+{
+    const dim3 grid((p.N + Cfg::BN - 1) / Cfg::BN, (p.M + Cfg::MAX_M - 1) / Cfg::MAX_M);
+    gemm_ragged_kernel<Cfg><<<grid, dim3(Cfg::THREADS), 0, s>>>(p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out, p.row_scale, p.col_scale, p.bias);
+    return hipGetLastError();
 }
 
 // The largest block that leaves more than half of the 256 CUs a workgroup of their own: it reads
@@ -429,8 +432,7 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
         ch = select_scaled(m, n, k, align, false);
         ch.ksplit = 1;
     }
-    const bool ragged = cfg == QM_CFG_AUTO && g_configs[ch.cfg].kind == KIND_GENERIC && ragged_fits(m, n, k);
-    if (cfg == QM_CFG_AUTO && has_ws && !(ragged && ragged_before_copies(m, n, k, align))) {
+    if (cfg == QM_CFG_AUTO && has_ws) {
         PadPlan pl = plan_padded_k(m, n, k, align, ch);
         if (pl.on && !launcher(pl.ch.cfg)) {
             // a pipelined configuration that has the scaled output, if the shape is one for those
@@ -443,7 +445,7 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
             return e == hipSuccess ? QM_OK : fail_launch(e);
         }
     }
-    if (ragged) {
+    if (cfg == QM_CFG_AUTO && g_configs[ch.cfg].kind == KIND_GENERIC && ragged_fits(m, n, k)) {
         const hipError_t e = launch_ragged(p, s);
         return e == hipSuccess ? QM_OK : fail_launch(e);
     }

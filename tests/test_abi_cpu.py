@@ -133,6 +133,25 @@ def test_workspace_sizes():
     assert qm.workspace_bytes(4096, 4096, 4162, qm.config_id("generic")) == 0   # explicit configuration: as asked
 
 
+@pytest.mark.parametrize("scaled", [False, True], ids=["int32", "scaled"])
+def test_no_workspace_for_calls_that_run_on_the_kernel_for_any_address(scaled):
+    """The size follows the choice that the launch makes: nothing is asked for where no copies are made, however
+    large they would be, and their whole size one row, one K or one byte of alignment further on."""
+    ws = lambda m, n, k, align=256: qm.workspace_bytes(m, n, k, scaled=scaled, ptr_align=align)
+    up = lambda v: (v + 255) // 256 * 256
+    copies = lambda m, n, k: up(m * ((k + 127) // 128 * 64)) + up(n * ((k + 127) // 128 * 64))
+    assert ws(1, 28672, 8194) == ws(1, 28672, 9002) == ws(2, 28672, 9002) == 0
+    assert ws(3, 28672, 9002) == copies(3, 28672, 9002) > qm.STATIC_SCRATCH_BYTES
+    # rows on multiples of four bytes: up to 64 rows, and as many more as the product has columns for
+    assert ws(64, 9000, 9000) == ws(300, 9000, 9000) == ws(32, 50000, 4104) == 0
+    assert ws(400, 9000, 9000) == copies(400, 9000, 9000) and ws(64, 9000, 9000, 2) == copies(64, 9000, 9000)
+    assert ws(300, 2000, 28672, 4) == 0 and ws(300, 8000, 28672, 4) == copies(300, 8000, 28672) and ws(300, 2000, 28672, 16) == 0
+    # rows that are not: a few bytes off a multiple of 1024 (4102 / 2 = 2051), and elsewhere (4000 / 2 - 48)
+    assert ws(16, 9000, 4102) == 0 and ws(17, 9000, 4102) == copies(17, 9000, 4102)
+    assert ws(32, 9000, 3902) == 0 and ws(33, 9000, 3902) == copies(33, 9000, 3902)
+    assert ws(117, 4732, 780) == 0 and ws(200, 6001, 780) == copies(200, 6001, 780)
+
+
 def test_version_names_the_compiler():
     v = qm.version()
     assert v.startswith("quadmul-amd") and "gfx950" in v and "HIP version" in v, v

@@ -109,3 +109,15 @@ def test_static_scratch_rejects_what_does_not_fit():
     assert b"scratch" in qm.library().qm_status_string(-7)
     with pytest.raises(qm.QuadmulError, match="scratch"):
         qm._check(-7, "qm_gemm_i4_static")
+
+
+def test_static_scratch_takes_calls_that_use_none(oracle_mod):
+    """One row against a weight whose zero-padded copy would not fit the array: the call makes no copy, so it runs."""
+    m, n, k = 1, 16390, 9002
+    a, b = make_operands(m, n, k, SEED_BASE + 7200)
+    ap, bp = pack_cpu(a), pack_cpu(b)
+    assert n * ((k + 127) // 128 * 64) > qm.STATIC_SCRATCH_BYTES
+    st, got = _static(ap.to(DEV), bp.to(DEV), m, n, k)
+    assert st == 0, qm.library().qm_status_string(st)
+    torch.cuda.synchronize()
+    assert oracle_mod.compare(got.cpu().numpy(), oracle_mod.gemm_i4(ap.numpy(), bp.numpy())) == -1
