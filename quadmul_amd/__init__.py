@@ -8,7 +8,7 @@ Two ways in, both ending in the same C ABI (``include/qm_abi.h``,
   (extension.cpp:8-29, call site test.py:40);
 * this package, which binds the C ABI with ctypes and takes torch tensors only to
   borrow their device pointers and the current stream; quantising, packing and the linear
-  layer go through the extension module, whose host side costs less per call.
+  layer go through the extension module, whose host side costs less per call, where it is there.
 
 There is no CPU or eager fallback for the GEMM: if the HIP library has not been
 built, every call raises.
@@ -111,21 +111,29 @@ def library() -> ctypes.CDLL:
     return lib
 
 
-_ext = None
+_EXT_FUNCTIONS = ("linear", "pack", "quantize_pack", "unpack")
+_ext = None  # the extension module; False: there is none, or it is not this package's
+
+
+def _extension():
+    """The extension module, or False where only the library was built (``python -m quadmul_amd.build --lib``) or
+    another module of its name is found first: the same kernels are then called through ctypes."""
+    global _ext
+    if _ext is None:
+        try:
+            import quadmul
+        except ImportError:
+            _ext = False
+        else:
+            _ext = quadmul if all(hasattr(quadmul, f) for f in _EXT_FUNCTIONS) else False
+    return _ext
 
 
 def _native(name: str, *args):
     """The extension module's function of this name.  From Python the same call costs two to three times as
     much on the host (device guard, stream, allocations, ctypes), more than a small one takes on the GPU."""
-    global _ext
-    if _ext is None:
-        try:
-            import quadmul
-        except ImportError as e:
-            raise QuadmulError(f"the extension module quadmul cannot be imported ({e}): build it with `python -m quadmul_amd.build`") from e
-        _ext = quadmul
     try:
-        return getattr(_ext, name)(*args)
+        return getattr(_extension(), name)(*args)
     except RuntimeError as e:
         if type(e) is RuntimeError:
             raise QuadmulError(str(e)) from None
@@ -236,7 +244,7 @@ def gemm_scaled(a: torch.Tensor, b: torch.Tensor, d: torch.Tensor, m: int, n: in
                                                  None if col_scale is None else col_scale.data_ptr(),
                                                  None if bias is None else bias.data_ptr(), out, _stream_ptr(a), cfg,
                                                  ws, ws_bytes)
-    _check(st, "qm_gemm_i4_scaled_ws")
+    _check(st, "qm_gemm_i4_scaled_bias_ws")
 
 
 def quantize_pack(x: torch.Tensor):
@@ -250,7 +258,16 @@ def quantize_pack(x: torch.Tensor):
         raise QuadmulError("quantize_pack: x must be float16, bfloat16 or float32")
     if x.shape[1] % 2:
         raise QuadmulError("quantize_pack: k must be even")
-    return _native("quantize_pack", x)
+    if _extension():
+        return _native("quantize_pack", x)
+    rows, k = x.shape
+    kind = {torch.float16: 1, torch.bfloat16: 2, torch.float32: 3}[x.dtype]
+    packed = torch.empty((rows, k // 2), dtype=torch.int8, device=x.device)
+    scales = torch.empty((rows,), dtype=torch.float32, device=x.device)
+    with torch.cuda.device(x.device):
+        st = library().qm_quantize_pack_i4(x.data_ptr(), kind, packed.data_ptr(), scales.data_ptr(), rows, k, _stream_ptr(x))
+    _check(st, "qm_quantize_pack_i4")
+    return packed, scales
 
 
 def config_has_scaled(cfg: int) -> bool:
@@ -294,8 +311,14 @@ def pack_int4(values: torch.Tensor) -> torch.Tensor:
     if k % 2:
         raise QuadmulError("pack_int4: K must be even")
     v = values.contiguous()
-    if v.is_cuda:
+    if v.is_cuda and _extension():
         return _native("pack", v)
+    if v.is_cuda:
+        out = torch.empty((rows, k // 2), dtype=torch.int8, device=v.device)
+        with torch.cuda.device(v.device):
+            st = library().qm_pack_i4(v.data_ptr(), out.data_ptr(), rows, k, _stream_ptr(v))
+        _check(st, "qm_pack_i4")
+        return out
     u = v.view(torch.uint8).reshape(-1)
     return ((u[0::2] & 0x0F) | ((u[1::2] & 0x0F) << 4)).reshape(rows, k // 2).view(torch.int8).contiguous()
 
@@ -307,8 +330,14 @@ def unpack_int4(packed: torch.Tensor) -> torch.Tensor:
         raise QuadmulError("unpack_int4: expects a 2-D int8/uint8 tensor")
     p = packed.contiguous()
     rows, half = p.shape
-    if p.is_cuda:
+    if p.is_cuda and _extension():
         return _native("unpack", p)
+    if p.is_cuda:
+        out = torch.empty((rows, 2 * half), dtype=torch.int8, device=p.device)
+        with torch.cuda.device(p.device):
+            st = library().qm_unpack_i4(p.data_ptr(), out.data_ptr(), rows, 2 * half, _stream_ptr(p))
+        _check(st, "qm_unpack_i4")
+        return out
     u = p.view(torch.uint8)
     lo = (u & 0x0F).to(torch.int16)
     hi = (u >> 4).to(torch.int16)

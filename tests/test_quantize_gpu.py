@@ -183,6 +183,29 @@ def test_w4a4_linear_forms_taken_and_refused():
         halved(x)
 
 
+@pytest.mark.parametrize("found", [None, "foreign"], ids=["no-module", "foreign-module"])
+def test_without_the_extension_module(monkeypatch, found):
+    """A build of the library alone, and another module of the extension's name on the path: the same kernels
+    through ctypes, the same bits."""
+    import sys
+    import types
+
+    from quadmul_amd.linear import W4A4Linear
+
+    g = torch.Generator().manual_seed(SEED_BASE + 8800)
+    w, x = torch.randn((96, 320), generator=g).half().to(DEV), torch.randn((6, 320), generator=g).half().to(DEV)
+    v = torch.randint(-8, 8, (5, 34), dtype=torch.int8, generator=g).to(DEV)
+    layers = [W4A4Linear.from_float(w, b) for b in (None, torch.randn(96, generator=g).to(DEV))]
+    calls = [lambda: qm.quantize_pack(x), lambda: (qm.pack_int4(v), qm.unpack_int4(qm.pack_int4(v))), lambda: [f(x) for f in layers]]
+    want = [t for c in calls for t in c()]
+    monkeypatch.setattr(qm, "_ext", None)
+    monkeypatch.setitem(sys.modules, "quadmul", None if found is None else types.ModuleType("quadmul"))
+    got = [t for c in calls for t in c()]
+    assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
+    with pytest.raises(qm.QuadmulError):
+        layers[0](x.double())
+
+
 def test_linear_chain_through_dispatcher_ops_traced(oracle_mod):
     """quantize_pack and gemm_scaled as dispatcher ops: the whole linear chain stays in one
     traced graph (aot_eager: fake tensors go through the Meta implementations) and gives the
