@@ -31,7 +31,7 @@ LIBDIR = os.path.join(PKG, "lib")
 OBJDIR = os.path.join(PKG, "build")
 LIB_PATH = os.path.join(LIBDIR, "libqm_hip.so")
 PROBE_PATH = os.path.join(LIBDIR, "libqm_probe.so")
-N_TILE_TUS = 14
+N_TILE_TUS = 22
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 HIP_FLAGS = [

@@ -478,6 +478,7 @@ QM_EXPORT int qm_gemm_i4_ws(const void *A, const void *B, void *C, int m, int n,
 QM_EXPORT int qm_init(void)
 {
     GemmArgs p{nullptr, nullptr, nullptr, 256, 256, 256};
+    const uint16_t no_bias = 0;
     for (int id = 0; id < g_num_configs; ++id) {
         if (g_configs[id].kind == KIND_GENERIC) continue;
         for (const int k : {256, 256 + 32}) {   // the kernel for whole K-steps and the one with a short last step
@@ -486,8 +487,11 @@ QM_EXPORT int qm_init(void)
                 const LaunchFn fn = out == OUT_I32 ? g_configs[id].launch : scaled_launcher(id);
                 if (!fn || (out != OUT_I32 && g_configs[id].kind != KIND_TILE16)) continue;
                 p.out = out;
-                const hipError_t e = fn(p, nullptr, QM_OPT_PREPARE);
-                if (e != hipSuccess) return fail_launch(e);
+                for (const uint16_t *bias : {(const uint16_t *)nullptr, &no_bias}) {   // (nothing is launched, nor read)
+                    p.bias = out == OUT_I32 ? nullptr : bias;
+                    const hipError_t e = fn(p, nullptr, QM_OPT_PREPARE);
+                    if (e != hipSuccess) return fail_launch(e);
+                }
             }
         }
     }

@@ -165,8 +165,11 @@ struct Tile16Cfg {
 };
 
 // TAIL: K % 128 may be 32, 64 or 96 (a short last K-step); the instantiation without it is
-// the same kernel with that code left out.
-template <class Cfg, int OUT = OUT_I32, bool TAIL = false>
+// the same kernel with that code left out.  BIAS: p.bias is added to the 16-bit output.  A kernel of
+// its own because it costs registers and instructions in the last K-step: as one kernel for both, adding
+// -0 where there is no bias, calls without one were slower (us, one kernel / two, scaled fp16 and bf16 output:
+// 8192 x 8192 x 8192 354 / 344 and 360 / 343, 4096 x 4096 x 4096 52.8 / 50.8 and 54.3 / 51.2).
+template <class Cfg, int OUT = OUT_I32, bool TAIL = false, bool BIAS = false>
 __global__ void __launch_bounds__(Cfg::THREADS, Cfg::OCC * Cfg::THREADS / 256)
 gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const int group_m, const int ksplit)
 {
@@ -225,12 +228,13 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
     const int ldc = c_stride(p);  // row stride of C in elements (N, unless this call computes a block of columns of a wider C)
     const bool vec_ok = (ldc & 3) == 0 && ((uintptr_t)p.C & (4 * ESZ - 1)) == 0;  // 4 elements per store
     // (The bias of a 16-bit output waits in registers for that; a configuration with no room for it
-    // -- 256 x 256 with the deepest ring: sixteen registers, one spilt -- writes the tiles of a call
-    // that has one through the guarded code.)
+    // -- 256 x 256 with the deepest ring: sixteen registers, one spilt -- writes its tiles through
+    // the guarded code.  4096 x 4096 x 4096 bf16: 83 us, 54 without a bias, 69 with a separate addition
+    // after it; no table row and no cost model picks that one.)
     constexpr int NBIAS = Cfg::XPOSE ? FN / 4 : Cfg::XHALF ? FN / 2 : FN;  // column quartets of a lane
-    constexpr bool BIAS_REGS = OUT != OUT_I32 && NBIAS <= 4;
+    constexpr bool BIAS_REGS = BIAS && NBIAS <= 4;
     const int last_n0 = vec_ok ? p.N : p.N - BN;  // no tile begins further right
-    const bool plain_c = last_n0 >= 0 && ksplit == 1 && ldc < (1 << 21) && (OUT == OUT_I32 || BIAS_REGS || p.bias == nullptr);
+    const bool plain_c = last_n0 >= 0 && ksplit == 1 && ldc < (1 << 21) && (BIAS_REGS || !BIAS);
     const int full_m = p.M / BM, full_n = p.N / BN;
     const int nwhole = __builtin_amdgcn_readfirstlane(plain_c ? full_m * full_n : 0);
     auto locate = [&](const int item, int &m0, int &n0, int &kt0, int &KT) __attribute__((always_inline)) {
@@ -496,10 +500,9 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
     float rs_reg[OUT != OUT_I32 ? FM : 1];
     v4f cs_reg[OUT != OUT_I32 ? FN : 1];
     // ... and the bias of the four columns it stores of every 64-column group (whole tiles through
-    // the LDS) or of every block, packed in the output's type.  No bias: -0, the value that
-    // changes nothing when it is added, so that the write-out has no branch.  (In registers
-    // because a load in the last K-step would drain the ring, see below.)
-    v2i bias_reg[OUT != OUT_I32 ? NBIAS : 1];
+    // the LDS) or of every block, packed in the output's type.  (In registers because a load in
+    // the last K-step would drain the ring, see below.)
+    v2i bias_reg[BIAS_REGS ? NBIAS : 1];
     v4i zero4;
     asm volatile("v_mov_b32 %0, 0" : "=v"(zero4.x));  // (opaque, so the MFMA operand is a plain register tuple)
     zero4.y = zero4.z = zero4.w = zero4.x;
@@ -529,8 +532,9 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
     auto with_bias = [&](const v2i o, const v2i b) __attribute__((always_inline)) -> v2i {
         return v2i{(int)add16_pair<OUT>((uint32_t)o.x, (uint32_t)b.x), (int)add16_pair<OUT>((uint32_t)o.y, (uint32_t)b.y)};
     };
-    auto pack_block = [&](const v4i v, auto j_) __attribute__((always_inline)) -> v2i {
-        if constexpr (BIAS_REGS) return with_bias(pack16(v), bias_reg[decltype(j_)::value]);
+    // what a whole tile stores: the bias of the lane's quartet i out of its register
+    auto finish = [&](const v4i v, auto i_) __attribute__((always_inline)) -> v2i {
+        if constexpr (BIAS_REGS) return with_bias(pack16(v), bias_reg[decltype(i_)::value]);
         else return pack16(v);
     };
     // byte offsets of this lane from the tile's corner (32 bits are enough for the rows of one
@@ -594,8 +598,8 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
                 if constexpr (edge) store_lanes(at, lane_row, v, std::integral_constant<int, ib * 16 + 4 * k>{}, std::integral_constant<int, grp * 64>{});
                 else *reinterpret_cast<v4i_elem_aligned *>(at + lane_row) = v;
             } else {
-                if constexpr (edge) store_lanes(at, lane_row, with_bias(pack16(xr[k]), bias_reg[grp]), std::integral_constant<int, ib * 16 + 4 * k>{}, std::integral_constant<int, grp * 64>{});
-                else *reinterpret_cast<v2i_half_aligned *>(at + lane_row) = with_bias(pack16(xr[k]), bias_reg[grp]);
+                if constexpr (edge) store_lanes(at, lane_row, finish(xr[k], std::integral_constant<int, grp>{}), std::integral_constant<int, ib * 16 + 4 * k>{}, std::integral_constant<int, grp * 64>{});
+                else *reinterpret_cast<v2i_half_aligned *>(at + lane_row) = finish(xr[k], std::integral_constant<int, grp>{});
             }
         };
         if constexpr (t < 4) {
@@ -633,8 +637,8 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
             if constexpr (edge) store_lanes(at, lane_half, v, std::integral_constant<int, ib * 16 + 8 * k>{}, std::integral_constant<int, h * 32>{});
             else *reinterpret_cast<v4i_elem_aligned *>(at + lane_half) = v;
         } else {
-            if constexpr (edge) store_lanes(at, lane_half, with_bias(pack16(xr[k]), bias_reg[h]), std::integral_constant<int, ib * 16 + 8 * k>{}, std::integral_constant<int, h * 32>{});
-            else *reinterpret_cast<v2i_half_aligned *>(at + lane_half) = with_bias(pack16(xr[k]), bias_reg[h]);
+            if constexpr (edge) store_lanes(at, lane_half, finish(xr[k], std::integral_constant<int, h>{}), std::integral_constant<int, ib * 16 + 8 * k>{}, std::integral_constant<int, h * 32>{});
+            else *reinterpret_cast<v2i_half_aligned *>(at + lane_half) = finish(xr[k], std::integral_constant<int, h>{});
         }
     };
     auto write_half = [&](auto ib_, auto h_, auto t_, auto edge_) __attribute__((always_inline)) {
@@ -667,10 +671,10 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
             char *const at = tile_c + ((size_t)(ib * 16) * ldc + j * 16) * ESZ;  // wave-uniform
             if constexpr (decltype(edge_)::value) {
                 if constexpr (OUT == OUT_I32) store_lanes(at, lane_blk, xr[0], std::integral_constant<int, ib * 16>{}, std::integral_constant<int, j * 16>{});
-                else store_lanes(at, lane_blk, pack_block(xr[0], j_), std::integral_constant<int, ib * 16>{}, std::integral_constant<int, j * 16>{});
+                else store_lanes(at, lane_blk, finish(xr[0], j_), std::integral_constant<int, ib * 16>{}, std::integral_constant<int, j * 16>{});
             } else {
                 if constexpr (OUT == OUT_I32) *reinterpret_cast<v4i_elem_aligned *>(at + lane_blk) = xr[0];
-                else *reinterpret_cast<v2i_half_aligned *>(at + lane_blk) = pack_block(xr[0], j_);
+                else *reinterpret_cast<v2i_half_aligned *>(at + lane_blk) = finish(xr[0], j_);
             }
         }
     };
@@ -697,9 +701,10 @@ gemm_tile16_kernel(const GemmArgs p, const int tiles_m, const int tiles_n, const
         if constexpr (OUT != OUT_I32) {
             if (m < p.M) {
                 uint16_t *drow = reinterpret_cast<uint16_t *>(p.C) + (size_t)m * ldc;
+                v2i o = pack16(v);
                 // (the columns of a block, not the order whole tiles are stored in: the bias is
                 // fetched here)
-                const v2i o = with_bias(pack16(v), bias4_at(p, n));
+                if constexpr (BIAS) o = with_bias(o, bias4_at(p, n));
                 if (vec_ok && n + 3 < p.N) {
                     *reinterpret_cast<v2i *>(drow + n) = o;
                 } else if (n + 3 < p.N) {

@@ -16,8 +16,8 @@ namespace qm {
 // default the grid is persistent: as many workgroups as the device holds at once, each
 // running several (K split, tile) items back to back.
 // (OUT is a template parameter so that every kernel gets launcher statics of its own.)
-// (... and TAIL: the kernel for K % 128 != 0 is another kernel with statics of its own)
-template <class Cfg, int OUT, bool TAIL, class Kernel>
+// (... and TAIL and BIAS: the kernels for K % 128 != 0 and with a bias are others, with statics of their own)
+template <class Cfg, int OUT, bool TAIL, bool BIAS, class Kernel>
 static hipError_t launch_tiled_persistent(Kernel kernel, const GemmArgs &p, hipStream_t stream, int opt)
 {
     static std::atomic<bool> lds_ok[QM_MAX_DEVICES] = {};
@@ -57,32 +57,45 @@ static hipError_t launch_tiled_persistent(Kernel kernel, const GemmArgs &p, hipS
 
 }  // namespace qm
 
+namespace qm {
+template <class Cfg, int OUT, bool BIAS>
+static hipError_t launch_tiled(const GemmArgs &p, hipStream_t s, int opt)
+{
+    if (p.K % 128) return launch_tiled_persistent<Cfg, OUT, true, BIAS>(&gemm_tile16_kernel<Cfg, OUT, true, BIAS>, p, s, opt);
+    return launch_tiled_persistent<Cfg, OUT, false, BIAS>(&gemm_tile16_kernel<Cfg, OUT, false, BIAS>, p, s, opt);
+}
+}  // namespace qm
+
 #define QM_TILE16_DEF(BM, BN, WGM, WGN, ST, OCC)                                                 \
     namespace qm {                                                                               \
     hipError_t QM_TILE16_FN(BM, BN, WGM, WGN, ST, OCC)(const GemmArgs &p, hipStream_t s, int gm) \
     {                                                                                            \
-        using Cfg = Tile16Cfg<BM, BN, WGM, WGN, ST, OCC>;                                        \
-        if (p.K % 128) return launch_tiled_persistent<Cfg, OUT_I32, true>(&gemm_tile16_kernel<Cfg, OUT_I32, true>, p, s, gm); \
-        return launch_tiled_persistent<Cfg, OUT_I32, false>(&gemm_tile16_kernel<Cfg, OUT_I32, false>, p, s, gm);  \
+        return launch_tiled<Tile16Cfg<BM, BN, WGM, WGN, ST, OCC>, OUT_I32, false>(p, s, gm);     \
     }                                                                                            \
     }
-// the same configuration with the scaled 16-bit float outputs
+// the same configuration with the scaled 16-bit float outputs, without a bias and (in a unit of
+// its own) with one
 #define QM_TILE16S_DEF(BM, BN, WGM, WGN, ST, OCC)                                                 \
     namespace qm {                                                                                \
     hipError_t QM_TILE16S_FN(BM, BN, WGM, WGN, ST, OCC)(const GemmArgs &p, hipStream_t s, int gm) \
     {                                                                                             \
         using Cfg = Tile16Cfg<BM, BN, WGM, WGN, ST, OCC>;                                         \
-        if (p.K % 128) {                                                                            \
-            if (p.out == OUT_F16) return launch_tiled_persistent<Cfg, OUT_F16, true>(&gemm_tile16_kernel<Cfg, OUT_F16, true>, p, s, gm); \
-            return launch_tiled_persistent<Cfg, OUT_BF16, true>(&gemm_tile16_kernel<Cfg, OUT_BF16, true>, p, s, gm); \
-        }                                                                                           \
-        if (p.out == OUT_F16) return launch_tiled_persistent<Cfg, OUT_F16, false>(&gemm_tile16_kernel<Cfg, OUT_F16, false>, p, s, gm); \
-        return launch_tiled_persistent<Cfg, OUT_BF16, false>(&gemm_tile16_kernel<Cfg, OUT_BF16, false>, p, s, gm); \
+        if (p.bias != nullptr) return QM_TILE16B_FN(BM, BN, WGM, WGN, ST, OCC)(p, s, gm);         \
+        return p.out == OUT_F16 ? launch_tiled<Cfg, OUT_F16, false>(p, s, gm) : launch_tiled<Cfg, OUT_BF16, false>(p, s, gm); \
+    }                                                                                             \
+    }
+#define QM_TILE16B_DEF(BM, BN, WGM, WGN, ST, OCC)                                                 \
+    namespace qm {                                                                                \
+    hipError_t QM_TILE16B_FN(BM, BN, WGM, WGN, ST, OCC)(const GemmArgs &p, hipStream_t s, int gm) \
+    {                                                                                             \
+        using Cfg = Tile16Cfg<BM, BN, WGM, WGN, ST, OCC>;                                         \
+        return p.out == OUT_F16 ? launch_tiled<Cfg, OUT_F16, true>(p, s, gm) : launch_tiled<Cfg, OUT_BF16, true>(p, s, gm); \
     }                                                                                             \
     }
 
 // An entry of qm_configs.inc is compiled here only when its unit number equals QM_TU:
-// QM_PICK*_<n> expands to nothing except for n == QM_TU.
+// QM_PICK*_<n> expands to nothing except for n == QM_TU.  The kernels with a bias of the
+// configurations of unit n are unit n + 8.
 #define QM_PICK16_0(...)
 #define QM_PICK16_1(...)
 #define QM_PICK16_2(...)
@@ -111,6 +124,14 @@ static hipError_t launch_tiled_persistent(Kernel kernel, const GemmArgs &p, hipS
 #define QM_PICK16S_11(...)
 #define QM_PICK16S_12(...)
 #define QM_PICK16S_13(...)
+#define QM_PICK16B_6(...)
+#define QM_PICK16B_7(...)
+#define QM_PICK16B_8(...)
+#define QM_PICK16B_9(...)
+#define QM_PICK16B_10(...)
+#define QM_PICK16B_11(...)
+#define QM_PICK16B_12(...)
+#define QM_PICK16B_13(...)
 #if QM_TU == 0
 #undef QM_PICK16_0
 #define QM_PICK16_0(...) QM_TILE16_DEF(__VA_ARGS__)
@@ -181,10 +202,34 @@ static hipError_t launch_tiled_persistent(Kernel kernel, const GemmArgs &p, hipS
 #define QM_PICK16_13(...) QM_TILE16_DEF(__VA_ARGS__)
 #undef QM_PICK16S_13
 #define QM_PICK16S_13(...) QM_TILE16S_DEF(__VA_ARGS__)
+#elif QM_TU == 14
+#undef QM_PICK16B_6
+#define QM_PICK16B_6(...) QM_TILE16B_DEF(__VA_ARGS__)
+#elif QM_TU == 15
+#undef QM_PICK16B_7
+#define QM_PICK16B_7(...) QM_TILE16B_DEF(__VA_ARGS__)
+#elif QM_TU == 16
+#undef QM_PICK16B_8
+#define QM_PICK16B_8(...) QM_TILE16B_DEF(__VA_ARGS__)
+#elif QM_TU == 17
+#undef QM_PICK16B_9
+#define QM_PICK16B_9(...) QM_TILE16B_DEF(__VA_ARGS__)
+#elif QM_TU == 18
+#undef QM_PICK16B_10
+#define QM_PICK16B_10(...) QM_TILE16B_DEF(__VA_ARGS__)
+#elif QM_TU == 19
+#undef QM_PICK16B_11
+#define QM_PICK16B_11(...) QM_TILE16B_DEF(__VA_ARGS__)
+#elif QM_TU == 20
+#undef QM_PICK16B_12
+#define QM_PICK16B_12(...) QM_TILE16B_DEF(__VA_ARGS__)
+#elif QM_TU == 21
+#undef QM_PICK16B_13
+#define QM_PICK16B_13(...) QM_TILE16B_DEF(__VA_ARGS__)
 #else
 #error "QM_TU out of range"
 #endif
 
 #define QM_TILE16(tu, ...) QM_PICK16_##tu(__VA_ARGS__)
-#define QM_TILE16S(tu, ...) QM_PICK16S_##tu(__VA_ARGS__)
+#define QM_TILE16S(tu, ...) QM_PICK16S_##tu(__VA_ARGS__) QM_PICK16B_##tu(__VA_ARGS__)
 #include "qm_configs.inc"
