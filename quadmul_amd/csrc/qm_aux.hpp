@@ -232,24 +232,38 @@ __device__ __forceinline__ uint32_t pack4(uint32_t w)  // 4 int8 -> 2 packed byt
 }
 
 // At least 8 packed bytes at any address; the last piece is the last 8 bytes, those that the one before
-// has written among them.  Two pieces per thread in flight, their loads non-temporal: nothing
-// reads the values again, and they leave the caches to the packed bytes (us, with one piece and plain
-// loads: 8192 x 8192 20.0 -> 17.3 = 5.8 TB/s, 16384 x 14336 65 -> 55).  Sizes and addresses that are not
-// multiples of 8 used to take one byte per thread: 8191 x 8190 42.6 us.
+// has written among them.  Two pieces per thread in flight.  Which two, and whether the loads are
+// non-temporal, follows from where the values are (us, on a box of 5.6 TB/s; "after": behind an
+// elementwise kernel that has just written the values, into the same buffer every time):
+//   - up to 24 MB of values may still be in the L2s of the XCDs that wrote them, 4 KB to a workgroup
+//     as elementwise kernels have it: workgroup b takes the 4 KB piece b and the one a grid (a
+//     multiple of 8 workgroups) further on, both on the XCD that wrote them.  8 KB in a row
+//     instead, 8 MB: after 10.1 (this way 6.8), and with unpack_i4_vec_kernel, whose 2 KB pieces of packed
+//     bytes fall on the XCD that packed them, 8.6 (6.4);
+//   - beyond that nothing reads the values again before they are gone, and non-temporal loads leave the
+//     caches to the packed bytes: 45 MB 14.6 -> 12.7, with unpack_i4_vec_kernel 24.7 -> 20.9;
+//   - from 56 MB on, whole 8 KB in a row: 64 MB 19.3 -> 17.0, 256 MB 68.7 -> 65.1.
+// Sizes and addresses that are not multiples of 8 once took one byte per thread: 8191 x 8190 42.6 us.
 constexpr int PACK_PIECES = 2, PACK_THREADS = 256;
-__global__ void __launch_bounds__(PACK_THREADS) pack_i4_vec_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t nbytes)
+constexpr size_t PACK_NT_BYTES = (size_t)12 << 20, PACK_IN_A_ROW_BYTES = (size_t)28 << 20;  // of packed bytes
+template <bool NT>
+__global__ void __launch_bounds__(PACK_THREADS) pack_i4_vec_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t nbytes, bool in_a_row)
 {
-    for (size_t i0 = (size_t)blockIdx.x * (PACK_THREADS * PACK_PIECES) + threadIdx.x; 8 * i0 < nbytes; i0 += (size_t)gridDim.x * (PACK_THREADS * PACK_PIECES)) {
+    const size_t apart = in_a_row ? PACK_THREADS : (size_t)gridDim.x * PACK_THREADS;  // between the pieces of a thread
+    const size_t first = (size_t)blockIdx.x * (PACK_THREADS * (in_a_row ? PACK_PIECES : 1)) + threadIdx.x;
+    for (size_t i0 = first; 8 * i0 < nbytes; i0 += (size_t)gridDim.x * (PACK_THREADS * PACK_PIECES)) {
         v4i v[PACK_PIECES];
 #pragma unroll
-        for (int u = 0; u < PACK_PIECES; ++u)
-            v[u] = __builtin_nontemporal_load(reinterpret_cast<const v4i_any_aligned *>(src + 2 * min(8 * (i0 + PACK_THREADS * u), nbytes - 8)));
+        for (int u = 0; u < PACK_PIECES; ++u) {
+            const v4i_any_aligned *from = reinterpret_cast<const v4i_any_aligned *>(src + 2 * min(8 * (i0 + apart * u), nbytes - 8));
+            v[u] = NT ? __builtin_nontemporal_load(from) : *from;
+        }
 #pragma unroll
         for (int u = 0; u < PACK_PIECES; ++u) {
             v2i o;
             o.x = (int)(pack4((uint32_t)v[u].x) | (pack4((uint32_t)v[u].y) << 16));
             o.y = (int)(pack4((uint32_t)v[u].z) | (pack4((uint32_t)v[u].w) << 16));
-            *reinterpret_cast<v2i_any_aligned *>(dst + min(8 * (i0 + PACK_THREADS * u), nbytes - 8)) = o;
+            *reinterpret_cast<v2i_any_aligned *>(dst + min(8 * (i0 + apart * u), nbytes - 8)) = o;
         }
     }
 }
@@ -277,7 +291,9 @@ __device__ __forceinline__ v2i unpack8(uint32_t w)
 
 // At least 8 packed bytes at any address, the last piece as in pack_i4_vec_kernel.  Bound: the stores, two
 // thirds of the traffic: 16 bytes per lane, non-temporal (us, 8 bytes per lane and plain stores / 16
-// and plain / 16 and non-temporal: 8192 x 8192 22.5 / 20.3 / 16.1 = 6.3 TB/s, 16384 x 14336 74 / 63 / 52.5).
+// and plain / 16 and non-temporal: 8192 x 8192 22.5 / 20.3 / 16.1 = 6.3 TB/s, 16384 x 14336 74 / 63 / 52.5; 8 MB
+// of values 4.2 / 3.8 / 3.4).  A kernel that reads the values next finds fewer of them in the caches: this kernel
+// and such a reader together 8 MB 8.2 / 7.7 / 7.9, 24 MB 19.4 / 18.2 / 20.0, 64 MB 43.1 / 40.5 / 43.4, 192 MB 126 / 121 / 116.
 __global__ void __launch_bounds__(PACK_THREADS) unpack_i4_vec_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t nbytes)
 {
     for (size_t i = (size_t)blockIdx.x * PACK_THREADS + threadIdx.x; 8 * i < nbytes; i += (size_t)gridDim.x * PACK_THREADS) {

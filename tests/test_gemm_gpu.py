@@ -259,6 +259,22 @@ def test_pack_unpack_any_address(oracle_mod, nbytes, off):
     assert (b[:8 + off] == 0x5A).all() and (b[8 + off + 2 * nbytes:] == 0x5A).all()
 
 
+@pytest.mark.parametrize("nbytes", [7 * 4096 + 5, (12 << 20) - 1, (12 << 20) + 2051, (28 << 20) - 4099, (28 << 20) + 4101])
+@pytest.mark.parametrize("off", [0, 1])
+def test_pack_every_piece_once(nbytes, off):
+    """Either side of the sizes where the loads become non-temporal and where a thread's pieces lie in a row, no
+    multiple of a workgroup's share: every byte, and the bytes around the output untouched."""
+    g = torch.Generator(device=DEV).manual_seed(SEED_BASE + 4200 + nbytes % 97)
+    src = torch.randint(-8, 8, (2 * nbytes + off,), dtype=torch.int8, device=DEV, generator=g)
+    v = src[off:]
+    out = torch.full((nbytes + 24,), 0x5A, dtype=torch.uint8, device=DEV)
+    s = torch.cuda.current_stream().cuda_stream
+    assert qm.library().qm_pack_i4(v.data_ptr(), out.data_ptr() + 8 + off, 1, 2 * nbytes, s) == 0
+    u = v.view(torch.uint8)
+    assert torch.equal(out[8 + off:8 + off + nbytes], (u[0::2] & 15) | ((u[1::2] & 15) << 4))
+    assert (out[:8 + off] == 0x5A).all() and (out[8 + off + nbytes:] == 0x5A).all()
+
+
 # ------------------------------------------------------------------ the named workloads
 NAMED_SHAPES = [
     (0, 1024, 1024, 1024), (1, 4096, 4096, 4096),
