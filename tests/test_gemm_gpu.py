@@ -68,11 +68,15 @@ GENERIC_SHAPES = [(1, 1, 2), (3, 5, 30), (17, 33, 34), (70, 33, 160 + 2), (100, 
 
 @pytest.mark.parametrize("shape", GENERIC_SHAPES, ids=lambda s: "x".join(map(str, s)))
 def test_k_not_multiple_of_32_takes_generic_path(oracle_mod, shape):
+    """No configuration but "generic" takes these: the automatic choice runs the kernel for operands at any
+    address (K < 32: one thread per element), the explicit id one thread per element whatever K is."""
     m, n, k = shape
     a, b = make_operands(m, n, k, SEED_BASE + 2000 + k)
     ap, bp = pack_cpu(a), pack_cpu(b)
     assert qm.config_name(qm.select_config(m, n, k) & 0xFFFF) == "generic"
-    assert oracle_mod.compare(run_gemm(ap, bp, m, n, k), oracle_mod.gemm_i4(ap.numpy(), bp.numpy())) == -1
+    want = oracle_mod.gemm_i4(ap.numpy(), bp.numpy())
+    assert oracle_mod.compare(run_gemm(ap, bp, m, n, k), want) == -1
+    assert oracle_mod.compare(run_gemm(ap, bp, m, n, k, qm.config_id("generic")), want) == -1
 
 
 def test_unaligned_operands_take_generic_path(oracle_mod):
@@ -86,8 +90,12 @@ def test_unaligned_operands_take_generic_path(oracle_mod):
     a_d.copy_(ap)
     b_d.copy_(bp)
     c_d = poisoned_c(m, n, DEV)
+    want = oracle_mod.gemm_i4(ap.numpy(), bp.numpy())
     qm.gemm(a_d, b_d, c_d, m, n, k)
-    assert oracle_mod.compare(c_d.cpu().numpy(), oracle_mod.gemm_i4(ap.numpy(), bp.numpy())) == -1
+    assert oracle_mod.compare(c_d.cpu().numpy(), want) == -1
+    c_d = poisoned_c(m, n, DEV)
+    qm.gemm_cfg(a_d, b_d, c_d, m, n, k, qm.config_id("generic"))   # (the explicit id: one thread per element)
+    assert oracle_mod.compare(c_d.cpu().numpy(), want) == -1
 
 
 @pytest.mark.parametrize("name", ["gemm_i4_32x48x64", "gemm_i4_70x33x160", "gemm_i4_5x130x34"])
@@ -434,7 +442,7 @@ def test_auto_choice_splits_k_and_matches(oracle_mod):
 
 def test_random_shapes_through_the_automatic_choice():
     """A seeded sweep of shapes nobody tuned for, through qm_gemm_i4's own choice of kernel
-    (table, cost model, K split with a workspace, generic fallback), against an fp32 matmul
+    (table, cost model, K split with a workspace, any even K), against an fp32 matmul
     on the GPU (exact: every partial sum is an integer below 2^24)."""
     import quadmul
 
@@ -502,7 +510,7 @@ def test_dot_product_kernel_one_and_two_rows(oracle_mod, shape):
 def test_k_padded_through_the_workspace(shape):
     """Large shapes whose K is not a multiple of 32, and unaligned operands: with a workspace
     the operands are copied with zero-padded rows and the pipelined kernel runs; without one
-    the generic kernel does.  (K % 32 == 0, first case: no copies, a short last K-step; a K of
+    the kernel for operands at any address does.  (K % 32 == 0, first case: no copies, a short last K-step; a K of
     less than one K-step: no copies either, 32 x 32 blocks of the wave-level kernel.)  Same
     result, against an exact fp32 matmul."""
     import quadmul
