@@ -336,12 +336,15 @@ def test_unaligned_rows_of_c_on_every_pipelined_configuration(oracle_mod, shape,
     assert ran >= 8
 
 
-# every epilogue: the dot, wave-level and persistent kernels (1 to 64 rows), the generic kernel (K % 32,
-# and too small to pad), zero-padded copies, each tile through its own way of writing whole tiles,
+# every epilogue: the dot, wave-level and persistent kernels (1 to 64 rows), the kernels for any address and
+# one thread per element (K % 32), each tile through its own way of writing whole tiles,
 # tiles that stick out of C, odd N, a short last K-step, a K split added up out of a workspace, k = 0,
 # several blocks of columns per workgroup of the persistent kernel with the last one cut short
 BIAS_SHAPES = [(1, 33, 256), (2, 64, 4096), (9, 130, 8192), (40, 96, 1152), (70, 33, 162), (2048, 520, 130), (256, 512, 256), (520, 780, 384),
                (300, 1021, 416), (257, 258, 640), (6, 10, 0), (5, 8263, 384)]
+# ... and zero-padded copies, the second time where the configuration that int32 takes on them has no scaled output
+COPIED_SHAPES = [(300, 1021, 4100), (1518, 4099, 506)]
+BIAS_SHAPES += COPIED_SHAPES
 
 
 @pytest.mark.parametrize("shape", BIAS_SHAPES, ids=lambda s: "x".join(map(str, s)))
@@ -349,6 +352,11 @@ def test_bias_in_every_epilogue(oracle_mod, shape):
     """The bias added in the epilogue gives, bit for bit, the rounded value plus the bias rounded
     once more; without one, a zero with a negative scale stays -0."""
     m, n, k = shape
+    if shape in COPIED_SHAPES:
+        kp = (k + 127) // 128 * 128
+        assert qm.workspace_bytes(m, n, k, scaled=True) >= (m + n) * kp // 2
+        alike = qm.library().qm_select_config_ex(m, n, kp, 256, 0, 0) & 0xFFFF
+        assert qm.config_has_scaled(alike) == (shape == COPIED_SHAPES[0]), qm.config_name(alike)
     a, b = make_operands(m, n, max(k, 2), SEED_BASE + 7600 + m + n + k)
     ap, bp = pack_cpu(a), pack_cpu(b)
     if k == 0:
@@ -380,6 +388,21 @@ def test_bias_in_every_epilogue(oracle_mod, shape):
                 assert (bits(d) == bits(w_)).all(), (name, code >> 16, dtype, b_ is None)
     with pytest.raises(qm.QuadmulError):
         qm.gemm_scaled(a_d, b_d, d, m, n, k, rs_d, cs_d, bias=torch.zeros(n + 1, dtype=d.dtype, device=DEV))
+
+
+def test_bf16_rounding_of_every_float():
+    """What the pipelined kernel's write-out makes of each of the 2^32 floats (a product of 1, the float its row's scale):
+    round to nearest even by the integer rule, a NaN its upper half with the quiet bit."""
+    rows, cfg = 1 << 22, qm.config_id("q64x64_w2x2_s8o2")
+    a, b = torch.zeros((rows, 64), dtype=torch.int8, device=DEV), torch.zeros((4, 64), dtype=torch.int8, device=DEV)
+    a[:, 0] = b[:, 0] = 1
+    d = torch.empty((rows, 4), dtype=torch.bfloat16, device=DEV)
+    for first in range(-(1 << 31), 1 << 31, rows):
+        x = torch.arange(first, first + rows, dtype=torch.int64, device=DEV)
+        qm.gemm_scaled(a, b, d, rows, 4, 128, x.to(torch.int32).view(torch.float32), None, cfg)
+        u = x & 0xFFFFFFFF
+        want = torch.where((u & 0x7FFFFFFF) > 0x7F800000, (u >> 16) | 0x40, (u + 0x7FFF + ((u >> 16) & 1)) >> 16)
+        assert torch.equal(d.view(torch.int16).long() & 0xFFFF, want[:, None].expand(rows, 4)), hex(first & 0xFFFFFFFF)
 
 
 def test_linear_bias_that_the_kernel_cannot_take(oracle_mod):
