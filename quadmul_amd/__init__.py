@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import types
 from typing import List, Optional
 
 import torch
@@ -112,28 +113,31 @@ def library() -> ctypes.CDLL:
 
 
 _EXT_FUNCTIONS = ("linear", "pack", "quantize_pack", "unpack")
-_ext = None  # the extension module; False: there is none, or it is not this package's
+_ext = None  # the extension module, once looked for
 
 
 def _extension():
-    """The extension module, or False where only the library was built (``python -m quadmul_amd.build --lib``) or
-    another module of its name is found first: the same kernels are then called through ctypes."""
+    """The extension module.  Where only the library was built (``python -m quadmul_amd.build --lib``), or another module
+    of its name is found first, functions that return None in its place: the same kernels are then called through
+    ctypes."""
     global _ext
-    if _ext is None:
-        try:
-            import quadmul
-        except ImportError:
-            _ext = False
-        else:
-            _ext = quadmul if all(hasattr(quadmul, f) for f in _EXT_FUNCTIONS) else False
+    try:
+        import quadmul
+    except ImportError:
+        quadmul = None
+    if not all(hasattr(quadmul, f) for f in _EXT_FUNCTIONS):
+        quadmul = types.SimpleNamespace(**dict.fromkeys(_EXT_FUNCTIONS, lambda *args: None))
+    _ext = quadmul
     return _ext
 
 
 def _native(name: str, *args):
-    """The extension module's function of this name.  From Python the same call costs two to three times as
-    much on the host (device guard, stream, allocations, ctypes), more than a small one takes on the GPU."""
+    """What the extension module's function of this name returns, or None where there is no such module.  From Python
+    the same call costs two to three times as much on the host (device guard, stream, allocations, ctypes), more
+    than a small one takes on the GPU."""
+    ext = _extension() if _ext is None else _ext
     try:
-        return getattr(_extension(), name)(*args)
+        return getattr(ext, name)(*args)
     except RuntimeError as e:
         if type(e) is RuntimeError:
             raise QuadmulError(str(e)) from None
@@ -258,8 +262,9 @@ def quantize_pack(x: torch.Tensor):
         raise QuadmulError("quantize_pack: x must be float16, bfloat16 or float32")
     if x.shape[1] % 2:
         raise QuadmulError("quantize_pack: k must be even")
-    if _extension():
-        return _native("quantize_pack", x)
+    found = _native("quantize_pack", x)
+    if found is not None:
+        return found
     rows, k = x.shape
     kind = {torch.float16: 1, torch.bfloat16: 2, torch.float32: 3}[x.dtype]
     packed = torch.empty((rows, k // 2), dtype=torch.int8, device=x.device)
@@ -311,9 +316,10 @@ def pack_int4(values: torch.Tensor) -> torch.Tensor:
     if k % 2:
         raise QuadmulError("pack_int4: K must be even")
     v = values.contiguous()
-    if v.is_cuda and _extension():
-        return _native("pack", v)
     if v.is_cuda:
+        out = _native("pack", v)
+        if out is not None:
+            return out
         out = torch.empty((rows, k // 2), dtype=torch.int8, device=v.device)
         with torch.cuda.device(v.device):
             st = library().qm_pack_i4(v.data_ptr(), out.data_ptr(), rows, k, _stream_ptr(v))
@@ -330,9 +336,10 @@ def unpack_int4(packed: torch.Tensor) -> torch.Tensor:
         raise QuadmulError("unpack_int4: expects a 2-D int8/uint8 tensor")
     p = packed.contiguous()
     rows, half = p.shape
-    if p.is_cuda and _extension():
-        return _native("unpack", p)
     if p.is_cuda:
+        out = _native("unpack", p)
+        if out is not None:
+            return out
         out = torch.empty((rows, 2 * half), dtype=torch.int8, device=p.device)
         with torch.cuda.device(p.device):
             st = library().qm_unpack_i4(p.data_ptr(), out.data_ptr(), rows, 2 * half, _stream_ptr(p))

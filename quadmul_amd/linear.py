@@ -15,7 +15,7 @@ from typing import Optional
 import torch
 from torch.autograd import forward_ad
 
-from . import QuadmulError, _extension, _native, gemm_scaled, quantize_pack
+from . import QuadmulError, _native, gemm_scaled, quantize_pack
 
 
 def _fusable(bias: torch.Tensor, x: torch.Tensor, out_dtype: torch.dtype, n: int) -> bool:
@@ -69,9 +69,8 @@ class W4A4Linear(torch.nn.Module):
             # (2048 x 11008: 21 us beside a GEMM of 73).  A bias that the kernel cannot take as
             # it is -- moved or cast after construction -- or that autograd follows is added apart.
             fused = bias is not None and _fusable(bias, x2, self.out_dtype, self.out_features)
-            if _extension():
-                y = _native("linear", x2, self.weight_packed, self.out_features, self.weight_scale, bias if fused else None, self.out_dtype == torch.bfloat16)
-            else:
+            y = _native("linear", x2, self.weight_packed, self.out_features, self.weight_scale, bias if fused else None, self.out_dtype == torch.bfloat16)
+            if y is None:
                 y = torch.empty((x2.shape[0], self.out_features), dtype=self.out_dtype, device=x.device)
                 xq, xs = quantize_pack(x2)
                 gemm_scaled(xq, self.weight_packed, y, x2.shape[0], self.out_features, self.in_features, xs, self.weight_scale,
