@@ -232,38 +232,33 @@ __device__ __forceinline__ uint32_t pack4(uint32_t w)  // 4 int8 -> 2 packed byt
 }
 
 // At least 8 packed bytes at any address; the last piece is the last 8 bytes, those that the one before
-// has written among them.  Two pieces per thread in flight.  Which two, and whether the loads are
-// non-temporal, follows from where the values are (us, on a box of 5.6 TB/s; "after": behind an
-// elementwise kernel that has just written the values, into the same buffer every time):
-//   - up to 24 MB of values may still be in the L2s of the XCDs that wrote them, 4 KB to a workgroup
-//     as elementwise kernels have it: workgroup b takes the 4 KB piece b and the one a grid (a
-//     multiple of 8 workgroups) further on, both on the XCD that wrote them.  8 KB in a row
-//     instead, 8 MB: after 10.1 (this way 6.8), and with unpack_i4_vec_kernel, whose 2 KB pieces of packed
-//     bytes fall on the XCD that packed them, 8.6 (6.4);
-//   - beyond that nothing reads the values again before they are gone, and non-temporal loads leave the
-//     caches to the packed bytes: 45 MB 14.6 -> 12.7, with unpack_i4_vec_kernel 24.7 -> 20.9;
-//   - from 56 MB on, whole 8 KB in a row: 64 MB 19.3 -> 17.0, 256 MB 68.7 -> 65.1.
-// Sizes and addresses that are not multiples of 8 once took one byte per thread: 8191 x 8190 42.6 us.
-constexpr int PACK_PIECES = 2, PACK_THREADS = 256;
-constexpr size_t PACK_NT_BYTES = (size_t)12 << 20, PACK_IN_A_ROW_BYTES = (size_t)28 << 20;  // of packed bytes
-template <bool NT>
-__global__ void __launch_bounds__(PACK_THREADS) pack_i4_vec_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t nbytes, bool in_a_row)
+// has written among them.  Two pieces per thread in flight, 32 KB of values apart: workgroup b takes the
+// 4 KB of values number 16 (b / 8) + b % 8 and those eight further on, so that
+//   - both are on the XCD of the workgroup that wrote them, if an elementwise kernel with 4 KB to a workgroup did, and
+//     are found in its L2 up to about 24 MB; unpack_i4_vec_kernel finds the packed bytes, 2 KB to a workgroup, in the same way;
+//   - eight workgroups read 64 KB in a row, which is what HBM wants.
+// Loads are non-temporal: they leave the caches to the packed bytes.  us, this way / 8 KB in a row to a workgroup,
+// non-temporal / the two pieces a grid apart, plain loads: an elementwise kernel and the packing behind it, same buffer,
+// 16 MB 8.9 / 13.7 / 8.9; packing and unpacking, same buffer, 16 MB 8.0 / 11.5 / 7.6, 32 MB 14.1 / 21.3 / 16.8, 48 MB
+// 21.5 / 26.7 / 23.8; packing from HBM 16 MB 5.7 / 5.7 / 6.6, 32 MB 9.5 / 9.4 / 11.4, 64 MB 16.8 / 17.1 / 20.3, 160 MB 38.6
+// (6.5 TB/s) / 38.4 / 45.5.  Sizes and addresses that are not multiples of 8 once took one byte per thread: 8191 x 8190 42.6 us.
+constexpr int PACK_PIECES = 2, PACK_THREADS = 256, PACK_APART = 8;  // (workgroups: one per XCD)
+__global__ void __launch_bounds__(PACK_THREADS) pack_i4_vec_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, size_t nbytes)
 {
-    const size_t apart = in_a_row ? PACK_THREADS : (size_t)gridDim.x * PACK_THREADS;  // between the pieces of a thread
-    const size_t first = (size_t)blockIdx.x * (PACK_THREADS * (in_a_row ? PACK_PIECES : 1)) + threadIdx.x;
-    for (size_t i0 = first; 8 * i0 < nbytes; i0 += (size_t)gridDim.x * (PACK_THREADS * PACK_PIECES)) {
+    static_assert(PACK_PIECES == 2, "the pieces of a group of PACK_APART workgroups");
+    // (the grid is a multiple of PACK_APART workgroups)
+    const size_t piece = (size_t)(blockIdx.x / PACK_APART) * (PACK_PIECES * PACK_APART) + blockIdx.x % PACK_APART;
+    for (size_t i0 = piece * PACK_THREADS + threadIdx.x; 8 * i0 < nbytes; i0 += (size_t)gridDim.x * (PACK_THREADS * PACK_PIECES)) {
+        const size_t at[PACK_PIECES] = {min(8 * i0, nbytes - 8), min(8 * (i0 + PACK_APART * PACK_THREADS), nbytes - 8)};
         v4i v[PACK_PIECES];
 #pragma unroll
-        for (int u = 0; u < PACK_PIECES; ++u) {
-            const v4i_any_aligned *from = reinterpret_cast<const v4i_any_aligned *>(src + 2 * min(8 * (i0 + apart * u), nbytes - 8));
-            v[u] = NT ? __builtin_nontemporal_load(from) : *from;
-        }
+        for (int u = 0; u < PACK_PIECES; ++u) v[u] = __builtin_nontemporal_load(reinterpret_cast<const v4i_any_aligned *>(src + 2 * at[u]));
 #pragma unroll
         for (int u = 0; u < PACK_PIECES; ++u) {
             v2i o;
             o.x = (int)(pack4((uint32_t)v[u].x) | (pack4((uint32_t)v[u].y) << 16));
             o.y = (int)(pack4((uint32_t)v[u].z) | (pack4((uint32_t)v[u].w) << 16));
-            *reinterpret_cast<v2i_any_aligned *>(dst + min(8 * (i0 + apart * u), nbytes - 8)) = o;
+            *reinterpret_cast<v2i_any_aligned *>(dst + at[u]) = o;
         }
     }
 }

@@ -631,11 +631,9 @@ QM_EXPORT int qm_pack_i4(const void *src_i8, void *dst_packed, int rows, int k, 
     if (!src_i8 || !dst_packed) return QM_ERR_NULL;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (nbytes >= 8) {
-        unsigned grid = flat_grid(nbytes, 8 * PACK_PIECES * PACK_THREADS, 1u << 22);
-        if (grid > 8) grid = (grid + 7) / 8 * 8;
-        const auto kernel = nbytes >= PACK_NT_BYTES ? &pack_i4_vec_kernel<true> : &pack_i4_vec_kernel<false>;
-        kernel<<<dim3(grid), dim3(PACK_THREADS), 0, s>>>(static_cast<const uint8_t *>(src_i8), static_cast<uint8_t *>(dst_packed), nbytes,
-                                                         nbytes >= PACK_IN_A_ROW_BYTES);
+        const unsigned grid = flat_grid(nbytes, 8 * PACK_PIECES * PACK_THREADS, 1u << 22);
+        pack_i4_vec_kernel<<<dim3((grid + PACK_APART - 1) / PACK_APART * PACK_APART), dim3(PACK_THREADS), 0, s>>>(
+            static_cast<const uint8_t *>(src_i8), static_cast<uint8_t *>(dst_packed), nbytes);
     } else {
         pack_i4_byte_kernel<<<dim3(flat_grid(nbytes, 256)), dim3(256), 0, s>>>(static_cast<const uint8_t *>(src_i8), static_cast<uint8_t *>(dst_packed), nbytes);
     }

@@ -267,11 +267,11 @@ def test_pack_unpack_any_address(oracle_mod, nbytes, off):
     assert (b[:8 + off] == 0x5A).all() and (b[8 + off + 2 * nbytes:] == 0x5A).all()
 
 
-@pytest.mark.parametrize("nbytes", [7 * 4096 + 5, (12 << 20) - 1, (12 << 20) + 2051, (28 << 20) - 4099, (28 << 20) + 4101])
+@pytest.mark.parametrize("nbytes", [7 * 4096 + 5, 2048 * 8 - 8, 2048 * 8 + 8, 2048 * 16 + 9, (12 << 20) - 1, (12 << 20) + 2051, (28 << 20) - 4099, (28 << 20) + 4101])
 @pytest.mark.parametrize("off", [0, 1])
 def test_pack_every_piece_once(nbytes, off):
-    """Either side of the sizes where the loads become non-temporal and where a thread's pieces lie in a row, no
-    multiple of a workgroup's share: every byte, and the bytes around the output untouched."""
+    """Groups of eight workgroups whose last one is cut short in its first or its second half: every byte, and the
+    bytes around the output untouched."""
     g = torch.Generator(device=DEV).manual_seed(SEED_BASE + 4200 + nbytes % 97)
     src = torch.randint(-8, 8, (2 * nbytes + off,), dtype=torch.int8, device=DEV, generator=g)
     v = src[off:]
