@@ -170,33 +170,53 @@ static bool ragged_fits(int m, int n, int k)
     return k >= 32 && k <= QM_MAX_K_X16 && (long long)m * kb < 0x7fffffffLL && (long long)n * kb < 0x7fffffffLL && (m + 15) / 16 <= 65535;
 }
 
-// With a workspace a large product can also run on zero-padded copies of A and B on the
-// aligned kernels.  The copies cost a launch and 2 x (M + N) K / 2 bytes whatever M is; the kernel
-// here costs more with every block of rows, and by how the rows lie:
-//   - on multiples of four bytes its loads are whole (us, here / on copies: 64 x 9000 x 9000 18.5 / 32,
-//     100 x 9000 x 9000 29 / 38, 300 x 5001 x 2056 15.2 / 19.5, 400 x 8191 x 1032 19.8 / 16.1, 64 x 28672 x 8200 49 / 77,
-//     129 x 28672 x 8200 99 / 90, 200 x 8192 x 28672 122 / 100), whatever K is up to 64 rows;
-//   - else every 16 bytes of a lane are split: 16 x 6001 x 4100 11.8 / 11.9, 32 x 6000 x 3002 8.4 / 11.4, 32 x 1000 x 6002
-//     11.6 / 7.5, 32 x 28672 x 8194 116 / 70, 48 x 8191 x 1030 7.4 / 8.8, 512 x 1001 x 1002 6.1 / 6.9, 512 x 8191 x 1030
-//     36 / 17;
-//   - and a few bytes off a multiple of 1024 from row to row the pieces of a block's rows meet
-//     in the same sets of the L1: 16 x 9000 x 2050 13.5 / 11.3, 32 x 5001 x 2050 10.2 / 9.3, 32 x 4100 x 4098
-//     17.1 / 11.0, 48 x 1500 x 2046 7.3 / 6.4.
-// One or two rows never take the copies, which are as large as the weights and at most a
-// fifth faster there (1 x 28672 x 8194 61 / 60, 1 x 11008 x 14338 53 / 44, 1 x 65536 x 4100 55 / 71).  A K of one or
-// two steps is mostly write-out: 160 x 5000 x 130 5.0 / 6.5, 300 x 5000 x 130 8.3 / 7.7.  Over 1088 products of
-// 1500 rows, this rule is 0.6 % behind the better of the two in the mean; one that took no account
-// of how the rows lie was 8 % behind.
+// Blocks of 16 fm rows and 16 fn columns of C, nw waves over K with u chunks in flight each: the largest block that
+// leaves more than half of the 256 CUs a workgroup of their own.  It reads (rows + columns) x K / 2
+// bytes per rows x columns of C, but a workgroup's time is its K loop and an idle CU helps nobody.
+// us, on blocks of 2x1, 2x2, 4x2 and 4x4 times 16: 17 x 3307 x 4100 10.0, 13.2, 15.4, 21.8; 64 x 3307 x 4100 23.0, 16.1,
+// 23.5, 30.1; 200 x 3307 x 4100 59, 43, 44, 31; 100 x 1001 x 1002 3.5, 4.2, 5.3, 6.7; 64 x 9000 x 9000 64, 45, 53, 34.  Up
+// to 16 rows, 1x1 and 1x2: 16 x 3307 x 4100 8.9, 12.1; 16 x 5001 x 2050 9.5, 7.8.  One thread per element, which
+// these calls used to run on: 1 x 9000 x 9000 264 us (here 14.5), 16 x 700 x 8998 195 (12.6), 64 x 1001 x 1002 19 (3.4).
+struct RaggedBlock {
+    int fm, fn, nw, u;
+    long long count(int m, int n) const { return (long long)((n + 16 * fn - 1) / (16 * fn)) * ((m + 16 * fm - 1) / (16 * fm)); }
+};
+static RaggedBlock ragged_block(int m, int n)
+{
+    const auto crowded = [&](const RaggedBlock &b) { return b.count(m, n) > 128; };
+    if (m <= 16) return crowded({1, 2, 8, 2}) ? RaggedBlock{1, 2, 8, 2} : RaggedBlock{1, 1, 16, 2};
+    if (m > 32 && crowded({4, 4, 8, 1})) return {4, 4, 8, 1};
+    if (m > 32 && crowded({4, 2, 8, 2})) return {4, 2, 8, 2};
+    return crowded({2, 2, 8, 2}) ? RaggedBlock{2, 2, 8, 2} : RaggedBlock{2, 1, 16, 2};
+}
+
+// With a workspace a large product can also run on zero-padded copies of A and B on the aligned kernels.
+// The faster of the two by what each costs (us), fitted to 3800 products of 1 to 1500 rows, timed both ways with B from HBM
+// and from the caches (rms of the fits 11 % here, 8 and 13 % on the copies; on 2500 others the choice is 1.4 % behind the
+// better one in the mean; up to 32 or 64 rows this kernel, which was the rule once, 7 %):
+//   - here it is the loads: every wave's 16 bytes per lane of the rows of a block go through the L1 of its CU, 0.66 clocks
+//     a lane where rows lie on multiples of four bytes and 1.94 where they do not (those are split); up to 0.35 x 5.5
+//     more where they lie within five bytes of a multiple of 128 from row to row, so that the rows of a block
+//     meet in the same banks (16 x 28672 x 4096 + 2 d, d = -1, -2, -3, -5, -7: 43.5, 38.4, 33.6, 28.5, 24.8; 17.5 at d = -8;
+//     the copies 34).  Rows of a block beyond m are copies of the last one and cost next to nothing (3, 8 and 16 x 65536 x
+//     4100: 58, 68, 78).  Workgroups beyond one per CU count whole rounds;
+//   - on copies, two launches, the rows of both operands read, written and read again, and the GEMM.
+// One or two rows never take the copies, which are as large as the weights and at most a fifth faster there.  Above
+// 512 rows only small products are left here, as before (809 x 708 x 1096 5.2 / 8.6, 939 x 1094 x 1596 17.7 / 12.7).
 static bool ragged_before_copies(int m, int n, int k, int ptr_align)
 {
-    const long long outs = (long long)m * n;
     if (m <= 2) return true;
-    if (k < 256) return outs <= (5 << 18);
-    const int kb = k / 2, off = kb & 1023;
-    if (kb % 4 == 0 && ptr_align >= 4) return m <= 64 || (m <= 512 && outs <= (k <= 10240 ? 3 << 20 : 1 << 20));
-    const bool near_1024 = off != 0 && (off < 8 || off >= 1016);
-    if (m <= (near_1024 ? 16 : 32) && (k <= 4224 || off == 0)) return true;
-    return k <= 2176 && outs * k < (near_1024 ? 1LL << 27 : 1LL << 29);
+    if (m > 512 && (long long)m * n * k >= (1LL << 29)) return false;
+    const RaggedBlock b = ragged_block(m, n);
+    const int kb = k / 2, off = std::min(kb % 128, 128 - kb % 128), kp = (k + 127) / 128 * 128;
+    const double chunks = (kb + 63) / 64, out = 4e-6 * m * n, rounds = (double)((b.count(m, n) + 255) / 256);
+    const double l1_clocks = kb % 4 == 0 && ptr_align >= 4 ? 0.66 : 1.94 + 0.35 * std::max(0.0, 5.5 - off);
+    const double rows16 = std::min(m / 16.0, (double)b.fm) + b.fn;
+    const double here = 1.56 + 0.33 * (double)(((kb + 63) / 64 + b.nw * b.u - 1) / (b.nw * b.u)) + 0.06e-6 * n * kb + 0.62 * out
+                        + rounds * chunks * (64 * rows16 * l1_clocks + 6 * b.fm * b.fn) / 2400;
+    const double moved = 1e-6 * ((double)m + n) * (kp / 2), mfma = 2.0 * m * n * kp / 4.5e9, steps = kp / 128;
+    const double copies = m <= 64 ? 5.35 + 0.425 * moved + 0.025 * steps + 0.54 * out + 1.9 * mfma : 6.7 + 0.52 * moved + 0.034 * steps + 0.18 * out + 1.66 * mfma;
+    return here < copies;
 }
 
 // Automatic choice only: K padded to a multiple of 128 (operands copied into the workspace) so
@@ -257,22 +277,12 @@ static hipError_t launch_ragged(const GemmArgs &p, hipStream_t s)
     return hipGetLastError();
 }
 
-// The largest block that leaves more than half of the 256 CUs a workgroup of their own: it reads
-// (rows + columns) x K / 2 bytes per rows x columns of C, but a workgroup's time is its K loop
-// and an idle CU helps nobody.  us, on blocks of 2x1, 2x2, 4x2 and 4x4 times 16: 17 x 3307 x 4100 10.0,
-// 13.2, 15.4, 21.8; 64 x 3307 x 4100 23.0, 16.1, 23.5, 30.1; 200 x 3307 x 4100 59, 43, 44, 31; 100 x 1001 x
-// 1002 3.5, 4.2, 5.3, 6.7; 64 x 9000 x 9000 64, 45, 53, 34.  Up to 16 rows, 1x1 and 1x2: 16 x 3307 x 4100 8.9,
-// 12.1; 16 x 5001 x 2050 9.5, 7.8.  One thread per element, which these calls used to run on: 1 x 9000
-// x 9000 264 us (here 14.5), 16 x 700 x 8998 195 (12.6), 64 x 1001 x 1002 19 (3.4).
 static hipError_t launch_ragged(const GemmArgs &p, hipStream_t s)
 {
-    const auto crowded = [&](int fm, int fn) { return (long long)((p.N + 16 * fn - 1) / (16 * fn)) * ((p.M + 16 * fm - 1) / (16 * fm)) > 128; };
-    if (p.M <= 16 && crowded(1, 2)) return launch_ragged<RaggedCfg<1, 2, 8, 2>>(p, s);
-    if (p.M <= 16) return launch_ragged<RaggedCfg<1, 1, 16, 2>>(p, s);
-    if (p.M > 32 && crowded(4, 4)) return launch_ragged<RaggedCfg<4, 4, 8, 1>>(p, s);
-    if (p.M > 32 && crowded(4, 2)) return launch_ragged<RaggedCfg<4, 2, 8, 2>>(p, s);
-    if (crowded(2, 2)) return launch_ragged<RaggedCfg<2, 2, 8, 2>>(p, s);
-    return launch_ragged<RaggedCfg<2, 1, 16, 2>>(p, s);
+    const RaggedBlock b = ragged_block(p.M, p.N);
+    if (b.fm == 1) return b.fn == 2 ? launch_ragged<RaggedCfg<1, 2, 8, 2>>(p, s) : launch_ragged<RaggedCfg<1, 1, 16, 2>>(p, s);
+    if (b.fm == 4) return b.fn == 4 ? launch_ragged<RaggedCfg<4, 4, 8, 1>>(p, s) : launch_ragged<RaggedCfg<4, 2, 8, 2>>(p, s);
+    return b.fn == 2 ? launch_ragged<RaggedCfg<2, 2, 8, 2>>(p, s) : launch_ragged<RaggedCfg<2, 1, 16, 2>>(p, s);
 }
 
 static Choice choice_from_code(int cfg)

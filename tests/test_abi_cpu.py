@@ -141,15 +141,16 @@ def test_no_workspace_for_calls_that_run_on_the_kernel_for_any_address(scaled):
     up = lambda v: (v + 255) // 256 * 256
     copies = lambda m, n, k: up(m * ((k + 127) // 128 * 64)) + up(n * ((k + 127) // 128 * 64))
     assert ws(1, 28672, 8194) == ws(1, 28672, 9002) == ws(2, 28672, 9002) == 0
-    assert ws(3, 28672, 9002) == copies(3, 28672, 9002) > qm.STATIC_SCRATCH_BYTES
-    # rows on multiples of four bytes: up to 64 rows, and as many more as the product has columns for
-    assert ws(64, 9000, 9000) == ws(300, 9000, 9000) == ws(32, 50000, 4104) == 0
-    assert ws(400, 9000, 9000) == copies(400, 9000, 9000) and ws(64, 9000, 9000, 2) == copies(64, 9000, 9000)
-    assert ws(300, 2000, 28672, 4) == 0 and ws(300, 8000, 28672, 4) == copies(300, 8000, 28672) and ws(300, 2000, 28672, 16) == 0
-    # rows that are not: a few bytes off a multiple of 1024 (4102 / 2 = 2051), and elsewhere (4000 / 2 - 48)
-    assert ws(16, 9000, 4102) == 0 and ws(17, 9000, 4102) == copies(17, 9000, 4102)
-    assert ws(32, 9000, 3902) == 0 and ws(33, 9000, 3902) == copies(33, 9000, 3902)
-    assert ws(117, 4732, 780) == 0 and ws(200, 6001, 780) == copies(200, 6001, 780)
+    # rows on multiples of four bytes: up to a hundred rows and more
+    assert ws(64, 9000, 9000) == ws(128, 9000, 9000) == ws(32, 50000, 4104) == 0
+    assert ws(400, 9000, 9000) == copies(400, 9000, 9000) > qm.STATIC_SCRATCH_BYTES // 2
+    # the same rows at an address that is not
+    assert ws(64, 9000, 9000, 2) == copies(64, 9000, 9000) and ws(64, 9000, 9000, 4) == 0
+    # rows that are not: fewer of them, and fewer still a byte off a multiple of 128 (2049), not seven (2055)
+    assert ws(32, 28672, 4110) == ws(16, 28672, 4110) == 0 and ws(200, 28672, 4110) == copies(200, 28672, 4110)
+    assert ws(16, 28672, 4098) == copies(16, 28672, 4098)
+    # above 512 rows small products only
+    assert ws(512, 700, 1096) == ws(513, 700, 1096) == 0 and ws(1000, 1000, 1000) == copies(1000, 1000, 1000)
 
 
 def test_version_names_the_compiler():
