@@ -115,8 +115,8 @@ int qm_config_has_scaled(int cfg); /* 1 / 0 */
  * C.  The second use (cfg = QM_CFG_AUTO only): large shapes whose K is not a multiple of
  * 32, or whose operands are not 16-byte aligned, get copies of A and B in the workspace
  * with every row padded with zeros to whole 128-nibble steps, and run on the pipelined
- * kernel, except where the kernel for operands at any address is faster.  Results are identical to the forms without a
- * workspace.
+ * kernel, except where the kernel for operands at any address is faster.  Results are identical
+ * to the forms without a workspace.
  *   workspace        device memory, 16-byte aligned, or NULL; used by the kernels of this
  *                    call only (in stream order): calls that may overlap on the GPU need
  *                    a workspace each, calls on one stream can share one
@@ -168,8 +168,13 @@ int qm_gemm_i4_static(const void *A, const void *B, void *C, int m, int n, int k
 
 /* The configuration qm_gemm_i4_ws picks for this shape when it is given a workspace
  * (the table lookup the reference does at kernel.cu:340-385, here with a heuristic
- * fallback instead of a silent no-op); without a workspace the K split may be lower.  ptr_align is the smallest alignment in bytes shared by A and
- * B (pass 16 or more when they come from a device allocator). */
+ * fallback instead of a silent no-op); without a workspace the K split may be lower.  ptr_align is the
+ * smallest alignment in bytes shared by A and B (pass 16 or more when they come from a device
+ * allocator).  "generic" (configuration 0) stands for operands that no other configuration takes:
+ * called with QM_CFG_AUTO they run on the kernel for operands at any address, which has no id of its
+ * own, or on zero-padded copies in the workspace, and where neither takes them (k < 32 or more than
+ * 16 x 65535 rows without copies, k > 131071, operands of 2 GiB and more) on one thread per element.
+ * Id 0 passed to qm_gemm_i4_cfg asks for one thread per element whatever the shape, many times slower. */
 int qm_select_config(int m, int n, int k, int ptr_align);
 /* The same for every form of the call: has_workspace = 0 gives what qm_gemm_i4 / qm_gemm_i4_cfg
  * (QM_CFG_AUTO) run, which never split K through a workspace; scaled = 1 the choice of the

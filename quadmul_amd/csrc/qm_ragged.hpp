@@ -4,8 +4,11 @@
 // The reference has no such path (its shapes are the rows of a table, kernel.cu:340-385).
 // Without it these calls ran on one thread per element of C (small products) or on
 // zero-padded copies of both operands (2 x (M + N) K / 2 bytes of extra traffic, which is
-// most of the time while M is small).  Bound: HBM for a few rows (3 x 9000 x 9000 12 us, 3.4 TB/s
-// of B), the latency of a wave's K loop otherwise.  The decomposition is that of gemm_skinny_kernel: a
+// most of the time while M is small).  Bound: where rows do not lie on multiples of four bytes the L1, which
+// takes the 16 bytes of such a lane in four accesses, one access per clock (16 x 65536 x 4100: 52.8 M accesses, 4.07 per
+// lane and load, 0.99 per clock and CU; 78 us, 1.7 TB/s of B, each byte of it fetched once); where they do (0.87 per lane and
+// load), HBM on a wide B (16 x 65536 x 8200 77 us, 3.5 TB/s; 3 x 9000 x 9000 12 us, 3.4 TB/s), the latency
+// of a wave's K loop otherwise.  The decomposition is that of gemm_skinny_kernel: a
 // workgroup owns 16*FM rows of A (grid.y walks over blocks of them) and 16*FN rows of B, its
 // NW waves split K in 128-nibble chunks, partial blocks meet in the LDS.  Lane (r, g) loads the
 // 16 bytes it feeds to the matrix core itself -- row r, bytes 16 g .. + 15 of the chunk's 64 --
