@@ -238,11 +238,13 @@ static PadPlan plan_padded_k(int m, int n, int k, int ptr_align, const Choice &d
     PadPlan pl;
     const int kind = g_configs[direct.cfg].kind;
     if (kind == KIND_TILE16 || kind == KIND_SKINNY) return pl;
-    if (ragged_fits(m, n, k) && ragged_before_copies(m, n, k, ptr_align)) return pl;
     const int kp = (k + 127) / 128 * 128;
-    if (kp > QM_MAX_K_X16 || !fast_path_ok(m, n, kp, 256)) return pl;
     const long long outs = (long long)m * n;
-    if (outs * kp < (1LL << 27)) return pl;  // (kp: a K below one K-step counts as the step it is padded to)
+    // (kp: a K below one K-step counts as the step it is padded to.  Before the costs, which are worked out
+    // twice a call, 30 to 50 ns each time: small products are bound by the host)
+    if (outs * kp < (1LL << 27)) return pl;
+    if (ragged_fits(m, n, k) && ragged_before_copies(m, n, k, ptr_align)) return pl;
+    if (kp > QM_MAX_K_X16 || !fast_path_ok(m, n, kp, 256)) return pl;
     Choice ch = heuristic(m, n, kp, 256, false);
     if (g_configs[ch.cfg].kind == KIND_GENERIC) return pl;
     ch.ksplit = 1;
