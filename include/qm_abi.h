@@ -42,6 +42,8 @@ extern "C" {
                                    QM_STATIC_SCRATCH_BYTES                                   */
 
 #define QM_CFG_AUTO          -1 /* let the shape table / heuristic choose                   */
+#define QM_CFG_RECODE        -2 /* 6-bit operands whether they pay or not: see
+                                   qm_gemm_recode_bytes                                      */
 
 /*
  * The hot path.  Replaces
@@ -142,6 +144,17 @@ int qm_gemm_i4_scaled_bias_ws(const void *A, const void *B, void *D, int m, int 
                               const float *col_scale, const void *bias, int out_dtype, void *stream, int cfg,
                               void *workspace, size_t workspace_bytes);
 size_t qm_gemm_workspace_bytes(int m, int n, int k, int ptr_align, int cfg, int scaled);
+/*
+ * The bytes of workspace with which a large product (cfg = QM_CFG_AUTO) runs faster still: A is re-coded
+ * there as 6-bit floats, three quarters of a byte per element, for a matrix instruction that takes twice
+ * as many of them as int8 values.  The results are the same bit for bit.  0 where that does not pay, or
+ * would take more than 256 MiB; the call itself never needs it: with a workspace of fewer bytes, it runs as
+ * described above.  A caller that wants both lends the larger of the two sizes.
+ * With cfg = QM_CFG_RECODE the two calls above run on them wherever they can: K a multiple of 32 from 256 to
+ * 65535, 256 columns and more, 16-byte aligned operands, a workspace of
+ * qm_gemm_workspace_bytes(..., QM_CFG_RECODE, scaled) bytes; QM_ERR_CONFIG elsewhere, and from the calls that take none.
+ */
+size_t qm_gemm_recode_bytes(int m, int n, int k, int ptr_align, int scaled);
 
 /*
  * qm_gemm_i4 for callers that cannot allocate and have no workspace to lend: code under HIP

@@ -34,10 +34,11 @@ _LIB_PATH = os.path.join(_PKG, "lib", "libqm_hip.so")
 _lib: Optional[ctypes.CDLL] = None
 
 CFG_AUTO = -1
+CFG_RECODE = -2
 #: every symbol include/qm_abi.h declares
 ABI_SYMBOLS = (
     "qm_gemm_i4", "qm_gemm_i4_cfg", "qm_gemm_i4_scaled", "qm_gemm_i4_scaled_cfg", "qm_config_has_scaled",
-    "qm_gemm_i4_ws", "qm_gemm_i4_static", "qm_gemm_i4_scaled_ws", "qm_gemm_i4_scaled_bias_ws", "qm_gemm_workspace_bytes", "qm_quantize_pack_i4", "qm_select_config", "qm_select_config_ex", "qm_num_configs", "qm_config_name",
+    "qm_gemm_i4_ws", "qm_gemm_i4_static", "qm_gemm_i4_scaled_ws", "qm_gemm_i4_scaled_bias_ws", "qm_gemm_workspace_bytes", "qm_gemm_recode_bytes", "qm_quantize_pack_i4", "qm_select_config", "qm_select_config_ex", "qm_num_configs", "qm_config_name",
     "qm_config_supports", "qm_pack_i4", "qm_unpack_i4", "qm_status_string", "qm_last_hip_error", "qm_version", "qm_init",
     "qm_debug_set_operand_limit",
 )
@@ -80,6 +81,8 @@ def library() -> ctypes.CDLL:
     lib.qm_gemm_i4_scaled_bias_ws.restype = ci
     lib.qm_gemm_workspace_bytes.argtypes = [ci, ci, ci, ci, ci, ci]
     lib.qm_gemm_workspace_bytes.restype = ctypes.c_size_t
+    lib.qm_gemm_recode_bytes.argtypes = [ci, ci, ci, ci, ci]
+    lib.qm_gemm_recode_bytes.restype = ctypes.c_size_t
     lib.qm_config_has_scaled.argtypes = [ci]
     lib.qm_config_has_scaled.restype = ci
     lib.qm_quantize_pack_i4.argtypes = [vp, ci, vp, vp, ci, ci, vp]
@@ -192,6 +195,11 @@ def workspace_bytes(m: int, n: int, k: int, cfg: int = CFG_AUTO, scaled: bool = 
     return int(library().qm_gemm_workspace_bytes(m, n, k, ptr_align, cfg, 1 if scaled else 0))
 
 
+def recode_bytes(m: int, n: int, k: int, scaled: bool = False, ptr_align: int = 256) -> int:
+    """Bytes of workspace with which a large product runs on 6-bit re-coded operands (0: that would not pay)."""
+    return int(library().qm_gemm_recode_bytes(m, n, k, ptr_align, 1 if scaled else 0))
+
+
 def _workspace(workspace, a, b, m, n, k, cfg, scaled):
     """(pointer, bytes, keep-alive) of the workspace argument: True = allocate what the call
     can use from torch's caching allocator (stream-ordered, so safe across streams and under
@@ -200,6 +208,8 @@ def _workspace(workspace, a, b, m, n, k, cfg, scaled):
         return None, 0, None
     if workspace is True:
         need = workspace_bytes(m, n, k, cfg, scaled, _ptr_align(a, b))
+        if cfg == CFG_AUTO:
+            need = max(need, recode_bytes(m, n, k, scaled, _ptr_align(a, b)))
         if need == 0:
             return None, 0, None
         workspace = torch.empty((need,), dtype=torch.uint8, device=a.device)

@@ -120,6 +120,7 @@ def build_lib(jobs: int = 8, verbose: bool = False) -> str:
     units = [("qm_dispatch.o", [f'-DQM_COMPILER_VERSION="{ver}"', "-mllvm", "-amdgpu-kernarg-preload-count=16", "-c", os.path.join(CSRC, "qm_dispatch.hip")]),
              ("qm_scratch.o", ["-c", os.path.join(CSRC, "qm_scratch.hip")])]
     # (the units with the scaled-output kernels, 6 and up, take longest: they go first)
+    units = [(f"qm_tile6_inst_{out}.o", [f"-DQM_TILE6_OUT={out}", "-c", os.path.join(CSRC, "qm_tile6_inst.hip")]) for out in (0, 1, 2)] + units
     units = [(f"qm_tile_inst_{tu}.o", [f"-DQM_TU={tu}", "-c", os.path.join(CSRC, "qm_tile_inst.hip")])
              for tu in sorted(range(N_TILE_TUS), key=lambda t: (t < 6, t))] + units
     # (a directory per unit: the compiler's intermediate files, kept for the scan below, are

@@ -64,7 +64,9 @@ int ptr_alignment(const torch::Tensor &a, const torch::Tensor &b)
 
 torch::Tensor workspace_for(const torch::Tensor &a, const torch::Tensor &b, int64_t m, int64_t n, int64_t k, int cfg, bool scaled)
 {
-    const size_t need = qm_gemm_workspace_bytes((int)m, (int)n, (int)k, ptr_alignment(a, b), cfg, scaled ? 1 : 0);
+    const int align = ptr_alignment(a, b);
+    size_t need = qm_gemm_workspace_bytes((int)m, (int)n, (int)k, align, cfg, scaled ? 1 : 0);
+    if (cfg == QM_CFG_AUTO) need = std::max(need, qm_gemm_recode_bytes((int)m, (int)n, (int)k, align, scaled ? 1 : 0));
     if (need == 0) return torch::Tensor();
     return torch::empty({(int64_t)need}, a.options().dtype(torch::kUInt8));
 }
@@ -168,7 +170,8 @@ torch::Tensor linear(torch::Tensor x, torch::Tensor weight, int64_t n, c10::opti
     const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     const size_t packed_bytes = up((size_t)m * (k / 2)), scale_bytes = up((size_t)m * sizeof(float));
     const int align = (int)std::min<uintptr_t>(256, weight.data_ptr() ? (uintptr_t)weight.data_ptr() & -(uintptr_t)weight.data_ptr() : 256);
-    const size_t ws_bytes = qm_gemm_workspace_bytes((int)m, (int)n, (int)k, align, QM_CFG_AUTO, 1);
+    const size_t ws_bytes = std::max(qm_gemm_workspace_bytes((int)m, (int)n, (int)k, align, QM_CFG_AUTO, 1),
+                                     qm_gemm_recode_bytes((int)m, (int)n, (int)k, align, 1));
     auto scratch = torch::empty({(int64_t)(packed_bytes + scale_bytes + ws_bytes)}, x.options().dtype(torch::kUInt8));
     uint8_t *const xq = scratch.data_ptr<uint8_t>();
     float *const xs = reinterpret_cast<float *>(xq + packed_bytes);

@@ -14,6 +14,7 @@
 #include "qm_skinny_dma.hpp"
 #include "qm_ragged.hpp"
 #include "qm_aux.hpp"
+#include "qm_expand6.hpp"
 
 #define QM_EXPORT extern "C" __attribute__((visibility("default")))
 
@@ -66,24 +67,6 @@ static hipError_t launch_skinny_dma(const GemmArgs &p, hipStream_t stream, int o
     gemm_skinny_dma_kernel<Cfg><<<dim3(blocks, row_blocks), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(
         p.A, p.B, p.C, pack_rows_out(p.M, p.out), p.N, p.K, p.ldc, p.row_scale, p.col_scale, p.bias);
     return hipGetLastError();
-}
-// Compute units of the current device (asked once per device).
-static hipError_t device_cus(int *cus)
-{
-    static std::atomic<int> cached[QM_MAX_DEVICES] = {};
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    if (dev < 0 || dev >= QM_MAX_DEVICES) return hipErrorInvalidDevice;
-    int n = cached[dev].load(std::memory_order_acquire);
-    if (n == 0) {
-        e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-        if (e != hipSuccess) return e;
-        if (n < 1) n = 1;
-        cached[dev].store(n, std::memory_order_release);
-    }
-    *cus = n;
-    return hipSuccess;
 }
 template <class Cfg>
 static hipError_t launch_skinny_stream_dma(const GemmArgs &p, hipStream_t stream, int opt)
@@ -271,6 +254,49 @@ static hipError_t launch_padded(GemmArgs &p, const PadPlan &pl, void *ws, hipStr
     return hipSuccess;
 }
 
+// The same product on the tile kernel for 6-bit floats (qm_tile6.hpp), A re-coded in the workspace ahead of it.
+static bool fp6_fits(int m, int n, int k, int ptr_align)
+{
+    if (k < 256 || k > QM_MAX_K_FP6 || !fast_path_ok(m, n, k, ptr_align)) return false;
+    return n >= 256 && n < (1 << 21) && fp6_layout(m, k).code_bytes <= QM_FP6_MAX_BYTES;
+}
+
+// What it takes (us), re-coding included, in the terms of modelled_us: fitted to 312 products of 200 to 8192 rows (rms
+// of the fit 7 %), 256 x 256 tiles, one workgroup per CU.  A K-step costs 0.83 us where the int8 tile of the same size takes
+// 1.19, a round of tiles 15 against 10, the re-coding 0.22 us per million elements of A and a launch of its own.
+static double fp6_us(int m, int n, int k)
+{
+    const double kt = (k + 127) / 128, share = (double)((m + 255) / 256) * (double)((n + 255) / 256) / 256;
+    const double rounds = 0.75 * std::ceil(share) + 0.25 * std::max(1.0, share);
+    return kt * (rounds * (k & 255 ? 0.612 : 0.539) + std::min(1.0, share) * 0.290) + rounds * 15.07 + 0.2203e-6 * m * k - 0.67;
+}
+
+// Automatic choice: where that is 5 % less than what the model says of the int8 configuration `direct`.  Of those 312
+// products it takes 66, on which the time falls by 14 % in the mean (1280 x 8192 x 14336 124 -> 91 us, 8192 x 8192 x 8192 336 -> 290,
+// 512 x 28672 x 4096 46.0 -> 41.8) and rises by more than 1 % on one (4.7 %).  Without the margin it takes ten more, seven of
+// them at a gain and nothing over all; below a K of 1280 the fit is off by up to 25 % and what it takes gains nothing.
+// (The bound on the product comes first: calls that the host bounds do not get as far as the model.)
+static bool fp6_pays(int m, int n, int k, int ptr_align, const Choice &direct)
+{
+    if ((double)m * n * k < 4e9 || k < 1280 || !fp6_fits(m, n, k, ptr_align)) return false;
+    const ConfigDesc &d = g_configs[direct.cfg];
+    for (const CostFit &f : g_cost_fits)
+        if (std::strcmp(f.name, d.name) == 0) return fp6_us(m, n, k) < 0.95 * modelled_us(f, d, m, n, k, direct.ksplit);
+    return false;
+}
+
+static auto tile6_launcher(int out) { return out == OUT_I32 ? &launch_tile6_i32 : out == OUT_F16 ? &launch_tile6_f16 : &launch_tile6_bf16; }
+
+static hipError_t launch_fp6(const GemmArgs &p, void *ws, hipStream_t s)
+{
+    const Fp6Operand a = fp6_operand(p.M, p.K, ws);
+    const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, a.layout.kt, a.layout.groups};
+    expand_a6_kernel<<<dim3(2 * a.layout.groups, a.layout.parts), dim3(512), 0, s>>>(q);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return tile6_launcher(p.out)(p, a, s, 0);
+}
+
 template <class Cfg>
 static hipError_t launch_ragged(const GemmArgs &p, hipStream_t s)
 {
@@ -414,6 +440,11 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
     p.out = out;
     p.ldc = strided ? row_stride : 0;
     if (strided && cfg != QM_CFG_AUTO) return QM_ERR_CONFIG;
+    if (cfg == QM_CFG_RECODE) {
+        if (!fp6_fits(m, n, k, align) || workspace == nullptr || ((uintptr_t)workspace & 15) || workspace_bytes < fp6_layout(m, k).bytes) return QM_ERR_CONFIG;
+        const hipError_t e = launch_fp6(p, workspace, s);
+        return e == hipSuccess ? QM_OK : fail_launch(e);
+    }
     const auto launcher = [&](int id) { return scaled ? scaled_launcher(id) : g_configs[id].launch; };
     Choice ch;
     if (strided) {
@@ -434,6 +465,10 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
         if (ch.ksplit > 1 && g_configs[ch.cfg].kind != KIND_TILE16) return QM_ERR_CONFIG;
     }
     ch.ksplit = effective_ksplit(g_configs[ch.cfg], k, ch.ksplit);
+    if (cfg == QM_CFG_AUTO && has_ws && ((uintptr_t)workspace & 15) == 0 && fp6_pays(m, n, k, align, ch) && workspace_bytes >= fp6_layout(m, k).bytes) {
+        const hipError_t e = launch_fp6(p, workspace, s);
+        return e == hipSuccess ? QM_OK : fail_launch(e);
+    }
     if (ch.ksplit > 1 && workspace_fits(g_configs[ch.cfg], m, n, ch.ksplit, workspace, workspace_bytes)) {
         const hipError_t e = launch_split_with_workspace(p, ch, workspace, s);
         return e == hipSuccess ? QM_OK : fail_launch(e);
@@ -507,6 +542,12 @@ QM_EXPORT int qm_init(void)
             }
         }
     }
+    for (const int out : {(int)OUT_I32, (int)OUT_F16, (int)OUT_BF16})
+        for (const uint16_t *bias : {(const uint16_t *)nullptr, &no_bias}) {
+            p.bias = out == OUT_I32 ? nullptr : bias;
+            const hipError_t e = tile6_launcher(out)(p, Fp6Operand{}, nullptr, QM_OPT_PREPARE);
+            if (e != hipSuccess) return fail_launch(e);
+        }
     void *ws = nullptr;
     const hipError_t e = static_scratch(&ws);
     return e == hipSuccess ? QM_OK : fail_launch(e);
@@ -524,8 +565,7 @@ QM_EXPORT int qm_gemm_i4_static(const void *A, const void *B, void *C, int m, in
         const hipError_t e = static_scratch(&ws);
         if (e != hipSuccess) return fail_launch(e);
     }
-    return run_gemm(A, B, C, m, n, k, nullptr, nullptr, OUT_I32, reinterpret_cast<hipStream_t>(stream), QM_CFG_AUTO, ws,
-                    ws ? (size_t)QM_STATIC_SCRATCH_BYTES : 0);
+    return run_gemm(A, B, C, m, n, k, nullptr, nullptr, OUT_I32, reinterpret_cast<hipStream_t>(stream), QM_CFG_AUTO, ws, ws ? need : 0);
 }
 
 QM_EXPORT int qm_gemm_i4_cfg(const void *A, const void *B, void *C, int m, int n, int k, void *stream, int cfg)
@@ -576,6 +616,7 @@ QM_EXPORT size_t qm_gemm_workspace_bytes(int m, int n, int k, int ptr_align, int
         return whole > rest ? whole : rest;
     }
     if (cfg == QM_CFG_AUTO && col_block_for_large_b(m, n, k, ptr_align)) return 0;  // blocks of columns: one launch each, no workspace
+    if (cfg == QM_CFG_RECODE) return fp6_fits(m, n, k, ptr_align) ? fp6_layout(m, k).bytes : 0;
     Choice ch;
     if (cfg == QM_CFG_AUTO) {
         ch = scaled ? select_scaled(m, n, k, ptr_align, true) : select_config(m, n, k, ptr_align, true);
@@ -590,6 +631,15 @@ QM_EXPORT size_t qm_gemm_workspace_bytes(int m, int n, int k, int ptr_align, int
         if (pl.on) return pl.bytes();
     }
     return 0;
+}
+
+QM_EXPORT size_t qm_gemm_recode_bytes(int m, int n, int k, int ptr_align, int scaled)
+{
+    if (m < 1 || n < 1 || (double)m * n * k < 4e9 || (k & 1) || !fp6_fits(m, n, k, ptr_align)) return 0;
+    if (row_block_for_large_a(m, n, k, ptr_align) || col_block_for_large_b(m, n, k, ptr_align)) return 0;
+    Choice ch = scaled ? select_scaled(m, n, k, ptr_align, true) : select_config(m, n, k, ptr_align, true);
+    ch.ksplit = effective_ksplit(g_configs[ch.cfg], k, ch.ksplit);
+    return fp6_pays(m, n, k, ptr_align, ch) ? fp6_layout(m, k).bytes : 0;
 }
 
 QM_EXPORT int qm_config_has_scaled(int cfg)

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <atomic>
 #include "qm_common.hpp"
+#include "qm_fp6.hpp"
 
 namespace qm {
 
@@ -56,6 +57,30 @@ constexpr size_t kernarg_bytes(void (*)(Args...))
     ((at = (at + alignof(Args) - 1) / alignof(Args) * alignof(Args) + sizeof(Args)), ...);
     return at;
 }
+
+// Compute units of the current device (asked once per device).
+inline hipError_t device_cus(int *cus)
+{
+    static std::atomic<int> cached[QM_MAX_DEVICES] = {};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    if (dev < 0 || dev >= QM_MAX_DEVICES) return hipErrorInvalidDevice;
+    int n = cached[dev].load(std::memory_order_acquire);
+    if (n == 0) {
+        e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+        if (e != hipSuccess) return e;
+        if (n < 1) n = 1;
+        cached[dev].store(n, std::memory_order_release);
+    }
+    *cus = n;
+    return hipSuccess;
+}
+
+// The tile kernel on 6-bit floats (qm_tile6_inst.hip).
+hipError_t launch_tile6_i32(const GemmArgs &p, const Fp6Operand &a, hipStream_t s, int opt);
+hipError_t launch_tile6_f16(const GemmArgs &p, const Fp6Operand &a, hipStream_t s, int opt);
+hipError_t launch_tile6_bf16(const GemmArgs &p, const Fp6Operand &a, hipStream_t s, int opt);
 
 // The address, on the current device, of the library's own scratch array (qm_scratch.hip).
 hipError_t static_scratch(void **out);
