@@ -225,6 +225,19 @@ int qm_unpack_i4(const void *src_packed, void *dst_i8, int rows, int k, void *st
 int qm_quantize_pack_i4(const void *x, int in_dtype, void *dst_packed, float *scales, int rows, int k, void *stream);
 
 /*
+ * The int4 linear layer in one call: the rows of x quantised as qm_quantize_pack_i4 quantises them, the GEMM with the scaled
+ * output on them -- D[m][n] as qm_gemm_i4_scaled_bias_ws gives it with their scales as row_scale -- and
+ * the same values bit for bit as those two calls one after the other.  The reference has no counterpart.
+ * Large products go from x to the 6-bit operands of qm_gemm_recode_bytes without the packed rows in between.
+ *   workspace    device memory, 256-byte aligned, at least qm_linear_workspace_bytes(...) bytes (weight_align: the
+ *                alignment of B in bytes), else QM_ERR_SCRATCH and nothing is enqueued; used in stream order by
+ *                the kernels of this call only
+ */
+size_t qm_linear_workspace_bytes(int m, int n, int k, int in_dtype, int weight_align);
+int qm_linear_i4(const void *x, int in_dtype, const void *B, void *D, int m, int n, int k, const float *col_scale,
+                 const void *bias, int out_dtype, void *stream, void *workspace, size_t workspace_bytes);
+
+/*
  * Optional: everything a first launch on the current device would otherwise do once -- the
  * LDS size attribute and the residency query of every kernel, the address of the library's
  * scratch array -- without launching anything.  No counterpart in the reference (its

@@ -40,7 +40,7 @@ ABI_SYMBOLS = (
     "qm_gemm_i4", "qm_gemm_i4_cfg", "qm_gemm_i4_scaled", "qm_gemm_i4_scaled_cfg", "qm_config_has_scaled",
     "qm_gemm_i4_ws", "qm_gemm_i4_static", "qm_gemm_i4_scaled_ws", "qm_gemm_i4_scaled_bias_ws", "qm_gemm_workspace_bytes", "qm_gemm_recode_bytes", "qm_quantize_pack_i4", "qm_select_config", "qm_select_config_ex", "qm_num_configs", "qm_config_name",
     "qm_config_supports", "qm_pack_i4", "qm_unpack_i4", "qm_status_string", "qm_last_hip_error", "qm_version", "qm_init",
-    "qm_debug_set_operand_limit",
+    "qm_debug_set_operand_limit", "qm_linear_workspace_bytes", "qm_linear_i4",
 )
 
 
@@ -83,6 +83,10 @@ def library() -> ctypes.CDLL:
     lib.qm_gemm_workspace_bytes.restype = ctypes.c_size_t
     lib.qm_gemm_recode_bytes.argtypes = [ci, ci, ci, ci, ci]
     lib.qm_gemm_recode_bytes.restype = ctypes.c_size_t
+    lib.qm_linear_workspace_bytes.argtypes = [ci, ci, ci, ci, ci]
+    lib.qm_linear_workspace_bytes.restype = ctypes.c_size_t
+    lib.qm_linear_i4.argtypes = [vp, ci, vp, vp, ci, ci, ci, vp, vp, ci, vp, vp, ctypes.c_size_t]
+    lib.qm_linear_i4.restype = ci
     lib.qm_config_has_scaled.argtypes = [ci]
     lib.qm_config_has_scaled.restype = ci
     lib.qm_quantize_pack_i4.argtypes = [vp, ci, vp, vp, ci, ci, vp]

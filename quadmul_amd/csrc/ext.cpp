@@ -149,8 +149,7 @@ std::tuple<torch::Tensor, torch::Tensor> quantize_pack(torch::Tensor x)
 }
 
 // The W4A4 linear layer (quadmul_amd/linear.py) in one call: quantise + pack the rows of x, then the
-// GEMM with the scaled output and the bias.  The packed rows, their scales and the workspace of a K split
-// share one allocation.
+// GEMM with the scaled output and the bias.  What lies between the two is in one allocation.
 torch::Tensor linear(torch::Tensor x, torch::Tensor weight, int64_t n, c10::optional<torch::Tensor> weight_scale, c10::optional<torch::Tensor> bias, bool bf16)
 {
     const auto t = x.scalar_type();
@@ -167,20 +166,13 @@ torch::Tensor linear(torch::Tensor x, torch::Tensor weight, int64_t n, c10::opti
                 "quadmul.linear: the bias must be a contiguous vector of ", n, " elements of the output's type on x's device");
     c10::OptionalDeviceGuard guard(x.device());
     auto y = torch::empty({m, n}, x.options().dtype(out));
-    const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
-    const size_t packed_bytes = up((size_t)m * (k / 2)), scale_bytes = up((size_t)m * sizeof(float));
-    const int align = (int)std::min<uintptr_t>(256, weight.data_ptr() ? (uintptr_t)weight.data_ptr() & -(uintptr_t)weight.data_ptr() : 256);
-    const size_t ws_bytes = std::max(qm_gemm_workspace_bytes((int)m, (int)n, (int)k, align, QM_CFG_AUTO, 1),
-                                     qm_gemm_recode_bytes((int)m, (int)n, (int)k, align, 1));
-    auto scratch = torch::empty({(int64_t)(packed_bytes + scale_bytes + ws_bytes)}, x.options().dtype(torch::kUInt8));
-    uint8_t *const xq = scratch.data_ptr<uint8_t>();
-    float *const xs = reinterpret_cast<float *>(xq + packed_bytes);
     const int in = t == torch::kFloat16 ? QM_IN_F16 : (t == torch::kBFloat16 ? QM_IN_BF16 : QM_IN_F32);
-    check_status(qm_quantize_pack_i4(x.data_ptr(), in, xq, xs, (int)m, (int)k, stream_of(x)), "quadmul.linear");
-    check_status(qm_gemm_i4_scaled_bias_ws(xq, weight.data_ptr(), y.data_ptr(), (int)m, (int)n, (int)k, xs,
-                                           weight_scale.has_value() ? weight_scale->data_ptr<float>() : nullptr,
-                                           bias.has_value() ? bias->data_ptr() : nullptr, bf16 ? QM_OUT_BF16 : QM_OUT_F16, stream_of(x), QM_CFG_AUTO,
-                                           ws_bytes ? xq + packed_bytes + scale_bytes : nullptr, ws_bytes),
+    const size_t need = qm_linear_workspace_bytes((int)m, (int)n, (int)k, in, ptr_alignment(weight, weight));
+    torch::Tensor scratch;
+    if (need > 0) scratch = torch::empty({(int64_t)need}, x.options().dtype(torch::kUInt8));
+    check_status(qm_linear_i4(x.data_ptr(), in, weight.data_ptr(), y.data_ptr(), (int)m, (int)n, (int)k,
+                              weight_scale.has_value() ? weight_scale->data_ptr<float>() : nullptr, bias.has_value() ? bias->data_ptr() : nullptr,
+                              bf16 ? QM_OUT_BF16 : QM_OUT_F16, stream_of(x), need > 0 ? scratch.data_ptr() : nullptr, need),
                  "quadmul.linear");
     return y;
 }

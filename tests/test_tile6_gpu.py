@@ -137,3 +137,49 @@ def test_what_it_cannot_take_is_refused():
     status(16, 256, 256, a_off=4)
     status(16, 256, 256, ws=None)
     status(16, 256, 256, ws=torch.empty(qm.workspace_bytes(16, 256, 256, qm.CFG_RECODE) - 1, dtype=torch.uint8, device=DEV))
+
+
+# rows that are no multiple of eight, K-steps short and odd in number, each number of chunks per lane, each type
+@pytest.mark.parametrize("m,n,k,dtype", [(1283, 8200, 4096, torch.float16), (1100, 8192, 4128, torch.bfloat16), (2048, 14336, 1984, torch.bfloat16),
+                                         (1100, 8192, 7200, torch.float16), (1031, 8192, 12320, torch.bfloat16), (2048, 14336, 2016, torch.float32),
+                                         (1283, 8192, 4000, torch.float32), (1283, 8192, 6176, torch.float32)], ids=str)
+def test_the_linear_layer_quantises_straight_to_codes(m, n, k, dtype):
+    """... with the values of the two calls one after the other, bit for bit."""
+    gen = torch.Generator(device=DEV).manual_seed(SEED_BASE + 34000 + k)
+    room = torch.randn(m * k + 1, device=DEV, generator=gen).to(dtype)
+    room[5:5 + k] = 0                       # (most of two rows)
+    x = room[1:].view(m, k)                 # aligned to an element only
+    x[7] = 0
+    x[9, 3] = 3e4
+    w, ws = quadmul.quantize_pack(torch.randn(n, k, device=DEV, generator=gen).to(dtype))
+    align = w.data_ptr() & -w.data_ptr()
+    groups, steps = (m + 31) // 32, -(-k // 128) + (-(-k // 128) & 1)
+    types = {torch.float16: 1, torch.bfloat16: 2, torch.float32: 3}
+    assert qm.library().qm_linear_workspace_bytes(m, n, k, types[dtype], align) - (4 * m + 255) // 256 * 256 >= groups * steps * 3072   # codes
+    xq, xs = quadmul.quantize_pack(x)
+    for out in (torch.float16, torch.bfloat16):
+        for bias in (None, torch.randn(n, device=DEV, generator=gen).to(out)):
+            want = torch.empty(m, n, dtype=out, device=DEV)
+            qm.gemm_scaled(xq, w, want, m, n, k, xs, ws, workspace=None, bias=bias)
+            got = quadmul.linear(x, w, n, ws, bias, out == torch.bfloat16)
+            assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (out, bias is None)
+
+
+def test_the_linear_call_refuses_what_it_cannot_do():
+    lib = qm.library()
+    m, n, k = 16, 64, 256
+    x = torch.randn(m, k, device=DEV, dtype=torch.float16)
+    w, ws = quadmul.quantize_pack(torch.randn(n, k, device=DEV, dtype=torch.float16))
+    d = torch.full((m, n), 7.0, dtype=torch.float16, device=DEV)
+    need = lib.qm_linear_workspace_bytes(m, n, k, 1, 256)
+    work = torch.empty(need + 256, dtype=torch.uint8, device=DEV)
+    call = lambda x_ptr, in_type, ws_ptr, ws_bytes, kk=k, out=1: lib.qm_linear_i4(x_ptr, in_type, w.data_ptr(), d.data_ptr(), m, n, kk, ws.data_ptr(), None, out, None,
+                                                                                  ws_ptr, ws_bytes)
+    assert call(x.data_ptr(), 1, work.data_ptr(), need - 1) == -7 and call(x.data_ptr(), 1, None, 0) == -7
+    assert call(x.data_ptr(), 1, work.data_ptr() + 16, need) == -7
+    assert call(x.data_ptr(), 4, work.data_ptr(), need) == call(x.data_ptr(), 1, work.data_ptr(), need, out=3) == -6
+    assert call(x.data_ptr(), 1, work.data_ptr(), need, kk=255) == -2
+    assert call(x.data_ptr() + 1, 1, work.data_ptr(), need) == -5 and call(None, 1, work.data_ptr(), need) == -1
+    torch.cuda.synchronize()
+    assert (d == 7.0).all()
+    assert lib.qm_linear_workspace_bytes(0, n, k, 1, 256) == 0
