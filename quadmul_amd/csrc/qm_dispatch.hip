@@ -15,6 +15,7 @@
 #include "qm_ragged.hpp"
 #include "qm_aux.hpp"
 #include "qm_expand6.hpp"
+#include "qm_dot_linear.hpp"
 
 #define QM_EXPORT extern "C" __attribute__((visibility("default")))
 
@@ -745,7 +746,7 @@ QM_EXPORT int qm_unpack_i4(const void *src_packed, void *dst_i8, int rows, int k
 // for the 6-bit tile kernel, or the packed rows and the GEMM's own workspace.
 namespace {
 struct LinearPlan {
-    bool coded;
+    bool one_launch, coded;
     int align;
     size_t scale_bytes, row_bytes, gemm_bytes;
     size_t bytes() const { return scale_bytes + row_bytes + gemm_bytes; }
@@ -754,6 +755,10 @@ LinearPlan linear_plan(int m, int n, int k, int in_dtype, int weight_align)
 {
     const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     LinearPlan pl{};
+    if (m <= 2 && fast_path_ok(m, n, k, weight_align) && n < (1 << 24) && k < (1 << 24) && dot_linear_lds_bytes(m, k) <= 48 * 1024) {
+        pl.one_launch = true;
+        return pl;
+    }
     pl.align = weight_align < 256 ? weight_align : 256;
     pl.scale_bytes = up((size_t)m * sizeof(float));
     if ((double)m * n * k >= 4e9 && quant6_fits(k, in_dtype) && row_block_for_large_a(m, n, k, pl.align) == 0 && col_block_for_large_b(m, n, k, pl.align) == 0) {
@@ -790,6 +795,13 @@ QM_EXPORT int qm_linear_i4(const void *x, int in_dtype, const void *B, void *D, 
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (k == 0) return run_gemm(nullptr, nullptr, D, m, n, 0, nullptr, col_scale, out, s, QM_CFG_AUTO, nullptr, 0, 0, static_cast<const uint16_t *>(bias));
     const LinearPlan pl = linear_plan(m, n, k, in_dtype, ptr_alignment(B, nullptr));
+    if (pl.one_launch) {
+        const uint16_t *b16 = static_cast<const uint16_t *>(bias);
+        const hipError_t e = in_dtype == QM_IN_F16 ? launch_dot_linear<QM_IN_F16>(x, B, D, m, n, k, col_scale, b16, out, s)
+                             : in_dtype == QM_IN_BF16 ? launch_dot_linear<QM_IN_BF16>(x, B, D, m, n, k, col_scale, b16, out, s)
+                                                      : launch_dot_linear<QM_IN_F32>(x, B, D, m, n, k, col_scale, b16, out, s);
+        return e == hipSuccess ? QM_OK : fail_launch(e);
+    }
     if (workspace == nullptr || ((uintptr_t)workspace & 255) || workspace_bytes < pl.bytes()) return QM_ERR_SCRATCH;
     float *scales = static_cast<float *>(workspace);
     uint8_t *rows = static_cast<uint8_t *>(workspace) + pl.scale_bytes;
