@@ -16,6 +16,15 @@ struct DotLinearCfg {
     static constexpr int NC = 4;  // chunks of eight elements per thread and row that stay in registers between the maximum and the quantisation
 };
 inline int dot_linear_lds_bytes(int mr, int k) { return mr * (k / 2); }
+// Against two launches (us inside a graph, weights from HBM, two / one): 1 x 1024 x 1024 4.46 / 3.18, 1 x 4096 x 4096 5.54 / 4.46,
+// 1 x 4096 x 11008 8.77 / 7.83, 1 x 28672 x 4096 14.2 / 13.1, but 1 x 8192 x 28672 27.1 / 28.2 -- seven turns over K, each waiting for its own
+// loads; two rows 1024 x 1024 4.90 / 3.71, 4096 x 4096 5.99 / 5.13, 4096 x 11008 9.14 / 8.74, but 22016 x 4096 12.6 / 14.2 (every workgroup
+// quantises, and there are 1376 of them) and 8192 x 8192 11.0 / 14.3 (the GEMM by itself runs on the matrix core there).
+inline bool dot_linear_pays(int m, int n, int k)
+{
+    if (k > 16384) return false;
+    return m == 1 || ((long long)n * k <= (3LL << 24) && !(k > 4096 && n >= 8192));
+}
 
 template <int IN, class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS)
@@ -149,7 +158,7 @@ static hipError_t launch_dot_linear(const void *x, const void *B, void *D, int m
 {
     if (m == 2) return k <= 4096 ? launch_dot_linear<IN, 2, 8, 4>(x, B, D, m, n, k, col_scale, bias, out, s) : launch_dot_linear<IN, 2, 16, 2>(x, B, D, m, n, k, col_scale, bias, out, s);
     if (k <= 2048) return launch_dot_linear<IN, 1, 8, 4>(x, B, D, m, n, k, col_scale, bias, out, s);
-    if (k <= 4096 || k > 16384) return launch_dot_linear<IN, 1, 4, 8>(x, B, D, m, n, k, col_scale, bias, out, s);
+    if (k <= 4096) return launch_dot_linear<IN, 1, 4, 8>(x, B, D, m, n, k, col_scale, bias, out, s);
     return launch_dot_linear<IN, 1, 16, 2>(x, B, D, m, n, k, col_scale, bias, out, s);
 }
 

@@ -22,10 +22,10 @@ def both(x, w, n, ws, out, bias):
 
 
 # a K of less than one chunk pair, of one, of part of one more; every number of waves; more elements than a workgroup keeps in
-# registers (8192 per row for four waves); columns that are no multiple of sixteen; the longest rows the LDS takes
+# registers (8192 per row for four waves); columns that are no multiple of sixteen; the longest rows it is given
 @pytest.mark.parametrize("m", [1, 2])
 @pytest.mark.parametrize("n,k", [(1, 32), (17, 96), (64, 256), (33, 288), (100, 2048), (250, 2080), (4096, 4096), (130, 4128), (77, 8192), (64, 11008),
-                                 (40, 16384), (40, 16416), (48, 28672), (16, 49152)], ids=str)
+                                 (40, 16384), (4096, 11008)], ids=str)
 def test_one_launch_gives_what_two_give(m, n, k):
     gen = torch.Generator(device=DEV).manual_seed(SEED_BASE + 35000 + k + m)
     w, ws = quadmul.quantize_pack(torch.randn(n, k, device=DEV, generator=gen))
@@ -56,7 +56,8 @@ def test_rows_of_zeros_infinities_and_nan():
 def test_three_rows_and_operands_it_cannot_take_run_as_before():
     gen = torch.Generator(device=DEV).manual_seed(SEED_BASE + 35600)
     lib = qm.library()
-    for m, n, k, off in ((3, 64, 512, 0), (1, 64, 514, 0), (2, 40, 512, 4), (2, 16, 49152 + 32, 0)):
+    for m, n, k, off in ((3, 64, 512, 0), (1, 64, 514, 0), (2, 40, 512, 4), (1, 16, 16384 + 32, 0), (2, 8192, 8192, 0),
+                         (2, 14336, 4096, 0)):
         assert lib.qm_linear_workspace_bytes(m, n, k, 1, 4 if off else 256) > 0
         x = torch.randn(m, k, device=DEV, generator=gen, dtype=torch.float16)
         w0, ws = quadmul.quantize_pack(torch.randn(n, k, device=DEV, generator=gen))
