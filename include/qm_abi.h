@@ -42,8 +42,9 @@ extern "C" {
                                    QM_STATIC_SCRATCH_BYTES                                   */
 
 #define QM_CFG_AUTO          -1 /* let the shape table / heuristic choose                   */
-#define QM_CFG_RECODE        -2 /* 6-bit operands whether they pay or not: see
-                                   qm_gemm_recode_bytes                                      */
+#define QM_CFG_RECODE        -2 /* 6-bit operands whether they pay or not, on tiles of 256 x 256:
+                                   see qm_gemm_recode_bytes                                  */
+#define QM_CFG_RECODE_NARROW -3 /* the same on tiles of 256 x 128                            */
 
 /*
  * The hot path.  Replaces
@@ -147,12 +148,13 @@ size_t qm_gemm_workspace_bytes(int m, int n, int k, int ptr_align, int cfg, int 
 /*
  * The bytes of workspace with which a large product (cfg = QM_CFG_AUTO) runs faster still: A is re-coded
  * there as 6-bit floats, three quarters of a byte per element, for a matrix instruction that takes twice
- * as many of them as int8 values.  The results are the same bit for bit.  0 where that does not pay, or
+ * as many of them as int8 values (and B is copied with zero-padded rows where the call would copy both operands).
+ * The results are the same bit for bit.  0 where that does not pay, or
  * would take more than 256 MiB; the call itself never needs it: with a workspace of fewer bytes, it runs as
  * described above.  A caller that wants both lends the larger of the two sizes.
- * With cfg = QM_CFG_RECODE the two calls above run on them wherever they can: K a multiple of 32 from 256 to
+ * With cfg = QM_CFG_RECODE or QM_CFG_RECODE_NARROW the two calls above run on them wherever they can: K a multiple of 32 from 256 to
  * 65535, 256 columns and more, 16-byte aligned operands, a workspace of
- * qm_gemm_workspace_bytes(..., QM_CFG_RECODE, scaled) bytes; QM_ERR_CONFIG elsewhere, and from the calls that take none.
+ * qm_gemm_workspace_bytes(..., cfg, scaled) bytes; QM_ERR_CONFIG elsewhere, and from the calls that take none.
  */
 size_t qm_gemm_recode_bytes(int m, int n, int k, int ptr_align, int scaled);
 

@@ -34,7 +34,7 @@ _LIB_PATH = os.path.join(_PKG, "lib", "libqm_hip.so")
 _lib: Optional[ctypes.CDLL] = None
 
 CFG_AUTO = -1
-CFG_RECODE = -2
+CFG_RECODE, CFG_RECODE_NARROW = -2, -3
 #: every symbol include/qm_abi.h declares
 ABI_SYMBOLS = (
     "qm_gemm_i4", "qm_gemm_i4_cfg", "qm_gemm_i4_scaled", "qm_gemm_i4_scaled_cfg", "qm_config_has_scaled",

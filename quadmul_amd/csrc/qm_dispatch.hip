@@ -262,48 +262,69 @@ static bool fp6_fits(int m, int n, int k, int ptr_align)
     return n >= 256 && n < (1 << 21) && fp6_layout(m, k).code_bytes <= QM_FP6_MAX_BYTES;
 }
 
-// What it takes (us), re-coding included, in the terms of modelled_us: fitted to 312 products of 200 to 8192 rows (rms
-// of the fit 7 %), 256 x 256 tiles, one workgroup per CU.  A K-step costs 0.83 us where the int8 tile of the same size takes
-// 1.19, a round of tiles 15 against 10, the re-coding 0.22 us per million elements of A and a launch of its own.
-static double fp6_us(int m, int n, int k)
+// What the GEMM takes (us), in the terms of modelled_us: fitted to 272 products of 200 to 8192 rows (rms of the fits 7.5 and 6.3 %).  Per K-step
+// and round 0.82 us on tiles of 256 x 256 (int8: 1.19) and 0.53 on 256 x 128 (0.72), per round 13.8 and 5.8.
+static double fp6_tile_us(int m, int n, int k, bool narrow)
 {
-    const double kt = (k + 127) / 128, share = (double)((m + 255) / 256) * (double)((n + 255) / 256) / 256;
-    const double rounds = 0.75 * std::ceil(share) + 0.25 * std::max(1.0, share);
-    return kt * (rounds * (k & 255 ? 0.612 : 0.539) + std::min(1.0, share) * 0.290) + rounds * 15.07 + 0.2203e-6 * m * k - 0.67;
+    const double kt = (k + 127) / 128, share = (double)((m + 255) / 256) * (double)((n + (narrow ? 127 : 255)) / (narrow ? 128 : 256)) / 256;
+    const double rounds = 0.75 * std::ceil(share) + 0.25 * std::max(1.0, share), fill = std::min(1.0, share);
+    if (narrow) return kt * (rounds * (k & 255 ? 0.4774 : 0.4506) + fill * 0.0829) + rounds * 5.82 + 1.04;
+    return kt * (rounds * (k & 255 ? 0.5784 : 0.5042) + fill * 0.3183) + rounds * 13.83 - 2.94;
 }
 
-// Automatic choice: where that is 5 % less than what the model says of the int8 configuration `direct`.  Of those 312
-// products it takes 66, on which the time falls by 14 % in the mean (1280 x 8192 x 14336 124 -> 91 us, 8192 x 8192 x 8192 336 -> 290,
-// 512 x 28672 x 4096 46.0 -> 41.8) and rises by more than 1 % on one (4.7 %).  Without the margin it takes ten more, seven of
-// them at a gain and nothing over all; below a K of 1280 the fit is off by up to 25 % and what it takes gains nothing.
+// Automatic choice: where the better of the two tiles is 5 % below what the model says of the int8 configuration `direct`.
+// A K split of the int8 tiles counts with what it costs.  `coded`: A comes as codes, or both ways copy their operands, so
+// that only the GEMM counts; else the re-coding is a launch of its own and 0.17 us per million elements of A.  Of those 272
+// products: coded, it takes 155, 18 % faster in the mean, none slower by 1 %; with the re-coding 98, 13 % faster, two slower by
+// more than 3 % (10.5 %).  Without the margin it gains the same on more of them, and loses on more; below a K of 512, or of 1280
+// with the re-coding, it gains nothing.  us, int8 / here: 1280 x 8192 x 14336 124 / 91, 8192 x 8192 x 8192 325 / 290,
+// 512 x 28672 x 4096 45.8 / 41.9, 2048 x 4096 x 11008 65.1 / 63.7 (coded 55.7).
 // (The bound on the product comes first: calls that the host bounds do not get as far as the model.)
-// `coded`: A comes as codes (the linear layer's quantisation writes them), so that only the GEMM counts, fitted by itself to the
-// same products: the rule takes 98 of them, 18 % faster in the mean, none slower.
-static double fp6_gemm_us(int m, int n, int k)
+enum Fp6Route { FP6_NO = 0, FP6_WIDE, FP6_NARROW };
+static Fp6Route fp6_route(int m, int n, int k, int ptr_align, const Choice &direct, bool coded)
 {
-    const double kt = (k + 127) / 128, share = (double)((m + 255) / 256) * (double)((n + 255) / 256) / 256;
-    const double rounds = 0.75 * std::ceil(share) + 0.25 * std::max(1.0, share);
-    return kt * (rounds * (k & 255 ? 0.576 : 0.498) + std::min(1.0, share) * 0.356) + rounds * 15.12 - 4.48;
-}
-static bool fp6_pays(int m, int n, int k, int ptr_align, const Choice &direct, bool coded = false)
-{
-    if ((double)m * n * k < 4e9 || k < (coded ? 768 : 1280) || !fp6_fits(m, n, k, ptr_align)) return false;
+    if ((double)m * n * k < 4e9 || m < 200 || k < (coded ? 512 : 1280) || !fp6_fits(m, n, k, ptr_align)) return FP6_NO;
     const ConfigDesc &d = g_configs[direct.cfg];
     for (const CostFit &f : g_cost_fits)
-        if (std::strcmp(f.name, d.name) == 0) return (coded ? fp6_gemm_us(m, n, k) : fp6_us(m, n, k)) < 0.95 * modelled_us(f, d, m, n, k, direct.ksplit);
-    return false;
+        if (std::strcmp(f.name, d.name) == 0) {
+            const double wide = fp6_tile_us(m, n, k, false), narrow = fp6_tile_us(m, n, k, true), first = coded ? 0.0 : 4.68 + 0.1685e-6 * m * k;
+            if (std::min(wide, narrow) + first >= 0.95 * modelled_us(f, d, m, n, k, direct.ksplit)) return FP6_NO;
+            return narrow < wide ? FP6_NARROW : FP6_WIDE;
+        }
+    return FP6_NO;
 }
+static Fp6Route fp6_asked_for(int cfg) { return cfg == QM_CFG_RECODE ? FP6_WIDE : cfg == QM_CFG_RECODE_NARROW ? FP6_NARROW : FP6_NO; }
 
 static auto tile6_launcher(int out) { return out == OUT_I32 ? &launch_tile6_i32 : out == OUT_F16 ? &launch_tile6_f16 : &launch_tile6_bf16; }
 
-static hipError_t launch_fp6(const GemmArgs &p, void *ws, hipStream_t s)
+static hipError_t launch_tile6(const GemmArgs &p, const Fp6Operand &a, Fp6Route route, hipStream_t s)
+{
+    return tile6_launcher(p.out)(p, a, s, route == FP6_NARROW ? QM_OPT_NARROW : 0);
+}
+
+static hipError_t launch_fp6(const GemmArgs &p, Fp6Route route, void *ws, hipStream_t s)
 {
     const Fp6Operand a = fp6_operand(p.M, p.K, ws);
     const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, a.layout.kt, a.layout.groups};
-    expand_a6_kernel<<<dim3(2 * a.layout.groups, a.layout.parts), dim3(512), 0, s>>>(q);
+    expand_a6_kernel<false><<<dim3(2 * a.layout.groups, a.layout.parts), dim3(512), 0, s>>>(q);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? launch_tile6(p, a, route, s) : e;
+}
+
+// The same where the operands would be copied (plan_padded_k): A's codes as of rows padded to kp, and the copy of B, in one launch.
+static size_t fp6_padded_bytes(int m, int kp, const PadPlan &pl) { return (fp6_layout(m, kp).bytes + 255) / 256 * 256 + pl.b_bytes; }
+static hipError_t launch_fp6_padded(GemmArgs p, const PadPlan &pl, Fp6Route route, void *ws, hipStream_t s)
+{
+    const Fp6Operand a = fp6_operand(p.M, pl.kp, ws);
+    uint8_t *b_copy = static_cast<uint8_t *>(ws) + fp6_padded_bytes(p.M, pl.kp, pl) - pl.b_bytes;
+    const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, a.layout.kt, a.layout.groups, p.B, reinterpret_cast<v4i *>(b_copy), p.N, pl.kp};
+    const long long per_row_of_blocks = 512LL * 2 * a.layout.groups, pieces = (long long)p.N * (pl.kp / 32);
+    expand_a6_kernel<true><<<dim3(2 * a.layout.groups, a.layout.parts + (unsigned)((pieces + per_row_of_blocks - 1) / per_row_of_blocks)), dim3(512), 0, s>>>(q);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return tile6_launcher(p.out)(p, a, s, 0);
+    p.B = b_copy;
+    p.K = pl.kp;
+    return launch_tile6(p, a, route, s);
 }
 
 template <class Cfg>
@@ -449,9 +470,9 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
     p.out = out;
     p.ldc = strided ? row_stride : 0;
     if (strided && cfg != QM_CFG_AUTO) return QM_ERR_CONFIG;
-    if (cfg == QM_CFG_RECODE) {
+    if (const Fp6Route route = fp6_asked_for(cfg)) {
         if (!fp6_fits(m, n, k, align) || workspace == nullptr || ((uintptr_t)workspace & 15) || workspace_bytes < fp6_layout(m, k).bytes) return QM_ERR_CONFIG;
-        const hipError_t e = launch_fp6(p, workspace, s);
+        const hipError_t e = launch_fp6(p, route, workspace, s);
         return e == hipSuccess ? QM_OK : fail_launch(e);
     }
     const auto launcher = [&](int id) { return scaled ? scaled_launcher(id) : g_configs[id].launch; };
@@ -474,9 +495,13 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
         if (ch.ksplit > 1 && g_configs[ch.cfg].kind != KIND_TILE16) return QM_ERR_CONFIG;
     }
     ch.ksplit = effective_ksplit(g_configs[ch.cfg], k, ch.ksplit);
-    if (cfg == QM_CFG_AUTO && has_ws && ((uintptr_t)workspace & 15) == 0 && fp6_pays(m, n, k, align, ch) && workspace_bytes >= fp6_layout(m, k).bytes) {
-        const hipError_t e = launch_fp6(p, workspace, s);
-        return e == hipSuccess ? QM_OK : fail_launch(e);
+    const bool auto_ws = cfg == QM_CFG_AUTO && has_ws && ((uintptr_t)workspace & 15) == 0;
+    if (auto_ws) {
+        const Fp6Route route = fp6_route(m, n, k, align, ch, false);
+        if (route && workspace_bytes >= fp6_layout(m, k).bytes) {
+            const hipError_t e = launch_fp6(p, route, workspace, s);
+            return e == hipSuccess ? QM_OK : fail_launch(e);
+        }
     }
     if (ch.ksplit > 1 && workspace_fits(g_configs[ch.cfg], m, n, ch.ksplit, workspace, workspace_bytes)) {
         const hipError_t e = launch_split_with_workspace(p, ch, workspace, s);
@@ -490,6 +515,13 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
     }
     if (cfg == QM_CFG_AUTO && has_ws) {
         PadPlan pl = plan_padded_k(m, n, k, align, ch);
+        if (pl.on && auto_ws) {
+            const Fp6Route route = fp6_route(m, n, pl.kp, 256, pl.ch, true);
+            if (route && workspace_bytes >= fp6_padded_bytes(m, pl.kp, pl)) {
+                const hipError_t e = launch_fp6_padded(p, pl, route, workspace, s);
+                return e == hipSuccess ? QM_OK : fail_launch(e);
+            }
+        }
         if (pl.on && !launcher(pl.ch.cfg)) {
             // a pipelined configuration that has the scaled output, if the shape is one for those
             const int id = find_config("q256x256_w2x2_s9o1");
@@ -554,8 +586,10 @@ QM_EXPORT int qm_init(void)
     for (const int out : {(int)OUT_I32, (int)OUT_F16, (int)OUT_BF16})
         for (const uint16_t *bias : {(const uint16_t *)nullptr, &no_bias}) {
             p.bias = out == OUT_I32 ? nullptr : bias;
-            const hipError_t e = tile6_launcher(out)(p, Fp6Operand{}, nullptr, QM_OPT_PREPARE);
-            if (e != hipSuccess) return fail_launch(e);
+            for (const int tile : {0, QM_OPT_NARROW}) {
+                const hipError_t e = tile6_launcher(out)(p, Fp6Operand{}, nullptr, QM_OPT_PREPARE | tile);
+                if (e != hipSuccess) return fail_launch(e);
+            }
         }
     void *ws = nullptr;
     const hipError_t e = static_scratch(&ws);
@@ -625,7 +659,7 @@ QM_EXPORT size_t qm_gemm_workspace_bytes(int m, int n, int k, int ptr_align, int
         return whole > rest ? whole : rest;
     }
     if (cfg == QM_CFG_AUTO && col_block_for_large_b(m, n, k, ptr_align)) return 0;  // blocks of columns: one launch each, no workspace
-    if (cfg == QM_CFG_RECODE) return fp6_fits(m, n, k, ptr_align) ? fp6_layout(m, k).bytes : 0;
+    if (fp6_asked_for(cfg)) return fp6_fits(m, n, k, ptr_align) ? fp6_layout(m, k).bytes : 0;
     Choice ch;
     if (cfg == QM_CFG_AUTO) {
         ch = scaled ? select_scaled(m, n, k, ptr_align, true) : select_config(m, n, k, ptr_align, true);
@@ -644,11 +678,13 @@ QM_EXPORT size_t qm_gemm_workspace_bytes(int m, int n, int k, int ptr_align, int
 
 QM_EXPORT size_t qm_gemm_recode_bytes(int m, int n, int k, int ptr_align, int scaled)
 {
-    if (m < 1 || n < 1 || (double)m * n * k < 4e9 || (k & 1) || !fp6_fits(m, n, k, ptr_align)) return 0;
+    if (m < 1 || n < 1 || (double)m * n * k < 3.5e9 || (k & 1)) return 0;   // (padded to 128, a K that counts here is a sixth longer at most)
     if (row_block_for_large_a(m, n, k, ptr_align) || col_block_for_large_b(m, n, k, ptr_align)) return 0;
     Choice ch = scaled ? select_scaled(m, n, k, ptr_align, true) : select_config(m, n, k, ptr_align, true);
     ch.ksplit = effective_ksplit(g_configs[ch.cfg], k, ch.ksplit);
-    return fp6_pays(m, n, k, ptr_align, ch) ? fp6_layout(m, k).bytes : 0;
+    if (fp6_route(m, n, k, ptr_align, ch, false)) return fp6_layout(m, k).bytes;
+    const PadPlan pl = plan_padded_k(m, n, k, ptr_align, ch);
+    return pl.on && fp6_route(m, n, pl.kp, 256, pl.ch, true) ? fp6_padded_bytes(m, pl.kp, pl) : 0;
 }
 
 QM_EXPORT int qm_config_has_scaled(int cfg)
@@ -746,7 +782,8 @@ QM_EXPORT int qm_unpack_i4(const void *src_packed, void *dst_i8, int rows, int k
 // for the 6-bit tile kernel, or the packed rows and the GEMM's own workspace.
 namespace {
 struct LinearPlan {
-    bool one_launch, coded;
+    bool one_launch;
+    Fp6Route coded;
     int align;
     size_t scale_bytes, row_bytes, gemm_bytes;
     size_t bytes() const { return scale_bytes + row_bytes + gemm_bytes; }
@@ -764,7 +801,7 @@ LinearPlan linear_plan(int m, int n, int k, int in_dtype, int weight_align)
     if ((double)m * n * k >= 4e9 && quant6_fits(k, in_dtype) && row_block_for_large_a(m, n, k, pl.align) == 0 && col_block_for_large_b(m, n, k, pl.align) == 0) {
         Choice ch = select_scaled(m, n, k, pl.align, true);
         ch.ksplit = effective_ksplit(g_configs[ch.cfg], k, ch.ksplit);
-        pl.coded = fp6_pays(m, n, k, pl.align, ch, true);
+        pl.coded = fp6_route(m, n, k, pl.align, ch, true);
     }
     if (pl.coded) {
         pl.row_bytes = fp6_layout(m, k).bytes;
@@ -817,7 +854,7 @@ QM_EXPORT int qm_linear_i4(const void *x, int in_dtype, const void *B, void *D, 
         p.col_scale = col_scale;
         p.bias = static_cast<const uint16_t *>(bias);
         p.out = out;
-        e = tile6_launcher(out)(p, a, s, 0);
+        e = launch_tile6(p, a, pl.coded, s);
         return e == hipSuccess ? QM_OK : fail_launch(e);
     }
     const int st = qm_quantize_pack_i4(x, in_dtype, rows, scales, m, k, stream);

@@ -6,34 +6,76 @@
 namespace qm {
 
 struct Expand6Args {
-    const uint8_t *A;  // [M, K/2] packed s4, rows 16-byte aligned, K a multiple of 32 and at least 256
+    const uint8_t *A;  // [M, K/2] packed s4; rows 16-byte aligned and K a multiple of 32, unless ANY
     uint8_t *codes;
     int *sums;
     int M, K, kt, groups;
+    // ANY only: B [N, K/2], and its copy with rows of Kp / 2 bytes, Kp a multiple of 128
+    const uint8_t *B;
+    v4i *b_copy;
+    int N, Kp;
 };
+
+// 16 bytes of a row of Kb from byte `at` on, zeros past its end
+__device__ __forceinline__ v4i row_piece(const uint8_t *row, const int at, const int Kb)
+{
+    const int left = Kb - at;  // bytes of the row from there on
+    v4i v = *reinterpret_cast<const v4i_any_aligned *>(row + min(at, Kb - 16));
+    if (left < 16) {
+        // the row's last 16 bytes: the wanted ones are its last `left`
+        const int down = 8 * (16 - max(left, 0));
+        uint64_t lo = (uint32_t)v.x | (uint64_t)(uint32_t)v.y << 32, hi = (uint32_t)v.z | (uint64_t)(uint32_t)v.w << 32;
+        if (down >= 64) {
+            lo = down < 128 ? hi >> (down - 64) : 0;
+            hi = 0;
+        } else {
+            lo = lo >> down | hi << (64 - down);
+            hi >>= down;
+        }
+        v = v4i{(int)lo, (int)(lo >> 32), (int)hi, (int)(hi >> 32)};
+    }
+    return v;
+}
 
 // One workgroup re-codes 16 rows over FP6_PART_STEPS K-steps (blockIdx.y), eight waves of two K-steps at a
 // time: 128 bytes of every row, whole lines.  Two K-steps that a row does not fill are its last 128
 // bytes, as the GEMM loads them of B, with zeros where the steps before have been.
+// ANY: rows of any K and at any address, as if padded with zeros to Kp; the workgroups beyond A's (blockIdx.y past the
+// parts) copy B with its rows padded, one 16-byte piece per thread, in the same launch.
+template <bool ANY>
 __global__ void __launch_bounds__(512) expand_a6_kernel(const Expand6Args q)
 {
     __shared__ int red[8][16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
-    const int half = blockIdx.x, row = half * 16 + r, Kb = q.K >> 1;
-    const uint8_t *src = q.A + (size_t)min(row, q.M - 1) * Kb + 16 * g;
+    const int Kb = q.K >> 1;
+    if constexpr (ANY) {
+        const int parts = (q.kt + FP6_PART_STEPS - 1) / FP6_PART_STEPS;
+        if ((int)blockIdx.y >= parts) {
+            const uint32_t per_row = (uint32_t)q.Kp >> 5, piece = ((blockIdx.y - parts) * gridDim.x + blockIdx.x) * 512u + threadIdx.x;  // (below 2^28)
+            const uint32_t n = piece / per_row;
+            if (n < (uint32_t)q.N) q.b_copy[piece] = row_piece(q.B + (size_t)n * Kb, 16 * (int)(piece - n * per_row), Kb);
+            return;
+        }
+    }
+    const int row_bytes = ANY ? q.Kp >> 1 : Kb;
+    const int half = blockIdx.x, row = half * 16 + r;
+    const uint8_t *src = q.A + (size_t)min(row, q.M - 1) * Kb;
     uint8_t *out = q.codes + (size_t)(half >> 1) * q.kt * FP6_GROUP_BYTES;
     constexpr int PAIRS = FP6_PART_STEPS / 16;  // per wave
     v4i v[PAIRS][2];
 #pragma unroll
     for (int t = 0; t < PAIRS; ++t) {
-        const int step = blockIdx.y * FP6_PART_STEPS + 2 * (wave + 8 * t), at = min(step * 64, Kb - 128);
+        const int step = blockIdx.y * FP6_PART_STEPS + 2 * (wave + 8 * t), at = min(step * 64, row_bytes - 128);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) v[t][u] = *reinterpret_cast<const v4i *>(src + at + 64 * u);
+        for (int u = 0; u < 2; ++u) {
+            if constexpr (ANY) v[t][u] = row_piece(src, at + 64 * u + 16 * g, Kb);
+            else v[t][u] = *reinterpret_cast<const v4i *>(src + at + 64 * u + 16 * g);
+        }
     }
     int sum = 0;
 #pragma unroll
     for (int t = 0; t < PAIRS; ++t) {
-        const int step = blockIdx.y * FP6_PART_STEPS + 2 * (wave + 8 * t), at = min(step * 64, Kb - 128);
+        const int step = blockIdx.y * FP6_PART_STEPS + 2 * (wave + 8 * t), at = min(step * 64, row_bytes - 128);
         if (step >= q.kt) break;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {

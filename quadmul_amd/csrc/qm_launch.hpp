@@ -14,6 +14,8 @@ constexpr int QM_MAX_DEVICES = 64;
 // bit of a launcher's third argument: do the kernel's one-off set-up on the current device
 // (LDS size attribute, residency query) and return without launching
 constexpr int QM_OPT_PREPARE = 1 << 17;
+// bit of the 6-bit kernel's: tiles of 256 x 128 instead of 256 x 256
+constexpr int QM_OPT_NARROW = 1 << 18;
 
 // K split of the pipelined kernel, normalised: kt K-steps of 128 nibbles (the last one may
 // be short); with kps steps per split only ceil(kt / kps) splits have work; and a split

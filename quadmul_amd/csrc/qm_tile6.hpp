@@ -74,12 +74,14 @@ struct Tile6Cfg {
     // A K-step of A per stage; B two K-steps at a time, whole 128-byte lines of its rows
     static constexpr int A_STAGES = 4, B_STAGES = 2, A_BYTES = BM * FP6_STEP_BYTES, B_BYTES = BN * 128;
     static constexpr int RING_BYTES = A_STAGES * A_BYTES + B_STAGES * B_BYTES;
-    static constexpr int XHALF_BYTES = 16 * 128;  // per wave, as in Tile16Cfg, in the stage of B that is free in an item's last step
-    static constexpr int SCALE_BYTES = WM * 4 + WN * 6;  // ... and its scales and biases, beside them
-    static constexpr int LDS_BYTES = RING_BYTES;
+    static constexpr int XHALF_BYTES = 16 * 128;           // the write-out's area, per wave, as in Tile16Cfg
+    static constexpr int SCALE_BYTES = WM * 4 + WN * 6;   // ... and its scales and biases, beside them
+    // Where the ring leaves no room for them they are in the stage of B that is free in an item's last step.
+    static constexpr bool OWN_AREA = RING_BYTES + WAVES * (XHALF_BYTES + SCALE_BYTES) <= 160 * 1024;
+    static constexpr int LDS_BYTES = RING_BYTES + (OWN_AREA ? WAVES * (XHALF_BYTES + SCALE_BYTES) : 0);
     static constexpr int A_GROUPS = BM / 32 / WAVES, A_PIECES = 3 * A_GROUPS, B_PIECES = BN / 8 / WAVES;
     static_assert(BM % (32 * WAVES) == 0 && BN % (8 * WAVES) == 0 && WAVES % 2 == 0, "loads divide evenly among the waves");
-    static_assert(WM % 64 == 0 && WN % 64 == 0 && WAVES * (XHALF_BYTES + SCALE_BYTES) <= B_BYTES, "the write-out fits the stage it borrows");
+    static_assert(WM % 64 == 0 && WN % 64 == 0 && (OWN_AREA || WAVES * (XHALF_BYTES + SCALE_BYTES) <= B_BYTES), "the write-out fits the stage it borrows");
     static_assert(LDS_BYTES <= 160 * 1024, "LDS budget of a gfx950 CU");
     static_assert(FM % 4 == 0 && FN % 2 == 0, "four fragments of A in rotation; blocks leave in pairs");
 };
@@ -331,7 +333,8 @@ gemm_tile6_kernel(const GemmArgs p, const uint8_t *const a6, const int *const ro
     __syncthreads();
 
     v6i bf[2][FN], af[4];
-    v4i b_pk[2];
+    constexpr int NPK = FM * FN >= 32 ? 2 : FN;  // packed fragments of B between their read and their re-coding
+    v4i b_pk[NPK];
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
         const v4i q = read_b(b_ring[0], false, j);
@@ -354,6 +357,7 @@ gemm_tile6_kernel(const GemmArgs p, const uint8_t *const a6, const int *const ro
         constexpr int bs = decltype(bs_tag)::value;
         constexpr bool first = decltype(first_tag)::value, last = decltype(last_tag)::value != 0, edge = decltype(last_tag)::value == 2;
         constexpr int SLOTS = FM * FN, OPS = W * FN;
+        constexpr bool loads_b = bs == 1 && (!last || Cfg::OWN_AREA);  // (else the stage is the write-out's)
         constexpr int LEAD = FN;               // the first fragment read in slot 0 is there by then
         static_for<0, SLOTS>([&](auto s_) __attribute__((always_inline)) {
             constexpr int s = decltype(s_)::value, i = s / FN, j = s % FN;
@@ -367,13 +371,13 @@ gemm_tile6_kernel(const GemmArgs p, const uint8_t *const a6, const int *const ro
             static_for<0, FN>([&](auto q_) __attribute__((always_inline)) {
                 constexpr int q = decltype(q_)::value;
                 constexpr int begin = LEAD + W * q * (SLOTS - LEAD) / OPS;
-                if constexpr (s == begin - LEAD) b_pk[q & 1] = read_b(b_ring[bs], bs == 0, q);
+                if constexpr (s == begin - LEAD) b_pk[q % NPK] = read_b(b_ring[bs], bs == 0, q);
             });
             if constexpr (s >= LEAD) {
                 constexpr int lo = (s - LEAD) * OPS / (SLOTS - LEAD), hi = (s - LEAD + 1) * OPS / (SLOTS - LEAD);
                 static_for<lo, hi>([&](auto o_) __attribute__((always_inline)) {
                     constexpr int o = decltype(o_)::value, q = o / W;
-                    code_op(std::integral_constant<int, o % W>{}, b_pk[q & 1], bf[bs ^ 1][q]);
+                    code_op(std::integral_constant<int, o % W>{}, b_pk[q % NPK], bf[bs ^ 1][q]);
                 });
             }
             // write-out of the accumulator row finished one sub-step ago: 4 NH parts over FN slots
@@ -383,8 +387,8 @@ gemm_tile6_kernel(const GemmArgs p, const uint8_t *const a6, const int *const ro
                     write_half(std::integral_constant<int, i - 1>{}, std::integral_constant<int, t / 4>{}, std::integral_constant<int, t % 4>{}, std::integral_constant<bool, edge>{});
                 });
             }
-            // the loads, spread over the step, M0 written two slots ahead (in a last step the stage of B is the write-out's)
-            constexpr int NB = bs == 1 && !last ? B_PIECES : 0;
+            // the loads, spread over the step, M0 written two slots ahead
+            constexpr int NB = loads_b ? B_PIECES : 0;
             static_for<0, NB + A_PIECES>([&](auto q_) __attribute__((always_inline)) {
                 constexpr int q = decltype(q_)::value, at = 3 + q * (SLOTS - 6) / (NB + A_PIECES);
                 if constexpr (s == at - 2 && q < NB) dma_setup_b(q, b_ring[0]);
@@ -399,14 +403,14 @@ gemm_tile6_kernel(const GemmArgs p, const uint8_t *const a6, const int *const ro
         // What the step after this one reads -- its A, the B of the step after it -- must be there: everything but this
         // step's own loads.  The counter is in order of issue and counts stores too: a last step's are all
         // younger, and may stay in flight (`edge`: a store without lanes may not count).
-        constexpr int pending = A_PIECES + (bs == 1 && !last ? B_PIECES : 0) + (last && !edge ? (FM - 1) * FN - 2 : 0);
+        constexpr int pending = A_PIECES + (loads_b ? B_PIECES : 0) + (last && !edge ? (FM - 1) * FN - 2 : 0);
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(pending > 63 ? 63 : pending) : "memory");
         const int ta = a_ring[0];
 #pragma unroll
         for (int u = 0; u + 1 < Cfg::A_STAGES; ++u) a_ring[u] = a_ring[u + 1];
         a_ring[Cfg::A_STAGES - 1] = ta;
-        if constexpr (bs == 1 && !last) swap_b();
-        if constexpr (!last) cursor_advance();
+        if constexpr (loads_b) swap_b();
+        if constexpr (!last || loads_b) cursor_advance();
     };
 
     auto run_item = [&](auto mode_) __attribute__((always_inline)) {
@@ -449,9 +453,10 @@ gemm_tile6_kernel(const GemmArgs p, const uint8_t *const a6, const int *const ro
             k_step(std::integral_constant<int, 1>{}, std::false_type{}, No{});
             k_step(std::integral_constant<int, 0>{}, std::false_type{}, No{});
         }
-        xh = b_ring[0] + wave * Cfg::XHALF_BYTES;
+        const int area = Cfg::OWN_AREA ? Cfg::RING_BYTES : b_ring[0];
+        xh = area + wave * Cfg::XHALF_BYTES;
         if constexpr (SCALED) {
-            sc = b_ring[0] + WAVES * Cfg::XHALF_BYTES + wave * Cfg::SCALE_BYTES;
+            sc = area + WAVES * Cfg::XHALF_BYTES + wave * Cfg::SCALE_BYTES;
 #pragma unroll
             for (int q = 0; q < Cfg::WM / 64; ++q) *reinterpret_cast<float *>(smem + sc + (q * 64 + lane) * 4) = rs_reg[q];
 #pragma unroll
@@ -471,11 +476,13 @@ gemm_tile6_kernel(const GemmArgs p, const uint8_t *const a6, const int *const ro
         });
         store_half(std::integral_constant<int, FM - 1>{}, std::integral_constant<int, NH - 1>{}, std::integral_constant<int, 0>{}, std::integral_constant<bool, edge>{});
         store_half(std::integral_constant<int, FM - 1>{}, std::integral_constant<int, NH - 1>{}, std::integral_constant<int, 1>{}, std::integral_constant<bool, edge>{});
-        // every wave is done with its area: the loads of B that the last step left out
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        load_b(b_ring[0]);
-        swap_b();
-        cursor_advance();
+        if constexpr (!Cfg::OWN_AREA) {
+            // every wave is done with its area: the loads of B that the last step left out
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            load_b(b_ring[0]);
+            swap_b();
+            cursor_advance();
+        }
         next_item(min(c_item + G, nitems - 1));
     };
     for (; c_item < nwhole; c_item += G) run_item(std::integral_constant<int, 1>{});

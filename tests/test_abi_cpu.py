@@ -285,11 +285,15 @@ def test_recoded_operands_are_an_offer_to_callers_with_more_workspace():
     assert qm.recode_bytes(8192, 8192, 8192) == groups * (steps * 3072 + parts * 32 * 4)
     assert qm.workspace_bytes(8192, 8192, 8192) == 0
     assert qm.workspace_bytes(100, 300, 288, qm.CFG_RECODE) == 4 * (4 * 3072 + 32 * 4)      # three K-steps, and one to make them even
-    for m, n, k, align in ((64, 4096, 4096, 256), (8192, 8192, 1024, 256), (8192, 8192, 8192 + 16, 256), (8192, 8192, 8192, 8),
+    for m, n, k, align in ((64, 4096, 4096, 256), (8192, 8192, 1024, 256), (150, 28672, 8192, 256),
                            (512, 8192, 8192, 256), (8192, 200, 8192, 256), (65536, 8192, 8192, 256), (8192, 8192, 65536, 256)):
         assert qm.recode_bytes(m, n, k, ptr_align=align) == 0 and qm.recode_bytes(m, n, k, True, align) == 0, (m, n, k, align)
     for bad in ((16, 255, 256), (16, 256, 224), (16, 256, 272), (0, 256, 256), (16, 256, 257)):
         assert qm.workspace_bytes(*bad, qm.CFG_RECODE) == 0, bad
+    # operands that would be copied with padded rows: the codes of rows padded to 8320, and the copy of B
+    for k, align in ((8192 + 16, 256), (8192 + 128, 8)):
+        assert qm.recode_bytes(8192, 8192, k, ptr_align=align) == groups * (66 * 3072 + 3 * 32 * 4) + 8192 * 8320 // 2
+        assert qm.workspace_bytes(8192, 8192, k, ptr_align=align) == 2 * 8192 * 8320 // 2
     # the library's own scratch array is lent for what that entry point has always used it for
     assert qm.workspace_bytes(2048, 11008, 4096) == 0 and qm.recode_bytes(2048, 11008, 4096) > 0
 

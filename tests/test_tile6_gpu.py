@@ -1,5 +1,5 @@
 """The tile kernel on 6-bit floats (csrc/qm_tile6.hpp): bit-exact against exact products, through the explicit
-configuration QM_CFG_RECODE, at the edges of its tiles, K-steps and work items, in every output form."""
+configurations QM_CFG_RECODE and QM_CFG_RECODE_NARROW, at the edges of its tiles, K-steps and work items, in every output form."""
 import numpy as np
 import pytest
 import torch
@@ -12,6 +12,7 @@ from util import SEED_BASE, make_operands, pack_cpu, poisoned_c
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
+both_tiles = pytest.mark.parametrize("cfg", [qm.CFG_RECODE, qm.CFG_RECODE_NARROW], ids=["256x256", "256x128"])
 
 # one row, one tile and one element more or less, K-steps short by 32, 64 and 96 nibbles, odd and even numbers of them, a K
 # of more than one part of the row sums and of more than four, columns that are no multiple of four, more tiles than CUs
@@ -24,18 +25,19 @@ def operands(m, n, k, seed):
     return a, b, pack_cpu(a).to(DEV), pack_cpu(b).to(DEV)
 
 
+@both_tiles
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
-def test_every_output_form_is_exact(shape):
+def test_every_output_form_is_exact(shape, cfg):
     m, n, k = shape
     a, b, a_d, b_d = operands(m, n, k, 31000 + m + n + k)
     want = fp32_matmul_on_gpu(a, b)   # (64 k < 2^24: exact)
     c = poisoned_c(m, n, DEV)
-    qm.gemm_cfg(a_d, b_d, c, m, n, k, qm.CFG_RECODE)
+    qm.gemm_cfg(a_d, b_d, c, m, n, k, cfg)
     assert torch.equal(c, want)
     # a C that is 4-byte aligned only
     room = torch.full((m * n + 1,), -1, dtype=torch.int32, device=DEV)
     c = room[1:].view(m, n)
-    qm.gemm_cfg(a_d, b_d, c, m, n, k, qm.CFG_RECODE)
+    qm.gemm_cfg(a_d, b_d, c, m, n, k, cfg)
     assert torch.equal(c, want) and room[0].item() == -1
     gen = torch.Generator(device=DEV).manual_seed(SEED_BASE + k)
     rs, cs = (torch.rand(x, device=DEV, generator=gen) * 1e-3 + 1e-4 for x in (m, n))
@@ -43,7 +45,7 @@ def test_every_output_form_is_exact(shape):
         for rows, cols in ((rs, cs), (None, cs), (rs, None)):
             for bias in (None, torch.randn(n, device=DEV, generator=gen).to(dtype)):
                 d = torch.empty(m, n, dtype=dtype, device=DEV)
-                qm.gemm_scaled(a_d, b_d, d, m, n, k, rows, cols, cfg=qm.CFG_RECODE, bias=bias)
+                qm.gemm_scaled(a_d, b_d, d, m, n, k, rows, cols, cfg=cfg, bias=bias)
                 e = want.float()
                 if rows is not None:
                     e = e * rows[:, None]
@@ -55,18 +57,20 @@ def test_every_output_form_is_exact(shape):
                 assert torch.equal(d.view(torch.int16), e.view(torch.int16)), (dtype, rows is None, cols is None, bias is None)
 
 
+@both_tiles
 @pytest.mark.parametrize("k", [256, 4096, 65504])
-def test_extremes_in_closed_form(k):
+def test_extremes_in_closed_form(k, cfg):
     """The largest and the most negative accumulators there are, up to the largest K."""
     m, n = 40, 260
     fill = lambda rows, v: pack_cpu(torch.full((rows, k), v, dtype=torch.int8)).to(DEV)
     for va, vb in ((-8, -8), (-8, 7), (7, -8), (7, 7), (0, 7), (-8, 0)):
         c = poisoned_c(m, n, DEV)
-        qm.gemm_cfg(fill(m, va), fill(n, vb), c, m, n, k, qm.CFG_RECODE)
+        qm.gemm_cfg(fill(m, va), fill(n, vb), c, m, n, k, cfg)
         assert (c == va * vb * k).all(), (va, vb)
 
 
-def test_every_product_of_two_nibbles_at_every_place_of_a_k_step():
+@both_tiles
+def test_every_product_of_two_nibbles_at_every_place_of_a_k_step(cfg):
     """One element of A against one of B: the place of each in its 6-bit fields, alone in its row."""
     k, n = 256, 256
     values = torch.arange(-8, 8, dtype=torch.int8)
@@ -77,7 +81,7 @@ def test_every_product_of_two_nibbles_at_every_place_of_a_k_step():
         b[:, pos] = values.repeat(n // 16)
         b[:, pos ^ 1] = 7   # (meets zeros of A only)
         c = poisoned_c(16, n, DEV)
-        qm.gemm_cfg(pack_cpu(a).to(DEV), pack_cpu(b).to(DEV), c, 16, n, k, qm.CFG_RECODE)
+        qm.gemm_cfg(pack_cpu(a).to(DEV), pack_cpu(b).to(DEV), c, 16, n, k, cfg)
         assert torch.equal(c.cpu(), values.int()[:, None] * b[:, pos].int()[None, :]), pos
 
 
@@ -123,20 +127,43 @@ def test_two_streams_have_a_workspace_each():
     assert all(torch.equal(c, w) for c, w in zip(outs, want))
 
 
-def test_what_it_cannot_take_is_refused():
+# K that fills its last 16-byte piece, K-step or pair of them by little, all but little, or not at all; operands at odd addresses
+@pytest.mark.parametrize("m,n,k,a_off,b_off", [(1531, 3307, 4100, 0, 0), (1531, 3307, 4098, 1, 2), (1531, 3307, 4222, 0, 0), (1500, 3300, 4224, 8, 0),
+                                               (1500, 3300, 4222, 0, 5), (1531, 3307, 4352 - 2, 0, 0), (1531, 3307, 4096, 3, 0), (1300, 8192, 1534, 0, 0)], ids=str)
+def test_rows_of_any_k_and_at_any_address(m, n, k, a_off, b_off):
+    """... are re-coded and copied padded, where the operands would be copied anyway."""
+    a, b = make_operands(m, n, k, SEED_BASE + 36000 + k)
+    place = lambda x, off: torch.full((x.numel() + 16,), 0x7F, dtype=torch.int8, device=DEV)[off:off + x.numel()].view(x.shape).copy_(x)
+    a_d, b_d = place(pack_cpu(a), a_off), place(pack_cpu(b), b_off)
+    align = min((x.data_ptr() & -x.data_ptr()) for x in (a_d, b_d))
+    assert qm.recode_bytes(m, n, k, ptr_align=align) > 0 and qm.recode_bytes(m, n, k, True, align) > 0
+    want = fp32_matmul_on_gpu(a, b)
+    for workspace in (True, torch.full((qm.recode_bytes(m, n, k, ptr_align=align),), 0x55, dtype=torch.uint8, device=DEV)):
+        c = poisoned_c(m, n, DEV)
+        qm.gemm(a_d, b_d, c, m, n, k, workspace=workspace)
+        assert torch.equal(c, want)
+    rs, cs = (torch.rand(x, device=DEV) * 1e-3 + 1e-4 for x in (m, n))
+    bias = torch.randn(n, device=DEV).to(torch.bfloat16)
+    d = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    qm.gemm_scaled(a_d, b_d, d, m, n, k, rs, cs, bias=bias)
+    assert torch.equal(d, ((want.float() * rs[:, None]) * cs[None, :]).to(torch.bfloat16) + bias)
+
+
+@both_tiles
+def test_what_it_cannot_take_is_refused(cfg):
     def status(m, n, k, a_off=0, ws=True):
         a = torch.zeros(m * (k // 2) + 16, dtype=torch.int8, device=DEV)[a_off:a_off + m * (k // 2)].view(m, k // 2)
         b = torch.zeros(n, k // 2, dtype=torch.int8, device=DEV)
         c = poisoned_c(m, n, DEV)
         with pytest.raises(qm.QuadmulError):
-            qm.gemm_cfg(a, b, c, m, n, k, qm.CFG_RECODE, ws)
+            qm.gemm_cfg(a, b, c, m, n, k, cfg, ws)
     status(16, 256, 224)
     status(16, 255, 256)
     status(16, 256, 272)
     status(16, 256, 65536)
     status(16, 256, 256, a_off=4)
     status(16, 256, 256, ws=None)
-    status(16, 256, 256, ws=torch.empty(qm.workspace_bytes(16, 256, 256, qm.CFG_RECODE) - 1, dtype=torch.uint8, device=DEV))
+    status(16, 256, 256, ws=torch.empty(qm.workspace_bytes(16, 256, 256, cfg) - 1, dtype=torch.uint8, device=DEV))
 
 
 # rows that are no multiple of eight, K-steps short and odd in number, each number of chunks per lane, each type
