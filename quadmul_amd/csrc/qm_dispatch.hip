@@ -284,14 +284,11 @@ enum Fp6Route { FP6_NO = 0, FP6_WIDE, FP6_NARROW };
 static Fp6Route fp6_route(int m, int n, int k, int ptr_align, const Choice &direct, bool coded)
 {
     if ((double)m * n * k < 4e9 || m < 200 || k < (coded ? 512 : 1280) || !fp6_fits(m, n, k, ptr_align)) return FP6_NO;
-    const ConfigDesc &d = g_configs[direct.cfg];
-    for (const CostFit &f : g_cost_fits)
-        if (std::strcmp(f.name, d.name) == 0) {
-            const double wide = fp6_tile_us(m, n, k, false), narrow = fp6_tile_us(m, n, k, true), first = coded ? 0.0 : 4.68 + 0.1685e-6 * m * k;
-            if (std::min(wide, narrow) + first >= 0.95 * modelled_us(f, d, m, n, k, direct.ksplit)) return FP6_NO;
-            return narrow < wide ? FP6_NARROW : FP6_WIDE;
-        }
-    return FP6_NO;
+    const CostFit *f = fit_of(direct.cfg);
+    if (f == nullptr) return FP6_NO;
+    const double wide = fp6_tile_us(m, n, k, false), narrow = fp6_tile_us(m, n, k, true), first = coded ? 0.0 : 4.68 + 0.1685e-6 * m * k;
+    if (std::min(wide, narrow) + first >= 0.95 * modelled_us(*f, g_configs[direct.cfg], m, n, k, direct.ksplit)) return FP6_NO;
+    return narrow < wide ? FP6_NARROW : FP6_WIDE;
 }
 static Fp6Route fp6_asked_for(int cfg) { return cfg == QM_CFG_RECODE ? FP6_WIDE : cfg == QM_CFG_RECODE_NARROW ? FP6_NARROW : FP6_NO; }
 

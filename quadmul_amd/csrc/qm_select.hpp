@@ -6,6 +6,8 @@
 #pragma once
 #include <cmath>
 #include <cstring>
+#include <string_view>
+#include <unordered_map>
 
 #include "qm_launch.hpp"
 
@@ -62,19 +64,30 @@ static const struct { const char *name; LaunchFn launch; } g_scaled_tile16[] = {
 // (not every configuration has them).
 static LaunchFn scaled_launcher(int cfg)
 {
-    const ConfigDesc &c = g_configs[cfg];
-    if (c.kind == KIND_GENERIC || c.kind == KIND_SKINNY) return c.launch;
-    if (c.kind == KIND_TILE16)
-        for (const auto &e : g_scaled_tile16)
-            if (std::strcmp(e.name, c.name) == 0) return e.launch;
-    return nullptr;
+    // (looked up by name once: a call asks several times which configurations have one)
+    static const auto launchers = [] {
+        struct { LaunchFn of[g_num_configs]; } t{};
+        for (int i = 0; i < g_num_configs; ++i) {
+            const ConfigDesc &c = g_configs[i];
+            if (c.kind == KIND_GENERIC || c.kind == KIND_SKINNY) t.of[i] = c.launch;
+            else
+                for (const auto &e : g_scaled_tile16)
+                    if (std::strcmp(e.name, c.name) == 0) t.of[i] = e.launch;
+        }
+        return t;
+    }();
+    return launchers.of[cfg];
 }
 
 static int find_config(const char *name)
 {
-    for (int i = 0; i < g_num_configs; ++i)
-        if (std::strcmp(g_configs[i].name, name) == 0) return i;
-    return -1;
+    static const std::unordered_map<std::string_view, int> ids = [] {
+        std::unordered_map<std::string_view, int> m;
+        for (int i = 0; i < g_num_configs; ++i) m.emplace(g_configs[i].name, i);
+        return m;
+    }();
+    const auto it = ids.find(name);
+    return it == ids.end() ? -1 : it->second;
 }
 
 // The 16-byte-load kernels need whole, aligned chunks and 32-bit row offsets,
@@ -161,6 +174,24 @@ static const CostFit g_cost_fits[] = {
 #undef QM_COST
 #undef QM_COST_SPLIT
 };
+static constexpr int g_num_fits = (int)(sizeof(g_cost_fits) / sizeof(g_cost_fits[0]));
+// the configuration of each, and of a configuration its fit or null (every choice outside the table goes through all of them: by
+// name each time they were half a microsecond of a call that the host bounds)
+static const int *fit_configs()
+{
+    static const auto ids = [] {
+        struct { int of[g_num_fits]; } t{};
+        for (int i = 0; i < g_num_fits; ++i) t.of[i] = find_config(g_cost_fits[i].name);
+        return t;
+    }();
+    return ids.of;
+}
+static const CostFit *fit_of(int cfg)
+{
+    for (int i = 0; i < g_num_fits; ++i)
+        if (fit_configs()[i] == cfg) return &g_cost_fits[i];
+    return nullptr;
+}
 static const float g_cost_split[2] = {
 #define QM_COST(name, slots, blend, step, busy, round, odd, ragged, reread, skew, launch)
 #define QM_COST_SPLIT(fixed, per_melem) fixed, per_melem
@@ -196,8 +227,9 @@ static Choice modelled_choice(int m, int n, int k, int ptr_align, bool has_ws, b
     Choice best{0, 1, 1};
     double best_us = 1e300;
     const int kt = (k + 127) / 128;
-    for (const CostFit &f : g_cost_fits) {
-        const int id = find_config(f.name);
+    for (int i = 0; i < g_num_fits; ++i) {
+        const CostFit &f = g_cost_fits[i];
+        const int id = fit_configs()[i];
         if (id < 0 || !config_supports(id, m, n, k, ptr_align)) continue;
         const ConfigDesc &d = g_configs[id];
         const bool tile = d.kind == KIND_TILE16;
