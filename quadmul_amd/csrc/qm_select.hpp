@@ -308,8 +308,21 @@ static Choice heuristic(int m, int n, int k, int ptr_align, bool has_ws)
         // multiply-adds, so the larger block moves half as much per product: 64 x 8192 x 4096
         // 6.5 us on 64 x 32 (32 x 32: 7.5) -- else blocks of 32 rows: 32 x 16 per workgroup while
         // that leaves one workgroup per CU, 32 x 32 (two to a CU) up to about three rounds.
-        const long long c64 = (n + 63) / 64, c32 = (n + 31) / 32;
+        const long long c64 = (n + 63) / 64, c48 = (n + 47) / 48, c32 = (n + 31) / 32;
         if (k <= 32768) {
+            // Rows and columns in blocks of 48: up to 48 rows a quarter less work than on blocks of 64, which is spent there on
+            // rows that are copies of the last one, and between 8192 and 12288 columns one round that fills the device, where
+            // blocks of 64 leave up to half of it idle and blocks of 32 start a second one.  Time against the choice below, B
+            // from HBM, K = 1024 .. 32768 (geometric mean, worst shape): 48 x 32 0.93, 0.99; 48 x 48 0.83, 0.98 (48 x 11008 x
+            // 4096 9.0 -> 7.3 us); 48 x 64 0.93, 0.99; 64 x 48 0.89, 0.99 (64 x 9600 x 4096 8.9 -> 8.0 us).  On a K of 1024
+            // 64 x 48 is 1 % behind (63 x 8230), beyond 224 workgroups up to 6 %; 48 x 64 on all 256 CUs gains 2 %: not taken.
+            if (m <= 48) {
+                if (c32 >= 140 && c32 <= 256) return pick("d3x2_w8_r1");
+                if (c32 > 256 && c48 <= 256) return pick("d3x3_w8_r1");
+                if (c48 > 256 && c64 < 256) return pick("d3x4_w8_r1");
+            } else if (k >= 2048 && c32 > 256 && c48 <= 224) {
+                return pick("d4x3_w8_r1");
+            }
             if (c64 >= 140 && c64 <= 256) return pick("d4x4_w8_r1");
             if (c64 > 256 && c64 <= 512 && (k <= 16384 || !has_ws)) return pick("d4x4_w4_r1");
             if (c32 >= 140 && c32 <= 256) return pick("d4x2_w8_r1");

@@ -852,3 +852,24 @@ def test_any_even_k_at_any_address(oracle_mod, shape):
     c_d = poisoned_c(m, n, DEV)
     qm.gemm(at(pack_cpu(lo), 1), at(pack_cpu(torch.full((n, k), 7, dtype=torch.int8)), 2), c_d, m, n, k)
     assert (c_d == -56 * k).all()
+
+
+@pytest.mark.parametrize("m,n,k,name", [
+    (33, 4449, 1024, "d3x2"), (48, 8192, 1056, "d3x2"), (33, 8193, 1184, "d3x3"), (47, 12288, 2048, "d3x3"), (48, 12289, 1024, "d3x4"),
+    (34, 16319, 1120, "d3x4"), (49, 8193, 2048, "d4x3"), (64, 10752, 2080, "d4x3"), (40, 4448, 1024, ""), (48, 16321, 1024, ""), (64, 10753, 2048, ""),
+])
+def test_blocks_of_48_rows_and_columns(m, n, k, name):
+    """First and last sizes that take 48-row / 48-column blocks and those next to them; columns that end inside a block,
+    every kind of short last K-step.  With integer and with scaled output, exact."""
+    chosen = qm.config_name(qm.select_config(m, n, k) & 0xFFFF)
+    assert chosen.startswith(name) if name else not any(s in chosen for s in ("d3x", "x3_"))
+    a = torch.randint(-8, 8, (m, k), dtype=torch.int8, generator=torch.Generator().manual_seed(SEED_BASE + 7100 + n))
+    b = torch.randint(-8, 8, (n, k), dtype=torch.int8, generator=torch.Generator().manual_seed(SEED_BASE + 7200 + n))
+    want = fp32_matmul_on_gpu(a, b)
+    ap, bp = pack_cpu(a), pack_cpu(b)
+    np.testing.assert_array_equal(run_gemm(ap, bp, m, n, k), want.cpu().numpy())
+    rs, cs = torch.rand(m, device=DEV) + 0.5, torch.rand(n, device=DEV) + 0.5
+    d = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    qm.gemm_scaled(ap.to(DEV), bp.to(DEV), d, m, n, k, rs, cs)
+    # (fp32 products of an exact integer and two scales, in either order: 2 roundings each, then one to bfloat16)
+    torch.testing.assert_close(d.float(), want.float() * rs[:, None] * cs[None, :], rtol=2.0 ** -8 + 4 * 2.0 ** -24, atol=0)
