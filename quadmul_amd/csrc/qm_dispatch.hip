@@ -65,7 +65,7 @@ static hipError_t launch_skinny_dma(const GemmArgs &p, hipStream_t stream, int o
     const int blocks = (p.N + Cfg::BN - 1) / Cfg::BN, row_blocks = (p.M + Cfg::MAX_M - 1) / Cfg::MAX_M;
     if (row_blocks > 65535) return hipErrorInvalidValue;
     static_assert(kernarg_bytes(&gemm_skinny_dma_kernel<Cfg>) <= 64, "see pack_rows_out");
-    gemm_skinny_dma_kernel<Cfg><<<dim3(blocks, row_blocks), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(
+    gemm_skinny_dma_kernel<Cfg><<<dim3(skinny_dma_columns(blocks, row_blocks), row_blocks), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(
         p.A, p.B, p.C, pack_rows_out(p.M, p.out), p.N, p.K, p.ldc, p.row_scale, p.col_scale, p.bias);
     return hipGetLastError();
 }

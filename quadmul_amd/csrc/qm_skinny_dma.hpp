@@ -38,7 +38,7 @@
 // slot is 8 KiB instead of 10, so that two runs per wave -- all of K = 4096 on eight waves --
 // are in flight at once within the 160 KiB of LDS.  The workgroups of one column block lie
 // gridDim.x apart in launch order, on the same XCD when gridDim.x is a multiple of 8: the
-// second reader of B's lines finds them in that XCD's L2.
+// second reader of B's lines finds them in that XCD's L2 (see skinny_dma_columns).
 #pragma once
 #include <type_traits>
 
@@ -62,6 +62,20 @@ struct SkinnyDmaCfg {
     static_assert(LOADS_PER_RUN * D <= 63, "the memory counter counts to 63");
 };
 
+// The grid's first dimension for so many column and row blocks.  With several row blocks it is rounded up to a multiple
+// of the 8 XCDs (the workgroups beyond N end at once), for the reason above: where the readers of one column block
+// sit on different XCDs, each of those fetches B's lines for itself.  Time with / without, B from HBM: 65 x 4100 x 4096 on 32 x 64
+// 5.8 / 6.8 us, 128 x 4100 x 28672 on 32 x 64 35 / 51, 320 x 5500 x 8192 on 64 x 64 21.5 / 24.7; geometric mean 0.90 over 270
+// cases with the rule, none more than 1 % slower.  The rule: an XCD then holds whole columns, the fullest of them one column of
+// row blocks more than the emptiest.  Below 24 columns, or where that column is a round more on the 32 CUs of its XCD than
+// all blocks are on 256 CUs, the imbalance costs more (41 columns of 6 row blocks: 1.25 times the time).
+inline int skinny_dma_columns(int cols, int rows)
+{
+    if (rows < 2 || cols < 24) return cols;
+    const long long per_xcd = (cols + 7) / 8;
+    return (per_xcd * rows + 31) / 32 <= ((long long)cols * rows + 255) / 256 ? (int)per_xcd * 8 : cols;
+}
+
 template <class Cfg>
 __global__ void __launch_bounds__(Cfg::THREADS)
 gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int rows_out, const int N, const int K, const int ldc,
@@ -82,6 +96,7 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
     const int n0 = blockIdx.x * Cfg::BN, m0 = blockIdx.y * Cfg::MAX_M;
+    if (n0 >= p.N) return;  // (a grid rounded up, see skinny_dma_columns)
     const bool b_read_once = p.M <= Cfg::MAX_M;  // one block of rows (gridDim.y == 1, without fetching the grid's size)
     const int Kb = p.K >> 1;             // bytes per row; a multiple of 16
     const int nruns = (Kb + 127) >> 7;   // 128-byte runs per row, the last one possibly short

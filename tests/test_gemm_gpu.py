@@ -873,3 +873,15 @@ def test_blocks_of_48_rows_and_columns(m, n, k, name):
     qm.gemm_scaled(ap.to(DEV), bp.to(DEV), d, m, n, k, rs, cs)
     # (fp32 products of an exact integer and two scales, in either order: 2 roundings each, then one to bfloat16)
     torch.testing.assert_close(d.float(), want.float() * rs[:, None] * cs[None, :], rtol=2.0 ** -8 + 4 * 2.0 ** -24, atol=0)
+
+
+@pytest.mark.parametrize("name", ["d2x2_w8_r1", "d4x4_w4_r1", "d3x4_w8_r1"])
+@pytest.mark.parametrize("cols,rows", [(23, 2), (24, 2), (25, 1), (25, 2), (31, 3), (33, 7), (33, 8), (41, 6)])
+def test_column_blocks_rounded_up_to_the_xcds(name, cols, rows):
+    """Grids on both sides of skinny_dma_columns' rule, with workgroups beyond N; the last column and row blocks are partly outside C."""
+    fm, fn = (int(x) for x in name[1:].split("_")[0].split("x"))
+    m, n, k = 16 * fm * rows - 5, 16 * fn * cols - 3, 288
+    a = torch.randint(-8, 8, (m, k), dtype=torch.int8, generator=torch.Generator().manual_seed(SEED_BASE + 7300 + cols))
+    b = torch.randint(-8, 8, (n, k), dtype=torch.int8, generator=torch.Generator().manual_seed(SEED_BASE + 7400 + rows))
+    want = fp32_matmul_on_gpu(a, b)
+    np.testing.assert_array_equal(run_gemm(pack_cpu(a), pack_cpu(b), m, n, k, qm.config_id(name)), want.cpu().numpy())
