@@ -44,7 +44,9 @@ The ten numbers per configuration and the two of the K split are least-squares f
     python -m quadmul_amd.cost_model fit --data benchmarks/cost_model_data.jsonl --emit quadmul_amd/csrc/qm_cost_model.inc
     python -m quadmul_amd.cost_model check --data benchmarks/cost_model_data.jsonl      # the built library's choices
 
-``collect`` needs the GPU (it appends to the data file); ``fit`` and ``check`` do not.
+``collect`` needs the GPU (it appends to the data file); ``fit`` and ``check`` do not.  The timings of the
+wave-level kernel's blocks of 48, 80 and 96 rows on these shapes, on those of them that they make one round of workgroups of, were taken later than the others, with the same settings, after
+its grid had come to be rounded up to the XCDs.
 ``check`` prints, for the choice the built library makes on every shape of the data, the
 measured time of that choice over the best measured time of any candidate.
 """
@@ -68,6 +70,7 @@ CANDIDATES = [
     "q256x256_w2x2_s9o1", "q256x128_w2x2_s9o1", "q256x128_w2x2_s3o2", "q128x256_w2x2_s9o1", "q128x128_w2x2_s9o1",
     "q128x64_w2x2_s6o2", "q64x128_w2x2_s6o2", "q64x64_w2x2_s8o2",
     "d4x4_w8_r1", "d4x4_w4_r1", "d4x2_w8_r1", "d2x4_w8_r1", "d2x2_w8_r1", "d2x2_w1_r1", "d2x1_w16_r1", "d1x2_w8_r2", "d1x1_w4_r4",
+    "d3x2_w8_r1", "d3x3_w8_r1", "d3x4_w8_r1", "d4x3_w8_r1", "d5x2_w8_r1", "d5x3_w8_r1", "d5x4_w7_r1", "d6x3_w4_r1", "d6x4_w6_r1",
 ]
 SLOTS = (256, 512, 1024)
 BLENDS = (0.0, 0.25, 0.5, 0.75, 1.0)
@@ -172,13 +175,30 @@ def predict(par: Dict, model: Optional[Dict], name: str, m: int, n: int, k: int,
     return us
 
 
+def between_blocks(name: str) -> bool:
+    """Blocks of the wave-level kernel between those of 32 and 64 rows and columns."""
+    bm, bn = block_of(name)
+    return name[0] == "d" and bm > 32 and (bm % 64 != 0 or bn == 48)
+
+
+def offered(name: str, m: int, n: int, k: int) -> bool:
+    """Those only in one round of workgroups, and a few sizes left out (one_round_between in csrc/qm_select.hpp)."""
+    if not between_blocks(name):
+        return True
+    bm, bn = block_of(name)
+    rows, cols = -(-m // bm), -(-n // bn)
+    if k < 1024 or (m > 1024 or k > 16384 if m > 384 else m % 32 == 0):
+        return False
+    return cols <= 256 and not (bn == 32 and k > 16384) if rows == 1 else cols >= 24 and -(-cols // 8) * rows <= 32
+
+
 def choose(model: Dict, row: Dict) -> Tuple[str, int]:
     """The model's choice among the variants that were timed for the shape."""
     best = None
     for (name, ks) in times_of(row):
-        if name not in model["configs"]:
+        if name not in model["configs"] or not offered(name, row["m"], row["n"], row["k"]):
             continue
-        us = predict(model["configs"], model, name, row["m"], row["n"], row["k"], ks)
+        us = predict(model["configs"], model, name, row["m"], row["n"], row["k"], ks) * (1.03 if between_blocks(name) else 1.0)
         if best is None or us < best[0]:
             best = (us, name, ks)
     return best[1], best[2]

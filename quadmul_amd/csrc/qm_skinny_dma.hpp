@@ -89,6 +89,7 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
     p.out = packed_out(rows_out);
     p.ldc = ldc;
     constexpr int FM = Cfg::FM, FN = Cfg::FN, NW = Cfg::NW, D = Cfg::D, LPR = Cfg::LOADS_PER_RUN;
+    constexpr bool EARLY = FM <= 4;  // A's fragments widened before B's have landed; more of them would not stay in registers, and each is widened ahead of its products
     extern __shared__ __align__(16) uint8_t smem[];
     int32_t *const red = reinterpret_cast<int32_t *>(smem + Cfg::RING_BYTES);
 
@@ -174,13 +175,12 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
         // widened while B's are still on their way from HBM.
         const int younger = min(D - 1, cnt - 1 - it);
         wait_loads(younger, std::integral_constant<int, 2 * FN>{});
-        v4i aev[FM][2], aod[FM][2];
-        {
-            v4i apk[FM][2];
+        v4i aev[EARLY ? FM : 1][2], aod[EARLY ? FM : 1][2], apk[FM][2];
 #pragma unroll
-            for (int i = 0; i < FM; ++i)
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) apk[i][j] = *reinterpret_cast<const v4i *>(at + i * 2048 + rd_at[j]);
+            for (int j = 0; j < 2; ++j) apk[i][j] = *reinterpret_cast<const v4i *>(at + i * 2048 + rd_at[j]);
+        if constexpr (EARLY) {
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -213,10 +213,11 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
             for (int b = 0; b < FN; ++b) x16_expand_pairs(bpk[b][j], bev[b], bod[b]);
 #pragma unroll
             for (int i = 0; i < FM; ++i) {
+                if constexpr (!EARLY) x16_expand_pairs(apk[i][j], aev[0][j], aod[0][j]);
 #pragma unroll
-                for (int b = 0; b < FN; ++b) acc[i][b] = mfma16(bev[b], aev[i][j], acc[i][b]);
+                for (int b = 0; b < FN; ++b) acc[i][b] = mfma16(bev[b], aev[EARLY ? i : 0][j], acc[i][b]);
 #pragma unroll
-                for (int b = 0; b < FN; ++b) acc[i][b] = mfma16(bod[b], aod[i][j], acc[i][b]);
+                for (int b = 0; b < FN; ++b) acc[i][b] = mfma16(bod[b], aod[EARLY ? i : 0][j], acc[i][b]);
             }
         }
     }

@@ -885,3 +885,16 @@ def test_column_blocks_rounded_up_to_the_xcds(name, cols, rows):
     b = torch.randint(-8, 8, (n, k), dtype=torch.int8, generator=torch.Generator().manual_seed(SEED_BASE + 7400 + rows))
     want = fp32_matmul_on_gpu(a, b)
     np.testing.assert_array_equal(run_gemm(pack_cpu(a), pack_cpu(b), m, n, k, qm.config_id(name)), want.cpu().numpy())
+
+
+@pytest.mark.parametrize("m,n,k,name", [
+    (65, 8192, 1024, "d5x2"), (79, 8193, 4096, "d5x3"), (80, 12288, 1056, "d5x3"), (81, 12285, 2080, "d6x3"), (95, 16384, 1024, "d6x4"),
+    (65, 12289, 2048, "d5x4"), (145, 4096, 2048, "d5x2"), (159, 8191, 1120, "d5x4"), (189, 8190, 1184, "d6x4"), (321, 4095, 2048, "d6x4"),
+])
+def test_blocks_of_80_and_96_rows(m, n, k, name):
+    """Sizes that take them, from one row block to four, with rows and columns that end inside a block and every kind of short last K-step."""
+    assert qm.config_name(qm.select_config(m, n, k) & 0xFFFF).startswith(name)
+    a = torch.randint(-8, 8, (m, k), dtype=torch.int8, generator=torch.Generator().manual_seed(SEED_BASE + 7500 + n))
+    b = torch.randint(-8, 8, (n, k), dtype=torch.int8, generator=torch.Generator().manual_seed(SEED_BASE + 7600 + n))
+    want = fp32_matmul_on_gpu(a, b)
+    np.testing.assert_array_equal(run_gemm(pack_cpu(a), pack_cpu(b), m, n, k), want.cpu().numpy())
