@@ -233,6 +233,14 @@ def workload_text(name):
             f"C=A.B^T int32, uniform [-8,7] seed {hex(SEED_BASE + row)}")
 
 
+def operands_of(m, n, k):
+    """What the matrix cores multiply in a call of quadmul.gemm: the configuration named as its kernel
+    runs on int8; where it pays the call re-codes A and runs on 6-bit floats instead, with the same integers as its result."""
+    import quadmul_amd as qm
+
+    return "6-bit floats, A re-coded in the call" if qm.recode_bytes(m, n, k) > 0 else "int8"
+
+
 def run_target(name, issue_peak_tops):
     """One configuration of the contract as a `targets` entry: graph-timed, median of the replays."""
     import torch
@@ -260,7 +268,7 @@ def run_target(name, issue_peak_tops):
     config = qm.config_name(qm.select_config(m, n, k) & 0xFFFF)
     out = {
         "workload": workload_text(name), "m": m, "n": n, "k": k,
-        "kernel": config,
+        "kernel": config, "operands": operands_of(m, n, k),
         "timing": f"HIP graph of {launches} launches, median of 5 replays",
         "ms_per_launch": round(med, 5), "ms_per_launch_min_max": [round(lo, 5), round(hi, 5)],
         "tops": round(2.0 * m * n * k / med / 1e9, 2),
@@ -524,9 +532,10 @@ def main(argv=None):
         "value": round(2.0 * m * n * k / wall_ms / 1e9, 2), "unit": "TOPS", "n_gpus": 1, "steps": a.steps, "warmup": a.warmup,
         "ms_per_step": round(wall_ms, 5), "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "i8 (s4 nibbles widened to 16*s4) x i8 -> i32 MFMA, exact",
+        "dtype": "s4 as E2M3 floats (every int4 is one) -> f32 MFMA whose bits count integer units -> i32, exact" if qm.recode_bytes(m, n, k) > 0
+                 else "i8 (s4 nibbles widened to 16*s4) x i8 -> i32 MFMA, exact",
         "data": "synthetic",
-        "config": {"workload": workload_text(a.workload), "kernel": config,
+        "config": {"workload": workload_text(a.workload), "kernel": config, "operands": operands_of(m, n, k),
                    "entry_point": "quadmul.gemm(a, b, c, m, n, k)",
                    # untimed launches of the same kernel before the warm-ups (see time_steps)
                    "preheat_ms": pre["preheat_ms"], "preheat_launches": pre["preheat_launches"],
