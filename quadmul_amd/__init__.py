@@ -212,11 +212,17 @@ def _workspace(workspace, a, b, m, n, k, cfg, scaled):
         return None, 0, None
     if workspace is True:
         need = workspace_bytes(m, n, k, cfg, scaled, _ptr_align(a, b))
-        if cfg == CFG_AUTO:
-            need = max(need, recode_bytes(m, n, k, scaled, _ptr_align(a, b)))
-        if need == 0:
-            return None, 0, None
-        workspace = torch.empty((need,), dtype=torch.uint8, device=a.device)
+        faster = recode_bytes(m, n, k, scaled, _ptr_align(a, b)) if cfg == CFG_AUTO else 0
+        workspace = None
+        if faster > need:   # (bytes that the call can do without)
+            try:
+                workspace = torch.empty((faster,), dtype=torch.uint8, device=a.device)
+            except torch.cuda.OutOfMemoryError:
+                pass
+        if workspace is None:
+            if need == 0:
+                return None, 0, None
+            workspace = torch.empty((need,), dtype=torch.uint8, device=a.device)
     if not (isinstance(workspace, torch.Tensor) and workspace.is_cuda and workspace.device == a.device and workspace.is_contiguous()):
         raise QuadmulError("gemm: workspace must be a contiguous tensor on a's device")
     return workspace.data_ptr(), workspace.numel() * workspace.element_size(), workspace
@@ -300,9 +306,10 @@ def gemm(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, m: int, n: int, k: i
     and is overwritten; enqueued on the current stream of ``a``'s device; returns None.
 
     ``workspace``: True (default) takes a temporary buffer from torch's allocator when the
-    shape runs with K split over several workgroups per tile (few tiles, long K); None runs
-    without one (the splits then meet in ``c`` through atomics); a uint8 tensor is used as
-    it is.  The result is the same in every case."""
+    shape runs with K split over several workgroups per tile (few tiles, long K), or is a large
+    product that runs faster on 6-bit operands (up to 256 MiB; without them where the allocator
+    has no such memory left); None runs without one (the splits then meet in ``c`` through
+    atomics); a uint8 tensor is used as it is.  The result is the same in every case."""
     gemm_cfg(a, b, c, m, n, k, CFG_AUTO, workspace)
 
 

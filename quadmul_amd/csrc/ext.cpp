@@ -14,6 +14,7 @@
 
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <c10/util/Exception.h>
 
 #include "qm_abi.h"
 
@@ -62,11 +63,26 @@ int ptr_alignment(const torch::Tensor &a, const torch::Tensor &b)
     return low > 4096 ? 4096 : (int)low;
 }
 
+// Bytes that only make a call faster: an undefined tensor where the allocator does not have them, and the call runs
+// without (in a capture too: what it asks for there is the graph's pool, and nothing has been enqueued yet).
+torch::Tensor bytes_if_there_are(size_t bytes, const torch::TensorOptions &options)
+{
+    try {
+        return torch::empty({(int64_t)bytes}, options.dtype(torch::kUInt8));
+    } catch (const c10::OutOfMemoryError &) {
+        return torch::Tensor();
+    }
+}
+
 torch::Tensor workspace_for(const torch::Tensor &a, const torch::Tensor &b, int64_t m, int64_t n, int64_t k, int cfg, bool scaled)
 {
     const int align = ptr_alignment(a, b);
-    size_t need = qm_gemm_workspace_bytes((int)m, (int)n, (int)k, align, cfg, scaled ? 1 : 0);
-    if (cfg == QM_CFG_AUTO) need = std::max(need, qm_gemm_recode_bytes((int)m, (int)n, (int)k, align, scaled ? 1 : 0));
+    const size_t need = qm_gemm_workspace_bytes((int)m, (int)n, (int)k, align, cfg, scaled ? 1 : 0);
+    const size_t faster = cfg == QM_CFG_AUTO ? qm_gemm_recode_bytes((int)m, (int)n, (int)k, align, scaled ? 1 : 0) : 0;
+    if (faster > need) {
+        const torch::Tensor ws = bytes_if_there_are(faster, a.options());
+        if (ws.defined()) return ws;
+    }
     if (need == 0) return torch::Tensor();
     return torch::empty({(int64_t)need}, a.options().dtype(torch::kUInt8));
 }
@@ -167,12 +183,28 @@ torch::Tensor linear(torch::Tensor x, torch::Tensor weight, int64_t n, c10::opti
     c10::OptionalDeviceGuard guard(x.device());
     auto y = torch::empty({m, n}, x.options().dtype(out));
     const int in = t == torch::kFloat16 ? QM_IN_F16 : (t == torch::kBFloat16 ? QM_IN_BF16 : QM_IN_F32);
-    const size_t need = qm_linear_workspace_bytes((int)m, (int)n, (int)k, in, ptr_alignment(weight, weight));
+    const float *const col_scale = weight_scale.has_value() ? weight_scale->data_ptr<float>() : nullptr;
+    const void *const bias_ptr = bias.has_value() ? bias->data_ptr() : nullptr;
+    const int y_type = bf16 ? QM_OUT_BF16 : QM_OUT_F16, align = ptr_alignment(weight, weight);
+    const size_t need = qm_linear_workspace_bytes((int)m, (int)n, (int)k, in, align);
     torch::Tensor scratch;
-    if (need > 0) scratch = torch::empty({(int64_t)need}, x.options().dtype(torch::kUInt8));
-    check_status(qm_linear_i4(x.data_ptr(), in, weight.data_ptr(), y.data_ptr(), (int)m, (int)n, (int)k,
-                              weight_scale.has_value() ? weight_scale->data_ptr<float>() : nullptr, bias.has_value() ? bias->data_ptr() : nullptr,
-                              bf16 ? QM_OUT_BF16 : QM_OUT_F16, stream_of(x), need > 0 ? scratch.data_ptr() : nullptr, need),
+    if (need > 0) scratch = bytes_if_there_are(need, x.options());
+    if (need == 0 || scratch.defined()) {
+        check_status(qm_linear_i4(x.data_ptr(), in, weight.data_ptr(), y.data_ptr(), (int)m, (int)n, (int)k, col_scale, bias_ptr, y_type, stream_of(x),
+                                  need > 0 ? scratch.data_ptr() : nullptr, need),
+                     "quadmul.linear");
+        return y;
+    }
+    // The two calls it stands for, which can do with less: the packed rows, their scales and what the GEMM must have.
+    const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    const size_t packed_bytes = up((size_t)m * (k / 2)), scale_bytes = up((size_t)m * sizeof(float));
+    const size_t ws_bytes = qm_gemm_workspace_bytes((int)m, (int)n, (int)k, std::min(align, 256), QM_CFG_AUTO, 1);
+    scratch = torch::empty({(int64_t)(packed_bytes + scale_bytes + ws_bytes)}, x.options().dtype(torch::kUInt8));
+    uint8_t *const xq = scratch.data_ptr<uint8_t>();
+    float *const xs = reinterpret_cast<float *>(xq + packed_bytes);
+    check_status(qm_quantize_pack_i4(x.data_ptr(), in, xq, xs, (int)m, (int)k, stream_of(x)), "quadmul.linear");
+    check_status(qm_gemm_i4_scaled_bias_ws(xq, weight.data_ptr(), y.data_ptr(), (int)m, (int)n, (int)k, xs, col_scale, bias_ptr, y_type, stream_of(x),
+                                           QM_CFG_AUTO, ws_bytes ? xq + packed_bytes + scale_bytes : nullptr, ws_bytes),
                  "quadmul.linear");
     return y;
 }
