@@ -6,8 +6,6 @@
 #pragma once
 #include <cmath>
 #include <cstring>
-#include <string_view>
-#include <unordered_map>
 
 #include "qm_launch.hpp"
 
@@ -79,15 +77,30 @@ static LaunchFn scaled_launcher(int cfg)
     return launchers.of[cfg];
 }
 
+// By name, in a table of hashes that is filled once: every choice looks a name up.  (An array, not a container: these
+// calls come through a C interface, where an allocation that fails has nobody to throw to.)
 static int find_config(const char *name)
 {
-    static const std::unordered_map<std::string_view, int> ids = [] {
-        std::unordered_map<std::string_view, int> m;
-        for (int i = 0; i < g_num_configs; ++i) m.emplace(g_configs[i].name, i);
-        return m;
+    constexpr uint32_t SLOTS = 256;
+    static_assert(2 * g_num_configs <= SLOTS, "at most half full");
+    const auto slot = [](const char *s) {
+        uint32_t h = 2166136261u;  // FNV-1a
+        for (; *s; ++s) h = (h ^ (uint8_t)*s) * 16777619u;
+        return (h ^ (h >> 16)) % SLOTS;
+    };
+    static const auto ids = [&] {
+        struct { int16_t of[SLOTS]; } t;
+        for (int16_t &id : t.of) id = -1;
+        for (int i = 0; i < g_num_configs; ++i) {
+            uint32_t at = slot(g_configs[i].name);
+            while (t.of[at] >= 0) at = (at + 1) % SLOTS;
+            t.of[at] = (int16_t)i;
+        }
+        return t;
     }();
-    const auto it = ids.find(name);
-    return it == ids.end() ? -1 : it->second;
+    for (uint32_t at = slot(name); ids.of[at] >= 0; at = (at + 1) % SLOTS)
+        if (std::strcmp(g_configs[ids.of[at]].name, name) == 0) return ids.of[at];
+    return -1;
 }
 
 // The 16-byte-load kernels need whole, aligned chunks and 32-bit row offsets,
