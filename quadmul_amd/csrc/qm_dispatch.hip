@@ -789,7 +789,7 @@ LinearPlan linear_plan(int m, int n, int k, int in_dtype, int weight_align)
 {
     const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     LinearPlan pl{};
-    if (m <= 2 && fast_path_ok(m, n, k, weight_align) && n < (1 << 24) && dot_linear_pays(m, n, k)) {
+    if (m <= 2 && fast_path_ok(m, n, k, weight_align) && n < (1 << 24) && dot_linear_pays(m, n, k, in_dtype)) {
         pl.one_launch = true;
         return pl;
     }

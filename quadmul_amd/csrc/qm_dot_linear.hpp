@@ -8,22 +8,33 @@ namespace qm {
 // gemm_dot_kernel with the quantisation of its rows in front: every workgroup quantises x by itself, with the arithmetic of
 // quantize_pack_kernel, while the first of its loads of B are on their way.  That is a few elements per
 // thread out of the L2; as a kernel of its own it is a second launch, 2.4 us and the gap between dependent kernels, in front of a
-// GEMM of 2 to 3 (1 x 4096 x 4096), and on the host half of a call.  From three rows on the matrix core does the GEMM,
-// and the elements a workgroup would quantise by itself take longer than its B.
+// GEMM of 2 to 3 (1 x 4096 x 4096), and on the host half of a call.  From three rows on the matrix core does the GEMM, in
+// kernels that take packed rows; whether those should quantise too has not been measured.
 template <int IN, int MR_, int NW_, int U_>
 struct DotLinearCfg {
     static constexpr int MR = MR_, NW = NW_, U = U_, THREADS = 64 * NW, BN = 16;
     static constexpr int NC = 4;  // chunks of eight elements per thread and row that stay in registers between the maximum and the quantisation
 };
 inline int dot_linear_lds_bytes(int mr, int k) { return mr * (k / 2); }
-// Against two launches (us inside a graph, weights from HBM, two / one): 1 x 1024 x 1024 4.46 / 3.18, 1 x 4096 x 4096 5.54 / 4.46,
-// 1 x 4096 x 11008 8.77 / 7.83, 1 x 28672 x 4096 14.2 / 13.1, but 1 x 8192 x 28672 27.1 / 28.2 -- seven turns over K, each waiting for its own
-// loads; two rows 1024 x 1024 4.90 / 3.71, 4096 x 4096 5.99 / 5.13, 4096 x 11008 9.14 / 8.74, but 22016 x 4096 12.6 / 14.2 (every workgroup
-// quantises, and there are 1376 of them) and 8192 x 8192 11.0 / 14.3 (the GEMM by itself runs on the matrix core there).
-inline bool dot_linear_pays(int m, int n, int k)
+// Against two launches, by the columns of one round of workgroups: every workgroup quantises x again, which costs little beside
+// its own B while it runs once, and the launch and more where the device takes a second round of them.  A
+// round is what registers leave room for (fp16 56, else 72 on 16 waves and one row: two workgroups of 1024
+// threads per CU, or one).  Time, one launch / two inside a graph, weights from HBM, the range over 2500 sizes in all:
+//   one row   K > 4096         fp16 to 8192 columns 0.81 .. 1.02, else to 4096 0.83 .. 0.92; beyond 0.91 .. 1.11 and 1.04 .. 1.38
+//             2048 < K <= 4096 0.83 .. 1.01 to 65536
+//             K <= 2048        fp16 to 16384 0.69 .. 1.01 (from a K of 1536, 24576), else to 12288 0.69 .. 0.95; beyond 0.98 .. 2.1
+//   two rows  K > 4096         to 4096 0.85 .. 1.00; beyond 1.17 .. 1.31
+//             K <= 4096        to 8192 0.74 .. 1.02 (fp16 from a K of 3072, 12288: 0.92 .. 1.00); beyond 0.96 .. 3.5
+// us, two / one: 1 x 1024 x 1024 4.46 / 3.18, 1 x 4096 x 4096 5.54 / 4.46, 1 x 28672 x 4096 14.2 / 13.1, but 1 x 10240 x 8192 12.2 / 15.0
+// and 2 x 174481 x 64 17 / 60.  Above a K of 16384 a row takes more turns than hide their loads: 1 x 8192 x 28672 27.1 / 28.2.
+inline bool dot_linear_pays(int m, int n, int k, int in)
 {
+    const bool f16 = in == QM_IN_F16;
     if (k > 16384) return false;
-    return m == 1 || ((long long)n * k <= (3LL << 24) && !(k > 4096 && n >= 8192));
+    if (m == 2) return n <= (k > 4096 ? 4096 : (f16 && k >= 3072 ? 12288 : 8192));
+    if (k > 4096) return n <= (f16 ? 8192 : 4096);
+    if (k > 2048) return n <= 65536;
+    return n <= (f16 ? (k >= 1536 ? 24576 : 16384) : 12288);
 }
 
 template <int IN, class Cfg>
