@@ -272,22 +272,32 @@ static double fp6_tile_us(int m, int n, int k, bool narrow)
     return kt * (rounds * (k & 255 ? 0.5784 : 0.5042) + fill * 0.3183) + rounds * 13.83 - 2.94;
 }
 
-// Automatic choice: where the better of the two tiles is 5 % below what the model says of the int8 configuration `direct`.
-// A K split of the int8 tiles counts with what it costs.  `coded`: A comes as codes, or both ways copy their operands, so
-// that only the GEMM counts; else the re-coding is a launch of its own and 0.17 us per million elements of A.  Of those 272
-// products: coded, it takes 155, 18 % faster in the mean, none slower by 1 %; with the re-coding 98, 13 % faster, two slower by
-// more than 3 % (10.5 %).  Without the margin it gains the same on more of them, and loses on more; below a K of 512, or of 1280
-// with the re-coding, it gains nothing.  us, int8 / here: 1280 x 8192 x 14336 124 / 91, 8192 x 8192 x 8192 325 / 290,
-// 512 x 28672 x 4096 45.8 / 41.9, 2048 x 4096 x 11008 65.1 / 63.7 (coded 55.7).
+// Automatic choice: where the better of the two tiles, with what its operands cost more than those of the int8 configuration
+// `direct`, is 5 % below what the model says of that.  A K split of the int8 tiles counts with what it costs.  What A's codes cost, by
+// where they come from (us; fitted to the same calls timed both ways):
+//   FP6_FROM_PACKED  a launch of its own: 4.7 and 0.17 per million elements of A;
+//   FP6_FROM_COPY    the launch that would copy both operands re-codes A instead: 0.5 and 0.3 per thousand rows more;
+//   FP6_FROM_X       the layer's quantisation writes codes instead of packed rows: 0.15 per million elements more.
+// The model's term for an N that is no multiple of four is left out: the int8 tiles have since come to lose a few percent on
+// such a C, the term says twenty.  One round of 256 x 128 that is more than half full has to be 10 % below: with most CUs at
+// work it loses more than the model says.  Below a K of 512, or of 1280 from packed rows, it gains nothing.
+// Measured against the int8 choice, B from HBM: from packed rows, 2450 products, taken on 2190 and 0.83 of the time in the mean, six more than
+// 2 % slower (5 %; 2816 x 2635 x 2112, once taken, 22.3 / 26.5 us); copied, 1260, 0.81 on 1105, three (4 %; 5386 x 938 x 1066, once taken, 19.0 / 23.7); layers, 460,
+// 0.82 on 425, one (2 %; 4381 x 951 x 15232, once taken, 99 / 117).  A wider margin loses gains of 8 % on average on ten times the calls it
+// saves from a loss.  us, int8 / here: 8192 x 8192 x 8192 356 / 297, 1280 x 8192 x 14336 124 / 91, 512 x 28672 x 4096 45.8 / 41.9.
 // (The bound on the product comes first: calls that the host bounds do not get as far as the model.)
 enum Fp6Route { FP6_NO = 0, FP6_WIDE, FP6_NARROW };
-static Fp6Route fp6_route(int m, int n, int k, int ptr_align, const Choice &direct, bool coded)
+enum Fp6Source { FP6_FROM_PACKED, FP6_FROM_COPY, FP6_FROM_X };
+static Fp6Route fp6_route(int m, int n, int k, int ptr_align, const Choice &direct, Fp6Source source)
 {
-    if ((double)m * n * k < 4e9 || m < 200 || k < (coded ? 512 : 1280) || !fp6_fits(m, n, k, ptr_align)) return FP6_NO;
+    if ((double)m * n * k < 4e9 || m < 200 || k < (source == FP6_FROM_PACKED ? 1280 : 512) || !fp6_fits(m, n, k, ptr_align)) return FP6_NO;
     const CostFit *f = fit_of(direct.cfg);
-    if (f == nullptr) return FP6_NO;
-    const double wide = fp6_tile_us(m, n, k, false), narrow = fp6_tile_us(m, n, k, true), first = coded ? 0.0 : 4.68 + 0.1685e-6 * m * k;
-    if (std::min(wide, narrow) + first >= 0.95 * modelled_us(*f, g_configs[direct.cfg], m, n, k, direct.ksplit)) return FP6_NO;
+    if (f == nullptr) return FP6_NO;  // (the choices for up to 64 rows and the any-address ones have none: neither gets here)
+    const double wide = fp6_tile_us(m, n, k, false), narrow = fp6_tile_us(m, n, k, true);
+    const double codes = source == FP6_FROM_PACKED ? 4.68 + 0.1685e-6 * m * k : source == FP6_FROM_COPY ? 0.5 + 0.3e-3 * m : 0.15e-6 * m * k;
+    const long long tiles = (long long)((m + 255) / 256) * ((n + 127) / 128);
+    const double margin = narrow < wide && tiles > 128 && tiles <= 256 ? 0.90 : 0.95;
+    if (std::min(wide, narrow) + codes >= margin * modelled_us(*f, g_configs[direct.cfg], m, (n + 3) & ~3, k, direct.ksplit)) return FP6_NO;
     return narrow < wide ? FP6_NARROW : FP6_WIDE;
 }
 static Fp6Route fp6_asked_for(int cfg) { return cfg == QM_CFG_RECODE ? FP6_WIDE : cfg == QM_CFG_RECODE_NARROW ? FP6_NARROW : FP6_NO; }
@@ -494,7 +504,7 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
     ch.ksplit = effective_ksplit(g_configs[ch.cfg], k, ch.ksplit);
     const bool auto_ws = cfg == QM_CFG_AUTO && has_ws && ((uintptr_t)workspace & 15) == 0;
     if (auto_ws) {
-        const Fp6Route route = fp6_route(m, n, k, align, ch, false);
+        const Fp6Route route = fp6_route(m, n, k, align, ch, FP6_FROM_PACKED);
         if (route && workspace_bytes >= fp6_layout(m, k).bytes) {
             const hipError_t e = launch_fp6(p, route, workspace, s);
             return e == hipSuccess ? QM_OK : fail_launch(e);
@@ -513,7 +523,7 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
     if (cfg == QM_CFG_AUTO && has_ws) {
         PadPlan pl = plan_padded_k(m, n, k, align, ch);
         if (pl.on && auto_ws) {
-            const Fp6Route route = fp6_route(m, n, pl.kp, 256, pl.ch, true);
+            const Fp6Route route = fp6_route(m, n, pl.kp, 256, pl.ch, FP6_FROM_COPY);
             if (route && workspace_bytes >= fp6_padded_bytes(m, pl.kp, pl)) {
                 const hipError_t e = launch_fp6_padded(p, pl, route, workspace, s);
                 return e == hipSuccess ? QM_OK : fail_launch(e);
@@ -679,9 +689,9 @@ QM_EXPORT size_t qm_gemm_recode_bytes(int m, int n, int k, int ptr_align, int sc
     if (row_block_for_large_a(m, n, k, ptr_align) || col_block_for_large_b(m, n, k, ptr_align)) return 0;
     Choice ch = scaled ? select_scaled(m, n, k, ptr_align, true) : select_config(m, n, k, ptr_align, true);
     ch.ksplit = effective_ksplit(g_configs[ch.cfg], k, ch.ksplit);
-    if (fp6_route(m, n, k, ptr_align, ch, false)) return fp6_layout(m, k).bytes;
+    if (fp6_route(m, n, k, ptr_align, ch, FP6_FROM_PACKED)) return fp6_layout(m, k).bytes;
     const PadPlan pl = plan_padded_k(m, n, k, ptr_align, ch);
-    return pl.on && fp6_route(m, n, pl.kp, 256, pl.ch, true) ? fp6_padded_bytes(m, pl.kp, pl) : 0;
+    return pl.on && fp6_route(m, n, pl.kp, 256, pl.ch, FP6_FROM_COPY) ? fp6_padded_bytes(m, pl.kp, pl) : 0;
 }
 
 QM_EXPORT int qm_config_has_scaled(int cfg)
@@ -798,7 +808,7 @@ LinearPlan linear_plan(int m, int n, int k, int in_dtype, int weight_align)
     if ((double)m * n * k >= 4e9 && quant6_fits(k, in_dtype) && row_block_for_large_a(m, n, k, pl.align) == 0 && col_block_for_large_b(m, n, k, pl.align) == 0) {
         Choice ch = select_scaled(m, n, k, pl.align, true);
         ch.ksplit = effective_ksplit(g_configs[ch.cfg], k, ch.ksplit);
-        pl.coded = fp6_route(m, n, k, pl.align, ch, true);
+        pl.coded = fp6_route(m, n, k, pl.align, ch, FP6_FROM_X);
     }
     if (pl.coded) {
         pl.row_bytes = fp6_layout(m, k).bytes;

@@ -21,3 +21,30 @@ def one_launch(m, n, k, dtype):
     (2, 8000, 896, BF16, True), (2, 11821, 1056, BF16, False), (3, 64, 64, F16, False)], ids=str)     # 0.98, 1.17
 def test_linear_layers_of_one_or_two_rows(m, n, k, dtype, one):
     assert one_launch(m, n, k, dtype) == one
+
+
+def recoded(m, n, k, align=256):
+    return qm.recode_bytes(m, n, k, ptr_align=align) > 0
+
+
+@pytest.mark.parametrize("m,n,k,codes", [
+    # time on 6-bit operands over that on the int8 choice, B from HBM.  A re-coded from packed rows
+    (8192, 8192, 8192, True), (1753, 8192, 8192, True), (3584, 4096, 4096, True), (5601, 2627, 13376, True),       # 0.83, 0.82, 0.94, 0.86
+    (2816, 2635, 2112, False), (6912, 5099, 1536, False), (5502, 1139, 4544, False), (964, 7321, 3456, False),   # 1.19, 1.15, 1.14, 1.13
+    (830, 5611, 3904, False), (4352, 1472, 17696, False), (2304, 3040, 8224, False), (1280, 4096, 11008, False),   # 1.09, 1.05, 1.05, 1.03
+    # both operands copied with padded rows
+    (1531, 3307, 4100, True), (2148, 27456, 1370, True), (6954, 1045, 604, False), (5386, 938, 1066, False),        # 0.91, 0.88, 1.27, 1.25
+    (1392, 11198, 682, False), (5096, 922, 1388, False), (2375, 3234, 2402, False)], ids=str)                      # 1.23, 1.21, 1.14
+def test_large_products_on_6_bit_operands(m, n, k, codes):
+    assert recoded(m, n, k) == codes
+
+
+@pytest.mark.parametrize("m,n,k,codes", [(2048, 11008, 4096, True), (3078, 2368, 4544, True), (4381, 951, 15232, False),          # 0.85, 0.94, 1.18
+                                         (3456, 1184, 11488, False), (6168, 1125, 5792, False), (2587, 1792, 13952, False)], ids=str)   # 1.11, 1.07, 1.07
+def test_large_layers_on_6_bit_operands(m, n, k, codes):
+    """... quantised straight to codes, or by way of packed rows."""
+    got = qm.library().qm_linear_workspace_bytes(m, n, k, BF16, 256) - (4 * m + 255) // 256 * 256
+    steps = -(-k // 128) + (-(-k // 128) & 1)
+    packed = (m * (k // 2) + 255) // 256 * 256
+    layout = (m + 31) // 32 * (steps * 3072 + -(-steps // 32) * 32 * 4)
+    assert got == (layout if codes else packed + max(qm.workspace_bytes(m, n, k, scaled=True), qm.recode_bytes(m, n, k, True)))
