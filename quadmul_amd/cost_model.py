@@ -187,7 +187,7 @@ def offered(name: str, m: int, n: int, k: int) -> bool:
         return True
     bm, bn = block_of(name)
     rows, cols = -(-m // bm), -(-n // bn)
-    if k < 1024 or (m > 1024 or k > 16384 if m > 384 else m % 32 == 0):
+    if k < 1024 or (k > 20480 and k % 256) or (m > 1024 or k > 16384 if m > 384 else m % 32 == 0):
         return False
     return cols <= 256 and not (bn == 32 and k > 16384) if rows == 1 else cols >= 24 and -(-cols // 8) * rows <= 32
 

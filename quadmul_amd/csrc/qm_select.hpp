@@ -232,19 +232,21 @@ static double modelled_us(const CostFit &f, const ConfigDesc &d, int m, int n, i
     return us;
 }
 
-// Blocks of 48, 80 and 96 rows, or of 48 columns, of the wave-level kernel, where they make one round of workgroups and blocks of 32 or 64 a
-// round and a part of one, or more rows that are copies of the last: 65 x 12288 x 4096 13.0 -> 9.9 us, 80 x 11008 x 8192 22.0 -> 15.1,
-// 144 x 8192 x 28672 60.7 -> 39.3; 0.86 of the time in the geometric mean of 250 random shapes that the rule takes, B from HBM, none of them more than
-// 2 % slower.  In a second round they are as often behind (75 x 28672 x 8192 31.6 -> 34.1, 482 x 2976 x 3328 10.8 -> 11.9).
-// Measured up to 1024 rows, above 384 of them up to a K of 16384.  Up to 384, whole blocks of 32 rows keep to blocks of 32 and 64, which leave none of theirs empty: 96 and 192 rows would gain
-// too (96 x 11008 x 4096 12.4 -> 10.2 us, 192 x 4096 x 4096 7.8 -> 7.2), but what those run on is promised.  One round of several row
-// blocks is one on each XCD, whole columns to an XCD (skinny_dma_columns): spread otherwise, B is read once more per XCD
-// (358 x 1568 x 12000 on 80 x 32 17.2 us, on 64 x 64 15.6).  Below a K of 1024 a launch is mostly its start and its end (759 x 1646 x 736
-// 6.3 -> 6.7); 80 x 32 in one row block falls behind on a very long K (75 x 8192 x 28672 32.3 us, 64 x 64 31.3, 48 x 64 27.4).
+// Blocks of 48, 80 and 96 rows, or of 48 columns, of the wave-level kernel, where they make one round of workgroups and
+// blocks of 32 or 64 a round and a part of one, or more rows that are copies of the last: 65 x 12288 x 4096 13.0 -> 9.9 us,
+// 80 x 11008 x 8192 22.0 -> 15.1, 144 x 8192 x 28672 60.7 -> 39.3; 0.83 of the time in the geometric mean of 1045 sizes that the
+// rule takes, B from HBM, two of them more than 2 % slower (7 %).  In a second round they are as often behind (75 x 28672 x 8192
+// 31.6 -> 34.1, 482 x 2976 x 3328 10.8 -> 11.9).  One round of several row blocks is one on each XCD, whole columns to an XCD
+// (skinny_dma_columns): spread otherwise, B is read once more per XCD (358 x 1568 x 12000 on 80 x 32 17.2 us, on 64 x 64 15.6).
+// Not taken: below a K of 1024, where a launch is mostly its start and its end (759 x 1646 x 736 6.3 -> 6.7); rows that are no whole
+// 128-byte lines on a very long K, where 17 of 149 lost up to 23 % (77 x 15034 x 30944 65 -> 80; whole lines gain there, 207 sizes, 0.79);
+// 80 x 32 in one row block on a very long K (75 x 8192 x 28672 32.3 us, 64 x 64 31.3, 48 x 64 27.4); above 384 rows, what was
+// not measured: more than 1024 rows, a K above 16384.  Up to 384, whole multiples of 32 rows, whose choices were there before these
+// blocks and are held by the tests of the selection: they would gain too (96 x 11008 x 4096 12.4 -> 10.2 us, 192 x 4096 x 4096 7.8 -> 7.2).
 static bool between_blocks(const ConfigDesc &d) { return d.bm > 32 && (d.bm % 64 != 0 || d.bn == 48); }
 static bool one_round_between(const ConfigDesc &d, int m, int n, int k)
 {
-    if (k < 1024 || (m > 384 ? m > 1024 || k > 16384 : m % 32 == 0)) return false;
+    if (k < 1024 || (k > 20480 && k % 256 != 0) || (m > 384 ? m > 1024 || k > 16384 : m % 32 == 0)) return false;
     const long long rows = (m + d.bm - 1) / d.bm, cols = (n + d.bn - 1) / d.bn;
     if (rows == 1) return cols <= 256 && !(d.bn == 32 && k > 16384);
     return cols >= 24 && (cols + 7) / 8 * rows <= 32;
@@ -267,7 +269,7 @@ static Choice modelled_choice(int m, int n, int k, int ptr_align, bool has_ws, b
         const bool between = !tile && between_blocks(d);
         if (between && !one_round_between(d, m, n, k)) continue;
         const auto offer = [&](double us, int ks) {
-            if (between) us *= 1.03;  // (ahead by more than a share of the fit's error)
+            if (between) us *= 1.03;  // (fitted to 20 to 62 sizes each, the others to 310: where the two are even, the others)
             if (us < best_us) { best_us = us; best = Choice{id, tile ? 4 : 1, ks}; }
         };
         if (!scaled || scaled_launcher(id)) offer(modelled_us(f, d, m, n, k, 1), 1);

@@ -48,3 +48,18 @@ def test_large_layers_on_6_bit_operands(m, n, k, codes):
     packed = (m * (k // 2) + 255) // 256 * 256
     layout = (m + 31) // 32 * (steps * 3072 + -(-steps // 32) * 32 * 4)
     assert got == (layout if codes else packed + max(qm.workspace_bytes(m, n, k, scaled=True), qm.recode_bytes(m, n, k, True)))
+
+
+def block(m, n, k):
+    """Rows and columns of a block of the wave-level kernel that the call runs on, or None: tiles of the pipelined one."""
+    name = qm.config_name(qm.select_config(m, n, k) & 0xFFFF)
+    return tuple(16 * int(x) for x in name[1:].split("_")[0].split("x")) if name[0] == "d" else None
+
+
+@pytest.mark.parametrize("m,n,k,between", [
+    (144, 8192, 28672, True), (82, 8192, 28672, True), (105, 4889, 32000, True), (79, 9088, 19168, True),              # 0.65, 0.98, 0.99, 1.02
+    (77, 15034, 30944, False), (80, 16074, 28704, False), (95, 8786, 24160, False), (377, 1787, 31040, False),         # 1.23, 1.22, 1.19, 1.09
+    (213, 4352, 24928, False), (248, 2445, 25120, False), (93, 8501, 21888, False)], ids=str)                          # 1.09, 1.07, 1.07
+def test_blocks_between_32_and_96_rows_on_a_very_long_k(m, n, k, between):
+    got = block(m, n, k)
+    assert (got is not None and got[0] > 32 and (got[0] % 64 != 0 or got[1] == 48)) == between
