@@ -65,10 +65,13 @@ struct SkinnyDmaCfg {
 // The grid's first dimension for so many column and row blocks.  With several row blocks it is rounded up to a multiple
 // of the 8 XCDs (the workgroups beyond N end at once), for the reason above: where the readers of one column block
 // sit on different XCDs, each of those fetches B's lines for itself.  Time with / without, B from HBM: 65 x 4100 x 4096 on 32 x 64
-// 5.8 / 6.8 us, 128 x 4100 x 28672 on 32 x 64 35 / 51, 320 x 5500 x 8192 on 64 x 64 21.5 / 24.7; geometric mean 0.90 over 270
-// cases with the rule, none more than 1 % slower.  The rule: an XCD then holds whole columns, the fullest of them one column of
-// row blocks more than the emptiest.  Below 24 columns, or where that column is a round more on the 32 CUs of its XCD than
-// all blocks are on 256 CUs, the imbalance costs more (41 columns of 6 row blocks: 1.25 times the time).
+// 5.8 / 6.8 us, 128 x 4100 x 28672 on 32 x 64 35 / 51, 320 x 5500 x 8192 on 64 x 64 21.5 / 24.7; geometric mean 0.94 over 1338
+// sizes with the rule, 0.88 where B is 4 to 16 MB, 1.00 below 1 MB; 84 of them more than 2 % slower (6 %), which only in part is the grid: the
+// check below costs the kernel up to 4 % on some sizes and gives as much on others (see there).  The rule: an XCD then holds whole
+// columns, the fullest of them one column of row blocks more than the emptiest.  Below 24 columns, or where that column is a round
+// more on the 32 CUs of its XCD than all blocks are on 256 CUs, the imbalance costs more (41 columns of 6 row blocks: 1.25 times
+// the time).  Without the rounding below 1.5 MB, or where four row blocks meet a number of columns that is 4 modulo 8, so that only two XCDs
+// read a column: 1.003 and 1.04 of the time.
 inline int skinny_dma_columns(int cols, int rows)
 {
     if (rows < 2 || cols < 24) return cols;
@@ -97,7 +100,10 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
     const int n0 = blockIdx.x * Cfg::BN, m0 = blockIdx.y * Cfg::MAX_M;
-    if (n0 >= p.N) return;  // (a grid rounded up, see skinny_dma_columns)
+    // A grid rounded up, see skinny_dma_columns.  (With a branch here the compiler moves the bodies of those around the loads to the end of the kernel, and
+    // each load waits for a jump.  A pause between the loads that refill the ring does the same: waves of three runs are 3 .. 8 % faster with it, 156 x
+    // 2824 x 5280 7.8 -> 7.2 us, those of two or of many 1 .. 4 % slower, 113 x 4096 x 4096 5.76 -> 5.97.  Over 2500 sizes the two forms are even.)
+    if (n0 >= p.N) return;
     const bool b_read_once = p.M <= Cfg::MAX_M;  // one block of rows (gridDim.y == 1, without fetching the grid's size)
     const int Kb = p.K >> 1;             // bytes per row; a multiple of 16
     const int nruns = (Kb + 127) >> 7;   // 128-byte runs per row, the last one possibly short
