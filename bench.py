@@ -20,8 +20,10 @@ resident in HBM.  Prints ONE JSON line:
   replay reported per launch.  HBM-bound shapes are reported with the launches rotating
   over copies of B that exceed the memory-side cache (B really comes from HBM), the
   figure on one cache-resident B beside it;
-* ``mfma_issue_peak`` / ``launch_floor``: what the part itself sustains (a loop of the
-  GEMM's MFMA instruction alone; an empty kernel and a read-only kernel per launch);
+* ``mfma_issue_peak`` / ``mfma6_issue_peak`` / ``launch_floor``: what the part itself sustains (loops of
+  the GEMM's two MFMA instructions alone; an empty kernel and a read-only kernel per launch).  A
+  ``roofline`` of a product that runs on 6-bit operands is against that instruction's nominal and
+  measured peaks; ``frac_of_int8_peak`` is its rate over the nominal int8 one, as for the others;
 * ``cpu_baseline``: the CPU oracle (a restatement of the reference's ``cpu_gemm_int8``)
   timed on this box's host cores on a bounded sample of the headline workload and on
   configuration [0] (1024^3) in full, which also checks the GPU result bit for bit.
@@ -42,6 +44,7 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 INT8_PEAK_TOPS = 5033.2   # dense int8 MFMA: 256 CU x 8192 op/clk/CU x 2.4 GHz
+FP6_PEAK_TOPS = 2 * INT8_PEAK_TOPS   # the same of the 6-bit float MFMA
 HBM_PEAK_GBS = 8000.0
 SEED_BASE = 0x51AD0000
 
@@ -165,9 +168,12 @@ _TITLE = re.compile(r"^# (\S+?)_kernel, configuration (\S+?),(?: [^\n]*?)? on (\
 _TOTAL = re.compile(r"^\| total \| \| (\d+) \|", re.M)
 
 
+_TILE6 = re.compile(r"^\| `gemm_tile6_kernel<Tile6Cfg<(\d+), (\d+),", re.M)
+
+
 def profile_summaries(root=None):
-    """{workload: {"path", "kernel", "config", "shape", "traffic"}} for every profiles/*__<workload>.md
-    with a traffic table."""
+    """{workload: {"path", "kernel", "config", "shape", "traffic", "tile6"}} for every profiles/*__<workload>.md
+    with a traffic table (``tile6``: the tile on 6-bit operands in its kernel trace, as ``kernel_name`` has it, or None)."""
     out = {}
     for path in sorted(glob.glob(os.path.join(root or ROOT, "profiles", "*__*.md"))):
         with open(path) as f:
@@ -177,7 +183,8 @@ def profile_summaries(root=None):
         if not title or not total:
             continue
         out[title.group(3)] = {"path": "profiles/" + os.path.basename(path), "kernel": title.group(1), "config": title.group(2),
-                               "shape": tuple(int(title.group(i)) for i in (4, 5, 6)), "traffic": int(total.group(1))}
+                               "shape": tuple(int(title.group(i)) for i in (4, 5, 6)), "traffic": int(total.group(1)),
+                               "tile6": next((f"t{t.group(1)}x{t.group(2)}" for t in _TILE6.finditer(text)), None)}
     return out
 
 
@@ -192,6 +199,13 @@ def profile_total(workload):
     return None
 
 
+def tile6_of(m, n, k, scaled=False):
+    """The tile on 6-bit operands that a call of this size runs on, or None: an int8 kernel."""
+    import quadmul_amd as qm
+
+    return qm.kernel_name(m, n, k, scaled) if qm.recode_bytes(m, n, k, scaled) > 0 else None
+
+
 def profiled_traffic(name, m, n, k, config):
     """(bytes per launch, where from) for workload `name` running configuration `config`."""
     prof = profile_summaries().get(name)
@@ -199,20 +213,28 @@ def profiled_traffic(name, m, n, k, config):
         return None, "no rocprofv3 summary of this workload under profiles/"
     if prof["shape"] != (m, n, k) or prof["config"] != config:
         return None, f"{prof['path']} profiled {prof['config']}, the library now chooses {config}: not used"
+    runs = tile6_of(m, n, k, name.endswith("_scaled_f16"))
+    if prof["tile6"] != runs:
+        return None, f"{prof['path']} profiled {prof['tile6'] or 'the int8 kernel'}, the call now runs on {runs or 'the int8 kernel'}: not used"
     return prof["traffic"], f"rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, profiled offline ({prof['path']})"
 
 
-def roofline_of(m, n, k, bound, ms, issue_peak_tops=None, name=None, config=None):
+def roofline_of(m, n, k, bound, ms, issue_peaks=None, name=None, config=None):
+    """`issue_peaks`: (int8, 6-bit) TOP/s of the loops of the instruction alone."""
     ops = 2.0 * m * n * k
     traffic, source = profiled_traffic(name, m, n, k, config) if name else (None, None)
+    six = tile6_of(m, n, k) is not None
     if bound == "mfma":
-        achieved, peak, unit = ops / ms / 1e9, INT8_PEAK_TOPS, "TOP/s"
+        achieved, peak, unit = ops / ms / 1e9, FP6_PEAK_TOPS if six else INT8_PEAK_TOPS, "TOP/s"
     else:
         achieved, peak, unit = algorithmic_bytes(m, n, k) / ms / 1e6, HBM_PEAK_GBS, "GB/s"
     r = {"bound": bound, "achieved": round(achieved, 1), "peak": peak, "unit": unit, "frac": round(achieved / peak, 4),
          "traffic": traffic, "traffic_source": source, "algorithmic_bytes": algorithmic_bytes(m, n, k), "launch_us": round(ms * 1e3, 3)}
-    if bound == "mfma" and issue_peak_tops:
-        r["frac_of_measured_issue_peak"] = round(achieved / issue_peak_tops, 4)
+    if bound == "mfma":
+        r["peak_of"] = "6-bit float MFMA" if six else "int8 MFMA"
+        r["frac_of_int8_peak"] = round(achieved / INT8_PEAK_TOPS, 4)
+        if issue_peaks:
+            r["frac_of_measured_issue_peak"] = round(achieved / issue_peaks[1 if six else 0], 4)
     return r
 
 
@@ -234,14 +256,18 @@ def workload_text(name):
 
 
 def operands_of(m, n, k):
-    """What the matrix cores multiply in a call of quadmul.gemm: the configuration named as its kernel
-    runs on int8; where it pays the call re-codes A and runs on 6-bit floats instead, with the same integers as its result."""
-    import quadmul_amd as qm
-
-    return "6-bit floats, A re-coded in the call" if qm.recode_bytes(m, n, k) > 0 else "int8"
+    """What the matrix cores multiply in a call of quadmul.gemm: int8, or, where it pays to re-code A in the call, 6-bit
+    floats, with the same integers as its result."""
+    return "int8" if tile6_of(m, n, k) is None else "6-bit floats, A re-coded in the call"
 
 
-def run_target(name, issue_peak_tops):
+def kernel_of(m, n, k, config):
+    """``kernel``: what runs; beside a tile on 6-bit operands the int8 configuration that runs without the workspace for them."""
+    six = tile6_of(m, n, k)
+    return {"kernel": config} if six is None else {"kernel": f"gemm_tile6 {six}", "kernel_without_workspace": config}
+
+
+def run_target(name, issue_peaks):
     """One configuration of the contract as a `targets` entry: graph-timed, median of the replays."""
     import torch
 
@@ -268,7 +294,7 @@ def run_target(name, issue_peak_tops):
     config = qm.config_name(qm.select_config(m, n, k) & 0xFFFF)
     out = {
         "workload": workload_text(name), "m": m, "n": n, "k": k,
-        "kernel": config, "operands": operands_of(m, n, k),
+        **kernel_of(m, n, k, config), "operands": operands_of(m, n, k),
         "timing": f"HIP graph of {launches} launches, median of 5 replays",
         "ms_per_launch": round(med, 5), "ms_per_launch_min_max": [round(lo, 5), round(hi, 5)],
         "tops": round(2.0 * m * n * k / med / 1e9, 2),
@@ -291,7 +317,7 @@ def run_target(name, issue_peak_tops):
                                    f"graph of {5 * ncopies} launches, median of 5 replays")
         out["roofline_b_cache_resident"] = roofline_of(m, n, k, bound, med, name=name, config=config)
     else:
-        out["roofline"] = roofline_of(m, n, k, bound, med, issue_peak_tops, name=name, config=config)
+        out["roofline"] = roofline_of(m, n, k, bound, med, issue_peaks, name=name, config=config)
     return out, (ap, bp, a_d, b_d, c_d)
 
 
@@ -514,13 +540,14 @@ def main(argv=None):
     torch.cuda.synchronize()
 
     probes = {}
-    issue_peak = None
+    issue_peaks = None
     if not a.no_probes:
         from quadmul_amd import probe
 
         probes["mfma_issue_peak"] = probe.mfma_issue_peak()
+        probes["mfma6_issue_peak"] = probe.mfma6_issue_peak()
         probes["launch_floor"] = probe.launch_floor()
-        issue_peak = probes["mfma_issue_peak"]["tops"]
+        issue_peaks = probes["mfma_issue_peak"]["tops"], probes["mfma6_issue_peak"]["tops"]
 
     # ---- the headline: exactly `steps` calls of quadmul.gemm after `warmup` untimed ones ----
     wall_ms, ev, pre = time_steps(fn, a.steps, a.warmup, a.preheat_ms)
@@ -535,7 +562,7 @@ def main(argv=None):
         "dtype": "s4 as E2M3 floats (every int4 is one) -> f32 MFMA whose bits count integer units -> i32, exact" if qm.recode_bytes(m, n, k) > 0
                  else "i8 (s4 nibbles widened to 16*s4) x i8 -> i32 MFMA, exact",
         "data": "synthetic",
-        "config": {"workload": workload_text(a.workload), "kernel": config, "operands": operands_of(m, n, k),
+        "config": {"workload": workload_text(a.workload), **kernel_of(m, n, k, config), "operands": operands_of(m, n, k),
                    "entry_point": "quadmul.gemm(a, b, c, m, n, k)",
                    # untimed launches of the same kernel before the warm-ups (see time_steps)
                    "preheat_ms": pre["preheat_ms"], "preheat_launches": pre["preheat_launches"],
@@ -543,7 +570,7 @@ def main(argv=None):
                    "ms_per_step_events_min_max": [round(ev["min"], 5), round(ev["max"], 5)],
                    "ms_per_launch_graph_median": round(graph_med, 5), "ms_per_launch_graph_min_max": [round(graph_lo, 5), round(graph_hi, 5)]},
         # average launch duration over the timed steps, from the HIP events around them
-        "roofline": roofline_of(m, n, k, bound, event_ms, issue_peak, name=a.workload, config=config),
+        "roofline": roofline_of(m, n, k, bound, event_ms, issue_peaks, name=a.workload, config=config),
     }
     line["roofline"]["duration_source"] = (f"one HIP event per step on the launch stream: first to last over the {a.steps} timed steps, average per launch "
                                            f"(after {pre['preheat_launches']} untimed launches = {pre['preheat_ms']} ms of the same kernel and {a.warmup} warm-ups)")
@@ -560,7 +587,7 @@ def main(argv=None):
         for name in WORKLOADS:
             if name == a.workload:
                 continue
-            res, (tap, tbp, ta_d, tb_d, tc_d) = run_target(name, issue_peak)
+            res, (tap, tbp, ta_d, tb_d, tc_d) = run_target(name, issue_peaks)
             if name == "square4096":
                 res.update(extras_4096(ta_d, tb_d, tc_d))
             targets.append(res)

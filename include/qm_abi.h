@@ -55,14 +55,15 @@ extern "C" {
  * is a no-op, k == 0 zero-fills C).
  *
  * Seven arguments leave no room for a workspace.  On every shape whose best schedule needs
- * none -- 40 of the 42 shapes of the reference's table (kernel.cu:343-384), every BASELINE
- * shape, K below one 128-nibble step -- this entry point runs exactly what qm_gemm_i4_ws
- * runs.  It is slower than qm_gemm_i4_ws / qm_gemm_i4_static (measured, MI355X, both columns
- * of benchmarks/mi355x.md's second table) in two cases:
+ * none -- 18 of the 42 shapes of the reference's table (kernel.cu:343-384), up to 64 rows, K below
+ * one 128-nibble step -- this entry point runs exactly what qm_gemm_i4_ws runs.  It is slower than qm_gemm_i4_ws / qm_gemm_i4_static (measured, MI355X, both columns
+ * of benchmarks/mi355x.md's second table) in three cases:
+ *   - large products, which run on 6-bit floats when they are lent qm_gemm_recode_bytes (not qm_gemm_i4_static):
+ *     22 of the table's shapes, 1.03 to 1.31 times as long here;
  *   - few output tiles and a long K, which those entry points split over several workgroups
  *     per tile through the workspace: here the best unsplit configuration runs instead.
- *     Two shapes of the reference's table are left that split K: 256 x 8192 x 28672, 59.3 us
- *     against 55.8 (1.06x), and 512 x 8192 x 28672, 96-105 us against 92-95 (1.04-1.11x);
+ *     Two shapes of the reference's table are left that split K: 256 x 8192 x 28672, 56.0 to 59.3 us
+ *     against 54.4 to 55.8, and 512 x 8192 x 28672, 94-105 us against 92-95 (1.02 to 1.11x);
  *   - K % 32 != 0, or A or B not 16-byte aligned: the kernel for operands at any address runs,
  *     several times slower on many rows than the zero-padded copies in a workspace.  Weight
  *     matrices of the reference's table all have K % 32 == 0.
@@ -157,6 +158,9 @@ size_t qm_gemm_workspace_bytes(int m, int n, int k, int ptr_align, int cfg, int 
  * qm_gemm_workspace_bytes(..., cfg, scaled) bytes; QM_ERR_CONFIG elsewhere, and from the calls that take none.
  */
 size_t qm_gemm_recode_bytes(int m, int n, int k, int ptr_align, int scaled);
+/* The tiles that a call with those bytes runs on: QM_CFG_RECODE, QM_CFG_RECODE_NARROW, or QM_CFG_AUTO where they are 0
+ * (qm_select_config_ex then names the kernel; it names the one that runs without them elsewhere). */
+int qm_recode_config(int m, int n, int k, int ptr_align, int scaled);
 
 /*
  * qm_gemm_i4 for callers that cannot allocate and have no workspace to lend: code under HIP
@@ -231,7 +235,7 @@ int qm_quantize_pack_i4(const void *x, int in_dtype, void *dst_packed, float *sc
  * output on them -- D[m][n] as qm_gemm_i4_scaled_bias_ws gives it with their scales as row_scale -- and
  * the same values bit for bit as those two calls one after the other.  The reference has no counterpart.
  * Large products go from x to the 6-bit operands of qm_gemm_recode_bytes without the packed rows in between; one or two
- * rows are one launch and want no workspace.
+ * rows are one launch, which wants no workspace, while its workgroups run in one round (qm_linear_workspace_bytes is 0).
  *   workspace    device memory, 256-byte aligned, at least qm_linear_workspace_bytes(...) bytes (weight_align: the
  *                alignment of B in bytes), else QM_ERR_SCRATCH and nothing is enqueued; used in stream order by
  *                the kernels of this call only

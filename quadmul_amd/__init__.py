@@ -38,7 +38,7 @@ CFG_RECODE, CFG_RECODE_NARROW = -2, -3
 #: every symbol include/qm_abi.h declares
 ABI_SYMBOLS = (
     "qm_gemm_i4", "qm_gemm_i4_cfg", "qm_gemm_i4_scaled", "qm_gemm_i4_scaled_cfg", "qm_config_has_scaled",
-    "qm_gemm_i4_ws", "qm_gemm_i4_static", "qm_gemm_i4_scaled_ws", "qm_gemm_i4_scaled_bias_ws", "qm_gemm_workspace_bytes", "qm_gemm_recode_bytes", "qm_quantize_pack_i4", "qm_select_config", "qm_select_config_ex", "qm_num_configs", "qm_config_name",
+    "qm_gemm_i4_ws", "qm_gemm_i4_static", "qm_gemm_i4_scaled_ws", "qm_gemm_i4_scaled_bias_ws", "qm_gemm_workspace_bytes", "qm_gemm_recode_bytes", "qm_recode_config", "qm_quantize_pack_i4", "qm_select_config", "qm_select_config_ex", "qm_num_configs", "qm_config_name",
     "qm_config_supports", "qm_pack_i4", "qm_unpack_i4", "qm_status_string", "qm_last_hip_error", "qm_version", "qm_init",
     "qm_debug_set_operand_limit", "qm_linear_workspace_bytes", "qm_linear_i4",
 )
@@ -83,6 +83,8 @@ def library() -> ctypes.CDLL:
     lib.qm_gemm_workspace_bytes.restype = ctypes.c_size_t
     lib.qm_gemm_recode_bytes.argtypes = [ci, ci, ci, ci, ci]
     lib.qm_gemm_recode_bytes.restype = ctypes.c_size_t
+    lib.qm_recode_config.argtypes = [ci, ci, ci, ci, ci]
+    lib.qm_recode_config.restype = ci
     lib.qm_linear_workspace_bytes.argtypes = [ci, ci, ci, ci, ci]
     lib.qm_linear_workspace_bytes.restype = ctypes.c_size_t
     lib.qm_linear_i4.argtypes = [vp, ci, vp, vp, ci, ci, ci, vp, vp, ci, vp, vp, ctypes.c_size_t]
@@ -202,6 +204,17 @@ def workspace_bytes(m: int, n: int, k: int, cfg: int = CFG_AUTO, scaled: bool = 
 def recode_bytes(m: int, n: int, k: int, scaled: bool = False, ptr_align: int = 256) -> int:
     """Bytes of workspace with which a large product runs on 6-bit re-coded operands (0: that would not pay)."""
     return int(library().qm_gemm_recode_bytes(m, n, k, ptr_align, 1 if scaled else 0))
+
+
+def recode_config(m: int, n: int, k: int, scaled: bool = False, ptr_align: int = 256) -> int:
+    """The tiles a call with :func:`recode_bytes` runs on: ``CFG_RECODE``, ``CFG_RECODE_NARROW``, or ``CFG_AUTO`` (neither)."""
+    return int(library().qm_recode_config(m, n, k, ptr_align, 1 if scaled else 0))
+
+
+def kernel_name(m: int, n: int, k: int, scaled: bool = False, ptr_align: int = 256) -> str:
+    """What ``gemm`` / ``gemm_scaled`` with ``workspace=True`` runs on: the configuration's name, or the tile on 6-bit operands."""
+    tile = {CFG_RECODE: "t256x256", CFG_RECODE_NARROW: "t256x128"}.get(recode_config(m, n, k, scaled, ptr_align))
+    return tile or config_name(select_config_ex(m, n, k, ptr_align, True, scaled) & 0xFFFF)
 
 
 def _workspace(workspace, a, b, m, n, k, cfg, scaled):

@@ -281,10 +281,11 @@ static double fp6_tile_us(int m, int n, int k, bool narrow)
 // The model's term for an N that is no multiple of four is left out: the int8 tiles have since come to lose a few percent on
 // such a C, the term says twenty.  One round of 256 x 128 that is more than half full has to be 10 % below: with most CUs at
 // work it loses more than the model says.  Below a K of 512, or of 1280 from packed rows, it gains nothing.
-// Measured against the int8 choice, B from HBM: from packed rows, 2450 products, taken on 2190 and 0.83 of the time in the mean, six more than
-// 2 % slower (5 %; 2816 x 2635 x 2112, once taken, 22.3 / 26.5 us); copied, 1260, 0.81 on 1105, three (4 %; 5386 x 938 x 1066, once taken, 19.0 / 23.7); layers, 460,
-// 0.82 on 425, one (2 %; 4381 x 951 x 15232, once taken, 99 / 117).  A wider margin loses gains of 8 % on average on ten times the calls it
-// saves from a loss.  us, int8 / here: 8192 x 8192 x 8192 356 / 297, 1280 x 8192 x 14336 124 / 91, 512 x 28672 x 4096 45.8 / 41.9.
+// Measured against the int8 choice, B from HBM: from packed rows, 2450 products, taken on 2190 and 0.83 of the time in the mean,
+// six more than 2 % slower (5 %; 2816 x 2635 x 2112, once taken, 22.3 / 26.5 us); copied, 1260, 0.81 on 1105, three (4 %; 5386 x
+// 938 x 1066, once taken, 19.0 / 23.7); layers, 460, 0.82 on 425, one (2 %; 4381 x 951 x 15232, once taken, 99 / 117).  A wider
+// margin loses gains of 8 % on average on ten times the calls it saves from a loss.  us, int8 / here: 8192 x 8192 x 8192
+// 356 / 297, 1280 x 8192 x 14336 124 / 91, 512 x 28672 x 4096 45.8 / 41.9.
 // (The bound on the product comes first: calls that the host bounds do not get as far as the model.)
 enum Fp6Route { FP6_NO = 0, FP6_WIDE, FP6_NARROW };
 enum Fp6Source { FP6_FROM_PACKED, FP6_FROM_COPY, FP6_FROM_X };
@@ -683,15 +684,36 @@ QM_EXPORT size_t qm_gemm_workspace_bytes(int m, int n, int k, int ptr_align, int
     return 0;
 }
 
-QM_EXPORT size_t qm_gemm_recode_bytes(int m, int n, int k, int ptr_align, int scaled)
+// The tiles that a call with enough workspace runs on as 6-bit floats (or none), and that workspace.
+static Fp6Route recode_route(int m, int n, int k, int ptr_align, int scaled, size_t *bytes)
 {
-    if (m < 1 || n < 1 || (double)m * n * k < 3.5e9 || (k & 1)) return 0;   // (padded to 128, a K that counts here is a sixth longer at most)
-    if (row_block_for_large_a(m, n, k, ptr_align) || col_block_for_large_b(m, n, k, ptr_align)) return 0;
+    *bytes = 0;
+    if (m < 1 || n < 1 || (double)m * n * k < 3.5e9 || (k & 1)) return FP6_NO;   // (padded to 128, a K that counts here is a sixth longer at most)
+    if (row_block_for_large_a(m, n, k, ptr_align) || col_block_for_large_b(m, n, k, ptr_align)) return FP6_NO;
     Choice ch = scaled ? select_scaled(m, n, k, ptr_align, true) : select_config(m, n, k, ptr_align, true);
     ch.ksplit = effective_ksplit(g_configs[ch.cfg], k, ch.ksplit);
-    if (fp6_route(m, n, k, ptr_align, ch, FP6_FROM_PACKED)) return fp6_layout(m, k).bytes;
+    if (const Fp6Route route = fp6_route(m, n, k, ptr_align, ch, FP6_FROM_PACKED)) {
+        *bytes = fp6_layout(m, k).bytes;
+        return route;
+    }
     const PadPlan pl = plan_padded_k(m, n, k, ptr_align, ch);
-    return pl.on && fp6_route(m, n, pl.kp, 256, pl.ch, FP6_FROM_COPY) ? fp6_padded_bytes(m, pl.kp, pl) : 0;
+    const Fp6Route route = pl.on ? fp6_route(m, n, pl.kp, 256, pl.ch, FP6_FROM_COPY) : FP6_NO;
+    if (route) *bytes = fp6_padded_bytes(m, pl.kp, pl);
+    return route;
+}
+
+QM_EXPORT size_t qm_gemm_recode_bytes(int m, int n, int k, int ptr_align, int scaled)
+{
+    size_t bytes;
+    recode_route(m, n, k, ptr_align, scaled, &bytes);
+    return bytes;
+}
+
+QM_EXPORT int qm_recode_config(int m, int n, int k, int ptr_align, int scaled)
+{
+    size_t bytes;
+    const Fp6Route route = recode_route(m, n, k, ptr_align, scaled, &bytes);
+    return route == FP6_WIDE ? QM_CFG_RECODE : route == FP6_NARROW ? QM_CFG_RECODE_NARROW : QM_CFG_AUTO;
 }
 
 QM_EXPORT int qm_config_has_scaled(int cfg)

@@ -10,6 +10,9 @@
 //                         issue peak of the matrix cores at the clock the part sustains,
 //                         with every MFMA on the same operand registers or rotating over
 //                         four pairs of them
+//   qm_probe_mfma6_issue  the same of v_mfma_f32_16x16x128_f8f6f4 on 6-bit floats that are
+//                         int4 values, the first operand as b + 8 (no sign bits) and the second as
+//                         sign and magnitude: the forms of the GEMM's tile kernel on them
 //   qm_probe_empty        a kernel that does nothing: the launch floor
 //   qm_probe_read         a kernel that only reads `bytes` (16 bytes per lane, whole lines)
 //                         and keeps a checksum: the floor of "launch + one pass over B"
@@ -19,11 +22,12 @@
 #define QM_PROBE_EXPORT extern "C" __attribute__((visibility("default")))
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v6i __attribute__((ext_vector_type(6)));
 
 namespace {
 
 constexpr int MFMA_PER_ITER = 16;   // independent accumulators: 16 x 4 AGPRs
-constexpr int MFMA_OPS = 2 * 16 * 16 * 64;
+constexpr int MFMA_OPS = 2 * 16 * 16 * 64, MFMA6_OPS = 2 * 16 * 16 * 128;
 
 // One workgroup of four waves (one per SIMD) per launch slot; `iters` trips of 16 MFMAs.
 // PAIRS: distinct operand register pairs the MFMAs of a trip rotate over (1: every MFMA reads
@@ -68,6 +72,58 @@ __global__ void __launch_bounds__(256) mfma_issue_kernel(uint64_t *out, int iter
     if (sum == 0x7fffffff && iters < 0) out[0] = (uint64_t)sum;  // keeps the accumulators alive
 }
 
+// 32 six-bit fields of a lane's operand, each `low` | sign << 5: E2M3 floats whose upper exponent bit is clear
+__device__ v6i random_codes(uint32_t &h, const bool has_sign)
+{
+    uint64_t bits[3] = {0, 0, 0};
+    for (int f = 0; f < 32; ++f) {
+        h ^= h << 13; h ^= h >> 17; h ^= h << 5;
+        const int value = (int)(h >> 28) - 8;  // an int4
+        const uint64_t code = has_sign ? (uint64_t)((value < 0 ? 32 : 0) | (value < 0 ? -value : value)) : (uint64_t)(value + 8);
+        const int at = 6 * f, w = at >> 6, b = at & 63;
+        bits[w] |= code << b;
+        if (b > 58) bits[w + 1] |= code >> (64 - b);
+    }
+    return v6i{(int)bits[0], (int)(bits[0] >> 32), (int)bits[1], (int)(bits[1] >> 32), (int)bits[2], (int)(bits[2] >> 32)};
+}
+
+__device__ __forceinline__ void mfma6(v4i &acc, const v6i &s0, const v6i &s1)
+{
+    asm volatile("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0 cbsz:2 blgp:2" : "+a"(acc) : "v"(s0), "v"(s1));
+}
+
+// mfma_issue_kernel with the other instruction: 16 independent accumulators a wave, PAIRS operand pairs in rotation.
+template <int PAIRS>
+__global__ void __launch_bounds__(256) mfma6_issue_kernel(uint64_t *out, int iters, uint32_t seed)
+{
+    uint32_t h = (threadIdx.x + 1) * 2654435761u + blockIdx.x * 40503u + seed;
+    v6i s0[PAIRS], s1[PAIRS];
+#pragma unroll
+    for (int q = 0; q < PAIRS; ++q) {
+        s0[q] = random_codes(h, false);
+        s1[q] = random_codes(h, true);
+    }
+    v4i acc[MFMA_PER_ITER];
+#pragma unroll
+    for (int i = 0; i < MFMA_PER_ITER; ++i) acc[i] = v4i{0x48400000, 0x48400000, 0x48400000, 0x48400000};  // 1.5 * 2^17, as the GEMM's
+    const uint64_t t0 = __builtin_readcyclecounter(), r0 = wall_clock64();
+    for (int it = 0; it < iters; ++it) {
+#pragma unroll
+        for (int i = 0; i < MFMA_PER_ITER; ++i)
+            mfma6(acc[i], s0[i % PAIRS], s1[i % PAIRS]);
+    }
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    const uint64_t t1 = __builtin_readcyclecounter(), r1 = wall_clock64();
+    int sum = 0;
+#pragma unroll
+    for (int i = 0; i < MFMA_PER_ITER; ++i) sum += acc[i].x ^ acc[i].y ^ acc[i].z ^ acc[i].w;
+    if (threadIdx.x == 0) {
+        out[2 * blockIdx.x] = t1 - t0;
+        out[2 * blockIdx.x + 1] = r1 - r0;
+    }
+    if (sum == 0x7fffffff && iters < 0) out[0] = (uint64_t)sum;
+}
+
 __global__ void empty_kernel() {}
 
 // (launched with 256 or 1024 threads per workgroup and any amount of dynamic LDS, which it
@@ -102,6 +158,17 @@ QM_PROBE_EXPORT double qm_probe_mfma_issue(void *out, int blocks, int iters, int
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return -(double)(int)e;
     return (double)blocks * 4.0 * (double)iters * MFMA_PER_ITER * (double)MFMA_OPS;
+}
+
+QM_PROBE_EXPORT double qm_probe_mfma6_issue(void *out, int blocks, int iters, int operand_pairs, void *stream)
+{
+    if (!out || blocks < 1 || iters < 1 || (operand_pairs != 1 && operand_pairs != 4)) return -1.0;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (operand_pairs == 1) mfma6_issue_kernel<1><<<dim3(blocks), dim3(256), 0, s>>>(static_cast<uint64_t *>(out), iters, 12345u);
+    else mfma6_issue_kernel<4><<<dim3(blocks), dim3(256), 0, s>>>(static_cast<uint64_t *>(out), iters, 12345u);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return -(double)(int)e;
+    return (double)blocks * 4.0 * (double)iters * MFMA_PER_ITER * (double)MFMA6_OPS;
 }
 
 QM_PROBE_EXPORT int qm_probe_empty(void *stream)

@@ -9,6 +9,8 @@ what the part sustains, measured on the box, to set beside the nominal peaks.
   reference's harness times its kernel (kernel.cu:468-497).  One such MFMA is 32768 integer
   operations and issues in 16 cycles of a SIMD, so the rate also gives the clock the part
   sustains under that load.
+* ``mfma6_issue_peak``: the same of ``v_mfma_f32_16x16x128_f8f6f4`` on 6-bit floats that are int4 values
+  (twice the operations per instruction, in the forms the GEMM's tile kernel feeds it).
 * ``launch_floor``: an empty kernel, and a kernel that only reads 8 MiB, per launch inside a
   graph of back-to-back launches -- what any kernel on an 8 MiB operand pays before it
   computes anything.
@@ -25,6 +27,7 @@ _LIB_PATH = os.path.join(_PKG, "lib", "libqm_probe.so")
 _lib = None
 
 INT8_PEAK_TOPS = 5033.2      # 256 CU x 8192 op/clk x 2.4 GHz
+FP6_PEAK_TOPS = 2 * INT8_PEAK_TOPS
 NOMINAL_MHZ = 2400.0
 
 
@@ -37,6 +40,8 @@ def library() -> ctypes.CDLL:
         vp, ci = ctypes.c_void_p, ctypes.c_int
         lib.qm_probe_mfma_issue.argtypes = [vp, ci, ci, ci, vp]
         lib.qm_probe_mfma_issue.restype = ctypes.c_double
+        lib.qm_probe_mfma6_issue.argtypes = [vp, ci, ci, ci, vp]
+        lib.qm_probe_mfma6_issue.restype = ctypes.c_double
         lib.qm_probe_empty.argtypes = [vp]
         lib.qm_probe_empty.restype = ci
         lib.qm_probe_read.argtypes = [vp, ctypes.c_size_t, vp, ci, ci, ci, vp]
@@ -45,16 +50,16 @@ def library() -> ctypes.CDLL:
     return _lib
 
 
-def _mfma_issue_rate(lib, out, blocks, iters, pairs, seconds):
+def _mfma_issue_rate(issue, out, blocks, iters, pairs, seconds):
     """(TOP/s, ms per launch, warm-up launches) of the MFMA-only loop on `pairs` operand register pairs."""
     import torch
 
     stream = torch.cuda.current_stream().cuda_stream
 
     def launch():
-        ops = lib.qm_probe_mfma_issue(out.data_ptr(), blocks, iters, pairs, stream)
+        ops = issue(out.data_ptr(), blocks, iters, pairs, stream)
         if ops < 0:
-            raise RuntimeError(f"qm_probe_mfma_issue: hipError_t {int(-ops)}")
+            raise RuntimeError(f"MFMA issue probe: hipError_t {int(-ops)}")
         return ops
 
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
@@ -94,8 +99,8 @@ def mfma_issue_peak(seconds: float = 0.6, blocks_per_cu: int = 1):
     blocks = cus * blocks_per_cu
     out = torch.zeros(2 * blocks, dtype=torch.int64, device=dev)
     iters = 12000   # x 16 MFMAs x 16 cycles = 3.07 M cycles: about 1.3 ms at 2.4 GHz
-    tops1, ms1, _ = _mfma_issue_rate(lib, out, blocks, iters, 1, seconds)
-    tops, ms, n_warm = _mfma_issue_rate(lib, out, blocks, iters, 4, seconds)
+    tops1, ms1, _ = _mfma_issue_rate(lib.qm_probe_mfma_issue, out, blocks, iters, 1, seconds)
+    tops, ms, n_warm = _mfma_issue_rate(lib.qm_probe_mfma_issue, out, blocks, iters, 4, seconds)
     counters = out.view(-1, 2).cpu()
     core, ref = int(counters[:, 0].max()), int(counters[:, 1].max())
     res = {
@@ -117,6 +122,27 @@ def mfma_issue_peak(seconds: float = 0.6, blocks_per_cu: int = 1):
         # s_memtime counts core cycles; reported as read
         res["memtime_per_100mhz_tick"] = round(core / ref, 3)
     return res
+
+
+def mfma6_issue_peak(seconds: float = 0.6, blocks_per_cu: int = 1):
+    """``mfma_issue_peak`` of the 6-bit instruction."""
+    import torch
+
+    lib = library()
+    dev = torch.device("cuda:0")
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    blocks = cus * blocks_per_cu
+    out = torch.zeros(2 * blocks, dtype=torch.int64, device=dev)
+    iters = 12000
+    tops1, _, _ = _mfma_issue_rate(lib.qm_probe_mfma6_issue, out, blocks, iters, 1, seconds)
+    tops, ms, n_warm = _mfma_issue_rate(lib.qm_probe_mfma6_issue, out, blocks, iters, 4, seconds)
+    return {
+        "tops": round(tops, 1), "frac_of_nominal_fp6_peak": round(tops / FP6_PEAK_TOPS, 4),
+        "implied_clock_mhz": round(tops / (FP6_PEAK_TOPS * cus / 256.0) * NOMINAL_MHZ, 0),
+        "instruction": "v_mfma_f32_16x16x128_f8f6f4 on E2M3 codes of random int4 values (b + 8 without sign bits, a as sign and magnitude), "
+                       "16 independent accumulators per wave, one wave per SIMD, consecutive MFMAs on four different pairs of operand registers",
+        "launch_ms_median_of_5": round(ms, 4), "warmup_launches": n_warm, "cus": cus, "tops_one_operand_pair": round(tops1, 1),
+    }
 
 
 def launch_floor(read_bytes: int = 8 << 20, launches: int = 200, replays: int = 5, blocks: int = 512, threads: int = 256, lds_bytes: int = 0):
@@ -171,7 +197,7 @@ def launch_floor(read_bytes: int = 8 << 20, launches: int = 200, replays: int = 
 
 
 def main():
-    print(json.dumps({"mfma_issue_peak": mfma_issue_peak(), "launch_floor": launch_floor()}))
+    print(json.dumps({"mfma_issue_peak": mfma_issue_peak(), "mfma6_issue_peak": mfma6_issue_peak(), "launch_floor": launch_floor()}))
 
 
 if __name__ == "__main__":

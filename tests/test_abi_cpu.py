@@ -320,6 +320,10 @@ def test_every_profile_summary_is_of_the_configuration_the_library_chooses():
         scaled = name.endswith("_scaled_f16")
         chosen = qm.config_name(qm.select_config_ex(m, n, k, scaled=scaled) & 0xFFFF)
         assert prof["config"] == chosen, f"{prof['path']} profiled {prof['config']}, the library now chooses {chosen} for {m}x{n}x{k}"
+        # ... and of the tile that runs, where the call runs on 6-bit operands instead
+        runs = qm.kernel_name(m, n, k, scaled)
+        assert prof["tile6"] == (runs if runs != chosen else None), f"{prof['path']} profiled {prof['tile6']}, {m}x{n}x{k} now runs on {runs}"
+        assert (prof["kernel"] == "gemm_tile6") == (runs != chosen), prof["path"]
         # the file is named for the kernel, the configuration and the workload it covers
         assert os.path.basename(prof["path"]).endswith(f"{prof['config']}__{name}.md"), prof["path"]
         total = prof["traffic"]
@@ -351,6 +355,8 @@ def test_benchmark_table_rows_name_the_kernels_the_library_chooses():
         cells = [c.strip() for c in l.strip("|").split("|")]
         m, n, k = int(cells[0]), int(cells[1]), int(cells[2])
         kernel = cells[-1]
+        if (m, n, k) not in seen:  # (the first table, whose calls may run on 6-bit operands)
+            assert cells[-2] == qm.kernel_name(m, n, k), f"benchmarks/mi355x.md row {m}x{n}x{k} ran on {cells[-2]}: regenerate the table"
         if (m, n, k) in seen:     # (the second table, timed through the bare seven-argument entry point)
             chosen = qm.config_name(qm.select_config_ex(m, n, k, workspace=False) & 0xFFFF)
         else:
