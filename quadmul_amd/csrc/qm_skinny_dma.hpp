@@ -100,9 +100,10 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
     const int n0 = blockIdx.x * Cfg::BN, m0 = blockIdx.y * Cfg::MAX_M;
-    // A grid rounded up, see skinny_dma_columns.  (With a branch here the compiler moves the bodies of those around the loads to the end of the kernel, and
-    // each load waits for a jump.  A pause between the loads that refill the ring does the same: waves of three runs are 3 .. 8 % faster with it, 156 x
-    // 2824 x 5280 7.8 -> 7.2 us, those of two or of many 1 .. 4 % slower, 113 x 4096 x 4096 5.76 -> 5.97.  Over 2500 sizes the two forms are even.)
+    // A grid rounded up, see skinny_dma_columns.  (With a branch here the compiler moves the bodies of those around the loads to
+    // the end of the kernel, and each load waits for a jump.  A pause between the loads that refill the ring does the same: waves
+    // of three runs are 3 .. 8 % faster with it, 156 x 2824 x 5280 7.8 -> 7.2 us, those of two or of many 1 .. 4 % slower, 113 x
+    // 4096 x 4096 5.76 -> 5.97.  Over 2500 sizes the two forms are even.)
     if (n0 >= p.N) return;
     const bool b_read_once = p.M <= Cfg::MAX_M;  // one block of rows (gridDim.y == 1, without fetching the grid's size)
     const int Kb = p.K >> 1;             // bytes per row; a multiple of 16

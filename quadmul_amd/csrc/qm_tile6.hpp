@@ -2,11 +2,11 @@
 //
 // A 6-bit E2M3 float with the upper exponent bit clear is a sign and a four-bit magnitude in
 // units of 1/8, so every int4 value is one of its codes, and the matrix core takes 128 of them per
-// instruction in the time it takes 64 int8: 8.0 against 4.5 POP/s on a loop of the instruction
-// alone.  Products are multiples of 1/64; the fp32 accumulators start from 1.5 * 2^17, where
+// instruction in the time it takes 64 int8: 7.3 to 7.9 against 4.4 to 4.5 POP/s, box to box, on a loop of the
+// instruction alone (quadmul_amd/probe.py; on one pair of operand registers, which do not toggle, 8.4 to 8.9).  Products are multiples of 1/64; the fp32 accumulators start from 1.5 * 2^17, where
 // one unit in the last place is 1/64, so their bit patterns count those units as an integer would
-// and every sum is exact (|C| <= 64 K < 2^22, K < 65536; checked against 64-bit integers on the
-// extremes up to K = 37248).
+// and every sum is exact (|C| <= 64 K < 2^22, K < 65536; checked on the
+// extremes, in closed form, up to K = 65504).
 //
 // The price is the re-coding, and each operand pays it where it is cheaper:
 //   * A is re-coded ahead of the GEMM by expand_a6_kernel into the caller's workspace, exactly
@@ -22,11 +22,14 @@
 // K-step -- it follows.  8192 x 8192 x 8192 runs at 1.80 GHz (int8: 2.15) in 459 thousand cycles, 390 of them
 // a loop of its matrix instructions alone; without its loads into the LDS the clock rises to 2.13 GHz and
 // the cycles stay.  us, this kernel / int8: 8192 x 8192 x 8192 264 / 336, 2048 x 11008 x 4096 64 / 77,
-// 4096 x 4096 x 4096 42.6 / 48.5; re-coding A costs 16, 4.4 and 5.3 more, and a launch.
+// 4096 x 4096 x 4096 42.6 / 48.5; the kernel that re-codes A takes 18 to 23, 5 to 10 and 7 to 8 more (traced).
 //
 // Eight waves, two per SIMD: a wave by itself issues a vector instruction every eight cycles (two every four),
 // and the 56 re-coding instructions per wave and K-step then take longer than the matrix ones (four waves
 // with 128 x 128 each: 281 us instead of 262).
+//
+// Registers: the 256 x 256 tile keeps 1 of them in scratch memory (int32), 10 (scaled) or 23 (scaled, bias), all of it
+// around an item's start and write-out: no reload, whose wait would drain the counted loads, lies in the loop over K.
 //
 // Tiles of 256 x 128 (4 x 2 waves) halve the grain where 256 x 256 leaves most of a round idle: per K-step and round 0.53 us
 // against 0.82, per round 5.8 against 13.8; their LDS has room for a write-out area of its own, where the large tile borrows a stage of B.
