@@ -19,22 +19,29 @@ inline int dot_linear_lds_bytes(int mr, int k) { return mr * (k / 2); }
 // Against two launches, by the columns of one round of workgroups: every workgroup quantises x again, which costs little beside
 // its own B while it runs once, and the launch and more where the device takes a second round of them.  A
 // round is what registers leave room for (fp16 56, else 72 on 16 waves and one row: two workgroups of 1024
-// threads per CU, or one).  Time, one launch / two inside a graph, weights from HBM, the range over 2500 sizes in all:
+// threads per CU, or one).  Some way into a second round the calls stay in one launch while that takes the GPU less than two take the
+// host, 8 to 9 us: called eagerly they then win by what the host saves, in a graph they lose the rest.
+// GPU time, one launch / two inside a graph, weights from HBM, the range over 2500 sizes in all, and eager calls in turn:
 //   one row   K > 4096         fp16 to 8192 columns 0.81 .. 1.02, else to 4096 0.83 .. 0.92; beyond 0.91 .. 1.11 and 1.04 .. 1.38
 //             2048 < K <= 4096 0.83 .. 1.01 to 65536
-//             K <= 2048        fp16 to 16384 0.69 .. 1.01 (from a K of 1536, 24576), else to 12288 0.69 .. 0.95; beyond 0.98 .. 2.1
+//             K <= 2048        fp16 to 16384 0.69 .. 1.01, else to 12288 0.69 .. 0.95; to 24576 0.93 .. 1.16, eager 0.65 .. 0.97
+//                              (24576 x 512 8.0 -> 6.2 us); beyond 1.0 .. 2.1
 //   two rows  K > 4096         to 4096 0.85 .. 1.00; beyond 1.17 .. 1.31
-//             K <= 4096        to 8192 0.74 .. 1.02 (fp16 from a K of 3072, 12288: 0.92 .. 1.00); beyond 0.96 .. 3.5
+//             K <= 4096        to 8192 0.74 .. 1.02 (fp16 from a K of 3072, 12288: 0.92 .. 1.00); below 3072 to 12288 (10240 below
+//                              1024) 0.96 .. 1.18 (1.30), eager 0.71 .. 0.90 (10240 x 1024 8.0 -> 5.8 us); beyond to 3.5
 // us, two / one: 1 x 1024 x 1024 4.46 / 3.18, 1 x 4096 x 4096 5.54 / 4.46, 1 x 28672 x 4096 14.2 / 13.1, but 1 x 10240 x 8192 12.2 / 15.0
 // and 2 x 174481 x 64 17 / 60.  Above a K of 16384 a row takes more turns than hide their loads: 1 x 8192 x 28672 27.1 / 28.2.
 inline bool dot_linear_pays(int m, int n, int k, int in)
 {
     const bool f16 = in == QM_IN_F16;
     if (k > 16384) return false;
-    if (m == 2) return n <= (k > 4096 ? 4096 : (f16 && k >= 3072 ? 12288 : 8192));
+    if (m == 2) {
+        if (k > 4096) return n <= 4096;
+        if (k >= 3072) return n <= (f16 ? 12288 : 8192);
+        return n <= (k >= 1024 ? 12288 : 10240);
+    }
     if (k > 4096) return n <= (f16 ? 8192 : 4096);
-    if (k > 2048) return n <= 65536;
-    return n <= (f16 ? (k >= 1536 ? 24576 : 16384) : 12288);
+    return n <= (k > 2048 ? 65536 : 24576);
 }
 
 template <int IN, class Cfg>
