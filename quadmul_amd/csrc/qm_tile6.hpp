@@ -2,7 +2,7 @@
 //
 // A 6-bit E2M3 float with the upper exponent bit clear is a sign and a four-bit magnitude in
 // units of 1/8, so every int4 value is one of its codes, and the matrix core takes 128 of them per
-// instruction in the time it takes 64 int8: 7.3 to 7.9 against 4.4 to 4.5 POP/s, box to box, on a loop of the
+// instruction in the time it takes 64 int8: 7.3 to 7.9 against 4.4 to 4.5 POP/s, card to card, on a loop of the
 // instruction alone (quadmul_amd/probe.py; on one pair of operand registers, which do not toggle, 8.4 to 8.9).  Products are multiples of 1/64; the fp32 accumulators start from 1.5 * 2^17, where
 // one unit in the last place is 1/64, so their bit patterns count those units as an integer would
 // and every sum is exact (|C| <= 64 K < 2^22, K < 65536; checked on the
