@@ -313,8 +313,9 @@ static hipError_t launch_tile6(const GemmArgs &p, const Fp6Operand &a, Fp6Route 
 static hipError_t launch_fp6(const GemmArgs &p, Fp6Route route, void *ws, hipStream_t s)
 {
     const Fp6Operand a = fp6_operand(p.M, p.K, ws);
-    const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, a.layout.kt, a.layout.groups};
-    expand_a6_kernel<false><<<dim3(2 * a.layout.groups, a.layout.parts), dim3(512), 0, s>>>(q);
+    const Fp6Layout &l = a.layout;
+    const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, l.kt, l.groups, l.parts};
+    expand_a6_kernel<false><<<dim3(l.groups * (32 / CODE_ROWS) * l.parts), dim3(EXPAND6_THREADS), 0, s>>>(q);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? launch_tile6(p, a, route, s) : e;
 }
@@ -325,9 +326,10 @@ static hipError_t launch_fp6_padded(GemmArgs p, const PadPlan &pl, Fp6Route rout
 {
     const Fp6Operand a = fp6_operand(p.M, pl.kp, ws);
     uint8_t *b_copy = static_cast<uint8_t *>(ws) + fp6_padded_bytes(p.M, pl.kp, pl) - pl.b_bytes;
-    const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, a.layout.kt, a.layout.groups, p.B, reinterpret_cast<v4i *>(b_copy), p.N, pl.kp};
-    const long long per_row_of_blocks = 512LL * 2 * a.layout.groups, pieces = (long long)p.N * (pl.kp / 32);
-    expand_a6_kernel<true><<<dim3(2 * a.layout.groups, a.layout.parts + (unsigned)((pieces + per_row_of_blocks - 1) / per_row_of_blocks)), dim3(512), 0, s>>>(q);
+    const Fp6Layout &l = a.layout;
+    const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, l.kt, l.groups, l.parts, p.B, reinterpret_cast<v4i *>(b_copy), p.N, pl.kp};
+    const long long pieces = (long long)p.N * (pl.kp / 32);
+    expand_a6_kernel<true><<<dim3(l.groups * (32 / CODE_ROWS) * l.parts + (unsigned)((pieces + EXPAND6_THREADS - 1) / EXPAND6_THREADS)), dim3(EXPAND6_THREADS), 0, s>>>(q);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     p.B = b_copy;
@@ -874,9 +876,9 @@ QM_EXPORT int qm_linear_i4(const void *x, int in_dtype, const void *B, void *D, 
     if (pl.coded) {
         Fp6Operand a = fp6_operand(m, k, rows);
         a.layout.parts = 1;
-        const Quant6Args q{static_cast<const uint8_t *>(x), a.codes, a.sums, scales, m, k, a.layout.kt};
-        hipError_t e = in_dtype == QM_IN_F16 ? launch_quantize_a6<QM_IN_F16>(q, a.layout.groups, s)
-                       : in_dtype == QM_IN_BF16 ? launch_quantize_a6<QM_IN_BF16>(q, a.layout.groups, s) : launch_quantize_a6<QM_IN_F32>(q, a.layout.groups, s);
+        const Quant6Args q{static_cast<const uint8_t *>(x), a.codes, a.sums, scales, m, k, a.layout.kt, a.layout.groups};
+        hipError_t e = in_dtype == QM_IN_F16 ? launch_quantize_a6<QM_IN_F16>(q, s)
+                       : in_dtype == QM_IN_BF16 ? launch_quantize_a6<QM_IN_BF16>(q, s) : launch_quantize_a6<QM_IN_F32>(q, s);
         if (e != hipSuccess) return fail_launch(e);
         GemmArgs p{nullptr, static_cast<const uint8_t *>(B), static_cast<int32_t *>(D), m, n, k};
         p.row_scale = scales;

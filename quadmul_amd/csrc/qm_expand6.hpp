@@ -9,7 +9,7 @@ struct Expand6Args {
     const uint8_t *A;  // [M, K/2] packed s4; rows 16-byte aligned and K a multiple of 32, unless ANY
     uint8_t *codes;
     int *sums;
-    int M, K, kt, groups;
+    int M, K, kt, groups, parts;
     // ANY only: B [N, K/2], and its copy with rows of Kp / 2 bytes, Kp a multiple of 128
     const uint8_t *B;
     v4i *b_copy;
@@ -37,70 +37,89 @@ __device__ __forceinline__ v4i row_piece(const uint8_t *row, const int at, const
     return v;
 }
 
-// One workgroup re-codes 16 rows over FP6_PART_STEPS K-steps (blockIdx.y), eight waves of two K-steps at a
-// time: 128 bytes of every row, whole lines.  Two K-steps that a row does not fill are its last 128
-// bytes, as the GEMM loads them of B, with zeros where the steps before have been.
-// ANY: rows of any K and at any address, as if padded with zeros to Kp; the workgroups beyond A's (blockIdx.y past the
-// parts) copy B with its rows padded, one 16-byte piece per thread, in the same launch.
-template <bool ANY>
-__global__ void __launch_bounds__(512) expand_a6_kernel(const Expand6Args q)
+// The eight rows of a workgroup: r0 .. r0 + 3 and r0 + 16 .. r0 + 19 of a group of 32, both halves of every 16 bytes of codes that they
+// share, 64 contiguous bytes of codes at a time.  (Workgroups of a group, which share 128-byte lines of codes, on one XCD: 8192 x 8192
+// 16.9 us, 2048 x 11008 6.5, against 14.8 and 6.0 with neighbours of any kind.)
+constexpr int CODE_ROWS = 8;
+__device__ __forceinline__ void code_rows(const int block, int &group, int &r0)
 {
-    __shared__ int red[8][16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    group = block >> 2;
+    r0 = (block & 3) * 4;
+}
+
+// One workgroup re-codes CODE_ROWS rows over FP6_PART_STEPS K-steps, eight waves of two K-steps at a time: 128 bytes of every row,
+// whole lines.  Two K-steps that a row does not fill are its last 128
+// bytes, as the GEMM loads them of B, with zeros where the steps before have been.
+// ANY: rows of any K and at any address, as if padded with zeros to Kp; the workgroups beyond A's
+// copy B with its rows padded, one 16-byte piece per thread, in the same launch.
+// Bound: HBM on large operands, the launch and one round trip on small ones.  us in a graph, by sixteen
+// neighbouring rows to a workgroup / now: 512 x 8192 3.9 / 3.2, 1536 x 4096 4.1 / 3.4, 4096 x 4096 5.8 / 5.7, 8192 x 8192 17.0 / 14.8 (5.7 TB/s).
+constexpr int EXPAND6_THREADS = 512;
+template <bool ANY>
+__global__ void __launch_bounds__(EXPAND6_THREADS) expand_a6_kernel(const Expand6Args q)
+{
+    constexpr int WAVES = EXPAND6_THREADS / 64, PAIRS = FP6_PART_STEPS / 2 / WAVES;  // (pairs of K-steps: per wave)
+    __shared__ int red[WAVES][CODE_ROWS];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int Kb = q.K >> 1;
+    const unsigned blocks = (unsigned)q.groups * (32 / CODE_ROWS);
+    const int part = blockIdx.x / blocks;
     if constexpr (ANY) {
-        const int parts = (q.kt + FP6_PART_STEPS - 1) / FP6_PART_STEPS;
-        if ((int)blockIdx.y >= parts) {
-            const uint32_t per_row = (uint32_t)q.Kp >> 5, piece = ((blockIdx.y - parts) * gridDim.x + blockIdx.x) * 512u + threadIdx.x;  // (below 2^28)
+        if (part >= q.parts) {
+            const uint32_t per_row = (uint32_t)q.Kp >> 5, piece = (blockIdx.x - q.parts * blocks) * (uint32_t)EXPAND6_THREADS + threadIdx.x;  // (below 2^28 and a workgroup)
             const uint32_t n = piece / per_row;
             if (n < (uint32_t)q.N) q.b_copy[piece] = row_piece(q.B + (size_t)n * Kb, 16 * (int)(piece - n * per_row), Kb);
             return;
         }
     }
-    const int row_bytes = ANY ? q.Kp >> 1 : Kb;
-    const int half = blockIdx.x, row = half * 16 + r;
+    int group, r0;
+    code_rows(blockIdx.x - part * blocks, group, r0);
+    // lane: row, 16 bytes of a K-step, step of the two
+    const int h = (lane >> 2) & 1, r = r0 + (lane & 3), g = (lane >> 3) & 3, second = lane >> 5;
+    const int row = group * 32 + h * 16 + r, row_bytes = ANY ? q.Kp >> 1 : Kb;
     const uint8_t *src = q.A + (size_t)min(row, q.M - 1) * Kb;
-    uint8_t *out = q.codes + (size_t)(half >> 1) * q.kt * FP6_GROUP_BYTES;
-    constexpr int PAIRS = FP6_PART_STEPS / 16;  // per wave
-    v4i v[PAIRS][2];
+    v4i v[PAIRS];
 #pragma unroll
     for (int t = 0; t < PAIRS; ++t) {
-        const int step = blockIdx.y * FP6_PART_STEPS + 2 * (wave + 8 * t), at = min(step * 64, row_bytes - 128);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            if constexpr (ANY) v[t][u] = row_piece(src, at + 64 * u + 16 * g, Kb);
-            else v[t][u] = *reinterpret_cast<const v4i *>(src + at + 64 * u + 16 * g);
-        }
+        const int at = min((part * FP6_PART_STEPS + 2 * (wave + WAVES * t)) * 64, row_bytes - 128) + 64 * second + 16 * g;
+        if constexpr (ANY) v[t] = row_piece(src, at, Kb);
+        else v[t] = *reinterpret_cast<const v4i *>(src + at);
     }
     int sum = 0;
 #pragma unroll
     for (int t = 0; t < PAIRS; ++t) {
-        const int step = blockIdx.y * FP6_PART_STEPS + 2 * (wave + 8 * t), at = min(step * 64, row_bytes - 128);
+        const int step = part * FP6_PART_STEPS + 2 * (wave + WAVES * t);
         if (step >= q.kt) break;
+        v4i w = v[t];
+        if (row >= q.M || min(step * 64, row_bytes - 128) + 64 * second + 16 * g < step * 64) w = v4i{0, 0, 0, 0};
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            v4i w = v[t][u];
-            if (row >= q.M || at + 64 * u + 16 * g < step * 64) w = v4i{0, 0, 0, 0};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_sdot8(w[e], 0x11111111, sum, false);
-            uint32_t lo[3], hi[3];
-            fp6_signed((uint32_t)w.x, (uint32_t)w.y, lo);
-            fp6_signed((uint32_t)w.z, (uint32_t)w.w, hi);
-            uint8_t *o = out + (size_t)(step + u) * FP6_GROUP_BYTES;
-            *reinterpret_cast<v4i *>(o + (half & 1) * 1024 + lane * 16) = v4i{(int)lo[0], (int)lo[1], (int)lo[2], (int)hi[0]};
-            *reinterpret_cast<v2i *>(o + 2048 + (half & 1) * 512 + lane * 8) = v2i{(int)hi[1], (int)hi[2]};
-        }
+        for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_sdot8(w[e], 0x11111111, sum, false);
+        uint32_t f[6];
+        fp6_fragment(w, f);
+        uint8_t *const o = q.codes + ((size_t)group * q.kt + step + second) * FP6_GROUP_BYTES + (r + 16 * g) * 16;
+        *reinterpret_cast<v4i *>(o + h * 2048) = h == 0 ? v4i{(int)f[0], (int)f[1], (int)f[2], (int)f[3]} : v4i{(int)f[2], (int)f[3], (int)f[4], (int)f[5]};
+        *reinterpret_cast<v2i *>(o + 1024 + h * 8) = h == 0 ? v2i{(int)f[4], (int)f[5]} : v2i{(int)f[0], (int)f[1]};
     }
+    sum += __shfl_xor(sum, 8);
     sum += __shfl_xor(sum, 16);
     sum += __shfl_xor(sum, 32);
-    if (lane < 16) red[wave][lane] = sum;
+    if (lane < CODE_ROWS) red[wave][lane] = sum;
     __syncthreads();
-    if (threadIdx.x < 16) {
+    if (threadIdx.x < CODE_ROWS) {
         int total = 0;
 #pragma unroll
-        for (int w = 0; w < 8; ++w) total += red[w][threadIdx.x];
-        q.sums[((size_t)blockIdx.y * q.groups * 2 + half) * 16 + threadIdx.x] = total;
+        for (int w = 0; w < WAVES; ++w) total += red[w][threadIdx.x];
+        q.sums[((size_t)part * q.groups + group) * 32 + h * 16 + r] = total;
     }
+}
+
+// the codes of a lane of a pair of fragments, at its place in the first of the three pieces
+__device__ __forceinline__ void put_pair(uint8_t *at, const uint32_t (&f)[2][6])
+{
+    v4i *const o = reinterpret_cast<v4i *>(at);
+    o[0] = v4i{(int)f[0][0], (int)f[0][1], (int)f[0][2], (int)f[0][3]};
+    o[64] = v4i{(int)f[0][4], (int)f[0][5], (int)f[1][0], (int)f[1][1]};
+    o[128] = v4i{(int)f[1][2], (int)f[1][3], (int)f[1][4], (int)f[1][5]};
 }
 
 struct Quant6Args {
@@ -108,21 +127,24 @@ struct Quant6Args {
     uint8_t *codes;
     int *sums;         // (one part)
     float *scales;
-    int M, K, kt;
+    int M, K, kt, groups;
 };
 
 // The rows of x quantised by the rule of quantize_pack_kernel, with the same arithmetic, and written as 6-bit codes: the linear
 // layer's activations on their way to the tile kernel, without the packed rows in between and the launch that re-codes
 // them.  Eight rows per workgroup, a wave on each, NC chunks of eight elements per lane (k <= 512 NC) in registers between
-// the maximum and the quantisation; the nibbles meet in the LDS, so that eight rows' codes leave as whole 128-byte lines.
-constexpr int QUANT6_ROWS = 8, QUANT6_THREADS = 64 * QUANT6_ROWS;
+// the maximum and the quantisation; the nibbles meet in the LDS, so that their
+// codes leave 64 contiguous bytes at a time.
+constexpr int QUANT6_ROWS = CODE_ROWS, QUANT6_THREADS = 64 * QUANT6_ROWS;
 inline int quant6_lds_bytes(int k) { return QUANT6_ROWS * (k / 2 + 16); }  // rows 16 bytes apart in banks
 template <int IN, int NC>
 __global__ void __launch_bounds__(QUANT6_THREADS, 2) quantize_a6_kernel(const Quant6Args q)
 {
     extern __shared__ __align__(16) uint8_t nibbles[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int row = blockIdx.x * QUANT6_ROWS + wave, Kb = q.K >> 1, pitch = Kb + 16, nchunks = q.K >> 3;
+    int group, r0;
+    code_rows(blockIdx.x, group, r0);
+    const int row = group * 32 + r0 + (wave & 3) + (wave >> 2) * 16, Kb = q.K >> 1, pitch = Kb + 16, nchunks = q.K >> 3;
     const uint8_t *src = q.x + (size_t)min(row, q.M - 1) * q.K * QuantIn<IN>::BYTES;
     Chunk8<IN> v[NC];
 #pragma unroll
@@ -152,38 +174,37 @@ __global__ void __launch_bounds__(QUANT6_THREADS, 2) quantize_a6_kernel(const Qu
         if (row < q.M) q.scales[row] = amax / 7.0f;
     }
     __syncthreads();
-    // rows 8 (b & 3) .. of group b >> 2: as expand_a6_kernel writes them
-    const int in_group = (blockIdx.x & 3) * QUANT6_ROWS, half = in_group >> 4;
-    uint8_t *out = q.codes + (size_t)(blockIdx.x >> 2) * q.kt * FP6_GROUP_BYTES;
-    for (int u = threadIdx.x; u < q.kt * 32; u += QUANT6_THREADS) {
-        const int r8 = u & 7, g = (u >> 3) & 3, step = u >> 5, pair = (step & ~1) * 64;
-        const int at = min(pair, Kb - 128) + 64 * (step & 1) + 16 * g, to = (in_group & 15) + r8 + 16 * g;
-        v4i w = *reinterpret_cast<const v4i *>(nibbles + r8 * pitch + at);
-        if (at < pair) w = v4i{0, 0, 0, 0};
-        uint32_t lo[3], hi[3];
-        fp6_signed((uint32_t)w.x, (uint32_t)w.y, lo);
-        fp6_signed((uint32_t)w.z, (uint32_t)w.w, hi);
-        uint8_t *o = out + (size_t)step * FP6_GROUP_BYTES;
-        *reinterpret_cast<v4i *>(o + half * 1024 + to * 16) = v4i{(int)lo[0], (int)lo[1], (int)lo[2], (int)hi[0]};
-        *reinterpret_cast<v2i *>(o + 2048 + half * 512 + to * 8) = v2i{(int)hi[1], (int)hi[2]};
+    uint8_t *const out = q.codes + (size_t)group * q.kt * FP6_GROUP_BYTES;
+    for (int u = threadIdx.x; u < q.kt * 16; u += QUANT6_THREADS) {
+        // (eight lanes together: four rows, 16 bytes apart in banks, of two steps, 64 bytes apart)
+        const int r4 = u & 3, g = (u >> 3) & 3, step = (u >> 5) * 2 + ((u >> 2) & 1), pair = (step & ~1) * 64;
+        const int at = min(pair, Kb - 128) + 64 * (step & 1) + 16 * g;
+        uint32_t f[2][6];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            v4i w = *reinterpret_cast<const v4i *>(nibbles + (h * 4 + r4) * pitch + at);
+            if (at < pair) w = v4i{0, 0, 0, 0};
+            fp6_fragment(w, f[h]);
+        }
+        put_pair(out + (size_t)step * FP6_GROUP_BYTES + (r0 + r4 + 16 * g) * 16, f);
     }
 }
 
 template <int IN, int NC>
-static hipError_t launch_quantize_a6(const Quant6Args &q, int groups, hipStream_t s)
+static hipError_t launch_quantize_a6_rows(const Quant6Args &q, hipStream_t s)
 {
-    quantize_a6_kernel<IN, NC><<<dim3(groups * 32 / QUANT6_ROWS), dim3(QUANT6_THREADS), quant6_lds_bytes(q.K), s>>>(q);
+    quantize_a6_kernel<IN, NC><<<dim3(q.groups * (32 / CODE_ROWS)), dim3(QUANT6_THREADS), quant6_lds_bytes(q.K), s>>>(q);
     return hipGetLastError();
 }
 // The K it holds: 64 KiB of LDS, and for fp32 128 registers of one wave per row.
 inline bool quant6_fits(int k, int in) { return quant6_lds_bytes(k) <= 64 * 1024 && (in != QM_IN_F32 || k <= 8192); }
 template <int IN>
-static hipError_t launch_quantize_a6(const Quant6Args &q, int groups, hipStream_t s)
+static hipError_t launch_quantize_a6(const Quant6Args &q, hipStream_t s)
 {
-    if (q.K <= 2048) return launch_quantize_a6<IN, 4>(q, groups, s);
-    if (q.K <= 4096) return launch_quantize_a6<IN, 8>(q, groups, s);
-    if (q.K <= 8192) return launch_quantize_a6<IN, 16>(q, groups, s);
-    if constexpr (IN != QM_IN_F32) return launch_quantize_a6<IN, 32>(q, groups, s);
+    if (q.K <= 2048) return launch_quantize_a6_rows<IN, 4>(q, s);
+    if (q.K <= 4096) return launch_quantize_a6_rows<IN, 8>(q, s);
+    if (q.K <= 8192) return launch_quantize_a6_rows<IN, 16>(q, s);
+    if constexpr (IN != QM_IN_F32) return launch_quantize_a6_rows<IN, 32>(q, s);
     return hipErrorInvalidValue;
 }
 

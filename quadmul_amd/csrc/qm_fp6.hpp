@@ -42,9 +42,23 @@ __device__ __forceinline__ void fp6_signed(const uint32_t w0, const uint32_t w1,
     f[2] |= (s[2] << 2) | (s[1] >> 30);
 }
 
+// a lane's 32 nibbles of a fragment -> its six dwords
+__device__ __forceinline__ void fp6_fragment(const v4i w, uint32_t (&f)[6])
+{
+    uint32_t lo[3], hi[3];
+    fp6_signed((uint32_t)w.x, (uint32_t)w.y, lo);
+    fp6_signed((uint32_t)w.z, (uint32_t)w.w, hi);
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+        f[e] = lo[e];
+        f[3 + e] = hi[e];
+    }
+}
+
 // ---- A re-coded, in a workspace ----
-// codes  [groups][kt][FP6_GROUP_BYTES]   groups of 32 rows, kt K-steps (an even number); within a group of one step the first
-//                                        four dwords of the lanes of its two halves, 1 KiB each, then the other two, 512 bytes each
+// codes  [groups][kt][FP6_GROUP_BYTES]   groups of 32 rows, kt K-steps (an even number); within a group of one step 48 bytes for
+//                                        each lane of the fragments that it is, first the one of rows 0..15, then the
+//                                        one of rows 16..31, in three pieces of 16 bytes per lane, 1 KiB each
 // sums   [parts][32 groups]              per row, over FP6_PART_STEPS K-steps each (a workgroup's share of the re-coding)
 constexpr int FP6_PART_STEPS = 32;
 struct Fp6Layout {

@@ -21,14 +21,14 @@
 // instruction each, the loads running ahead through item boundaries, the write-out inside an item's last
 // K-step -- it follows.  8192 x 8192 x 8192 runs at 1.80 GHz (int8: 2.15) in 459 thousand cycles, 390 of them
 // a loop of its matrix instructions alone; without its loads into the LDS the clock rises to 2.13 GHz and
-// the cycles stay.  us, this kernel / int8: 8192 x 8192 x 8192 264 / 336, 2048 x 11008 x 4096 64 / 77,
-// 4096 x 4096 x 4096 42.6 / 48.5; the kernel that re-codes A takes 18 to 23, 5 to 10 and 7 to 8 more (traced).
+// the cycles stay (taken before A was read as it is now, see read_a).  us, this kernel / int8: 8192 x 8192 x 8192 262 / 336,
+// 2048 x 11008 x 4096 60 / 77, 4096 x 4096 x 4096 39.3 / 48.5; the kernel that re-codes A takes 14.8, 3.7 and 5.7 in a graph of its own.
 //
 // Eight waves, two per SIMD: a wave by itself issues a vector instruction every eight cycles (two every four),
 // and the 56 re-coding instructions per wave and K-step then take longer than the matrix ones (four waves
 // with 128 x 128 each: 281 us instead of 262).
 //
-// Registers: the 256 x 256 tile keeps 1 of them in scratch memory (int32), 10 (scaled) or 23 (scaled, bias), all of it
+// Registers: the 256 x 256 tile keeps none of them in scratch memory (int32), 10 (scaled) or 24 (scaled, bias), all of it
 // around an item's start and write-out: no reload, whose wait would drain the counted loads, lies in the loop over K.
 //
 // Tiles of 256 x 128 (4 x 2 waves) halve the grain where 256 x 256 leaves most of a round idle: per K-step and round 0.53 us
@@ -89,7 +89,7 @@ struct Tile6Cfg {
     static_assert(BM % (32 * WAVES) == 0 && BN % (8 * WAVES) == 0 && WAVES % 2 == 0, "loads divide evenly among the waves");
     static_assert(WM % 64 == 0 && WN % 64 == 0 && (OWN_AREA || WAVES * (XHALF_BYTES + SCALE_BYTES) <= B_BYTES), "the write-out fits the stage it borrows");
     static_assert(LDS_BYTES <= 160 * 1024, "LDS budget of a gfx950 CU");
-    static_assert(FM % 4 == 0 && FN % 2 == 0, "four fragments of A in rotation; blocks leave in pairs");
+    static_assert(FM % 4 == 0 && FN >= 4 && FN % 2 == 0, "two pairs of fragments of A in rotation; blocks leave in pairs");
 };
 
 template <class Cfg, int OUT = OUT_I32, bool BIAS = false>
@@ -189,13 +189,16 @@ gemm_tile6_kernel(const GemmArgs p, const uint8_t *const a6, const int *const ro
 
     // ---- fragment reads ----
     constexpr int B_BASE = Cfg::A_STAGES * Cfg::A_BYTES;
-    const int a_rd = wm * (Cfg::WM / 32) * FP6_GROUP_BYTES + lane * 16, a_rd8 = wm * (Cfg::WM / 32) * FP6_GROUP_BYTES + 2048 + lane * 8;
+    // A: two fragments, 32 rows, are three reads of 16 bytes per lane into twelve registers, the second fragment behind the
+    // first.  (As a read of 16 and one of 8 bytes per fragment, which the LDS serves at less than its full rate, the same bytes took
+    // longer: us, before -> now, 8192 x 8192 x 8192 266 -> 262, 2048 x 11008 x 4096 62.3 -> 60.4, 2048 x 4096 x 11008 62.5 -> 59.7, all on 256 x 256.)
+    const int a_rd = wm * (Cfg::WM / 32) * FP6_GROUP_BYTES + lane * 16;
     const int b_row = wn * Cfg::WN + r;
     const int b_rd = b_row * 128 + ((g ^ ((b_row >> 1) & 7)) << 4);  // of the first of two steps; the second's differs in bit 6
-    auto read_a = [&](int stage, int i) __attribute__((always_inline)) -> v6i {
-        const v4i x = *reinterpret_cast<const v4i *>(smem + stage + a_rd + (i >> 1) * FP6_GROUP_BYTES + (i & 1) * 1024);
-        const v2i y = *reinterpret_cast<const v2i *>(smem + stage + a_rd8 + (i >> 1) * FP6_GROUP_BYTES + (i & 1) * 512);
-        return v6i{x.x, x.y, x.z, x.w, y.x, y.y};
+    typedef int v12i __attribute__((ext_vector_type(12)));
+    auto read_a = [&](int stage, int q, int t, v12i &pair) __attribute__((always_inline)) {  // third t of pair q
+        const v4i x = *reinterpret_cast<const v4i *>(smem + stage + a_rd + q * FP6_GROUP_BYTES + t * 1024);
+        pair[4 * t] = x.x; pair[4 * t + 1] = x.y; pair[4 * t + 2] = x.z; pair[4 * t + 3] = x.w;
     };
     const int b_rd2 = b_rd ^ 64;
     auto read_b = [&](int stage, bool second, int j) __attribute__((always_inline)) -> v4i {
@@ -338,7 +341,8 @@ gemm_tile6_kernel(const GemmArgs p, const uint8_t *const a6, const int *const ro
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(A_PIECES + B_PIECES) : "memory");
     __syncthreads();
 
-    v6i bf[2][FN], af[4];
+    v6i bf[2][FN];
+    v12i ap[2];
     constexpr int NPK = FM * FN >= 32 ? 2 : FN;  // packed fragments of B between their read and their re-coding
     v4i b_pk[NPK];
 #pragma unroll
@@ -346,8 +350,15 @@ gemm_tile6_kernel(const GemmArgs p, const uint8_t *const a6, const int *const ro
         const v4i q = read_b(b_ring[0], false, j);
         static_for<0, W>([&](auto k_) __attribute__((always_inline)) { code_op(k_, q, bf[0][j]); });
     }
-    af[0] = read_a(a_ring[0], 0);
-    af[1] = read_a(a_ring[0], 1);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) read_a(a_ring[0], 0, t, ap[0]);
+    // (one register tuple, before its halves are used: else the compiler gives each half one of its own and copies)
+    asm volatile("" : "+v"(ap[0]));
+    auto frag_a = [&](auto i_) __attribute__((always_inline)) -> v6i {
+        constexpr int i = decltype(i_)::value, q = (i >> 1) & 1;
+        if constexpr (i & 1) return __builtin_shufflevector(ap[q], ap[q], 6, 7, 8, 9, 10, 11);
+        else return __builtin_shufflevector(ap[q], ap[q], 0, 1, 2, 3, 4, 5);
+    };
     float one;
     asm volatile("v_mov_b32 %0, 1.0" : "=v"(one));
 
@@ -367,12 +378,10 @@ gemm_tile6_kernel(const GemmArgs p, const uint8_t *const a6, const int *const ro
         constexpr int LEAD = FN;               // the first fragment read in slot 0 is there by then
         static_for<0, SLOTS>([&](auto s_) __attribute__((always_inline)) {
             constexpr int s = decltype(s_)::value, i = s / FN, j = s % FN;
-            mfma6_acc(acc[i][j], bf[bs][j], af[i & 3]);
+            mfma6_acc(acc[i][j], bf[bs][j], frag_a(std::integral_constant<int, i>{}));
             if constexpr (first && i + 1 < FM) mfma6_start(acc[i + 1][j], one, start_reg[i + 1]);
-            if constexpr (j == 0) {
-                constexpr int i2 = i + 2;
-                af[i2 & 3] = read_a(i2 >= FM ? a_ring[1] : a_ring[0], i2 % FM);
-            }
+            if constexpr (i % 2 == 0 && j < 3) read_a(i + 2 >= FM ? a_ring[1] : a_ring[0], (i + 2) % FM / 2, j, ap[(i / 2 + 1) & 1]);
+            if constexpr (i % 2 == 1 && j == FN - 1) asm volatile("" : "+v"(ap[(i / 2 + 1) & 1]));
             // fragment q of B is re-coded in ops [W q, W (q + 1)), which begin at slot LEAD + W q (SLOTS - LEAD) / OPS
             static_for<0, FN>([&](auto q_) __attribute__((always_inline)) {
                 constexpr int q = decltype(q_)::value;
