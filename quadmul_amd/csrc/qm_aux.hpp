@@ -384,6 +384,66 @@ __device__ __forceinline__ uint32_t quant8(const Chunk8<IN> &c, float inv)
     return __builtin_amdgcn_perm(hi, lo, 0x05040100u) ^ 0x88888888u;
 }
 
+// The same for fp16 in fewer instructions, where no clamp is needed: no NaN among the elements, the row's maximum and inv finite (|c inv|
+// <= 7 and a rounding).  The product is rounded as above, then to an integer, half to even, by the addition of 1.5 * 2^23 + 8, whose
+// last bits then count n + 8; the bits of eight such sums are added up sixteen-fold, and what the constant leaves in them is taken
+// away.  With the maximum on bit patterns (chunks_amax) 4.1 vector instructions per element where one
+// element after the other takes 8: in a graph, us, before -> now, 2048 x 4096 5.76 -> 5.46, 2048 x 8192 8.94 -> 8.56, 8192 x 1024 5.77 ->
+// 5.41.  bf16, which needs an instruction more to widen and had one less, was no faster (2048 x 8192 8.66 / 8.67).
+__device__ __forceinline__ uint32_t quant8_plain(const Chunk8<QM_IN_F16> &c, const float inv)
+{
+    constexpr float round_to = 12582912.0f + 8.0f;
+    constexpr uint32_t left = 0x4B400000u + (0x4B400000u << 4) + (0x4B400000u << 8);  // (further up it has no bits)
+    uint32_t sum = 0;
+#pragma unroll
+    for (int e = 7; e >= 0; --e) {
+        // (the widening and the product in one; + 0 only makes a zero positive)
+        float t;
+        if (e & 1) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(t) : "v"(c.w[0][e >> 1]), "v"(inv));
+        else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(t) : "v"(c.w[0][e >> 1]), "v"(inv));
+        sum = (sum << 4) + __builtin_bit_cast(uint32_t, t + round_to);
+    }
+    return (sum - left) ^ 0x88888888u;
+}
+
+// The largest magnitude among a lane's chunks, NaNs left out.  fp16: on the bit patterns, two at a time; `plain` comes back false where
+// the wave has a NaN, and for the other types.
+template <int IN, int NC>
+__device__ __forceinline__ float chunks_amax(const Chunk8<IN> (&v)[NC], bool &plain)
+{
+    plain = false;
+    if constexpr (IN == QM_IN_F16) {
+        typedef uint16_t v2u __attribute__((ext_vector_type(2)));
+        v2u m = {0, 0};
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int w = v[i].w[0][e] & 0x7FFF7FFF;
+                m = __builtin_elementwise_max(m, __builtin_bit_cast(v2u, w));
+            }
+        const uint16_t most = m.x > m.y ? m.x : m.y;
+        plain = !__any(most > 0x7C00);
+        if (plain) return QuantIn<IN>::widen(most);
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) amax = v[i].amax(amax);
+    return amax;
+}
+// put(quant) with the quantisation of a chunk that does for these, the same for the whole wave
+template <int IN, class Put>
+__device__ __forceinline__ void quantise_chunks(const bool plain, const float amax, const float inv, Put &&put)
+{
+    if constexpr (IN == QM_IN_F16) {
+        if (plain && fmaxf(amax, inv) < __builtin_inff()) {
+            put([&](const Chunk8<IN> &c) __attribute__((always_inline)) { return quant8_plain(c, inv); });
+            return;
+        }
+    }
+    put([&](const Chunk8<IN> &c) __attribute__((always_inline)) { return quant8(c, inv); });
+}
+
 // maximum over the NW waves that share a row (one row per workgroup unless NW == 1)
 template <int NW>
 __device__ __forceinline__ float row_max(float x, float *lds)
@@ -418,17 +478,18 @@ __global__ void __launch_bounds__(NW == 1 ? 256 : 64 * NW) quantize_pack_kernel(
         Chunk8<IN> v[NC];
 #pragma unroll
         for (int i = 0; i < NC; ++i) v[i].load(xr + first(lane + i * 64 * NW) * QuantIn<IN>::BYTES);
-#pragma unroll
-        for (int i = 0; i < NC; ++i) amax = v[i].amax(amax);
-        amax = row_max<NW>(amax, red);
+        bool plain;
+        amax = row_max<NW>(chunks_amax(v, plain), red);
         const float inv = amax > 0.0f ? 7.0f / amax : 0.0f;
         if (lane == 0) scales[row] = amax / 7.0f;
+        quantise_chunks<IN>(plain, amax, inv, [&](auto quant) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < NC; ++i) {
-            const int c = lane + i * 64 * NW;
-            const uint32_t q = quant8(v[i], inv);
-            if (c < nchunks) *reinterpret_cast<u32_any_aligned *>(out + (first(c) >> 1)) = q;
-        }
+            for (int i = 0; i < NC; ++i) {
+                const int c = lane + i * 64 * NW;
+                const uint32_t q = quant(v[i]);
+                if (c < nchunks) *reinterpret_cast<u32_any_aligned *>(out + (first(c) >> 1)) = q;
+            }
+        });
     } else {
         Chunk8<IN> v;
         for (int c = lane; c < nchunks; c += 64 * NW) {

@@ -149,24 +149,24 @@ __global__ void __launch_bounds__(QUANT6_THREADS, 2) quantize_a6_kernel(const Qu
     Chunk8<IN> v[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) v[i].load(src + (size_t)min(lane + i * 64, nchunks - 1) * 8 * QuantIn<IN>::BYTES);
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NC; ++i) amax = v[i].amax(amax);
-    amax = row_max<1>(amax, nullptr);
+    bool plain;
+    const float amax = row_max<1>(chunks_amax(v, plain), nullptr);
     const float inv = amax > 0.0f ? 7.0f / amax : 0.0f;
     int sum = 0;
+    quantise_chunks<IN>(plain, amax, inv, [&](auto quant) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        const int c = lane + i * 64;
-        // (the elements as loaded: widened for the maximum, the compiler would keep all of them as floats)
+        for (int i = 0; i < NC; ++i) {
+            const int c = lane + i * 64;
+            // (the elements as loaded: widened for the maximum, the compiler would keep all of them as floats)
 #pragma unroll
-        for (int w = 0; w < QuantIn<IN>::WORDS / 4; ++w) asm volatile("" : "+v"(v[i].w[w]));
-        const uint32_t n8 = quant8(v[i], inv);
-        if (c < nchunks) {
-            sum = __builtin_amdgcn_sdot8((int)n8, 0x11111111, sum, false);
-            *reinterpret_cast<uint32_t *>(nibbles + wave * pitch + 4 * c) = n8;
+            for (int w = 0; w < QuantIn<IN>::WORDS / 4; ++w) asm volatile("" : "+v"(v[i].w[w]));
+            const uint32_t n8 = quant(v[i]);
+            if (c < nchunks) {
+                sum = __builtin_amdgcn_sdot8((int)n8, 0x11111111, sum, false);
+                *reinterpret_cast<uint32_t *>(nibbles + wave * pitch + 4 * c) = n8;
+            }
         }
-    }
+    });
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off);
     if (lane == 0) {

@@ -1,0 +1,23 @@
+"""fp16 rows, which are quantised by an arithmetic of their own where they hold no NaN and no infinity (quant8_plain in csrc/qm_aux.hpp)."""
+import pytest
+import torch
+
+import quadmul
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+# every fp16 pattern as an element of rows with a maximum above it, the shorter arithmetic, and of rows with infinities and NaN, the longer
+def test_every_fp16_value_is_quantised_as_the_same_value_in_fp32_is():
+    k = 2048
+    for top in (1.0, 7.0, 65504.0, 6.1e-5):
+        x = torch.arange(65536, dtype=torch.int32, device=DEV).to(torch.int16).view(torch.float16).view(32, k).clone()
+        special = ~(x.float().abs() <= top)
+        finite = torch.where(special, torch.zeros_like(x), x)
+        finite[:, 0] = top
+        for rows in (finite, x):
+            q16, s16 = quadmul.quantize_pack(rows)
+            q32, s32 = quadmul.quantize_pack(rows.float())   # (the same values, by the other arithmetic)
+            assert torch.equal(q16, q32) and torch.equal(s16.view(torch.int32), s32.view(torch.int32)), top
