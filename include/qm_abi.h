@@ -235,7 +235,7 @@ int qm_quantize_pack_i4(const void *x, int in_dtype, void *dst_packed, float *sc
  * output on them -- D[m][n] as qm_gemm_i4_scaled_bias_ws gives it with their scales as row_scale -- and
  * the same values bit for bit as those two calls one after the other.  The reference has no counterpart.
  * Large products go from x to the 6-bit operands of qm_gemm_recode_bytes without the packed rows in between; one or two
- * rows are one launch, which wants no workspace, while its workgroups run in one round (qm_linear_workspace_bytes is 0).
+ * rows, and up to sixteen of 16-bit types on few columns, are one launch, which wants no workspace (qm_linear_workspace_bytes is 0).
  *   workspace    device memory, 256-byte aligned, at least qm_linear_workspace_bytes(...) bytes (weight_align: the
  *                alignment of B in bytes), else QM_ERR_SCRATCH and nothing is enqueued; used in stream order by
  *                the kernels of this call only

@@ -16,6 +16,7 @@
 #include "qm_aux.hpp"
 #include "qm_expand6.hpp"
 #include "qm_dot_linear.hpp"
+#include "qm_skinny_linear.hpp"
 
 #define QM_EXPORT extern "C" __attribute__((visibility("default")))
 
@@ -601,8 +602,11 @@ QM_EXPORT int qm_init(void)
                 if (e != hipSuccess) return fail_launch(e);
             }
         }
+    hipError_t e = ready_skinny_linear<QM_IN_F16>();
+    if (e == hipSuccess) e = ready_skinny_linear<QM_IN_BF16>();
+    if (e != hipSuccess) return fail_launch(e);
     void *ws = nullptr;
-    const hipError_t e = static_scratch(&ws);
+    e = static_scratch(&ws);
     return e == hipSuccess ? QM_OK : fail_launch(e);
 }
 
@@ -823,7 +827,7 @@ LinearPlan linear_plan(int m, int n, int k, int in_dtype, int weight_align)
 {
     const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     LinearPlan pl{};
-    if (m <= 2 && fast_path_ok(m, n, k, weight_align) && n < (1 << 24) && dot_linear_pays(m, n, k, in_dtype)) {
+    if (m <= 16 && fast_path_ok(m, n, k, weight_align) && n < (1 << 24) && (m <= 2 ? dot_linear_pays(m, n, k, in_dtype) : skinny_linear_pays(m, n, k, in_dtype))) {
         pl.one_launch = true;
         return pl;
     }
@@ -865,9 +869,14 @@ QM_EXPORT int qm_linear_i4(const void *x, int in_dtype, const void *B, void *D, 
     const LinearPlan pl = linear_plan(m, n, k, in_dtype, ptr_alignment(B, nullptr));
     if (pl.one_launch) {
         const uint16_t *b16 = static_cast<const uint16_t *>(bias);
-        const hipError_t e = in_dtype == QM_IN_F16 ? launch_dot_linear<QM_IN_F16>(x, B, D, m, n, k, col_scale, b16, out, s)
-                             : in_dtype == QM_IN_BF16 ? launch_dot_linear<QM_IN_BF16>(x, B, D, m, n, k, col_scale, b16, out, s)
-                                                      : launch_dot_linear<QM_IN_F32>(x, B, D, m, n, k, col_scale, b16, out, s);
+        const auto launch = [&](auto in) {
+            constexpr int IN = decltype(in)::value;
+            if constexpr (IN != QM_IN_F32)
+                if (m > 2) return launch_skinny_linear<IN>(x, B, D, m, n, k, col_scale, b16, out, s);
+            return launch_dot_linear<IN>(x, B, D, m, n, k, col_scale, b16, out, s);
+        };
+        const hipError_t e = in_dtype == QM_IN_F16 ? launch(std::integral_constant<int, QM_IN_F16>{})
+                             : in_dtype == QM_IN_BF16 ? launch(std::integral_constant<int, QM_IN_BF16>{}) : launch(std::integral_constant<int, QM_IN_F32>{});
         return e == hipSuccess ? QM_OK : fail_launch(e);
     }
     if (workspace == nullptr || ((uintptr_t)workspace & 255) || workspace_bytes < pl.bytes()) return QM_ERR_SCRATCH;

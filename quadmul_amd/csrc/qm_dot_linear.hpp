@@ -8,8 +8,7 @@ namespace qm {
 // gemm_dot_kernel with the quantisation of its rows in front: every workgroup quantises x by itself, with the arithmetic of
 // quantize_pack_kernel, while the first of its loads of B are on their way.  That is a few elements per
 // thread out of the L2; as a kernel of its own it is a second launch, 2.4 us and the gap between dependent kernels, in front of a
-// GEMM of 2 to 3 (1 x 4096 x 4096), and on the host half of a call.  From three rows on the matrix core does the GEMM, in
-// kernels that take packed rows; whether those should quantise too has not been measured.
+// GEMM of 2 to 3 (1 x 4096 x 4096), and on the host half of a call.  From three rows on: qm_skinny_linear.hpp.
 template <int IN, int MR_, int NW_, int U_>
 struct DotLinearCfg {
     static constexpr int MR = MR_, NW = NW_, U = U_, THREADS = 64 * NW, BN = 16;
