@@ -221,6 +221,39 @@ __device__ __forceinline__ v4i mfma16(const v4i s0, const v4i s1, const v4i acc)
 // sit in front of a wave's first load).
 __device__ __forceinline__ uint32_t row_bytes24(int row, int Kb) { return __umul24((uint32_t)row, (uint32_t)Kb); }
 
+// 16 bytes at any byte address, as five aligned dwords shifted into place.  The memory pipeline takes 16 bytes per lane at any
+// multiple of four in one access and at other addresses in four, so four dwords from the
+// multiple of four below and a fifth are less than half the work.  No dword is read that lies partly outside the `bytes`
+// from `base` on: where the 16 bytes begin or end too close to them, they are loaded as they are.
+// Addresses are 32-bit offsets from `base` rounded down to a multiple of four, which `low` to `high` are inside (dword_span).
+struct DwordSpan {
+    const uint8_t *base;
+    uint32_t lead, low, count;  // bytes from `base` to the operand; offsets low .. low + count - 1 are far enough from both ends
+};
+__device__ __forceinline__ DwordSpan dword_span(const uint8_t *operand, const uint32_t bytes)
+{
+    const uint32_t lead = (uint32_t)(uintptr_t)operand & 3u, low = lead != 0 ? 4u : 0u, end = lead + bytes;
+    return {operand - lead, lead, low, end >= low + 19u ? end - 18u - low : 0u};
+}
+struct Shifted16 {
+    v4i w;
+    int next;
+    uint32_t by;
+    __device__ __forceinline__ void load(const DwordSpan &s, const uint32_t at)  // `at` bytes into the operand
+    {
+        const uint32_t off = at + s.lead;
+        const bool near = off - s.low >= s.count;
+        by = near ? 0u : off & 3u;
+        w = *reinterpret_cast<const v4i_any_aligned *>(s.base + (off - by));
+        next = *reinterpret_cast<const int *>(s.base + ((near ? off + 3u : off + 15u) & ~3u));
+    }
+    __device__ __forceinline__ v4i value() const
+    {
+        return v4i{(int)__builtin_amdgcn_alignbyte((uint32_t)w.y, (uint32_t)w.x, by), (int)__builtin_amdgcn_alignbyte((uint32_t)w.z, (uint32_t)w.y, by),
+                   (int)__builtin_amdgcn_alignbyte((uint32_t)w.w, (uint32_t)w.z, by), (int)__builtin_amdgcn_alignbyte((uint32_t)next, (uint32_t)w.w, by)};
+    }
+};
+
 // Workgroups are dealt round-robin to the 8 XCDs (id % 8), each with a private
 // L2.  Renumber so that every XCD owns one contiguous range of tile ids.
 __device__ __forceinline__ int xcd_contiguous_id(int bid, int nblocks)

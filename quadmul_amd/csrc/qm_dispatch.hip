@@ -177,31 +177,38 @@ static RaggedBlock ragged_block(int m, int n)
 
 // With a workspace a large product can also run on zero-padded copies of A and B on the aligned kernels.
 // The faster of the two by what each costs (us), fitted to 3800 products of 1 to 1500 rows, timed both ways with B from HBM
-// and from the caches (rms of the fits 11 % here, 8 and 13 % on the copies; on 2500 others the choice is 1.4 % behind the
-// better one in the mean; up to 32 or 64 rows this kernel, which was the rule once, 7 %):
+// and from the caches (rms of the fits 11 % here, 8 and 13 % on the copies), the clocks of rows off the multiples of four to 700
+// since those are loaded as shifted dwords (7 %; with them the choice is 0.9 % behind the better one in the mean, at the clocks of
+// before, 1.94 and 0.35, 3.3 %):
 //   - here it is the loads: every wave's 16 bytes per lane of the rows of a block go through the L1 of its CU, 0.66 clocks
-//     a lane where rows lie on multiples of four bytes and 1.94 where they do not (those are split); up to 0.35 x 5.5
+//     a lane where rows lie on multiples of four bytes and 1.18 where they do not (a dword more each); up to 0.07 x 5.5
 //     more where they lie within five bytes of a multiple of 128 from row to row, so that the rows of a block
-//     meet in the same banks (16 x 28672 x 4096 + 2 d, d = -1, -2, -3, -5, -7: 43.5, 38.4, 33.6, 28.5, 24.8; 17.5 at d = -8;
-//     the copies 34).  Rows of a block beyond m are copies of the last one and cost next to nothing (3, 8 and 16 x 65536 x
-//     4100: 58, 68, 78).  Workgroups beyond one per CU count whole rounds;
+//     meet in the same banks.  From 40 MB of B on the clocks are those of before, to which the tests of the selection hold such calls (few
+//     rows would gain: 13 x 22589 x 3282 takes 0.58 of the time on copies, 9 x 52926 x 3886 0.55).  Rows of a block beyond m are copies of the last one and cost next to nothing.  Workgroups
+//     beyond one per CU count whole rounds;
 //   - on copies, two launches, the rows of both operands read, written and read again, and the GEMM.
 // One or two rows never take the copies, which are as large as the weights and at most a fifth faster there.  Above
-// 512 rows only small products are left here, as before (809 x 708 x 1096 5.2 / 8.6, 939 x 1094 x 1596 17.7 / 12.7).
+// 512 rows only small products are left here (809 x 708 x 1096 5.2 / 8.6, 939 x 1094 x 1596 17.7 / 12.7); to 1500 rows off the multiples of four, where the
+// rule was measured, up to 2^32 multiplications.  What the clocks of before left to the copies has to be a tenth below them: with none 20 of 700 were more
+// than 2 % slower than on the copies they had run on, so 7 (14 %).
 static bool ragged_before_copies(int m, int n, int k, int ptr_align)
 {
     if (m <= 2) return true;
-    if (m > 512 && (long long)m * n * k >= (1LL << 29)) return false;
+    const bool dwords = k / 2 % 4 == 0 && ptr_align >= 4;
+    const bool shifted = !dwords && (long long)n * (k / 2) < 40000000;
     const RaggedBlock b = ragged_block(m, n);
     const int kb = k / 2, off = std::min(kb % 128, 128 - kb % 128), kp = (k + 127) / 128 * 128;
     const double chunks = (kb + 63) / 64, out = 4e-6 * m * n, rounds = (double)((b.count(m, n) + 255) / 256);
-    const double l1_clocks = kb % 4 == 0 && ptr_align >= 4 ? 0.66 : 1.94 + 0.35 * std::max(0.0, 5.5 - off);
-    const double rows16 = std::min(m / 16.0, (double)b.fm) + b.fn;
-    const double here = 1.56 + 0.33 * (double)(((kb + 63) / 64 + b.nw * b.u - 1) / (b.nw * b.u)) + 0.06e-6 * n * kb + 0.62 * out
-                        + rounds * chunks * (64 * rows16 * l1_clocks + 6 * b.fm * b.fn) / 2400;
+    const double rows16 = std::min(m / 16.0, (double)b.fm) + b.fn, near_line = std::max(0.0, 5.5 - off);
+    const auto here = [&](double l1_clocks) {
+        return 1.56 + 0.33 * (double)(((kb + 63) / 64 + b.nw * b.u - 1) / (b.nw * b.u)) + 0.06e-6 * n * kb + 0.62 * out
+               + rounds * chunks * (64 * rows16 * l1_clocks + 6 * b.fm * b.fn) / 2400;
+    };
     const double moved = 1e-6 * ((double)m + n) * (kp / 2), mfma = 2.0 * m * n * kp / 4.5e9, steps = kp / 128;
     const double copies = m <= 64 ? 5.35 + 0.425 * moved + 0.025 * steps + 0.54 * out + 1.9 * mfma : 6.7 + 0.52 * moved + 0.034 * steps + 0.18 * out + 1.66 * mfma;
-    return here < copies;
+    const bool small = m <= 512 || (long long)m * n * k < (1LL << 29);
+    if (small && here(dwords ? 0.66 : 1.94 + 0.35 * near_line) < copies) return true;
+    return shifted && (small || (m <= 1500 && (long long)m * n * k < (1LL << 32))) && here(1.18 + 0.072 * near_line) < 0.9 * copies;
 }
 
 // Automatic choice only: K padded to a multiple of 128 (operands copied into the workspace) so
@@ -240,6 +247,9 @@ static PadPlan plan_padded_k(int m, int n, int k, int ptr_align, const Choice &d
     pl.b_bytes = ((size_t)n * (kp / 2) + 255) / 256 * 256;
     return pl;
 }
+
+// Rows on multiples of four: they are loaded as they are, others as shifted dwords (Shifted16).
+static bool rows_on_dwords(const GemmArgs &p) { return (((uintptr_t)p.A | (uintptr_t)p.B | (uintptr_t)(p.K >> 1)) & 3) == 0; }
 
 // The padded copies of A and B in the workspace, and the arguments of the GEMM on them.
 static hipError_t launch_padded(GemmArgs &p, const PadPlan &pl, void *ws, hipStream_t s)
@@ -330,7 +340,8 @@ static hipError_t launch_fp6_padded(GemmArgs p, const PadPlan &pl, Fp6Route rout
     const Fp6Layout &l = a.layout;
     const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, l.kt, l.groups, l.parts, p.B, reinterpret_cast<v4i *>(b_copy), p.N, pl.kp};
     const long long pieces = (long long)p.N * (pl.kp / 32);
-    expand_a6_kernel<true><<<dim3(l.groups * (32 / CODE_ROWS) * l.parts + (unsigned)((pieces + EXPAND6_THREADS - 1) / EXPAND6_THREADS)), dim3(EXPAND6_THREADS), 0, s>>>(q);
+    const auto kernel = rows_on_dwords(p) ? &expand_a6_kernel<true, false> : &expand_a6_kernel<true, true>;
+    kernel<<<dim3(l.groups * (32 / CODE_ROWS) * l.parts + (unsigned)((pieces + EXPAND6_THREADS - 1) / EXPAND6_THREADS)), dim3(EXPAND6_THREADS), 0, s>>>(q);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     p.B = b_copy;
@@ -342,7 +353,8 @@ template <class Cfg>
 static hipError_t launch_ragged(const GemmArgs &p, hipStream_t s)
 {
     const dim3 grid((p.N + Cfg::BN - 1) / Cfg::BN, (p.M + Cfg::MAX_M - 1) / Cfg::MAX_M);
-    gemm_ragged_kernel<Cfg><<<grid, dim3(Cfg::THREADS), 0, s>>>(p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out, p.row_scale, p.col_scale, p.bias);
+    const auto kernel = rows_on_dwords(p) ? &gemm_ragged_kernel<Cfg, false> : &gemm_ragged_kernel<Cfg, true>;
+    kernel<<<grid, dim3(Cfg::THREADS), 0, s>>>(p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out, p.row_scale, p.col_scale, p.bias);
     return hipGetLastError();
 }
 

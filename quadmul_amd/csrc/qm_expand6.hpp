@@ -16,11 +16,24 @@ struct Expand6Args {
     int N, Kp;
 };
 
-// 16 bytes of a row of Kb from byte `at` on, zeros past its end
-__device__ __forceinline__ v4i row_piece(const uint8_t *row, const int at, const int Kb)
+// 16 bytes of a row of Kb from byte `at` on, zeros past its end.  Loaded by row_load -- SHIFT: rows that do not lie on multiples of four --
+// and put right once it is there.
+template <bool SHIFT>
+using RowPiece = std::conditional_t<SHIFT, Shifted16, v4i>;
+template <bool SHIFT>
+__device__ __forceinline__ void row_load(RowPiece<SHIFT> &v, const DwordSpan &s, const uint32_t row, const int at, const int Kb)
+{
+    const uint32_t from = row * (uint32_t)Kb + (uint32_t)min(at, Kb - 16);
+    if constexpr (SHIFT) v.load(s, from);
+    else v = *reinterpret_cast<const v4i_any_aligned *>(s.base + (s.lead + from));
+}
+template <bool SHIFT>
+__device__ __forceinline__ v4i row_value(const RowPiece<SHIFT> &piece, const int at, const int Kb)
 {
     const int left = Kb - at;  // bytes of the row from there on
-    v4i v = *reinterpret_cast<const v4i_any_aligned *>(row + min(at, Kb - 16));
+    v4i v;
+    if constexpr (SHIFT) v = piece.value();
+    else v = piece;
     if (left < 16) {
         // the row's last 16 bytes: the wanted ones are its last `left`
         const int down = 8 * (16 - max(left, 0));
@@ -54,8 +67,9 @@ __device__ __forceinline__ void code_rows(const int block, int &group, int &r0)
 // copy B with its rows padded, one 16-byte piece per thread, in the same launch.
 // Bound: HBM on large operands, the launch and one round trip on small ones.  us in a graph, by sixteen
 // neighbouring rows to a workgroup / now: 512 x 8192 3.9 / 3.2, 1536 x 4096 4.1 / 3.4, 4096 x 4096 5.8 / 5.7, 8192 x 8192 17.0 / 14.8 (5.7 TB/s).
+// SHIFT (rows of A off the multiples of four): with B's copy 1531 x 3307 x 4100 6.8 -> 5.0, the whole product 35.5 -> 33.0.
 constexpr int EXPAND6_THREADS = 512;
-template <bool ANY>
+template <bool ANY, bool SHIFT = false>
 __global__ void __launch_bounds__(EXPAND6_THREADS) expand_a6_kernel(const Expand6Args q)
 {
     constexpr int WAVES = EXPAND6_THREADS / 64, PAIRS = FP6_PART_STEPS / 2 / WAVES;  // (pairs of K-steps: per wave)
@@ -68,7 +82,11 @@ __global__ void __launch_bounds__(EXPAND6_THREADS) expand_a6_kernel(const Expand
         if (part >= q.parts) {
             const uint32_t per_row = (uint32_t)q.Kp >> 5, piece = (blockIdx.x - q.parts * blocks) * (uint32_t)EXPAND6_THREADS + threadIdx.x;  // (below 2^28 and a workgroup)
             const uint32_t n = piece / per_row;
-            if (n < (uint32_t)q.N) q.b_copy[piece] = row_piece(q.B + (size_t)n * Kb, 16 * (int)(piece - n * per_row), Kb);
+            if (n < (uint32_t)q.N) {
+                const int at = 16 * (int)(piece - n * per_row);
+                // (one load per thread, as it is also where that is four accesses: shifted dwords are no faster here)
+                q.b_copy[piece] = row_value<false>(*reinterpret_cast<const v4i_any_aligned *>(q.B + (n * (uint32_t)Kb + (uint32_t)min(at, Kb - 16))), at, Kb);
+            }
             return;
         }
     }
@@ -77,21 +95,24 @@ __global__ void __launch_bounds__(EXPAND6_THREADS) expand_a6_kernel(const Expand
     // lane: row, 16 bytes of a K-step, step of the two
     const int h = (lane >> 2) & 1, r = r0 + (lane & 3), g = (lane >> 3) & 3, second = lane >> 5;
     const int row = group * 32 + h * 16 + r, row_bytes = ANY ? q.Kp >> 1 : Kb;
-    const uint8_t *src = q.A + (size_t)min(row, q.M - 1) * Kb;
-    v4i v[PAIRS];
+    const DwordSpan span = dword_span(q.A, (uint32_t)q.M * (uint32_t)Kb);
+    RowPiece<SHIFT> v[PAIRS];
 #pragma unroll
     for (int t = 0; t < PAIRS; ++t) {
         const int at = min((part * FP6_PART_STEPS + 2 * (wave + WAVES * t)) * 64, row_bytes - 128) + 64 * second + 16 * g;
-        if constexpr (ANY) v[t] = row_piece(src, at, Kb);
-        else v[t] = *reinterpret_cast<const v4i *>(src + at);
+        if constexpr (ANY) row_load<SHIFT>(v[t], span, min(row, q.M - 1), at, Kb);
+        else v[t] = *reinterpret_cast<const v4i *>(q.A + (size_t)min(row, q.M - 1) * Kb + at);
     }
     int sum = 0;
 #pragma unroll
     for (int t = 0; t < PAIRS; ++t) {
         const int step = part * FP6_PART_STEPS + 2 * (wave + WAVES * t);
         if (step >= q.kt) break;
-        v4i w = v[t];
-        if (row >= q.M || min(step * 64, row_bytes - 128) + 64 * second + 16 * g < step * 64) w = v4i{0, 0, 0, 0};
+        const int at = min(step * 64, row_bytes - 128) + 64 * second + 16 * g;
+        v4i w;
+        if constexpr (ANY) w = row_value<SHIFT>(v[t], at, Kb);
+        else w = v[t];
+        if (row >= q.M || at < step * 64) w = v4i{0, 0, 0, 0};
 #pragma unroll
         for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_sdot8(w[e], 0x11111111, sum, false);
         uint32_t f[6];

@@ -5,15 +5,16 @@
 // Without it these calls ran on one thread per element of C (small products) or on
 // zero-padded copies of both operands (2 x (M + N) K / 2 bytes of extra traffic, which is
 // most of the time while M is small).  Bound: where rows do not lie on multiples of four bytes the L1, which
-// takes the 16 bytes of such a lane in four accesses, one access per clock (16 x 65536 x 4100: 52.8 M accesses, 4.07 per
-// lane and load, 0.99 per clock and CU; 78 us, 1.7 TB/s of B, each byte of it fetched once); where they do (0.87 per lane and
+// takes the 16 bytes of such a lane in four accesses, one access per clock (16 x 65536 x 4100: 4.07 accesses per
+// lane and load, 0.99 per clock and CU; 78 us): those rows are loaded as aligned dwords, four and the one after them, and shifted (SHIFT; us, before ->
+// now: 16 x 5001 x 2050 7.5 -> 4.3, 17 x 3307 x 4100 8.9 -> 5.2, 9 x 7085 x 7390 13.4 -> 9.0, 143 x 1003 x 1788 7.7 -> 4.6); where they
+// do (0.87 per lane and
 // load), HBM on a wide B (16 x 65536 x 8200 77 us, 3.5 TB/s; 3 x 9000 x 9000 12 us, 3.4 TB/s), the latency
 // of a wave's K loop otherwise.  The decomposition is that of gemm_skinny_kernel: a
 // workgroup owns 16*FM rows of A (grid.y walks over blocks of them) and 16*FN rows of B, its
 // NW waves split K in 128-nibble chunks, partial blocks meet in the LDS.  Lane (r, g) loads the
 // 16 bytes it feeds to the matrix core itself -- row r, bytes 16 g .. + 15 of the chunk's 64 --
-// as one global_load_dwordx4 at whatever byte address that is: the memory pipeline takes
-// those at any alignment and splits them at cache lines.  (Direct global -> LDS loads, which
+// as one global_load_dwordx4, or that and a dword.  (Direct global -> LDS loads, which
 // the aligned kernels use, want aligned addresses.)  U chunks are in flight per wave, no more than it has: with every wave
 // loading U chunks whether or not they exist, 1 x 5001 x 2050 -- seventeen chunks on sixteen waves --
 // took 10.5 us instead of 6.7.
@@ -35,7 +36,7 @@ struct RaggedCfg {
     static_assert((FM + FN) * U <= 16, "staging registers: four per load in flight");
 };
 
-template <class Cfg>
+template <class Cfg, bool SHIFT>
 __global__ void __launch_bounds__(Cfg::THREADS)
 gemm_ragged_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int M, const int N, const int K, const int ldc, const int out,
                    const float *row_scale, const float *col_scale, const uint16_t *bias)
@@ -72,22 +73,36 @@ gemm_ragged_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int M, 
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = v4i{0, 0, 0, 0};
 
+    const DwordSpan a_span = dword_span(A, (uint32_t)M * (uint32_t)Kb), b_span = dword_span(B, (uint32_t)N * (uint32_t)Kb);
     // chunks wave, wave + NW, ... of this wave, U at a time
     for (int c0 = wave; c0 < nchunks; c0 += NW * U) {
         v4i aq[U][FM], bq[U][FN];
+        Shifted16 as[SHIFT ? U : 1][FM], bs[SHIFT ? U : 1][FN];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (c0 + u * NW >= nchunks) break;  // (wave-uniform)
             const uint32_t at = (uint32_t)min((c0 + u * NW) * 64 + g * 16, Kb - 16);
 #pragma unroll
-            for (int j = 0; j < FN; ++j) bq[u][j] = *reinterpret_cast<const v4i_any_aligned *>(B + (b_off[j] + at));
+            for (int j = 0; j < FN; ++j) {
+                if constexpr (SHIFT) bs[u][j].load(b_span, b_off[j] + at);
+                else bq[u][j] = *reinterpret_cast<const v4i_any_aligned *>(B + (b_off[j] + at));
+            }
 #pragma unroll
-            for (int i = 0; i < FM; ++i) aq[u][i] = *reinterpret_cast<const v4i_any_aligned *>(A + (a_off[i] + at));
+            for (int i = 0; i < FM; ++i) {
+                if constexpr (SHIFT) as[u][i].load(a_span, a_off[i] + at);
+                else aq[u][i] = *reinterpret_cast<const v4i_any_aligned *>(A + (a_off[i] + at));
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int c = c0 + u * NW;
             if (c >= nchunks) break;
+            if constexpr (SHIFT) {
+#pragma unroll
+                for (int j = 0; j < FN; ++j) bq[u][j] = bs[u][j].value();
+#pragma unroll
+                for (int i = 0; i < FM; ++i) aq[u][i] = as[u][i].value();
+            }
             if ((c + 1) * 64 > Kb) {
                 // the short last chunk: of the 16 bytes loaded the first `seen` belong to lanes
                 // before this one
