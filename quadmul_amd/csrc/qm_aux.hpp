@@ -54,8 +54,7 @@ static hipError_t launch_generic(const GemmArgs &p, hipStream_t stream, int)
 {
     const long long tiles_m = (p.M + 15) / 16, tiles_n = (p.N + 15) / 16;
     if (tiles_m * tiles_n > 0x7fffffffLL) return hipErrorInvalidValue;
-    gemm_generic_kernel<<<dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream>>>(p, (int)tiles_n);
-    return hipGetLastError();
+    return enqueue(&gemm_generic_kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, p, (int)tiles_n);
 }
 
 // --------------------------------------------------------------------------
@@ -532,16 +531,17 @@ __global__ void __launch_bounds__(256) quantize_pack_scalar_kernel(const uint8_t
 }
 
 template <int IN, int NW, int NC>
-static void launch_quantize_rows(const uint8_t *x, uint8_t *dst, float *scales, int rows, int k, hipStream_t s)
+static hipError_t launch_quantize_rows(const uint8_t *x, uint8_t *dst, float *scales, int rows, int k, hipStream_t s)
 {
     constexpr int threads = NW == 1 ? 256 : 64 * NW, rows_per_block = NW == 1 ? 4 : 1;
     constexpr int most = (1 << 21) * rows_per_block;  // a grid has less than 2^32 threads
     for (int r0 = 0; r0 < rows; r0 += most) {
         const int n = rows - r0 < most ? rows - r0 : most;
-        quantize_pack_kernel<IN, NW, NC><<<dim3((unsigned)(n + rows_per_block - 1) / rows_per_block), dim3(threads), 0, s>>>(
+        const hipError_t e = enqueue(&quantize_pack_kernel<IN, NW, NC>, dim3((unsigned)(n + rows_per_block - 1) / rows_per_block), dim3(threads), 0, s,
             x + (size_t)r0 * k * QuantIn<IN>::BYTES, dst + (size_t)r0 * (k / 2), scales + r0, n, k);
-        if (r0 > 0x7fffffff - most) break;
+        if (e != hipSuccess || r0 > 0x7fffffff - most) return e;
     }
+    return hipSuccess;
 }
 
 // Four waves per row: as many chunks per lane as the row takes, none of them empty.  A workgroup per row is
@@ -556,19 +556,18 @@ static hipError_t launch_quantize_pack(const void *x, void *dst, float *scales, 
 {
     const uint8_t *xb = static_cast<const uint8_t *>(x);
     uint8_t *db = static_cast<uint8_t *>(dst);
-    if (k < 8) quantize_pack_scalar_kernel<IN><<<dim3(rows), dim3(256), 0, s>>>(xb, db, scales, k);
-    else if (k > 16384) launch_quantize_rows<IN, 16, 0>(xb, db, scales, rows, k, s);
-    else if (k > 12288) launch_quantize_rows<IN, 16, 2>(xb, db, scales, rows, k, s);
-    else if (rows > 1024 && k <= 512) launch_quantize_rows<IN, 1, 1>(xb, db, scales, rows, k, s);
-    else if (rows > 1024 && k <= 1024) launch_quantize_rows<IN, 1, 2>(xb, db, scales, rows, k, s);
-    else if (rows > 1024 && k <= 1536) launch_quantize_rows<IN, 1, 3>(xb, db, scales, rows, k, s);
-    else if (k <= 2048) launch_quantize_rows<IN, 4, 1>(xb, db, scales, rows, k, s);
-    else if (k <= 4096) launch_quantize_rows<IN, 4, 2>(xb, db, scales, rows, k, s);
-    else if (k <= 6144) launch_quantize_rows<IN, 4, 3>(xb, db, scales, rows, k, s);
-    else if (k <= 8192) launch_quantize_rows<IN, 4, 4>(xb, db, scales, rows, k, s);
-    else if (k <= 10240) launch_quantize_rows<IN, 4, 5>(xb, db, scales, rows, k, s);
-    else launch_quantize_rows<IN, 4, 6>(xb, db, scales, rows, k, s);
-    return hipGetLastError();
+    if (k < 8) return enqueue(&quantize_pack_scalar_kernel<IN>, dim3(rows), dim3(256), 0, s, xb, db, scales, k);
+    if (k > 16384) return launch_quantize_rows<IN, 16, 0>(xb, db, scales, rows, k, s);
+    if (k > 12288) return launch_quantize_rows<IN, 16, 2>(xb, db, scales, rows, k, s);
+    if (rows > 1024 && k <= 512) return launch_quantize_rows<IN, 1, 1>(xb, db, scales, rows, k, s);
+    if (rows > 1024 && k <= 1024) return launch_quantize_rows<IN, 1, 2>(xb, db, scales, rows, k, s);
+    if (rows > 1024 && k <= 1536) return launch_quantize_rows<IN, 1, 3>(xb, db, scales, rows, k, s);
+    if (k <= 2048) return launch_quantize_rows<IN, 4, 1>(xb, db, scales, rows, k, s);
+    if (k <= 4096) return launch_quantize_rows<IN, 4, 2>(xb, db, scales, rows, k, s);
+    if (k <= 6144) return launch_quantize_rows<IN, 4, 3>(xb, db, scales, rows, k, s);
+    if (k <= 8192) return launch_quantize_rows<IN, 4, 4>(xb, db, scales, rows, k, s);
+    if (k <= 10240) return launch_quantize_rows<IN, 4, 5>(xb, db, scales, rows, k, s);
+    return launch_quantize_rows<IN, 4, 6>(xb, db, scales, rows, k, s);
 }
 
 static unsigned flat_grid(size_t items, unsigned block, size_t most = 256u * 32u)

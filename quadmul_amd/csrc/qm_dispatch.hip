@@ -36,12 +36,10 @@ static hipError_t launch_skinny(const GemmArgs &p, hipStream_t stream, int opt)
     if constexpr (Cfg::U % 2 == 0) {
         if (blocks > resident && (p.K + 127) / 128 <= Cfg::NW * Cfg::U) {
             const int turns = (blocks + resident - 1) / resident;
-            gemm_skinny_stream_kernel<Cfg><<<dim3((blocks + turns - 1) / turns), dim3(Cfg::THREADS), 0, stream>>>(p, blocks);
-            return hipGetLastError();
+            return enqueue(&gemm_skinny_stream_kernel<Cfg>, dim3((blocks + turns - 1) / turns), dim3(Cfg::THREADS), 0, stream, p, blocks);
         }
     }
-    gemm_skinny_kernel<Cfg><<<dim3(blocks), dim3(Cfg::THREADS), 0, stream>>>(p);
-    return hipGetLastError();
+    return enqueue(&gemm_skinny_kernel<Cfg>, dim3(blocks), dim3(Cfg::THREADS), 0, stream, p);
 }
 #define QM_SKINNY(FM, FN, NW, U) \
     hipError_t QM_SKINNY_FN(FM, FN, NW, U)(const GemmArgs &p, hipStream_t s, int gm) { return launch_skinny<SkinnyCfg<FM, FN, NW, U>>(p, s, gm); }
@@ -51,8 +49,7 @@ static hipError_t launch_dot(const GemmArgs &p, hipStream_t stream, int opt)
     if (opt & QM_OPT_PREPARE) return hipSuccess;
     const int blocks = (p.N + Cfg::BN - 1) / Cfg::BN;
     static_assert(kernarg_bytes(&gemm_dot_kernel<Cfg>) <= 64, "see pack_rows_out");
-    gemm_dot_kernel<Cfg><<<dim3(blocks), dim3(Cfg::THREADS), 0, stream>>>(p.A, p.B, p.C, pack_rows_out(p.M, p.out), p.N, p.K, p.ldc, p.row_scale, p.col_scale, p.bias);
-    return hipGetLastError();
+    return enqueue(&gemm_dot_kernel<Cfg>, dim3(blocks), dim3(Cfg::THREADS), 0, stream, p.A, p.B, p.C, pack_rows_out(p.M, p.out), p.N, p.K, p.ldc, p.row_scale, p.col_scale, p.bias);
 }
 #define QM_DOT(MR, FN, NW, U) \
     hipError_t QM_DOT_FN(MR, FN, NW, U)(const GemmArgs &p, hipStream_t s, int gm) { return launch_dot<DotCfg<MR, FN, NW, U>>(p, s, gm); }
@@ -66,9 +63,8 @@ static hipError_t launch_skinny_dma(const GemmArgs &p, hipStream_t stream, int o
     const int blocks = (p.N + Cfg::BN - 1) / Cfg::BN, row_blocks = (p.M + Cfg::MAX_M - 1) / Cfg::MAX_M;
     if (row_blocks > 65535) return hipErrorInvalidValue;
     static_assert(kernarg_bytes(&gemm_skinny_dma_kernel<Cfg>) <= 64, "see pack_rows_out");
-    gemm_skinny_dma_kernel<Cfg><<<dim3(skinny_dma_columns(blocks, row_blocks), row_blocks), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(
+    return enqueue(&gemm_skinny_dma_kernel<Cfg>, dim3(skinny_dma_columns(blocks, row_blocks), row_blocks), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream,
         p.A, p.B, p.C, pack_rows_out(p.M, p.out), p.N, p.K, p.ldc, p.row_scale, p.col_scale, p.bias);
-    return hipGetLastError();
 }
 template <class Cfg>
 static hipError_t launch_skinny_stream_dma(const GemmArgs &p, hipStream_t stream, int opt)
@@ -84,9 +80,8 @@ static hipError_t launch_skinny_stream_dma(const GemmArgs &p, hipStream_t stream
     const int resident = cus * (160 * 1024 / Cfg::LDS_BYTES);  // workgroups the device holds at once (the LDS decides)
     const int grid = blocks < resident ? blocks : resident;
     static_assert(kernarg_bytes(&gemm_skinny_stream_dma_kernel<Cfg>) <= 64, "see pack_rows_out");
-    gemm_skinny_stream_dma_kernel<Cfg><<<dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(
+    return enqueue(&gemm_skinny_stream_dma_kernel<Cfg>, dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream,
         p.A, p.B, p.C, p.out | (p.M << 2) | (grid << 8), p.N, p.K, p.ldc, p.row_scale, p.col_scale, p.bias);
-    return hipGetLastError();
 }
 #define QM_SKINNYP(FM, FN, NW, D, R) \
     hipError_t QM_SKINNYP_FN(FM, FN, NW, D, R)(const GemmArgs &p, hipStream_t s, int gm) { return launch_skinny_stream_dma<SkinnyStreamCfg<FM, FN, NW, D, R>>(p, s, gm); }
@@ -257,8 +252,7 @@ static hipError_t launch_padded(GemmArgs &p, const PadPlan &pl, void *ws, hipStr
     uint8_t *a_p = static_cast<uint8_t *>(ws), *b_p = a_p + pl.a_bytes;
     const PadRowsArgs q{p.A, p.B, reinterpret_cast<v4i *>(a_p), reinterpret_cast<v4i *>(b_p), p.M, p.N, p.K / 2, pl.kp / 32};
     const long long pieces = ((long long)p.M + p.N) * q.ppr;
-    pad_rows_kernel<<<dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, s>>>(q);
-    const hipError_t e = hipGetLastError();
+    const hipError_t e = enqueue(&pad_rows_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, s, q);
     if (e != hipSuccess) return e;
     p.A = a_p;
     p.B = b_p;
@@ -326,8 +320,7 @@ static hipError_t launch_fp6(const GemmArgs &p, Fp6Route route, void *ws, hipStr
     const Fp6Operand a = fp6_operand(p.M, p.K, ws);
     const Fp6Layout &l = a.layout;
     const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, l.kt, l.groups, l.parts};
-    expand_a6_kernel<false><<<dim3(l.groups * (32 / CODE_ROWS) * l.parts), dim3(EXPAND6_THREADS), 0, s>>>(q);
-    const hipError_t e = hipGetLastError();
+    const hipError_t e = enqueue(&expand_a6_kernel<false>, dim3(l.groups * (32 / CODE_ROWS) * l.parts), dim3(EXPAND6_THREADS), 0, s, q);
     return e == hipSuccess ? launch_tile6(p, a, route, s) : e;
 }
 
@@ -341,8 +334,7 @@ static hipError_t launch_fp6_padded(GemmArgs p, const PadPlan &pl, Fp6Route rout
     const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, l.kt, l.groups, l.parts, p.B, reinterpret_cast<v4i *>(b_copy), p.N, pl.kp};
     const long long pieces = (long long)p.N * (pl.kp / 32);
     const auto kernel = rows_on_dwords(p) ? &expand_a6_kernel<true, false> : &expand_a6_kernel<true, true>;
-    kernel<<<dim3(l.groups * (32 / CODE_ROWS) * l.parts + (unsigned)((pieces + EXPAND6_THREADS - 1) / EXPAND6_THREADS)), dim3(EXPAND6_THREADS), 0, s>>>(q);
-    const hipError_t e = hipGetLastError();
+    const hipError_t e = enqueue(kernel, dim3(l.groups * (32 / CODE_ROWS) * l.parts + (unsigned)((pieces + EXPAND6_THREADS - 1) / EXPAND6_THREADS)), dim3(EXPAND6_THREADS), 0, s, q);
     if (e != hipSuccess) return e;
     p.B = b_copy;
     p.K = pl.kp;
@@ -354,8 +346,7 @@ static hipError_t launch_ragged(const GemmArgs &p, hipStream_t s)
 {
     const dim3 grid((p.N + Cfg::BN - 1) / Cfg::BN, (p.M + Cfg::MAX_M - 1) / Cfg::MAX_M);
     const auto kernel = rows_on_dwords(p) ? &gemm_ragged_kernel<Cfg, false> : &gemm_ragged_kernel<Cfg, true>;
-    kernel<<<grid, dim3(Cfg::THREADS), 0, s>>>(p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out, p.row_scale, p.col_scale, p.bias);
-    return hipGetLastError();
+    return enqueue(kernel, grid, dim3(Cfg::THREADS), 0, s, p.A, p.B, p.C, p.M, p.N, p.K, p.ldc, p.out, p.row_scale, p.col_scale, p.bias);
 }
 
 static hipError_t launch_ragged(const GemmArgs &p, hipStream_t s)
@@ -410,8 +401,7 @@ static hipError_t launch_split_with_workspace(GemmArgs p, const Choice &ch, void
     if (e != hipSuccess) return e;
     const size_t pieces = (size_t)q.tiles_m * q.tiles_n * (size_t)(d.bm * d.bn / 4);
     if (pieces > 0x7fffff00ULL) return hipErrorInvalidValue;
-    splitk_reduce_kernel<<<dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, s>>>(q);
-    return hipGetLastError();
+    return enqueue(&splitk_reduce_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, s, q);
 }
 
 // Operands of this many bytes or more are cut into blocks (below).  2^31 - 1 in production: what
@@ -459,10 +449,10 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
     const int row_stride = ldc != 0 ? ldc : n;   // of the output, in elements
     const bool strided = row_stride != n;        // a block of columns of a wider output
     if (k == 0) {
-        if (scaled && bias) fill_bias16_kernel<<<dim3(flat_grid(cnt, 256)), dim3(256), 0, s>>>(static_cast<uint16_t *>(dst), bias, n, row_stride, cnt, out);
-        else if (scaled) fill_zero16_kernel<<<dim3(flat_grid(cnt, 256)), dim3(256), 0, s>>>(static_cast<uint16_t *>(dst), cnt);
-        else fill_zero_kernel<<<dim3(flat_grid(cnt, 256)), dim3(256), 0, s>>>(static_cast<int32_t *>(dst), cnt);
-        const hipError_t e = hipGetLastError();
+        const dim3 grid(flat_grid(cnt, 256)), block(256);
+        const hipError_t e = scaled && bias ? enqueue(&fill_bias16_kernel, grid, block, 0, s, static_cast<uint16_t *>(dst), bias, n, row_stride, cnt, out)
+                             : scaled       ? enqueue(&fill_zero16_kernel, grid, block, 0, s, static_cast<uint16_t *>(dst), cnt)
+                                            : enqueue(&fill_zero_kernel, grid, block, 0, s, static_cast<int32_t *>(dst), cnt);
         return e == hipSuccess ? QM_OK : fail_launch(e);
     }
     const int align = ptr_alignment(A, B);
@@ -562,8 +552,7 @@ static int run_gemm(const void *A, const void *B, void *dst, int m, int n, int k
     }
     if (ch.ksplit > 1) {
         // int32, no workspace: the partial sums meet in C by integer atomic adds, C starts from zero
-        fill_zero_kernel<<<dim3(flat_grid(cnt, 256)), dim3(256), 0, s>>>(static_cast<int32_t *>(dst), cnt);
-        const hipError_t ez = hipGetLastError();
+        const hipError_t ez = enqueue(&fill_zero_kernel, dim3(flat_grid(cnt, 256)), dim3(256), 0, s, static_cast<int32_t *>(dst), cnt);
         if (ez != hipSuccess) return fail_launch(ez);
     }
     const LaunchFn launch = launcher(ch.cfg);
@@ -784,14 +773,14 @@ QM_EXPORT int qm_pack_i4(const void *src_i8, void *dst_packed, int rows, int k, 
     if (nbytes == 0) return QM_OK;
     if (!src_i8 || !dst_packed) return QM_ERR_NULL;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    hipError_t e;
     if (nbytes >= 8) {
         const unsigned grid = flat_grid(nbytes, 8 * PACK_PIECES * PACK_THREADS, 1u << 22);
-        pack_i4_vec_kernel<<<dim3((grid + PACK_APART - 1) / PACK_APART * PACK_APART), dim3(PACK_THREADS), 0, s>>>(
+        e = enqueue(&pack_i4_vec_kernel, dim3((grid + PACK_APART - 1) / PACK_APART * PACK_APART), dim3(PACK_THREADS), 0, s,
             static_cast<const uint8_t *>(src_i8), static_cast<uint8_t *>(dst_packed), nbytes);
     } else {
-        pack_i4_byte_kernel<<<dim3(flat_grid(nbytes, 256)), dim3(256), 0, s>>>(static_cast<const uint8_t *>(src_i8), static_cast<uint8_t *>(dst_packed), nbytes);
+        e = enqueue(&pack_i4_byte_kernel, dim3(flat_grid(nbytes, 256)), dim3(256), 0, s, static_cast<const uint8_t *>(src_i8), static_cast<uint8_t *>(dst_packed), nbytes);
     }
-    const hipError_t e = hipGetLastError();
     return e == hipSuccess ? QM_OK : fail_launch(e);
 }
 
@@ -817,11 +806,11 @@ QM_EXPORT int qm_unpack_i4(const void *src_packed, void *dst_i8, int rows, int k
     if (nbytes == 0) return QM_OK;
     if (!src_packed || !dst_i8) return QM_ERR_NULL;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    hipError_t e;
     if (nbytes >= 8)
-        unpack_i4_vec_kernel<<<dim3(flat_grid(nbytes, 8 * PACK_THREADS, 1u << 22)), dim3(PACK_THREADS), 0, s>>>(static_cast<const uint8_t *>(src_packed), static_cast<uint8_t *>(dst_i8), nbytes);
+        e = enqueue(&unpack_i4_vec_kernel, dim3(flat_grid(nbytes, 8 * PACK_THREADS, 1u << 22)), dim3(PACK_THREADS), 0, s, static_cast<const uint8_t *>(src_packed), static_cast<uint8_t *>(dst_i8), nbytes);
     else
-        unpack_i4_byte_kernel<<<dim3(flat_grid(nbytes, 256)), dim3(256), 0, s>>>(static_cast<const uint8_t *>(src_packed), static_cast<int8_t *>(dst_i8), nbytes);
-    const hipError_t e = hipGetLastError();
+        e = enqueue(&unpack_i4_byte_kernel, dim3(flat_grid(nbytes, 256)), dim3(256), 0, s, static_cast<const uint8_t *>(src_packed), static_cast<int8_t *>(dst_i8), nbytes);
     return e == hipSuccess ? QM_OK : fail_launch(e);
 }
 

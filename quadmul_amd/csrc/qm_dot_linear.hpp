@@ -166,9 +166,8 @@ template <int IN, int MR, int NW, int U>
 static hipError_t launch_dot_linear(const void *x, const void *B, void *D, int m, int n, int k, const float *col_scale, const uint16_t *bias, int out, hipStream_t s)
 {
     using Cfg = DotLinearCfg<IN, MR, NW, U>;
-    dot_linear_kernel<IN, Cfg><<<dim3((n + Cfg::BN - 1) / Cfg::BN), dim3(Cfg::THREADS), dot_linear_lds_bytes(MR, k), s>>>(
+    return enqueue(&dot_linear_kernel<IN, Cfg>, dim3((n + Cfg::BN - 1) / Cfg::BN), dim3(Cfg::THREADS), dot_linear_lds_bytes(MR, k), s,
         static_cast<const uint8_t *>(x), static_cast<const uint8_t *>(B), static_cast<int32_t *>(D), pack_rows_out(m, out), n, k, col_scale, bias);
-    return hipGetLastError();
 }
 template <int IN>
 static hipError_t launch_dot_linear(const void *x, const void *B, void *D, int m, int n, int k, const float *col_scale, const uint16_t *bias, int out, hipStream_t s)

@@ -214,8 +214,7 @@ __global__ void __launch_bounds__(QUANT6_THREADS, 2) quantize_a6_kernel(const Qu
 template <int IN, int NC>
 static hipError_t launch_quantize_a6_rows(const Quant6Args &q, hipStream_t s)
 {
-    quantize_a6_kernel<IN, NC><<<dim3(q.groups * (32 / CODE_ROWS)), dim3(QUANT6_THREADS), quant6_lds_bytes(q.K), s>>>(q);
-    return hipGetLastError();
+    return enqueue(&quantize_a6_kernel<IN, NC>, dim3(q.groups * (32 / CODE_ROWS)), dim3(QUANT6_THREADS), quant6_lds_bytes(q.K), s, q);
 }
 // The K it holds: 64 KiB of LDS, and for fp32 128 registers of one wave per row.
 inline bool quant6_fits(int k, int in) { return quant6_lds_bytes(k) <= 64 * 1024 && (in != QM_IN_F32 || k <= 8192); }

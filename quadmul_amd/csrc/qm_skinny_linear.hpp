@@ -209,9 +209,8 @@ static hipError_t launch_skinny_linear(const void *x, const void *B, void *Y, in
     e = device_cus(&cus);
     if (e != hipSuccess) return e;
     const int blocks = (n + Cfg::BN - 1) / Cfg::BN, grid = blocks < cus ? blocks : cus;
-    skinny_linear_kernel<Cfg><<<dim3(grid), dim3(Cfg::THREADS), Cfg::lds_bytes(k), s>>>(
+    return enqueue(&skinny_linear_kernel<Cfg>, dim3(grid), dim3(Cfg::THREADS), Cfg::lds_bytes(k), s,
         static_cast<const uint8_t *>(x), static_cast<const uint8_t *>(B), static_cast<int32_t *>(Y), grid << 8 | m << 2 | out, n, k, col_scale, bias);
-    return hipGetLastError();
 }
 template <int IN>
 static hipError_t launch_skinny_linear(const void *x, const void *B, void *Y, int m, int n, int k, const float *col_scale, const uint16_t *bias, int out, hipStream_t s)

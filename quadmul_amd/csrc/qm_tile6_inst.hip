@@ -31,8 +31,7 @@ static hipError_t launch_tile6_kernel(Kernel kernel, const GemmArgs &p, const Fp
     // Tiles are numbered in columns of four tile rows: of the 32 that an XCD works on at a time, 4 x 8 share the fewest
     // bytes (4 x 24 KiB of A and 8 x 16 of B per K-step, of B 8 on the narrow tiles)
     const int group_m = tiles_m < 4 ? tiles_m : 4;
-    kernel<<<dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, s>>>(p, a.codes, a.sums, a.layout.parts, a.layout.kt, tiles_m, tiles_n, group_m);
-    return hipGetLastError();
+    return enqueue(kernel, dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, s, p, a.codes, a.sums, a.layout.parts, a.layout.kt, tiles_m, tiles_n, group_m);
 }
 
 template <int OUT, bool BIAS>

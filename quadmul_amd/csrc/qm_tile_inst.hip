@@ -51,8 +51,7 @@ static hipError_t launch_tiled_persistent(Kernel kernel, const GemmArgs &p, hipS
     if (items > 0x7FFFFFFF) return hipErrorInvalidValue;
     int grid = (int)items;
     if (!(opt & 0x10000) && grid > held) grid = held;
-    kernel<<<dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream>>>(p, tiles_m, tiles_n, group_m, ksplit);
-    return hipGetLastError();
+    return enqueue(kernel, dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream, p, tiles_m, tiles_n, group_m, ksplit);
 }
 
 }  // namespace qm
