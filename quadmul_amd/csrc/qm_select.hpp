@@ -318,20 +318,38 @@ static Choice heuristic(int m, int n, int k, int ptr_align, bool has_ws)
         // operands streamed global -> LDS; with A resident in registers and a persistent grid
         // while the waves hold all of K
         if (k <= 4096) return pick(k > 2048 || n >= 8192 ? "p1x1_w8_r2k2" : "d1x1_w16_r1");
-        if (k <= 8192 && n >= 8192) return pick("p1x1_w16_r2k2");
-        // a very long K: every workgroup re-reads A over all of it; 32 columns per workgroup
-        // halve that (16 x 8192 x 28672 19.1 us against 21.7)
-        if (k > 16384) return pick("d1x2_w8_r2");
+        // (below 8192 columns where sixteen waves are busy with it: 10 x 4448 x 6720 7.26 -> 6.14 us, 5 x 7584 x 6304 7.32 -> 6.97; on a K
+        // of 4096 to 6144 0.89 .. 1.03, and to 2048 columns, a few workgroups of either kernel, 1.05 .. 1.12)
+        if (k <= 8192 && (n >= 8192 || (n > 4096 && k >= 6144))) return pick("p1x1_w16_r2k2");
+        // A very long K: every workgroup re-reads A over all of it; 32 columns per workgroup
+        // halve that (16 x 8192 x 28672 19.1 us against 21.7), as long as 16 columns make more than one round
+        // of workgroups (13 x 1216 x 20448 16.3 -> 11.1, 10 x 4000 x 16480 13.5 -> 9.6 on 16) and 32 not
+        // little more than one (12 x 9120 x 21152 33.7 -> 30.4).
+        if (k > 16384) return pick(n <= 4096 || (n > 8192 && n <= 12288) ? "d1x1_w16_r1" : "d1x2_w8_r2");
         return pick("d1x1_w16_r1");
     }
     if (m <= 32) {
         // tens of thousands of columns on a long K: one wave per workgroup, thousands of them
         // (32 x 57344 x 8192 39.9 us against 49.2 on eight waves)
         if (k > 4096 && n >= 32768) return pick("d2x2_w1_r1");
-        if (k <= 2048) return pick("p2x1_w16_r2k1");
-        // few column blocks and a long K: two blocks of 16 rows each double the workgroups
-        if (n <= 2048) return pick("d1x1_w16_r1");
-        if (k <= 4096) return pick("p2x1_w8_r2k2");
+        // few column blocks: two blocks of 16 rows each double the workgroups (from a K of 2048 on; on 1024 to 2048 22 x 1792 x
+        // 2016 3.21 -> 2.82 us, 0.86 .. 0.95 over 50 sizes)
+        if (n <= 2048 && k >= 1024) return pick("d1x1_w16_r1");
+        if (k <= 2048) {
+            // (16 rows x 32 columns in as many workgroups as 32 x 16: 23 x 3232 x 1440 3.22 -> 2.84 us, 0.87 .. 1.00 over 26 sizes)
+            return pick(n <= 4096 && k >= 1024 && k < 2048 ? "d1x2_w8_r2" : "p2x1_w16_r2k1");
+        }
+        // Many columns: sixteen waves with one run of K each instead of eight with two, either one workgroup per CU:
+        // twice the bytes of B on their way.  23 x 54624 x 2464 18.7 -> 16.6 us, 0.85 .. 1.01 over 46 sizes; near the whole K of 4096 0.98 .. 1.05.
+        if (k <= 4096) return pick(n > 16384 && k <= 3584 ? "p2x1_w16_r2k1" : "p2x1_w8_r2k2");
+        // One round of wider blocks that fills the device, where 32 columns start a second one.  48 columns, a third block of
+        // rows idle: 32 x 10240 x 8192 12.9 -> 10.9 us, 0.72 .. 0.90 over 55 sizes; 64 columns: 28 x 13920 x 7680 13.0 -> 12.1, 0.87 .. 1.00
+        // over 40.
+        {
+            const int c32 = (n + 31) / 32, c48 = (n + 47) / 48, c64 = (n + 63) / 64;
+            if (c32 > 256 && c48 <= 256) return pick("d3x3_w8_r1");
+            if (c48 > 256 && c64 <= 256) return pick("d2x4_w8_r1");
+        }
         // a long K: every workgroup re-reads the rows of A it owns over all of K; 32 columns
         // per workgroup halve that against 16
         return pick(n <= 4096 ? "d2x1_w16_r1" : "d2x2_w8_r1");
@@ -351,12 +369,16 @@ static Choice heuristic(int m, int n, int k, int ptr_align, bool has_ws)
             // blocks of 64 leave up to half of it idle and blocks of 32 start a second one.  Time against the choice below, B
             // from HBM, K = 1024 .. 32768 (geometric mean, worst shape): 48 x 32 0.93, 0.99; 48 x 48 0.83, 0.98 (48 x 11008 x
             // 4096 9.0 -> 7.3 us); 48 x 64 0.93, 0.99; 64 x 48 0.89, 0.99 (64 x 9600 x 4096 8.9 -> 8.0 us).  On a K of 1024
-            // 64 x 48 is 1 % behind (63 x 8230), beyond 224 workgroups up to 6 %; 48 x 64 on all 256 CUs gains 2 %: not taken.
+            // 64 x 48 is 1 % behind (63 x 8230), beyond 224 workgroups up to 6 % from 60 rows on
+            // (below that 0.88 .. 0.95); 48 x 64 on all 256 CUs gains 2 %: not taken.
             if (m <= 48) {
                 if (c32 >= 140 && c32 <= 256) return pick("d3x2_w8_r1");
                 if (c32 > 256 && c48 <= 256) return pick("d3x3_w8_r1");
                 if (c48 > 256 && c64 < 256) return pick("d3x4_w8_r1");
-            } else if (k >= 2048 && c32 > 256 && c48 <= 224) {
+                // (48 columns also into a second round, to 1.8 of them: 37 x 22016 x 4096 14.0 -> 12.8 us, 0.87 .. 1.01 over 14 sizes;
+                // beyond 1.10 .. 1.23)
+                if (k >= 2048 && c64 > 256 && n <= 22528) return pick("d3x3_w8_r1");
+            } else if (k >= 2048 && c32 > 256 && (c48 <= 224 || (c48 <= 256 && m < 60))) {
                 return pick("d4x3_w8_r1");
             }
             if (c64 >= 140 && c64 <= 256) return pick("d4x4_w8_r1");
@@ -414,7 +436,10 @@ static Choice select_config(int m, int n, int k, int ptr_align, bool has_ws)
 // heuristic says for skinny shapes, else the generic kernel.
 static Choice select_scaled(int m, int n, int k, int ptr_align, bool has_ws)
 {
-    const Choice ch = select_config(m, n, k, ptr_align, has_ws);
+    Choice ch = select_config(m, n, k, ptr_align, has_ws);
+    // (The persistent kernel of 17 to 32 rows on many columns: a block's epilogue takes longer with scales, and sixteen
+    // waves are ahead through a K of 4096: linear layer of 26 x 22016 x 4096, its quantisation included, 14.4 -> 13.1 us, 0.91 .. 0.96 over 24 sizes.)
+    if (m > 16 && m <= 32 && n > 20480 && k > 3584 && k <= 4096 && ch.cfg == find_config("p2x1_w8_r2k2")) ch.cfg = find_config("p2x1_w16_r2k1");
     if (ch.ksplit <= 1 && scaled_launcher(ch.cfg)) return ch;
     // K split: the int32 kernel of any pipelined configuration leaves partial sums in the
     // workspace, and the kernel that adds them up scales and rounds
