@@ -56,21 +56,29 @@ static hipError_t launch_dot(const GemmArgs &p, hipStream_t stream, int opt)
 template <class Cfg>
 static hipError_t launch_skinny_dma(const GemmArgs &p, hipStream_t stream, int opt)
 {
-    static std::atomic<bool> lds_ok[QM_MAX_DEVICES] = {};
-    const hipError_t e = ensure_dynamic_lds(&gemm_skinny_dma_kernel<Cfg>, Cfg::LDS_BYTES, lds_ok);
-    if (e != hipSuccess) return e;
-    if (opt & QM_OPT_PREPARE) return hipSuccess;
+    static std::atomic<bool> lds_ok[2][QM_MAX_DEVICES] = {};
+    const bool prepare = (opt & QM_OPT_PREPARE) != 0, round = skinny_dma_goes_round(p.M, p.N, p.K);
+    const auto kernel = round ? &gemm_skinny_dma_kernel<Cfg, true> : &gemm_skinny_dma_kernel<Cfg, false>;
+    hipError_t e = ensure_dynamic_lds(kernel, Cfg::LDS_BYTES, lds_ok[round]);
+    if (e == hipSuccess && prepare) e = ensure_dynamic_lds(round ? &gemm_skinny_dma_kernel<Cfg, false> : &gemm_skinny_dma_kernel<Cfg, true>, Cfg::LDS_BYTES, lds_ok[!round]);
+    if (e != hipSuccess || prepare) return e;
     const int blocks = (p.N + Cfg::BN - 1) / Cfg::BN, row_blocks = (p.M + Cfg::MAX_M - 1) / Cfg::MAX_M;
     if (row_blocks > 65535) return hipErrorInvalidValue;
-    static_assert(kernarg_bytes(&gemm_skinny_dma_kernel<Cfg>) <= 64, "see pack_rows_out");
-    return enqueue(&gemm_skinny_dma_kernel<Cfg>, dim3(skinny_dma_columns(blocks, row_blocks), row_blocks), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream,
+    static_assert(kernarg_bytes(&gemm_skinny_dma_kernel<Cfg, true>) <= 64, "see pack_rows_out");
+    return enqueue(kernel, dim3(skinny_dma_columns(blocks, row_blocks), row_blocks), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream,
         p.A, p.B, p.C, pack_rows_out(p.M, p.out), p.N, p.K, p.ldc, p.row_scale, p.col_scale, p.bias);
 }
 template <class Cfg>
 static hipError_t launch_skinny_stream_dma(const GemmArgs &p, hipStream_t stream, int opt)
 {
-    static std::atomic<bool> lds_ok[QM_MAX_DEVICES] = {};
-    hipError_t e = ensure_dynamic_lds(&gemm_skinny_stream_dma_kernel<Cfg>, Cfg::LDS_BYTES, lds_ok);
+    // (rows of 4096 bytes fit the waves of some only)
+    constexpr bool CAN_ROUND = Cfg::MAX_K >= 8192;
+    static std::atomic<bool> lds_ok[2][QM_MAX_DEVICES] = {};
+    const bool round = CAN_ROUND && skinny_dma_goes_round(p.M, p.N, p.K);
+    const auto kernel = round ? &gemm_skinny_stream_dma_kernel<Cfg, CAN_ROUND> : &gemm_skinny_stream_dma_kernel<Cfg, false>;
+    hipError_t e = ensure_dynamic_lds(kernel, Cfg::LDS_BYTES, lds_ok[round]);
+    if (e == hipSuccess && CAN_ROUND && (opt & QM_OPT_PREPARE))
+        e = ensure_dynamic_lds(round ? &gemm_skinny_stream_dma_kernel<Cfg, false> : &gemm_skinny_stream_dma_kernel<Cfg, CAN_ROUND>, Cfg::LDS_BYTES, lds_ok[!round]);
     if (e != hipSuccess) return e;
     int cus = 0;
     e = device_cus(&cus);
@@ -79,8 +87,8 @@ static hipError_t launch_skinny_stream_dma(const GemmArgs &p, hipStream_t stream
     const int blocks = (p.N + Cfg::BN - 1) / Cfg::BN;
     const int resident = cus * (160 * 1024 / Cfg::LDS_BYTES);  // workgroups the device holds at once (the LDS decides)
     const int grid = blocks < resident ? blocks : resident;
-    static_assert(kernarg_bytes(&gemm_skinny_stream_dma_kernel<Cfg>) <= 64, "see pack_rows_out");
-    return enqueue(&gemm_skinny_stream_dma_kernel<Cfg>, dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream,
+    static_assert(kernarg_bytes(&gemm_skinny_stream_dma_kernel<Cfg, false>) <= 64, "see pack_rows_out");
+    return enqueue(kernel, dim3(grid), dim3(Cfg::THREADS), Cfg::LDS_BYTES, stream,
         p.A, p.B, p.C, p.out | (p.M << 2) | (grid << 8), p.N, p.K, p.ldc, p.row_scale, p.col_scale, p.bias);
 }
 #define QM_SKINNYP(FM, FN, NW, D, R) \

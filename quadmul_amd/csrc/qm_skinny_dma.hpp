@@ -46,6 +46,22 @@
 
 namespace qm {
 
+// Which of its `cnt` runs a wave begins with.  Rows of 4096 bytes or multiples of them have the same columns in the same channels of the
+// L2 and of the memory, and workgroups that begin together want the same columns of all their rows: a
+// kilobyte of eight waves comes from a quarter of the channels.  There the workgroups of an XCD (every eighth) begin at different
+// runs and go round.  us, before -> now, B from HBM: 48 x 8192 x 8192 9.63 -> 8.50, 16 x 4096 x 8192 5.38 -> 4.88, 33 x 8192 x 16384 16.0 -> 13.5, 17 x
+// 6144 x 32768 23.9 -> 17.9; 0.93 in the geometric mean over 114 sizes to 64 rows on a K of 8192 to 57344.  Not taken: rows of other lengths, which
+// their length spreads (1 % slower in the mean, 16 x 4096 x 11008 3.6); few columns, whose workgroups share A while it is there
+// (592 columns 3.5 % slower); many rows, where B's second reader comes too late (380 x 8192 x 16384 2.7 %, 108 x 6144 x 57344 5; to 256
+// rows and 16384 bytes 0.98 in the mean).  (A form of the kernels of its own: the few instructions before the first load are 0.8 % of 37 x 11008 x 4096.)
+inline bool skinny_dma_goes_round(const int m, const int n, const int k) { return k % 8192 == 0 && n >= 2048 && m <= (k > 32768 ? 64 : 256); }
+__device__ __forceinline__ int first_of_runs(const int cnt, const int waves)
+{
+    const int turn = blockIdx.x >> 3;
+    // (one wave's runs are short and many: with sixteen places 32 x 57344 x 8192 39.5 -> 44.7 us, with four 38.8)
+    return waves == 1 ? (turn & 3) * cnt >> 2 : (turn * 5 & 15) * cnt >> 4;
+}
+
 template <int FM_, int FN_, int NW_, int D_>
 struct SkinnyDmaCfg {
     static constexpr int FM = FM_, FN = FN_, NW = NW_, D = D_;  // D: runs in flight per wave (ring depth)
@@ -79,7 +95,7 @@ inline int skinny_dma_columns(int cols, int rows)
     return (per_xcd * rows + 31) / 32 <= ((long long)cols * rows + 255) / 256 ? (int)per_xcd * 8 : cols;
 }
 
-template <class Cfg>
+template <class Cfg, bool ROUND>
 __global__ void __launch_bounds__(Cfg::THREADS)
 gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int rows_out, const int N, const int K, const int ldc,
                        const float *row_scale, const float *col_scale, const uint16_t *bias)
@@ -110,6 +126,8 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
     const int nruns = (Kb + 127) >> 7;   // 128-byte runs per row, the last one possibly short
     // this wave's runs: wave, wave + NW, ...
     const int cnt = wave < nruns ? (nruns - wave + NW - 1) / NW : 0;
+    const int first_run = ROUND ? wave + first_of_runs(cnt, NW) * NW : wave;
+    const auto run_after = [&](const int run) __attribute__((always_inline)) { return !ROUND || run + NW < nruns ? run + NW : wave; };
 
     // ---- global side of a load: lane -> row l / 8 of the 8 rows, position l % 8 in the line.
     // Half h of a block holds its rows 8 h .. 8 h + 7; the piece fetched is the logical one
@@ -146,9 +164,13 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
     };
 
     // ---- all loads the ring holds go out first ----
+    int load_run = first_run;
 #pragma unroll
     for (int d = 0; d < D; ++d)
-        if (d < cnt) issue_run(wave + d * NW, d);
+        if (d < cnt) {
+            issue_run(load_run, d);
+            load_run = run_after(load_run);
+        }
 
     // (the sums start from zero; cleared while the loads are in flight, and the barrier comes
     // while every wave is still waiting for its data anyway)
@@ -174,8 +196,8 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
         else if (younger == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPR + extra > 63 ? 63 : 2 * LPR + extra) : "memory");
         else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * LPR + extra > 63 ? 63 : 3 * LPR + extra) : "memory");
     };
-    for (int it = 0; it < cnt; ++it) {
-        const int run = wave + it * NW, slot = it % D;
+    for (int it = 0, run = first_run; it < cnt; ++it, run = run_after(run)) {
+        const int slot = it % D;
         const uint8_t *const at = smem + wave * D * Cfg::SLOT_BYTES + slot * Cfg::SLOT_BYTES;
         // the loads of this run have landed when at most those of the younger runs are in
         // flight.  A's were issued first and come from the L2s: its fragments are read and
@@ -202,7 +224,8 @@ gemm_skinny_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int
         if (it + D < cnt) {
             // the slot is free once its fragments are in registers: refill it
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            issue_run(run + D * NW, slot);
+            issue_run(load_run, slot);
+            load_run = run_after(load_run);
         }
         // a short last run: pieces past the end of K hold bytes that belong to other pieces
         if (run == nruns - 1 && (Kb & 127) != 0) {
@@ -317,7 +340,7 @@ struct SkinnyStreamCfg {
 // into SGPRs before the first wave starts -- the library is built with
 // -amdgpu-kernarg-preload-count=16 -- where a structure is fetched by the waves themselves;
 // measured 1.5 % at M = 16, N = K = 4096 with B from HBM.)
-template <class Cfg>
+template <class Cfg, bool ROUND>
 __global__ void __launch_bounds__(Cfg::THREADS)
 gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int grid_rows_out, const int N, const int K, const int ldc,
                               const float *row_scale, const float *col_scale, const uint16_t *bias)  // 16 dwords: all preloaded
@@ -343,6 +366,9 @@ gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, co
     const int Kb = p.K >> 1;
     const int nruns = (Kb + 127) >> 7;
     const int cnt = wave < nruns ? (nruns - wave + NW - 1) / NW : 0;  // this wave's runs: wave, wave + NW, ... (at most R)
+    // (ROUND: see first_of_runs.  The fragments of A are held in the order of the runs, so that is turned round)
+    const bool back = ROUND && first_of_runs(2, NW) != 0;
+    const int first_run = back ? wave + (cnt - 1) * NW : wave, next_run = back ? -NW : NW;
     // (set after A's loads are on their way: the number of blocks takes a division)
     int G, my_blocks, units;
 
@@ -358,7 +384,7 @@ gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, co
     const uint32_t ring_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * D * Cfg::UNIT_BYTES);
     int ld_u = 0, ld_blk = blockIdx.x, ld_run = 0;
     auto issue_unit = [&]() __attribute__((always_inline)) {
-        const int slot = ld_u % D, run = wave + ld_run * NW, n0 = ld_blk * Cfg::BN;
+        const int slot = ld_u % D, run = first_run + ld_run * next_run, n0 = ld_blk * Cfg::BN;
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
@@ -384,7 +410,7 @@ gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, co
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const uint32_t dst = a_lds + (q * FM + i) * 2048 + h * 1024;
-                    const uint32_t goff = row_bytes24(min(i * 16 + 8 * h + row8, p.M - 1), Kb) + min((uint32_t)(wave + q * NW) * 128u + piece_off[h], last16);
+                    const uint32_t goff = row_bytes24(min(i * 16 + 8 * h + row8, p.M - 1), Kb) + min((uint32_t)(first_run + q * next_run) * 128u + piece_off[h], last16);
                     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(goff), "s"(p.A) : "memory", "m0");
                 }
         }
@@ -439,7 +465,7 @@ gemm_skinny_stream_dma_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, co
 #pragma unroll
         for (int q = 0; q < R; ++q) {
             if (q < cnt) {
-                const int slot = u % D, run = wave + q * NW;
+                const int slot = u % D, run = first_run + q * next_run;
                 wait_b(min(D - 1, units - 1 - u));
                 const uint8_t *const at = smem + (wave * D + slot) * Cfg::UNIT_BYTES;
                 v4i bpk[FN][2];
