@@ -48,8 +48,10 @@ static hipError_t launch_dot(const GemmArgs &p, hipStream_t stream, int opt)
 {
     if (opt & QM_OPT_PREPARE) return hipSuccess;
     const int blocks = (p.N + Cfg::BN - 1) / Cfg::BN;
-    static_assert(kernarg_bytes(&gemm_dot_kernel<Cfg>) <= 64, "see pack_rows_out");
-    return enqueue(&gemm_dot_kernel<Cfg>, dim3(blocks), dim3(Cfg::THREADS), 0, stream, p.A, p.B, p.C, pack_rows_out(p.M, p.out), p.N, p.K, p.ldc, p.row_scale, p.col_scale, p.bias);
+    static_assert(8192 / 128 % (Cfg::NW * Cfg::U) == 0, "rows that go round are whole turns");
+    const auto kernel = goes_round(p.M, p.N, p.K) ? &gemm_dot_kernel<Cfg, true> : &gemm_dot_kernel<Cfg, false>;
+    static_assert(kernarg_bytes(&gemm_dot_kernel<Cfg, false>) <= 64, "see pack_rows_out");
+    return enqueue(kernel, dim3(blocks), dim3(Cfg::THREADS), 0, stream, p.A, p.B, p.C, pack_rows_out(p.M, p.out), p.N, p.K, p.ldc, p.row_scale, p.col_scale, p.bias);
 }
 #define QM_DOT(MR, FN, NW, U) \
     hipError_t QM_DOT_FN(MR, FN, NW, U)(const GemmArgs &p, hipStream_t s, int gm) { return launch_dot<DotCfg<MR, FN, NW, U>>(p, s, gm); }
@@ -57,7 +59,7 @@ template <class Cfg>
 static hipError_t launch_skinny_dma(const GemmArgs &p, hipStream_t stream, int opt)
 {
     static std::atomic<bool> lds_ok[2][QM_MAX_DEVICES] = {};
-    const bool prepare = (opt & QM_OPT_PREPARE) != 0, round = skinny_dma_goes_round(p.M, p.N, p.K);
+    const bool prepare = (opt & QM_OPT_PREPARE) != 0, round = goes_round(p.M, p.N, p.K);
     const auto kernel = round ? &gemm_skinny_dma_kernel<Cfg, true> : &gemm_skinny_dma_kernel<Cfg, false>;
     hipError_t e = ensure_dynamic_lds(kernel, Cfg::LDS_BYTES, lds_ok[round]);
     if (e == hipSuccess && prepare) e = ensure_dynamic_lds(round ? &gemm_skinny_dma_kernel<Cfg, false> : &gemm_skinny_dma_kernel<Cfg, true>, Cfg::LDS_BYTES, lds_ok[!round]);
@@ -74,7 +76,7 @@ static hipError_t launch_skinny_stream_dma(const GemmArgs &p, hipStream_t stream
     // (rows of 4096 bytes fit the waves of some only)
     constexpr bool CAN_ROUND = Cfg::MAX_K >= 8192;
     static std::atomic<bool> lds_ok[2][QM_MAX_DEVICES] = {};
-    const bool round = CAN_ROUND && skinny_dma_goes_round(p.M, p.N, p.K);
+    const bool round = CAN_ROUND && goes_round(p.M, p.N, p.K);
     const auto kernel = round ? &gemm_skinny_stream_dma_kernel<Cfg, CAN_ROUND> : &gemm_skinny_stream_dma_kernel<Cfg, false>;
     hipError_t e = ensure_dynamic_lds(kernel, Cfg::LDS_BYTES, lds_ok[round]);
     if (e == hipSuccess && CAN_ROUND && (opt & QM_OPT_PREPARE))

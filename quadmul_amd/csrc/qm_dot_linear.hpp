@@ -43,7 +43,7 @@ inline bool dot_linear_pays(int m, int n, int k, int in)
     return n <= (k > 2048 ? 65536 : 24576);
 }
 
-template <int IN, class Cfg>
+template <int IN, class Cfg, bool ROUND>
 __global__ void __launch_bounds__(Cfg::THREADS)
 dot_linear_kernel(const uint8_t *x, const uint8_t *B, int32_t *D, const int rows_out, const int N, const int K, const float *col_scale, const uint16_t *bias)
 {
@@ -82,7 +82,10 @@ dot_linear_kernel(const uint8_t *x, const uint8_t *B, int32_t *D, const int rows
             for (int h = 0; h < 2; ++h) bq[pu][h] = ok ? __builtin_nontemporal_load(reinterpret_cast<const v4i *>(p.B + b_off[h] + kofs)) : v4i{0, 0, 0, 0};
         }
     };
-    load_b(wave * U);
+    // (ROUND: as in gemm_dot_kernel; us in a graph, before -> now: 1 x 4096 x 8192 6.59 -> 6.35, 2 x 4096 x 8192 7.48 -> 6.87, 1 x 8192 x 8192
+    // fp16 8.68 -> 8.00)
+    const int first = ROUND ? wave * U + first_of_runs(nchunks / (NW * U), NW) * NW * U : wave * U;
+    load_b(first);
     __builtin_amdgcn_sched_barrier(0);
 
     float scale[MR];
@@ -124,8 +127,9 @@ dot_linear_kernel(const uint8_t *x, const uint8_t *B, int32_t *D, const int rows
     int32_t acc[MR][2];
 #pragma unroll
     for (int i = 0; i < MR; ++i) acc[i][0] = acc[i][1] = 0;
-    for (int c0 = wave * U; c0 < nchunks; c0 += NW * U) {
-        if (c0 != wave * U) load_b(c0);
+    for (int part = 0; part < (ROUND ? 2 : 1); ++part)
+    for (int c0 = part == 0 ? first : wave * U; c0 < (part == 0 ? nchunks : first); c0 += NW * U) {
+        if (c0 != first) load_b(c0);
 #pragma unroll
         for (int pu = 0; pu < U / 2; ++pu) {
             const int kofs = (c0 + 2 * pu) * 64 + ld_ch * 16;
@@ -166,7 +170,10 @@ template <int IN, int MR, int NW, int U>
 static hipError_t launch_dot_linear(const void *x, const void *B, void *D, int m, int n, int k, const float *col_scale, const uint16_t *bias, int out, hipStream_t s)
 {
     using Cfg = DotLinearCfg<IN, MR, NW, U>;
-    return enqueue(&dot_linear_kernel<IN, Cfg>, dim3((n + Cfg::BN - 1) / Cfg::BN), dim3(Cfg::THREADS), dot_linear_lds_bytes(MR, k), s,
+    // (the rows that go round are longer than those of the others)
+    constexpr bool CAN_ROUND = NW == 16;
+    static_assert(8192 / 128 % (NW * U) == 0, "whole turns");
+    return enqueue(CAN_ROUND && goes_round(m, n, k) ? &dot_linear_kernel<IN, Cfg, CAN_ROUND> : &dot_linear_kernel<IN, Cfg, false>, dim3((n + Cfg::BN - 1) / Cfg::BN), dim3(Cfg::THREADS), dot_linear_lds_bytes(MR, k), s,
         static_cast<const uint8_t *>(x), static_cast<const uint8_t *>(B), static_cast<int32_t *>(D), pack_rows_out(m, out), n, k, col_scale, bias);
 }
 template <int IN>

@@ -339,7 +339,7 @@ struct DotCfg {
     static constexpr int MAX_M = MR, BN = 16 * FN;
 };
 
-template <class Cfg>
+template <class Cfg, bool ROUND>
 __global__ void __launch_bounds__(Cfg::THREADS)
 gemm_dot_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int rows_out, const int N, const int K, const int ldc,
                        const float *row_scale, const float *col_scale, const uint16_t *bias)
@@ -375,7 +375,11 @@ gemm_dot_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int rows_o
     for (int i = 0; i < MR; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j][0] = acc[i][j][1] = 0;
-    for (int c0 = wave * U; c0 < nchunks; c0 += NW * U) {
+    // ROUND: from a turn of the workgroup's own on and round to it, see goes_round; K is a multiple of all waves' chunks.
+    // us, before -> now, B from HBM: 1 x 4096 x 8192 4.81 -> 4.48, 2 x 4096 x 8192 5.18 -> 4.57, 1 x 28672 x 16384 36.4 -> 34.4, 1 x 4096 x 32768 15.7 -> 13.3.
+    const int first = ROUND ? wave * U + first_of_runs(nchunks / (NW * U), NW) * NW * U : wave * U;
+    for (int part = 0; part < (ROUND ? 2 : 1); ++part)
+    for (int c0 = part == 0 ? first : wave * U; c0 < (part == 0 ? nchunks : first); c0 += NW * U) {
         v4i bq[U / 2][FN][2], aq[U / 2][MR];
 #pragma unroll
         for (int pu = 0; pu < U / 2; ++pu) {
