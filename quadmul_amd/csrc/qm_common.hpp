@@ -284,7 +284,7 @@ __device__ __forceinline__ int xcd_contiguous_id(int bid, int nblocks)
 // kilobyte of eight waves comes from a quarter of the channels.  There the workgroups of an XCD (every eighth) begin at different
 // runs and go round.  us, before -> now, B from HBM: 48 x 8192 x 8192 9.63 -> 8.50, 16 x 4096 x 8192 5.38 -> 4.88, 33 x 8192 x 16384 16.0 -> 13.5, 17 x
 // 6144 x 32768 23.9 -> 17.9; 0.93 in the geometric mean over 114 sizes to 64 rows on a K of 8192 to 57344.  Not taken: rows of other lengths, which
-// their length spreads (1 % slower in the mean, 16 x 4096 x 11008 3.6); few columns, whose workgroups share A while it is there
+// their length spreads (1 % slower in the mean, 16 x 4096 x 11008 3.6), odd multiples of 2048 bytes among them (1.004 over 24 sizes); few columns, whose workgroups share A while it is there
 // (592 columns 3.5 % slower); many rows, where B's second reader comes too late (380 x 8192 x 16384 2.7 %, 108 x 6144 x 57344 5; to 256
 // rows and 16384 bytes 0.98 in the mean).  (A form of the kernels of its own: the few instructions before the first load are 0.8 % of 37 x 11008 x 4096.)
 inline bool goes_round(const int m, const int n, const int k) { return k % 8192 == 0 && n >= 2048 && m <= (k > 32768 ? 64 : 256); }
