@@ -66,8 +66,13 @@ class W4A4Linear(torch.nn.Module):
             if out_dtype not in (torch.float16, torch.bfloat16):
                 raise QuadmulError("W4A4Linear: out_dtype must be float16 or bfloat16")
             # (out of the dictionary: an attribute that is a buffer is found after everything else has been looked through, 0.28 us each of the
-            # 6.2 of a small call.  One that is no buffer any more -- replaced by a parameter, parametrized -- is looked up as ever)
-            held = self._buffers
+            # 6.2 of a small call.  Only where nothing would be found ahead of it -- not in a subclass, nor with an attribute of that
+            # name beside the buffer, on the layer or on the class.  One that is no buffer any more -- replaced by a parameter,
+            # parametrized -- is looked up as ever)
+            own = self.__dict__
+            shadowed = (type(self) is not W4A4Linear or "weight_packed" in own or "weight_scale" in own or "bias" in own
+                        or "weight_packed" in _CLASS or "weight_scale" in _CLASS or "bias" in _CLASS)
+            held = {} if shadowed else own["_buffers"]
             try:
                 weight, weight_scale, bias = held["weight_packed"], held["weight_scale"], held["bias"]
             except KeyError:
@@ -90,3 +95,6 @@ class W4A4Linear(torch.nn.Module):
 
     def extra_repr(self) -> str:
         return f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, out_dtype={self.out_dtype}"
+
+
+_CLASS = W4A4Linear.__dict__  # (as it is at the time of a call)

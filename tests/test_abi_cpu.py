@@ -403,3 +403,36 @@ def test_bias_that_the_kernel_cannot_read_as_it_is_is_added_apart():
     assert _fusable(b, x, torch.float16, 4) and _fusable(torch.nn.Parameter(b, requires_grad=False), x, torch.float16, 4)
     for other in (torch._neg_view(b), b.to_sparse(), b.float(), b[:3], torch.zeros(8, dtype=torch.float16)[::2], b.reshape(1, 4), torch.nn.Parameter(b)):
         assert not _fusable(other, x, torch.float16, 4)
+
+
+def test_linear_layer_reads_what_shadows_a_buffer(monkeypatch):
+    """Weight, scales and bias are found as attributes are: one set beside a buffer that is still registered, on the layer, on a
+    subclass or on the class itself, comes before the buffer."""
+    from quadmul_amd import linear
+
+    n, k = 4, 8
+    w, ws, b, other = torch.zeros(n, k // 2, dtype=torch.int8), torch.ones(n), torch.zeros(n, dtype=torch.float16), torch.ones(n, dtype=torch.float16)
+    called = []
+    monkeypatch.setattr(linear, "_native", lambda name, x, weight, rows, scale, bias, bf16: called.append((weight, scale, bias)) or torch.zeros(x.shape[0], rows, dtype=torch.float16))
+
+    def used(layer):
+        layer(torch.zeros(2, k, dtype=torch.float16))
+        return called.pop()
+
+    names = ("weight_packed", "weight_scale", "bias")
+    plain = linear.W4A4Linear(w, ws, b)
+    assert all(got is plain._buffers[name] for got, name in zip(used(plain), names))
+    for i, (name, value) in enumerate(zip(names, (w + 1, ws * 2, other))):
+        layer = linear.W4A4Linear(w, ws, b)
+        layer.__dict__[name] = value
+        assert used(layer)[i] is value and name in layer._buffers, name
+        derived = linear.W4A4Linear(w, ws, b)
+        derived.__class__ = type("Derived", (linear.W4A4Linear,), {name: property(lambda self: value)})
+        assert used(derived)[i] is value and name in derived._buffers, name
+        with monkeypatch.context() as patch:
+            patch.setattr(linear.W4A4Linear, name, property(lambda self: value), raising=False)
+            assert used(plain)[i] is value, name
+        assert used(plain)[i] is plain._buffers[name], name
+    layer = linear.W4A4Linear(w, ws, b)
+    layer.__dict__["bias"] = None
+    assert used(layer)[2] is None
