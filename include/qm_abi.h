@@ -239,6 +239,8 @@ int qm_quantize_pack_i4(const void *x, int in_dtype, void *dst_packed, float *sc
  *   workspace    device memory, 256-byte aligned, at least qm_linear_workspace_bytes(...) bytes (weight_align: the
  *                alignment of B in bytes), else QM_ERR_SCRATCH and nothing is enqueued; used in stream order by
  *                the kernels of this call only
+ *   D            may overlap x (a square layer in place).  A call of one launch then is two, with a workspace of 4 m and m k / 2
+ *                bytes, each rounded up to 256; with less, QM_ERR_SCRATCH
  */
 size_t qm_linear_workspace_bytes(int m, int n, int k, int in_dtype, int weight_align);
 int qm_linear_i4(const void *x, int in_dtype, const void *B, void *D, int m, int n, int k, const float *col_scale,

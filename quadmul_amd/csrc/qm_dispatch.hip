@@ -834,11 +834,12 @@ struct LinearPlan {
     size_t scale_bytes, row_bytes, gemm_bytes;
     size_t bytes() const { return scale_bytes + row_bytes + gemm_bytes; }
 };
-LinearPlan linear_plan(int m, int n, int k, int in_dtype, int weight_align)
+// `apart`: D does not overlap x.  In one launch some workgroups write D while others still read x; in two x is read before.
+LinearPlan linear_plan(int m, int n, int k, int in_dtype, int weight_align, bool apart = true)
 {
     const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     LinearPlan pl{};
-    if (m <= 16 && fast_path_ok(m, n, k, weight_align) && n < (1 << 24) && (m <= 2 ? dot_linear_pays(m, n, k, in_dtype) : skinny_linear_pays(m, n, k, in_dtype))) {
+    if (apart && m <= 16 && fast_path_ok(m, n, k, weight_align) && n < (1 << 24) && (m <= 2 ? dot_linear_pays(m, n, k, in_dtype) : skinny_linear_pays(m, n, k, in_dtype))) {
         pl.one_launch = true;
         return pl;
     }
@@ -877,7 +878,8 @@ QM_EXPORT int qm_linear_i4(const void *x, int in_dtype, const void *B, void *D, 
     const int out = out_dtype == QM_OUT_F16 ? OUT_F16 : OUT_BF16;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (k == 0) return run_gemm(nullptr, nullptr, D, m, n, 0, nullptr, col_scale, out, s, QM_CFG_AUTO, nullptr, 0, 0, static_cast<const uint16_t *>(bias));
-    const LinearPlan pl = linear_plan(m, n, k, in_dtype, ptr_alignment(B, nullptr));
+    const uintptr_t x0 = (uintptr_t)x, x1 = x0 + (uintptr_t)m * k * (in_dtype == QM_IN_F32 ? 4 : 2), d0 = (uintptr_t)D, d1 = d0 + (uintptr_t)m * n * 2;
+    const LinearPlan pl = linear_plan(m, n, k, in_dtype, ptr_alignment(B, nullptr), x1 <= d0 || d1 <= x0);
     if (pl.one_launch) {
         const uint16_t *b16 = static_cast<const uint16_t *>(bias);
         const auto launch = [&](auto in) {

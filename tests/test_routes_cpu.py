@@ -64,3 +64,15 @@ def block(m, n, k):
 def test_blocks_between_32_and_96_rows_on_a_very_long_k(m, n, k, between):
     got = block(m, n, k)
     assert (got is not None and got[0] > 32 and (got[0] % 64 != 0 or got[1] == 48)) == between
+
+
+@pytest.mark.parametrize("m,k,dtype,esz", [(1, 4096, F16, 2), (2, 2048, BF16, 2), (2, 2048, F32, 4), (4, 4096, F16, 2), (8, 4096, BF16, 2), (16, 2048, F16, 2)], ids=str)
+def test_a_layer_that_overwrites_its_rows_is_never_one_launch(m, k, dtype, esz):
+    """One launch reads x while it writes D.  (Without the workspace of two launches such a call is refused, whatever part of x it is that D overlaps;
+    nothing is enqueued.)"""
+    assert one_launch(m, k, k, dtype)
+    lib, x, size, out = qm.library(), 1 << 30, m * k * esz, 2 * m * k
+    call = lambda d, ws, ws_bytes: lib.qm_linear_i4(x, dtype, 2 << 30, d, m, k, k, None, None, 1, None, ws, ws_bytes)
+    need = (4 * m + 255) // 256 * 256 + (m * k // 2 + 255) // 256 * 256
+    for d in (x, x + 2, x + size - 2, x - out + 2):
+        assert call(d, None, 0) == -7 and call(d, 3 << 30, need - 1) == -7, hex(d)

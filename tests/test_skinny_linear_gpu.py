@@ -67,3 +67,18 @@ def test_captured_and_replayed():
         got, want = both(x, w, n, ws, torch.float16, None)
         assert torch.equal(y.view(torch.int16), want) and torch.equal(got, want), i
 
+
+@pytest.mark.parametrize("m,k,shift", [(1, 4096, 0), (2, 2048, 0), (4, 4096, 0), (4, 4096, 2048), (8, 4096, -2048), (16, 2048, 0)], ids=str)
+def test_in_place(m, k, shift):
+    """The output over the rows, or some of them."""
+    gen = torch.Generator(device=DEV).manual_seed(SEED_BASE + 42900 + m)
+    w, ws = quadmul.quantize_pack(torch.randn(k, k, device=DEV, generator=gen))
+    room = torch.randn(3, m * k, device=DEV, generator=gen).to(torch.float16)
+    x = room.flatten()[m * k:2 * m * k].view(m, k)
+    _, want = both(x, w, k, ws, torch.float16, None)
+    assert one_launch(m, k, k, torch.float16)
+    need = (4 * m + 255) // 256 * 256 + m * k // 2
+    scratch = torch.empty(need, dtype=torch.uint8, device=DEV)
+    d = room.flatten()[m * k + shift:2 * m * k + shift]
+    assert qm.library().qm_linear_i4(x.data_ptr(), 1, w.data_ptr(), d.data_ptr(), m, k, k, ws.data_ptr(), None, 1, torch.cuda.current_stream().cuda_stream, scratch.data_ptr(), need) == 0
+    assert torch.equal(d.view(m, k).view(torch.int16), want)
