@@ -37,7 +37,8 @@ HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    "-Wno-unused-command-line-argument", "-Wno-inline-asm", "-I", os.path.join(ROOT, "include"), "-I", CSRC,
+    # (a reference to a 16-byte vector at an address that is not aligned: the compiler may take it that it is)
+    "-Werror=align-mismatch", "-Wno-unused-command-line-argument", "-Wno-inline-asm", "-I", os.path.join(ROOT, "include"), "-I", CSRC,
 ]
 
 

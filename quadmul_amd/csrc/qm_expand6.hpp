@@ -85,7 +85,8 @@ __global__ void __launch_bounds__(EXPAND6_THREADS) expand_a6_kernel(const Expand
             if (n < (uint32_t)q.N) {
                 const int at = 16 * (int)(piece - n * per_row);
                 // (one load per thread, as it is also where that is four accesses: shifted dwords are no faster here)
-                q.b_copy[piece] = row_value<false>(*reinterpret_cast<const v4i_any_aligned *>(q.B + (n * (uint32_t)Kb + (uint32_t)min(at, Kb - 16))), at, Kb);
+                const v4i w = *reinterpret_cast<const v4i_any_aligned *>(q.B + (n * (uint32_t)Kb + (uint32_t)min(at, Kb - 16)));
+                q.b_copy[piece] = row_value<false>(w, at, Kb);
             }
             return;
         }
