@@ -839,7 +839,7 @@ LinearPlan linear_plan(int m, int n, int k, int in_dtype, int weight_align, bool
 {
     const auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     LinearPlan pl{};
-    if (apart && m <= 16 && fast_path_ok(m, n, k, weight_align) && n < (1 << 24) && (m <= 2 ? dot_linear_pays(m, n, k, in_dtype) : skinny_linear_pays(m, n, k, in_dtype))) {
+    if (apart && m <= 16 && fast_path_ok(m, n, k, weight_align) && n < (1 << 24) && (m <= 2 ? dot_linear_pays(m, n, k, in_dtype) : skinny_linear_fits(m, k, in_dtype) && skinny_linear_pays(m, n, k, in_dtype))) {
         pl.one_launch = true;
         return pl;
     }

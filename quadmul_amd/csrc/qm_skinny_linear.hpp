@@ -203,6 +203,8 @@ template <int IN, int ROWS, int NC, int R, int D>
 static hipError_t launch_skinny_linear(const void *x, const void *B, void *Y, int m, int n, int k, const float *col_scale, const uint16_t *bias, int out, hipStream_t s)
 {
     using Cfg = SkinnyLinearCfg<IN, ROWS, NC, R, D>;
+    // (of a longer row the kernel would leave the rest out, of more rows all but ROWS)
+    if (m > Cfg::ROWS || k > Cfg::MAX_K) return hipErrorInvalidValue;
     hipError_t e = ready_skinny_linear<IN, ROWS, NC, R, D>();
     if (e != hipSuccess) return e;
     int cus = 0;
@@ -229,13 +231,19 @@ static hipError_t ready_skinny_linear()
     }
     return hipSuccess;
 }
+// What the kernels that launch_skinny_linear has can do, whether it pays or not
+constexpr bool skinny_linear_fits(int m, int k, int in)
+{
+    if (in == QM_IN_F32 || m < 1 || m > 16) return false;
+    return k <= (m > 8 ? SkinnyLinearCfg<QM_IN_F16, 16, 4, 1, 3>::MAX_K : m > 4 ? SkinnyLinearCfg<QM_IN_F16, 8, 4, 1, 3>::MAX_K : SkinnyLinearCfg<QM_IN_F16, 4, 4, 2, 3>::MAX_K);
+}
 // Against two launches, in a graph with the weights from HBM, one / two over 75 sizes and both types (us: 4 x 4096 x 4096 5.9 -> 4.5,
 // 8 x 6144 x 4096 7.1 -> 6.2, 16 x 2048 x 2048 5.1 -> 4.7); called eagerly they gain more, the host half of a call:
 //   3, 4 rows    K <= 4096 to 12288 columns 0.73 .. 0.97, beyond 0.90 .. 1.27; K <= 8192 to 4096 0.85 .. 0.94, beyond 0.96 .. 1.11; a longer K 1.03 .. 1.16
 //   5 .. 8       K <= 4096 to 8192 columns 0.79 .. 1.00, beyond 0.96 .. 1.33; a longer K 1.05 .. 1.21
 //   9 .. 16      K <= 2048 to 8192 columns 0.75 .. 0.94, beyond 0.94 .. 1.34; a longer K 0.93 .. 1.18
 // (Below 1024 columns nothing was measured.  fp32 has twice the bytes of x and no shorter arithmetic.)
-inline bool skinny_linear_pays(int m, int n, int k, int in)
+constexpr bool skinny_linear_pays(int m, int n, int k, int in)
 {
     if (in == QM_IN_F32 || m < 3 || m > 16 || n < 1024) return false;
     if (m > 8) return k <= 2048 && n <= 8192;
