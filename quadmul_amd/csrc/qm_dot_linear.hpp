@@ -128,21 +128,21 @@ dot_linear_kernel(const uint8_t *x, const uint8_t *B, int32_t *D, const int rows
 #pragma unroll
     for (int i = 0; i < MR; ++i) acc[i][0] = acc[i][1] = 0;
     for (int part = 0; part < (ROUND ? 2 : 1); ++part)
-    for (int c0 = part == 0 ? first : wave * U; c0 < (part == 0 ? nchunks : first); c0 += NW * U) {
-        if (c0 != first) load_b(c0);
+        for (int c0 = part == 0 ? first : wave * U; c0 < (part == 0 ? nchunks : first); c0 += NW * U) {
+            if (c0 != first) load_b(c0);
 #pragma unroll
-        for (int pu = 0; pu < U / 2; ++pu) {
-            const int kofs = (c0 + 2 * pu) * 64 + ld_ch * 16;
+            for (int pu = 0; pu < U / 2; ++pu) {
+                const int kofs = (c0 + 2 * pu) * 64 + ld_ch * 16;
 #pragma unroll
-            for (int i = 0; i < MR; ++i) {
-                const v4i a = *reinterpret_cast<const v4i *>(rows + i * Kb + min(kofs, Kb - 16));  // (past the row's end B is zero)
+                for (int i = 0; i < MR; ++i) {
+                    const v4i a = *reinterpret_cast<const v4i *>(rows + i * Kb + min(kofs, Kb - 16));  // (past the row's end B is zero)
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
+                    for (int h = 0; h < 2; ++h)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][h] = __builtin_amdgcn_sdot8(a[e], bq[pu][h][e], acc[i][h], false);
+                        for (int e = 0; e < 4; ++e) acc[i][h] = __builtin_amdgcn_sdot8(a[e], bq[pu][h][e], acc[i][h], false);
+                }
             }
         }
-    }
 #pragma unroll
     for (int i = 0; i < MR; ++i)
 #pragma unroll

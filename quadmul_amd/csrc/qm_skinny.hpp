@@ -379,32 +379,32 @@ gemm_dot_kernel(const uint8_t *A, const uint8_t *B, int32_t *C, const int rows_o
     // us, before -> now, B from HBM: 1 x 4096 x 8192 4.81 -> 4.48, 2 x 4096 x 8192 5.18 -> 4.57, 1 x 28672 x 16384 36.4 -> 34.4, 1 x 4096 x 32768 15.7 -> 13.3.
     const int first = ROUND ? wave * U + first_of_runs(nchunks / (NW * U), NW) * NW * U : wave * U;
     for (int part = 0; part < (ROUND ? 2 : 1); ++part)
-    for (int c0 = part == 0 ? first : wave * U; c0 < (part == 0 ? nchunks : first); c0 += NW * U) {
-        v4i bq[U / 2][FN][2], aq[U / 2][MR];
+        for (int c0 = part == 0 ? first : wave * U; c0 < (part == 0 ? nchunks : first); c0 += NW * U) {
+            v4i bq[U / 2][FN][2], aq[U / 2][MR];
 #pragma unroll
-        for (int pu = 0; pu < U / 2; ++pu) {
-            const int kofs = (c0 + 2 * pu) * 64;
-            const bool ok = kofs + ld_ch * 16 < Kb;  // also false for chunks past the last; zeros add nothing
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    bq[pu][j][h] = ok ? __builtin_nontemporal_load(reinterpret_cast<const v4i *>(p.B + b_off[j][h] + kofs)) : v4i{0, 0, 0, 0};
-#pragma unroll
-            for (int i = 0; i < MR; ++i)
-                aq[pu][i] = ok ? *reinterpret_cast<const v4i *>(p.A + a_off[i] + kofs) : v4i{0, 0, 0, 0};
-        }
-#pragma unroll
-        for (int pu = 0; pu < U / 2; ++pu)
-#pragma unroll
-            for (int i = 0; i < MR; ++i)
+            for (int pu = 0; pu < U / 2; ++pu) {
+                const int kofs = (c0 + 2 * pu) * 64;
+                const bool ok = kofs + ld_ch * 16 < Kb;  // also false for chunks past the last; zeros add nothing
 #pragma unroll
                 for (int j = 0; j < FN; ++j)
 #pragma unroll
                     for (int h = 0; h < 2; ++h)
+                        bq[pu][j][h] = ok ? __builtin_nontemporal_load(reinterpret_cast<const v4i *>(p.B + b_off[j][h] + kofs)) : v4i{0, 0, 0, 0};
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[i][j][h] = __builtin_amdgcn_sdot8(aq[pu][i][e], bq[pu][j][h][e], acc[i][j][h], false);
-    }
+                for (int i = 0; i < MR; ++i)
+                    aq[pu][i] = ok ? *reinterpret_cast<const v4i *>(p.A + a_off[i] + kofs) : v4i{0, 0, 0, 0};
+            }
+#pragma unroll
+            for (int pu = 0; pu < U / 2; ++pu)
+#pragma unroll
+                for (int i = 0; i < MR; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[i][j][h] = __builtin_amdgcn_sdot8(aq[pu][i][e], bq[pu][j][h][e], acc[i][j][h], false);
+        }
 
     // the eight lanes of a row hold the eight 32-nibble pieces of a pair of chunks: add them
     // up (within the quads, then the two quads through the mirror image of the eight), then
