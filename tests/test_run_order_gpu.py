@@ -1,4 +1,4 @@
-"""Rows of 4096 bytes and multiples of them, whose workgroups begin at different places of K (first_of_runs in csrc/qm_skinny_dma.hpp): every
+"""Rows of 4096 bytes and multiples of them, whose workgroups begin at different places of K (first_of_runs in csrc/qm_common.hpp): every
 kernel that does so, waves with one, two and many runs, numbers of waves that do and do not divide the runs."""
 import pytest
 import torch
