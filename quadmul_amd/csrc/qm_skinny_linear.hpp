@@ -239,10 +239,10 @@ constexpr bool skinny_linear_fits(int m, int k, int in)
 }
 // Against two launches, in a graph with the weights from HBM, one / two over 75 sizes and both types (us: 4 x 4096 x 4096 5.9 -> 4.5,
 // 8 x 6144 x 4096 7.1 -> 6.2, 16 x 2048 x 2048 5.1 -> 4.7); called eagerly they gain more, the host half of a call:
-//   3, 4 rows    K <= 4096 to 12288 columns 0.73 .. 0.97, beyond 0.90 .. 1.27; K <= 8192 to 4096 0.85 .. 0.94, beyond 0.96 .. 1.11; a longer K 1.03 .. 1.16
-//   5 .. 8       K <= 4096 to 8192 columns 0.79 .. 1.00, beyond 0.96 .. 1.33; a longer K 1.05 .. 1.21
-//   9 .. 16      K <= 2048 to 8192 columns 0.75 .. 0.94, beyond 0.94 .. 1.34; a longer K 0.93 .. 1.18
-// (Below 1024 columns nothing was measured.  fp32 has twice the bytes of x and no shorter arithmetic.)
+//   3, 4 rows    K <= 4096 to 12288 columns 0.73 .. 0.97, beyond 0.90 .. 1.27; K <= 8192 to 4096 0.85 .. 0.94, beyond 0.96 .. 1.11
+//   5 .. 8       K <= 4096 to 8192 columns 0.79 .. 1.00, beyond 0.96 .. 1.33
+//   9 .. 16      K <= 2048 to 8192 columns 0.75 .. 0.94, beyond 0.94 .. 1.34
+// A longer K has no kernel (skinny_linear_fits).  (Below 1024 columns nothing was measured.  fp32 has twice the bytes of x and no shorter arithmetic.)
 constexpr bool skinny_linear_pays(int m, int n, int k, int in)
 {
     if (in == QM_IN_F32 || m < 3 || m > 16 || n < 1024) return false;
