@@ -187,14 +187,14 @@ static RaggedBlock ragged_block(int m, int n)
 //   - here it is the loads: every wave's 16 bytes per lane of the rows of a block go through the L1 of its CU, 0.66 clocks
 //     a lane where rows lie on multiples of four bytes and 1.18 where they do not (a dword more each); up to 0.07 x 5.5
 //     more where they lie within five bytes of a multiple of 128 from row to row, so that the rows of a block
-//     meet in the same banks.  From 40 MB of B on the clocks are those of before, to which the tests of the selection hold such calls.  Rows of a block beyond m are copies of the last one and cost next to nothing.  Workgroups
+//     meet in the same banks.  Rows of a block beyond m are copies of the last one and cost next to nothing.  Workgroups
 //     beyond one per CU count whole rounds;
 //   - on copies, two launches, the rows of both operands read, written and read again, and the GEMM.
 // One or two rows never take the copies, which are as large as the weights and at most a fifth faster there.  Above
 // 512 rows only small products are left here (809 x 708 x 1096 5.2 / 8.6, 939 x 1094 x 1596 17.7 / 12.7), to 1500 rows off the multiples of four, where the
 // rule was measured.  What the loads as they were before, at 1.94 and 0.35 clocks, left to the copies has to be a twentieth below them, an eighth where
 // the fits are furthest off: few blocks on a long K, whose GEMM on the copies is one short round (93 x 799 x 6400 at an odd address 10.3 / 7.9), and several rounds of a few
-// chunks (76 x 16590 x 448 11.2 / 9.7).  Of the 21587, time against that choice of before: 0.797 in the mean where it is another, 21 of those more than 2 % slower (2 more than 10).
+// chunks (76 x 16590 x 448 11.2 / 9.7).  Of the 21587, time against that choice of before: 0.782 in the mean where it is another, 29 of those more than 2 % slower (4 more than 10).
 static bool ragged_before_copies(int m, int n, int k, int ptr_align)
 {
     if (m <= 2) return true;
@@ -211,7 +211,7 @@ static bool ragged_before_copies(int m, int n, int k, int ptr_align)
     const double copies = m <= 64 ? 5.35 + 0.425 * moved + 0.025 * steps + 0.54 * out + 1.9 * mfma : 6.7 + 0.52 * moved + 0.034 * steps + 0.18 * out + 1.66 * mfma;
     const bool small = m <= 512 || (long long)m * n * k < (1LL << 29);
     if (small && here(dwords ? 0.66 : 1.94 + 0.35 * near_line) < copies) return true;
-    if (dwords || m > 1500 || (long long)n * kb >= 40000000) return false;
+    if (dwords || m > 1500) return false;
     const double shifted_copies = m <= 64 ? 5.06 + 0.45 * moved + 0.0242 * steps + 0.656 * out + 1.553 * mfma : 5.41 + 0.4224 * moved + 0.0325 * steps + 0.279 * out + 2.546 * mfma;
     const bool few_long = (long long)((m + 31) / 32) * ((n + 31) / 32) <= 128 && k > 5000, many_short = k <= 640 && rounds >= 2;
     return here(1.18 + 0.072 * near_line) < (few_long || many_short ? 0.87 : 0.95) * shifted_copies;
