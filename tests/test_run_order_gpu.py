@@ -35,3 +35,24 @@ def test_automatic_choice(m, n, k):
     c = poisoned_c(m, n, DEV)
     qm.gemm(pack_cpu(a).to(DEV), pack_cpu(b).to(DEV), c, m, n, k)
     assert torch.equal(c, fp32_matmul_on_gpu(a, b))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=lambda d: str(d)[6:])
+@pytest.mark.parametrize("m,n,k", [(2, 2049, 8192), (16, 2065, 8192), (31, 2050, 16384), (64, 2063, 8192), (100, 2049, 8192)], ids=str)
+def test_scaled_output_with_and_without_a_bias(m, n, k, dtype):
+    a, b = make_operands(m, n, k, SEED_BASE + 45700 + m + n + k)
+    gen = torch.Generator(device=DEV).manual_seed(SEED_BASE + 45800 + m)
+    rs, cs = (torch.rand(r, device=DEV, generator=gen) * 1e-3 + 1e-4 for r in (m, n))
+    bias = torch.randn(n, device=DEV, generator=gen).to(dtype)
+    plain = (fp32_matmul_on_gpu(a, b).float() * rs[:, None] * cs[None]).to(dtype)
+    ap, bp = pack_cpu(a).to(DEV), pack_cpu(b).to(DEV)
+    ran = 0
+    for cfg, name in enumerate(qm.config_names()):
+        if name[0] not in "dpv" or not qm.config_supports(cfg, m, n, k):
+            continue
+        for extra, want in ((None, plain), (bias, plain + bias)):
+            d = torch.full((m, n), float("nan"), dtype=dtype, device=DEV)
+            qm.gemm_scaled(ap, bp, d, m, n, k, rs, cs, cfg, bias=extra)
+            assert torch.equal(d.view(torch.int16), want.view(torch.int16)), (name, extra is None)
+        ran += 1
+    assert ran >= 10
