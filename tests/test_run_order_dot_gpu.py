@@ -11,7 +11,7 @@ from util import SEED_BASE, make_operands, pack_cpu, poisoned_c
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
-SIZES = [(1, 2048, 8192), (2, 2065, 8192), (1, 4099, 16384), (2, 2048, 24576), (1, 2049, 57344)]
+SIZES = [(1, 2048, 8192), (2, 2065, 8192), (1, 4099, 16384), (2, 2048, 24576), (1, 2049, 57344), (1, 2561, 57344), (2, 2579, 8192)]
 
 
 @pytest.mark.parametrize("m,n,k", SIZES, ids=str)
@@ -29,7 +29,7 @@ def test_every_dot_kernel(m, n, k):
     assert ran >= 2
 
 
-@pytest.mark.parametrize("m,n,k", SIZES[:3], ids=str)
+@pytest.mark.parametrize("m,n,k", SIZES[:3] + SIZES[5:], ids=str)
 def test_linear_layer(m, n, k):
     gen = torch.Generator(device=DEV).manual_seed(SEED_BASE + 46500 + k)
     w, ws = quadmul.quantize_pack(torch.randn(n, k, device=DEV, generator=gen))

@@ -13,7 +13,8 @@ DEV = "cuda:0"
 KERNELS = [i for i, name in enumerate(qm.config_names()) if name[0] in "dp"]
 
 
-@pytest.mark.parametrize("m,n,k", [(3, 2048, 8192), (16, 2049, 8192), (17, 2065, 8192), (32, 2048, 16384), (48, 2049, 24576), (64, 2063, 8192), (65, 2048, 16384), (256, 2048, 8192)], ids=str)
+@pytest.mark.parametrize("m,n,k", [(3, 2048, 8192), (16, 2049, 8192), (17, 2065, 8192), (32, 2048, 16384), (48, 2049, 24576), (64, 2063, 8192), (65, 2048, 16384), (256, 2048, 8192),
+                                   (16, 2561, 8192), (17, 3073, 8192), (24, 4097, 16384), (48, 3081, 24576), (64, 3087, 8192), (32, 3077, 49152)], ids=str)
 def test_every_kernel(m, n, k):
     a, b = make_operands(m, n, k, SEED_BASE + 45000 + m + n + k)
     want = fp32_matmul_on_gpu(a, b)
@@ -38,7 +39,7 @@ def test_automatic_choice(m, n, k):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=lambda d: str(d)[6:])
-@pytest.mark.parametrize("m,n,k", [(2, 2049, 8192), (16, 2065, 8192), (31, 2050, 16384), (64, 2063, 8192), (100, 2049, 8192)], ids=str)
+@pytest.mark.parametrize("m,n,k", [(2, 2561, 8192), (16, 2577, 8192), (31, 4098, 16384), (64, 3087, 8192), (100, 3073, 8192)], ids=str)
 def test_scaled_output_with_and_without_a_bias(m, n, k, dtype):
     a, b = make_operands(m, n, k, SEED_BASE + 45700 + m + n + k)
     gen = torch.Generator(device=DEV).manual_seed(SEED_BASE + 45800 + m)
