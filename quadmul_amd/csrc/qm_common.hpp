@@ -283,18 +283,16 @@ __device__ __forceinline__ int xcd_contiguous_id(int bid, int nblocks)
 // L2 and of the memory, and workgroups that begin together want the same columns of all their rows: a
 // kilobyte of eight waves comes from a quarter of the channels.  There the workgroups of an XCD (every eighth) begin at different
 // runs and go round.  us, before -> now, B from HBM: 48 x 8192 x 8192 9.63 -> 8.50, 16 x 4096 x 8192 5.38 -> 4.88, 33 x 8192 x 16384 16.0 -> 13.5, 17 x
-// 6144 x 32768 23.9 -> 17.9; 0.956 in the geometric mean over 11304 sizes to 256 rows on a K of 8192 to 57344, 0.956 too with B in the caches as far as it fits;
-// 56 and 20 of them are more than 2 % slower (5.3 and 3).  Not taken: rows of other lengths, which
+// 6144 x 32768 23.9 -> 17.9; over 7463 sizes to 256 rows on a K of 8192 to 57344 0.956 in the geometric mean, 0.959 with B in the caches as far as it fits,
+// 9 and 39 of them more than 2 % slower (6 and 7).  Not taken: rows of other lengths, which
 // their length spreads (1 % slower in the mean, 16 x 4096 x 11008 3.6), odd multiples of 2048 bytes among them (1.004 over 24 sizes); few columns, whose workgroups share A while it is there
-// (592 columns 3.5 % slower), up to 3072 where they are no whole multiple of 256 and some XCDs have a workgroup more (29 x 2064 x 8192 4.82 -> 5.35;
-// 28 x 2048 x 8192 0.98); many rows, where B's second reader comes too late, the fewer the longer K (238 x 6095 x 32768 60 -> 74, B in the caches 233 x
-// 7945 x 32768 63 -> 94; 33 to 64 rows above 32768 1.03 in the mean with B in the caches, 0.99 from HBM); blocks of 48 columns in one round on a K
-// of 32768 (60 sizes, 1.02).  (A form of the kernels of its own: the few instructions before the first load are 0.8 % of 37 x 11008 x 4096.)
+// (592 columns 3.5 % slower); many rows, where B's second reader comes too late, the fewer the longer K (233 x 7945 x 32768 75 -> 92, with B in the caches
+// 64 -> 96; 216 x 2117 x 24576 23.2 -> 25.9; 33 to 64 rows on many columns above 32768 1.04 in the mean with B in the caches, 0.99 from HBM); blocks of 48 columns in one
+// round on a K of 32768 (50 x 12039 39.2 -> 40.9).  (A form of the kernels of its own: the few instructions before the first load are 0.8 % of 37 x 11008 x 4096.)
 constexpr bool goes_round(const int m, const int n, const int k)
 {
-    if (k % 8192 != 0 || n < 2048 || m > (k <= 8192 ? 256 : k <= 16384 ? 160 : k <= 32768 ? 64 : 32)) return false;
-    if (n % 256 != 0 && n < (m <= 16 ? 2560 : m <= 32 && k == 16384 ? 4096 : 3072)) return false;
-    return !(k == 32768 && m > 16 && n > 8192 && n <= 12288);
+    const int rows = k <= 8192 ? 256 : k <= 16384 ? 160 : k <= 32768 ? 96 : n <= 4096 ? 64 : 32;
+    return k % 8192 == 0 && n >= 2048 && m <= rows && !(k == 32768 && m > 16 && n > 8192 && n <= 12288);
 }
 __device__ __forceinline__ int first_of_runs(const int cnt, const int waves)
 {

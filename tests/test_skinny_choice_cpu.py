@@ -25,11 +25,12 @@ def test_kernel_by_size(m, n, k, int32, scaled):
 def test_sizes_whose_workgroups_go_round(tmp_path):
     """Sizes of the same kernels that were measured with workgroups that begin at different places of K over all at the same, B from HBM and in the caches."""
     sizes = {
-        # 0.88, 0.99; 0.97, 1.02; 0.90, 0.99; 0.87, 0.91; 0.91, 0.96; 0.97, 0.96; 0.94, 0.91 ...
-        True: [(2, 4096, 8192), (1, 2048, 8192), (2, 3584, 8192), (1, 2304, 32768), (16, 4096, 8192), (32, 2048, 8192), (56, 4096, 32768), (8, 2560, 57344), (256, 4096, 8192), (160, 4096, 16384)],
-        # 1.19, 1.32; 1.24, 1.30; 1.17, 1.18; 1.11, 1.00; 1.09, 1.00; 1.05, 1.05; 1.08, 1.04; 0.99, 1.06 and more; rows that are no whole 4096 bytes
-        False: [(220, 8374, 32768), (201, 9667, 32768), (210, 2103, 24576), (29, 2064, 8192), (27, 2307, 16384), (26, 10223, 32768), (50, 12039, 32768), (48, 8192, 49152), (48, 4096, 57344),
-                (257, 4096, 8192), (161, 4096, 16384), (16, 4096, 12288), (16, 4096, 11008)]}
+        # 0.88, 0.99; 0.97, 1.02; 0.90, 0.99; 0.85, 0.92; 0.91, 0.97; 0.97, 0.96; 0.99, 1.00; 0.91, 0.71; 0.97, 0.91; 0.99, 0.99; many sizes: 0.96, 0.97; 0.96, 0.99
+        True: [(2, 4096, 8192), (1, 2048, 8192), (2, 3584, 8192), (1, 2304, 32768), (16, 4096, 8192), (32, 2048, 8192), (24, 2304, 8192), (56, 4096, 32768), (80, 3072, 32768), (160, 4096, 16384),
+               (256, 4096, 8192), (8, 2560, 57344), (64, 3584, 57344)],
+        # 1.24, 1.49; 1.15, 1.35; 1.12, 1.21; 1.13, 1.13; 1.04, 1.05; 1.04, 1.06; 1.01, 1.08; many sizes: 0.99, 1.09; 1.00, 1.00; rows that are no whole 4096 bytes
+        False: [(233, 7945, 32768), (201, 9667, 32768), (216, 2117, 24576), (149, 3260, 24576), (46, 9903, 32768), (50, 12039, 32768), (47, 9203, 49152), (48, 4097, 57344), (257, 4096, 8192),
+                (161, 8200, 16384), (16, 4096, 12288), (16, 4096, 11008)]}
     source = tmp_path / "round.hip"
     source.write_text('#include "qm_common.hpp"\n' + "".join(f"static_assert({'' if yes else '!'}qm::goes_round({m}, {n}, {k}));\n" for yes, of in sizes.items() for m, n, k in of))
     r = subprocess.run([build.HIPCC, *build.HIP_FLAGS, "--cuda-host-only", "-fsyntax-only", str(source)], capture_output=True, text=True, timeout=120)
