@@ -388,7 +388,7 @@ __device__ __forceinline__ uint32_t quant8(const Chunk8<IN> &c, float inv)
 // last bits then count n + 8; the bits of eight such sums are added up sixteen-fold, and what the constant leaves in them is taken
 // away.  With the maximum on bit patterns (chunks_amax) 4.1 vector instructions per element where one
 // element after the other takes 8: in a graph, us, before -> now, 2048 x 4096 5.76 -> 5.46, 2048 x 8192 8.94 -> 8.56, 8192 x 1024 5.77 ->
-// 5.41.  bf16, which needs an instruction more to widen and had one less, was no faster (2048 x 8192 8.66 / 8.67).
+// 5.41 (few rows and short ones lose: quantise_many).  bf16, which needs an instruction more to widen and had one less, was no faster (2048 x 8192 8.66 / 8.67).
 __device__ __forceinline__ uint32_t quant8_plain(const Chunk8<QM_IN_F16> &c, const float inv)
 {
     constexpr float round_to = 12582912.0f + 8.0f;
@@ -461,7 +461,8 @@ __device__ __forceinline__ float row_max(float x, float *lds)
 
 // NW waves per row (4 rows per workgroup if one), NC chunks of 8 elements per lane: k <= 512 * NW * NC.
 // NC == 0: any k, the row read twice (the second time out of the L2).
-template <int IN, int NW, int NC>
+// MANY: fp16 by quant8_plain, which has fewer instructions and a longer chain of them (see quantise_many).
+template <int IN, int NW, int NC, bool MANY>
 __global__ void __launch_bounds__(NW == 1 ? 256 : 64 * NW) quantize_pack_kernel(const uint8_t *__restrict__ x, uint8_t *__restrict__ dst, float *__restrict__ scales, int rows, int k)
 {
     __shared__ float red[NW];
@@ -477,18 +478,34 @@ __global__ void __launch_bounds__(NW == 1 ? 256 : 64 * NW) quantize_pack_kernel(
         Chunk8<IN> v[NC];
 #pragma unroll
         for (int i = 0; i < NC; ++i) v[i].load(xr + first(lane + i * 64 * NW) * QuantIn<IN>::BYTES);
-        bool plain;
-        amax = row_max<NW>(chunks_amax(v, plain), red);
+        bool plain = false;
+        if constexpr (MANY) {
+            amax = chunks_amax(v, plain);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NC; ++i) amax = v[i].amax(amax);
+        }
+        amax = row_max<NW>(amax, red);
         const float inv = amax > 0.0f ? 7.0f / amax : 0.0f;
         if (lane == 0) scales[row] = amax / 7.0f;
-        quantise_chunks<IN>(plain, amax, inv, [&](auto quant) __attribute__((always_inline)) {
+        if constexpr (MANY) {
+            quantise_chunks<IN>(plain, amax, inv, [&](auto quant) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < NC; ++i) {
+                    const int c = lane + i * 64 * NW;
+                    const uint32_t q = quant(v[i]);
+                    if (c < nchunks) *reinterpret_cast<u32_any_aligned *>(out + (first(c) >> 1)) = q;
+                }
+            });
+        } else {
+            // (not through the same function: bf16 and fp32 lost 1 to 2 % on three and four chunks to the order that the compiler gave the loads)
 #pragma unroll
             for (int i = 0; i < NC; ++i) {
                 const int c = lane + i * 64 * NW;
-                const uint32_t q = quant(v[i]);
+                const uint32_t q = quant8(v[i], inv);
                 if (c < nchunks) *reinterpret_cast<u32_any_aligned *>(out + (first(c) >> 1)) = q;
             }
-        });
+        }
     } else {
         Chunk8<IN> v;
         for (int c = lane; c < nchunks; c += 64 * NW) {
@@ -530,14 +547,20 @@ __global__ void __launch_bounds__(256) quantize_pack_scalar_kernel(const uint8_t
     }
 }
 
+// Where the arithmetic of fp16 rows, and not the launch and the way there and back, is what they take.  quant8_plain over quant8, in a graph, over
+// 7000 sizes: to a K of 2048 1.03 on 16 to 512 rows, 1.01 on 513 to 1024, 0.95 beyond; to 4096 1.01, 0.99 from 257 rows on, 0.92 from 1025 on; above 1.00 to
+// 0.94 on few rows, 0.96 to 0.87 on more.
+inline bool quantise_many(int rows, int k) { return k > 4096 || rows > (k > 2048 ? 256 : 1024); }
+
 template <int IN, int NW, int NC>
 static hipError_t launch_quantize_rows(const uint8_t *x, uint8_t *dst, float *scales, int rows, int k, hipStream_t s)
 {
+    const auto kernel = IN == QM_IN_F16 && NC > 0 && quantise_many(rows, k) ? &quantize_pack_kernel<IN, NW, NC, IN == QM_IN_F16 && NC != 0> : &quantize_pack_kernel<IN, NW, NC, false>;
     constexpr int threads = NW == 1 ? 256 : 64 * NW, rows_per_block = NW == 1 ? 4 : 1;
     constexpr int most = (1 << 21) * rows_per_block;  // a grid has less than 2^32 threads
     for (int r0 = 0; r0 < rows; r0 += most) {
         const int n = rows - r0 < most ? rows - r0 : most;
-        const hipError_t e = enqueue(&quantize_pack_kernel<IN, NW, NC>, dim3((unsigned)(n + rows_per_block - 1) / rows_per_block), dim3(threads), 0, s,
+        const hipError_t e = enqueue(kernel, dim3((unsigned)(n + rows_per_block - 1) / rows_per_block), dim3(threads), 0, s,
             x + (size_t)r0 * k * QuantIn<IN>::BYTES, dst + (size_t)r0 * (k / 2), scales + r0, n, k);
         if (e != hipSuccess || r0 > 0x7fffffff - most) return e;
     }

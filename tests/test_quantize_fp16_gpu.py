@@ -21,3 +21,12 @@ def test_every_fp16_value_is_quantised_as_the_same_value_in_fp32_is():
             q16, s16 = quadmul.quantize_pack(rows)
             q32, s32 = quadmul.quantize_pack(rows.float())   # (the same values, by the other arithmetic)
             assert torch.equal(q16, q32) and torch.equal(s16.view(torch.int32), s32.view(torch.int32)), top
+
+
+@pytest.mark.parametrize("rows,k", [(1024, 2048), (1025, 2048), (1025, 510), (256, 4096), (257, 4096), (1025, 2050), (1, 4098), (3, 16384), (2, 16386)], ids=str)
+def test_both_sides_of_the_choice_between_the_arithmetics(rows, k):
+    x = torch.randn(rows, k, device=DEV, generator=torch.Generator(device=DEV).manual_seed(rows + k)).half()
+    x[0, 1], x[rows // 2, k - 1], x[rows - 1, 0] = float("inf"), float("nan"), -0.0
+    q16, s16 = quadmul.quantize_pack(x)
+    q32, s32 = quadmul.quantize_pack(x.float())
+    assert torch.equal(q16, q32) and torch.equal(s16.view(torch.int32), s32.view(torch.int32))
