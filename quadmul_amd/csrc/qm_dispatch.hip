@@ -331,7 +331,9 @@ static hipError_t launch_fp6(const GemmArgs &p, Fp6Route route, void *ws, hipStr
     const Fp6Operand a = fp6_operand(p.M, p.K, ws);
     const Fp6Layout &l = a.layout;
     const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, l.kt, l.groups, l.parts};
-    const hipError_t e = enqueue(&expand_a6_kernel<false>, dim3(l.groups * (32 / CODE_ROWS) * l.parts), dim3(EXPAND6_THREADS), 0, s, q);
+    const int rows = expand_rows(p.M, p.K);
+    const auto kernel = rows == 16 ? &expand_a6_kernel<false, false, 16> : &expand_a6_kernel<false, false, 8>;
+    const hipError_t e = enqueue(kernel, dim3(l.groups * (32 / rows) * l.parts), dim3(EXPAND6_THREADS), 0, s, q);
     return e == hipSuccess ? launch_tile6(p, a, route, s) : e;
 }
 
@@ -344,8 +346,10 @@ static hipError_t launch_fp6_padded(GemmArgs p, const PadPlan &pl, Fp6Route rout
     const Fp6Layout &l = a.layout;
     const Expand6Args q{p.A, a.codes, a.sums, p.M, p.K, l.kt, l.groups, l.parts, p.B, reinterpret_cast<v4i *>(b_copy), p.N, pl.kp};
     const long long pieces = (long long)p.N * (pl.kp / 32);
-    const auto kernel = rows_on_dwords(p) ? &expand_a6_kernel<true, false> : &expand_a6_kernel<true, true>;
-    const hipError_t e = enqueue(kernel, dim3(l.groups * (32 / CODE_ROWS) * l.parts + (unsigned)((pieces + EXPAND6_THREADS - 1) / EXPAND6_THREADS)), dim3(EXPAND6_THREADS), 0, s, q);
+    const int rows = expand_rows(p.M, pl.kp);
+    const auto kernel = rows_on_dwords(p) ? (rows == 16 ? &expand_a6_kernel<true, false, 16> : &expand_a6_kernel<true, false, 8>)
+                                          : (rows == 16 ? &expand_a6_kernel<true, true, 16> : &expand_a6_kernel<true, true, 8>);
+    const hipError_t e = enqueue(kernel, dim3(l.groups * (32 / rows) * l.parts + (unsigned)((pieces + EXPAND6_THREADS - 1) / EXPAND6_THREADS)), dim3(EXPAND6_THREADS), 0, s, q);
     if (e != hipSuccess) return e;
     p.B = b_copy;
     p.K = pl.kp;

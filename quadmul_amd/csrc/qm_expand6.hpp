@@ -50,17 +50,23 @@ __device__ __forceinline__ v4i row_value(const RowPiece<SHIFT> &piece, const int
     return v;
 }
 
-// The eight rows of a workgroup: r0 .. r0 + 3 and r0 + 16 .. r0 + 19 of a group of 32, both halves of every 16 bytes of codes that they
-// share, 64 contiguous bytes of codes at a time.  (Workgroups of a group, which share 128-byte lines of codes, on one XCD: 8192 x 8192
-// 16.9 us, 2048 x 11008 6.5, against 14.8 and 6.0 with neighbours of any kind.)
+// The rows of a workgroup: half of them from r0 on and the other half 16 further in a group of 32, both halves of every 16 bytes of codes that they
+// share: of eight rows 64 contiguous bytes of codes at a time, of sixteen 128, whole lines.  (Eight: workgroups of a group, which share 128-byte lines of codes, on
+// one XCD: 8192 x 8192 16.9 us, 2048 x 11008 6.5, against 14.8 and 6.0 with neighbours of any kind.)
+// Eight fill the device where there is little to do; where the codes do not stay in the L2s with what else is there, half lines leave them twice: 11008 x
+// 8192 traced in front of its GEMM 23.6 us by sixteen neighbouring rows, 34.0 by eight, and the whole product on 4096 columns, us, 191.7, 198.1, 189.8 by sixteen
+// as here.  The whole product over 686 sizes, by eight / by sixteen over sixteen neighbouring ones: 0.961 / 0.971 below 4 million
+// elements of A, 0.978 / 0.983 to 32 million, 0.983 / 0.978 beyond.
 constexpr int CODE_ROWS = 8;
+inline int expand_rows(int m, int k) { return (long long)m * k >= 32000000 ? 16 : 8; }
+template <int ROWS>
 __device__ __forceinline__ void code_rows(const int block, int &group, int &r0)
 {
-    group = block >> 2;
-    r0 = (block & 3) * 4;
+    group = block / (32 / ROWS);
+    r0 = (block & (32 / ROWS - 1)) * (ROWS / 2);
 }
 
-// One workgroup re-codes CODE_ROWS rows over FP6_PART_STEPS K-steps, eight waves of two K-steps at a time: 128 bytes of every row,
+// One workgroup re-codes ROWS rows over FP6_PART_STEPS K-steps, eight waves of two K-steps at a time: 128 bytes of every row,
 // whole lines.  Two K-steps that a row does not fill are its last 128
 // bytes, as the GEMM loads them of B, with zeros where the steps before have been.
 // ANY: rows of any K and at any address, as if padded with zeros to Kp; the workgroups beyond A's
@@ -69,14 +75,15 @@ __device__ __forceinline__ void code_rows(const int block, int &group, int &r0)
 // neighbouring rows to a workgroup / now: 512 x 8192 3.9 / 3.2, 1536 x 4096 4.1 / 3.4, 4096 x 4096 5.8 / 5.7, 8192 x 8192 17.0 / 14.8 (5.7 TB/s).
 // SHIFT (rows of A off the multiples of four): with B's copy 1531 x 3307 x 4100 6.8 -> 5.0, the whole product 35.5 -> 33.0.
 constexpr int EXPAND6_THREADS = 512;
-template <bool ANY, bool SHIFT = false>
+template <bool ANY, bool SHIFT, int ROWS>
 __global__ void __launch_bounds__(EXPAND6_THREADS) expand_a6_kernel(const Expand6Args q)
 {
     constexpr int WAVES = EXPAND6_THREADS / 64, PAIRS = FP6_PART_STEPS / 2 / WAVES;  // (pairs of K-steps: per wave)
-    __shared__ int red[WAVES][CODE_ROWS];
+    constexpr int HALF = ROWS / 2, U = ROWS / 8;  // rows of a fragment, K-steps of a pair that a lane has
+    __shared__ int red[WAVES][ROWS];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int Kb = q.K >> 1;
-    const unsigned blocks = (unsigned)q.groups * (32 / CODE_ROWS);
+    const unsigned blocks = (unsigned)q.groups * (32 / ROWS);
     const int part = blockIdx.x / blocks;
     if constexpr (ANY) {
         if (part >= q.parts) {
@@ -92,42 +99,49 @@ __global__ void __launch_bounds__(EXPAND6_THREADS) expand_a6_kernel(const Expand
         }
     }
     int group, r0;
-    code_rows(blockIdx.x - part * blocks, group, r0);
+    code_rows<ROWS>(blockIdx.x - part * blocks, group, r0);
     // lane: row, 16 bytes of a K-step, step of the two
-    const int h = (lane >> 2) & 1, r = r0 + (lane & 3), g = (lane >> 3) & 3, second = lane >> 5;
+    const int h = (lane / HALF) & 1, r = r0 + (lane & (HALF - 1)), g = (lane / ROWS) & 3;
+    const auto step_of = [&](int u) { return U == 2 ? u : lane >> 5; };
     const int row = group * 32 + h * 16 + r, row_bytes = ANY ? q.Kp >> 1 : Kb;
     const DwordSpan span = dword_span(q.A, (uint32_t)q.M * (uint32_t)Kb);
-    RowPiece<SHIFT> v[PAIRS];
+    RowPiece<SHIFT> v[PAIRS][U];
 #pragma unroll
-    for (int t = 0; t < PAIRS; ++t) {
-        const int at = min((part * FP6_PART_STEPS + 2 * (wave + WAVES * t)) * 64, row_bytes - 128) + 64 * second + 16 * g;
-        if constexpr (ANY) row_load<SHIFT>(v[t], span, min(row, q.M - 1), at, Kb);
-        else v[t] = *reinterpret_cast<const v4i *>(q.A + (size_t)min(row, q.M - 1) * Kb + at);
-    }
+    for (int t = 0; t < PAIRS; ++t)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int at = min((part * FP6_PART_STEPS + 2 * (wave + WAVES * t)) * 64, row_bytes - 128) + 64 * step_of(u) + 16 * g;
+            if constexpr (ANY) row_load<SHIFT>(v[t][u], span, min(row, q.M - 1), at, Kb);
+            else v[t][u] = *reinterpret_cast<const v4i *>(q.A + (size_t)min(row, q.M - 1) * Kb + at);
+        }
     int sum = 0;
 #pragma unroll
     for (int t = 0; t < PAIRS; ++t) {
         const int step = part * FP6_PART_STEPS + 2 * (wave + WAVES * t);
         if (step >= q.kt) break;
-        const int at = min(step * 64, row_bytes - 128) + 64 * second + 16 * g;
-        v4i w;
-        if constexpr (ANY) w = row_value<SHIFT>(v[t], at, Kb);
-        else w = v[t];
-        if (row >= q.M || at < step * 64) w = v4i{0, 0, 0, 0};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_sdot8(w[e], 0x11111111, sum, false);
-        uint32_t f[6];
-        fp6_fragment(w, f);
-        uint8_t *const o = q.codes + ((size_t)group * q.kt + step + second) * FP6_GROUP_BYTES + (r + 16 * g) * 16;
-        *reinterpret_cast<v4i *>(o + h * 2048) = h == 0 ? v4i{(int)f[0], (int)f[1], (int)f[2], (int)f[3]} : v4i{(int)f[2], (int)f[3], (int)f[4], (int)f[5]};
-        *reinterpret_cast<v2i *>(o + 1024 + h * 8) = h == 0 ? v2i{(int)f[4], (int)f[5]} : v2i{(int)f[0], (int)f[1]};
+        for (int u = 0; u < U; ++u) {
+            const int at = min(step * 64, row_bytes - 128) + 64 * step_of(u) + 16 * g;
+            v4i w;
+            if constexpr (ANY) w = row_value<SHIFT>(v[t][u], at, Kb);
+            else w = v[t][u];
+            if (row >= q.M || at < step * 64) w = v4i{0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_sdot8(w[e], 0x11111111, sum, false);
+            uint32_t f[6];
+            fp6_fragment(w, f);
+            uint8_t *const o = q.codes + ((size_t)group * q.kt + step + step_of(u)) * FP6_GROUP_BYTES + (r + 16 * g) * 16;
+            const v4i four = h == 0 ? v4i{(int)f[0], (int)f[1], (int)f[2], (int)f[3]} : v4i{(int)f[2], (int)f[3], (int)f[4], (int)f[5]};
+            const v2i two = h == 0 ? v2i{(int)f[4], (int)f[5]} : v2i{(int)f[0], (int)f[1]};
+            *reinterpret_cast<v4i *>(o + h * 2048) = four;
+            *reinterpret_cast<v2i *>(o + 1024 + h * 8) = two;
+        }
     }
-    sum += __shfl_xor(sum, 8);
-    sum += __shfl_xor(sum, 16);
-    sum += __shfl_xor(sum, 32);
-    if (lane < CODE_ROWS) red[wave][lane] = sum;
+#pragma unroll
+    for (int apart = ROWS; apart < 64; apart <<= 1) sum += __shfl_xor(sum, apart);
+    if (lane < ROWS) red[wave][lane] = sum;
     __syncthreads();
-    if (threadIdx.x < CODE_ROWS) {
+    if (threadIdx.x < ROWS) {
         int total = 0;
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) total += red[w][threadIdx.x];
@@ -165,7 +179,7 @@ __global__ void __launch_bounds__(QUANT6_THREADS, 2) quantize_a6_kernel(const Qu
     extern __shared__ __align__(16) uint8_t nibbles[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int group, r0;
-    code_rows(blockIdx.x, group, r0);
+    code_rows<CODE_ROWS>(blockIdx.x, group, r0);
     const int row = group * 32 + r0 + (wave & 3) + (wave >> 2) * 16, Kb = q.K >> 1, pitch = Kb + 16, nchunks = q.K >> 3;
     const uint8_t *src = q.x + (size_t)min(row, q.M - 1) * q.K * QuantIn<IN>::BYTES;
     Chunk8<IN> v[NC];
