@@ -194,7 +194,8 @@ static RaggedBlock ragged_block(int m, int n)
 // 512 rows only small products are left here (809 x 708 x 1096 5.2 / 8.6, 939 x 1094 x 1596 17.7 / 12.7), to 1500 rows off the multiples of four, where the
 // rule was measured.  What the loads as they were before, at 1.94 and 0.35 clocks, left to the copies has to be a twentieth below them, an eighth where
 // the fits are furthest off: few blocks on a long K, whose GEMM on the copies is one short round (93 x 799 x 6400 at an odd address 10.3 / 7.9), and several rounds of a few
-// chunks (76 x 16590 x 448 11.2 / 9.7).  Of the 21587, time against that choice of before: 0.782 in the mean where it is another, 29 of those more than 2 % slower (4 more than 10).
+// chunks (76 x 16590 x 448 11.2 / 9.7).  On 5578 others, time against that choice of before: 0.778 in the mean where it is another, 10 of those more than 2 % slower (2 more than 10: 127 x
+// 40507 x 5898 79.0 -> 94.7).
 static bool ragged_before_copies(int m, int n, int k, int ptr_align)
 {
     if (m <= 2) return true;
@@ -278,7 +279,8 @@ static bool fp6_fits(int m, int n, int k, int ptr_align)
     return n >= 256 && n < (1 << 21) && fp6_layout(m, k).code_bytes <= QM_FP6_MAX_BYTES;
 }
 
-// What the GEMM takes (us), in the terms of modelled_us: fitted to 272 products of 200 to 8192 rows (rms of the fits 7.5 and 6.3 %).  Per K-step
+// What the GEMM takes (us), in the terms of modelled_us: fitted to 272 products of 200 to 8192 rows (rms of the fits 7.5 and 6.3 %), before A's codes
+// were read in whole 16-byte pieces, which is 1.5 to 4 % less; the terms of fp6_route for the codes are from before that too (up to 2 us less now).  Per K-step
 // and round 0.82 us on tiles of 256 x 256 (int8: 1.19) and 0.53 on 256 x 128 (0.72), per round 13.8 and 5.8.
 static double fp6_tile_us(int m, int n, int k, bool narrow)
 {

@@ -72,8 +72,8 @@ __device__ __forceinline__ void code_rows(const int block, int &group, int &r0)
 // ANY: rows of any K and at any address, as if padded with zeros to Kp; the workgroups beyond A's
 // copy B with its rows padded, one 16-byte piece per thread, in the same launch.
 // Bound: HBM on large operands, the launch and one round trip on small ones.  us in a graph, by sixteen
-// neighbouring rows to a workgroup / now: 512 x 8192 3.9 / 3.2, 1536 x 4096 4.1 / 3.4, 4096 x 4096 5.8 / 5.7, 8192 x 8192 17.0 / 14.8 (5.7 TB/s).
-// SHIFT (rows of A off the multiples of four): with B's copy 1531 x 3307 x 4100 6.8 -> 5.0, the whole product 35.5 -> 33.0.
+// neighbouring rows to a workgroup / by eight as here: 512 x 8192 3.9 / 3.2, 1536 x 4096 4.1 / 3.4, 4096 x 4096 5.8 / 5.7, 8192 x 8192 17.0 / 14.8 (5.7 TB/s).
+// SHIFT (rows of A off the multiples of four): with B's copy 1531 x 3307 x 4100 6.8 -> 5.0, the whole product 35.6 -> 32.7 with A's new split.
 constexpr int EXPAND6_THREADS = 512;
 template <bool ANY, bool SHIFT, int ROWS>
 __global__ void __launch_bounds__(EXPAND6_THREADS) expand_a6_kernel(const Expand6Args q)

@@ -17,12 +17,13 @@
 //     without a sign.  The 8 that every b has too much is 8 * (sum of the row of A) in C, taken out
 //     where an item's accumulators get their start value.
 //
-// What bounds it: power, as with the int8 tile (qm_tile16.hpp), whose schedule -- slots of one matrix
+// What bounds it: no unit is full, the LDS nearest to it.  The schedule is the int8 tile's (qm_tile16.hpp) -- slots of one matrix
 // instruction each, the loads running ahead through item boundaries, the write-out inside an item's last
-// K-step -- it follows.  8192 x 8192 x 8192 runs at 1.80 GHz (int8: 2.15) in 459 thousand cycles, 390 of them
-// a loop of its matrix instructions alone; without its loads into the LDS the clock rises to 2.13 GHz and
+// K-step.  8192 x 8192 x 8192 runs at 1.8 to 1.9 GHz (int8: 2.15) in 469 thousand cycles: 264 of its matrix instructions, 16 each; fragments of
+// 34.7 MB per CU read out of the LDS, 271 at 128 bytes a cycle, and 10.5 MB loaded into it, 82; no bank conflicts; a wave issues for a third of its time and waits to issue
+// for 39 % (counters of the traced kernel).  Without its loads into the LDS the clock rises to 2.13 GHz and
 // the cycles stay (taken before A was read as it is now, see read_a).  us, this kernel / int8: 8192 x 8192 x 8192 262 / 336,
-// 2048 x 11008 x 4096 60 / 77, 4096 x 4096 x 4096 39.3 / 48.5; the kernel that re-codes A takes 14.8, 3.7 and 5.7 in a graph of its own.
+// 2048 x 11008 x 4096 60 / 77, 4096 x 4096 x 4096 39.3 / 48.5; the kernel that re-codes A takes 22.6, 7.9 and 7.2 traced in front of it.
 //
 // Eight waves, two per SIMD: a wave by itself issues a vector instruction every eight cycles (two every four),
 // and the 56 re-coding instructions per wave and K-step then take longer than the matrix ones (four waves
