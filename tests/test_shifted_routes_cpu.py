@@ -13,6 +13,8 @@ import quadmul_amd as qm
     # ... and on a B of 40 MB and more
     (7, 44701, 3582, False), (26, 25086, 4630, False), (36, 49813, 9482, False), (59, 22887, 7090, False),                               # 0.59, 0.71, 0.72, 0.90
     (117, 28679, 4998, True), (152, 16876, 6878, True),                                                                                  # 1.25, 1.29
-    (1501, 660, 1210, True), (470, 33870, 2452, True), (225, 13824, 6110, True)], ids=str)                                     # (not measured), 1.97, 1.52
+    (470, 33870, 2452, True), (225, 13824, 6110, True),                                                                                 # 1.97, 1.52
+    # the last rows that the rule was fitted on, and one more, which would gain as much (B in the caches)
+    (1500, 552, 1126, False), (1501, 552, 1126, True)], ids=str)                                                                        # 0.74, 0.73
 def test_rows_off_the_multiples_of_four(m, n, k, copied):
     assert (qm.workspace_bytes(m, n, k) > 0) == copied
