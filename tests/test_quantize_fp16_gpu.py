@@ -10,10 +10,11 @@ DEV = "cuda:0"
 
 
 # every fp16 pattern as an element of rows with a maximum above it, the shorter arithmetic, and of rows with infinities and NaN, the longer
-def test_every_fp16_value_is_quantised_as_the_same_value_in_fp32_is():
-    k = 2048
+# (k: rows that take the shorter arithmetic only, and rows too short for it)
+@pytest.mark.parametrize("k", [8192, 2048])
+def test_every_fp16_value_is_quantised_as_the_same_value_in_fp32_is(k):
     for top in (1.0, 7.0, 65504.0, 6.1e-5):
-        x = torch.arange(65536, dtype=torch.int32, device=DEV).to(torch.int16).view(torch.float16).view(32, k).clone()
+        x = torch.arange(65536, dtype=torch.int32, device=DEV).to(torch.int16).view(torch.float16).view(-1, k).clone()
         special = ~(x.float().abs() <= top)
         finite = torch.where(special, torch.zeros_like(x), x)
         finite[:, 0] = top
