@@ -55,15 +55,17 @@ class W4A4Linear(torch.nn.Module):
         return cls(wq, ws, bias, out_dtype)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if x.shape[-1] != self.in_features:
-            raise QuadmulError(f"W4A4Linear: last dimension of x must be {self.in_features}")
-        flat = x.dim() == 2 and self.in_features > 0
-        x2 = x if flat else x.reshape(-1, self.in_features)
+        in_features = self.in_features
+        if x.shape[-1] != in_features:
+            raise QuadmulError(f"W4A4Linear: last dimension of x must be {in_features}")
+        flat = x.dim() == 2 and in_features > 0
+        x2 = x if flat else x.reshape(-1, in_features)
         if not x2.is_contiguous():
             x2 = x2.contiguous()
         if x2.shape[0]:
             out_dtype = self.out_dtype
-            if out_dtype not in (torch.float16, torch.bfloat16):
+            bf16 = out_dtype is torch.bfloat16
+            if not bf16 and out_dtype is not torch.float16:
                 raise QuadmulError("W4A4Linear: out_dtype must be float16 or bfloat16")
             # (out of the dictionary: an attribute that is a buffer is found after everything else has been looked through, 0.28 us each of the
             # 6.2 of a small call.  Only where nothing would be found ahead of it -- not in a subclass, nor with an attribute of that
@@ -81,7 +83,7 @@ class W4A4Linear(torch.nn.Module):
             # (2048 x 11008: 21 us beside a GEMM of 73).  A bias that the kernel cannot take as
             # it is -- moved or cast after construction -- or that autograd follows is added apart.
             fused = bias is not None and _fusable(bias, x2, out_dtype, self.out_features)
-            y = _native("linear", x2, weight, self.out_features, weight_scale, bias if fused else None, out_dtype == torch.bfloat16)
+            y = _native("linear", x2, weight, self.out_features, weight_scale, bias if fused else None, bf16)
             if y is None:
                 y = torch.empty((x2.shape[0], self.out_features), dtype=out_dtype, device=x.device)
                 xq, xs = quantize_pack(x2)
